@@ -38,6 +38,8 @@ struct LaunchClass {
   int half_max = 64;  // largest pack half (the block of an unsplit launch)
   size_t lds = 0;    // dynamic LDS bytes
   KParams lay{};     // LDS offsets and exchange-buffer fields
+  size_t lds_flat = 0;  // the same with the receptor as units of the flat
+  KParams lay_flat{};   // pair loop (0: none)
 };
 
 struct HostComplex {
@@ -46,7 +48,9 @@ struct HostComplex {
   int lpr = 0, apl = 0, n_chunks = 0;
   bool tiled = false;  // receptor streamed through LDS tiles
   bool ref_built = false;
+  int flat_n = 0;      // units of the flat pair loop (0: no list)
   bool shape_final = false;  // lane shape fixed (the complex's energies have bits)
+  std::vector<int4> chunks;  // receptor chunks (host copy)
   std::vector<int> lig_t;  // ligand atom types (host copy)
   std::vector<int> lig_ns;  // receptor split of each ligand conformer's MC packs
   DevComplex dev{};
@@ -413,6 +417,7 @@ gd_status gd_add_complex(gd_ctx *ctx, const gd_complex_desc *d, int *complex_id)
     i = j;
   }
   h.n_chunks = (int)chunks.size();
+  h.chunks = chunks;
 
   // type-pair parameter records [receptor type][ligand type]
   const gd_enepara &ep = *d->enepara;
@@ -674,9 +679,82 @@ gd_status widen_shapes(gd_ctx *ctx) {
   return GD_OK;
 }
 
+// Unit list of the flat pair loop (gd_mc.h) for lane groups of a split of 8:
+// group g's share of every chunk, in chunk order, cut into units of one
+// receptor type, an even number for each type. `apl` sets the groups of NP
+// points that chunk_pairs forms (4, 2 and 1 for 1, 2 and more atoms per lane),
+// which the units' modes keep.
+std::vector<int4> build_flat_units(const std::vector<int4> &chunks, int apl, int (&off)[9]) {
+  std::vector<int4> U;
+  const int np = apl >= 3 ? 1 : (apl == 2 ? 2 : 4);
+  for (int g = 0; g < 8; ++g) {
+    off[g] = (int)U.size();
+    std::vector<int> first, types;  // each type's first unit
+    int lone = -1;                  // a unit of one point that may take a second
+    auto even = [&] {
+      if (!first.empty() && ((int)U.size() - first.back()) % 2 != 0)
+        U.push_back(make_int4(FLAT_EMPTY, U.back().y, 0, 0));
+    };
+    for (const int4 &ch : chunks) {
+      const int fb = ch.x + (ch.y * g) / 8, fe = ch.x + (ch.y * (g + 1)) / 8;
+      if (fb >= fe) continue;
+      if (types.empty() || types.back() != ch.z) {
+        even();
+        first.push_back((int)U.size());
+        types.push_back(ch.z);
+        lone = -1;
+      }
+      const int hpc = ch.w >= KIND_HPC ? FLAT_HPC : 0;
+      auto emit = [&](int p0, int p1, int flags) {
+        U.push_back(make_int4(flags | hpc, p0 | (p1 << 16), 0, 0));
+      };
+      int p = fb;
+      for (; np == 4 && p + 4 <= fe; p += 4) {
+        emit(p, p + 1, FLAT_FIRST);
+        emit(p + 2, p + 3, FLAT_SECOND | (p + 4 == fe ? FLAT_END1 : 0));
+        lone = -1;
+      }
+      for (; np == 2 && p + 2 <= fe; p += 2) {
+        emit(p, p + 1, FLAT_BLOCK | (p + 2 == fe ? FLAT_END1 : 0));
+        lone = -1;
+      }
+      for (; p < fe; ++p) {
+        const bool last = p + 1 == fe;
+        if (lone >= 0) {
+          int4 &u = U[lone];
+          u.x = (u.x & ~FLAT_ONE) | (last ? FLAT_END1 : 0) | hpc;
+          u.y = (u.y & 0xffff) | (p << 16);
+          lone = -1;
+        } else {
+          emit(p, p, FLAT_SINGLES | FLAT_ONE | (last ? FLAT_END0 : 0));
+          lone = (int)U.size() - 1;
+        }
+      }
+    }
+    even();
+    for (size_t i = 0; i < first.size(); ++i) {
+      const int end = i + 1 < first.size() ? first[i + 1] : (int)U.size();
+      U[first[i]].x |= types[i] | (((end - first[i]) / 2) << FLAT_PAIRS);
+    }
+  }
+  off[8] = (int)U.size();
+  return U;
+}
+
 gd_status sync_complexes(gd_ctx *ctx) {
   if (!ctx->cx_dirty) return GD_OK;
   TRY(widen_shapes(ctx));
+  // spread packing splits every receptor eight ways: its complexes get unit
+  // lists (points and PSP columns are 16-bit there, a type has at most
+  // FLAT_PAIR_MASK unit pairs in a group; receptors in LDS are far below that)
+  if (spread_packing(ctx))
+    for (HostComplex &h : ctx->cx) {
+      if (h.tiled || h.flat_n > 0 || h.d.pnp > 4096 * 4 || h.d.n_res > 0x7fff) continue;
+      const std::vector<int4> U = build_flat_units(h.chunks, h.apl, h.dev.flat_off);
+      TRY(dev_upload(ctx, h, (int4 **)&h.dev.flat, U.data(), U.size()));
+      HIPCHK(hipStreamSynchronize(ctx->stream));
+      h.flat_n = (int)U.size();
+    }
   if (ctx->d_cx) HIPCHK(hipFree(ctx->d_cx));
   ctx->d_cx = nullptr;
   for (auto &g : ctx->gslot) g.valid = false;  // captured launches hold the old pointer
@@ -730,9 +808,10 @@ int complex_tile(const gd_ctx *ctx, const HostComplex &h) {
 // `block` lanes; `split` adds the partial-sum exchange buffers of packs with
 // more than one lane group ([ns*half][4] HPC sums and [ns][half/8][12] replica
 // sums, ns*half = block). With tile > 0 the receptor arrays are two tiles of
-// `tile` points and KDE stays in HBM.
+// `tile` points and KDE stays in HBM; with flat_max > 0 the receptor is that many
+// units of the flat pair loop (and a pad, which its reads run into).
 void layout(KParams &P, size_t *bytes, int pnp_max, int pnk_max, int nch_max, int slots_max,
-            int block, bool split, int tile = 0) {
+            int block, bool split, int tile = 0, int flat_max = 0) {
   auto al = [](size_t v) { return (v + 15) & ~(size_t)15; };
   P.tile = tile;
   if (tile > 0) {
@@ -744,6 +823,7 @@ void layout(KParams &P, size_t *bytes, int pnp_max, int pnk_max, int nch_max, in
   o = al(o + (size_t)pnp_max * 4);
   P.off_psp = (int)o;
   o = al(o + (size_t)pnp_max * 4);
+  if (flat_max > 0) o = (size_t)(flat_max + 1) * FLAT_F4 * 16;
   P.off_par = (int)o;
   o = al(o + (size_t)PAR_FLOATS * 4);
   P.off_kde = (int)o;
@@ -846,8 +926,8 @@ void pack_finish(const gd_ctx *ctx, PackSet &ps) {
     lc.begin = (int)b;
     lc.block = block[o0];
     lc.tile = tile[o0];
-    int pnp_max = 0, pnk_max = 0, nch_max = 0, slots_max = 1, half_max = 64;
-    bool split = false;
+    int pnp_max = 0, pnk_max = 0, nch_max = 0, slots_max = 1, half_max = 64, flat_max = 0;
+    bool split = false, flat = lc.tile == 0;
     size_t e = b;
     for (; e < n_pk; ++e) {
       const int oe = order[e];
@@ -869,11 +949,18 @@ void pack_finish(const gd_ctx *ctx, PackSet &ps) {
       slots_max = ns;
       split = sp;
       half_max = std::max(half_max, p.half);
+      flat_max = std::max(flat_max, h.flat_n);
+      flat = flat && p.ns == 8 && h.flat_n > 0;
     }
     lc.end = (int)e;
     lc.half_max = half_max;
     layout(lc.lay, &lc.lds, (pnp_max + 3) & ~3, pnk_max, nch_max, slots_max, lc.block, split,
            lc.tile);
+    if (flat) {
+      layout(lc.lay_flat, &lc.lds_flat, 0, pnk_max, nch_max, slots_max, lc.block, split, 0,
+             flat_max);
+      if (lc.lds_flat > ctx->max_lds) lc.lds_flat = 0;
+    }
     ps.classes.push_back(lc);
     b = e;
   }
@@ -1147,12 +1234,12 @@ KParams base_params(gd_ctx *ctx) {
 // Kernel instance for atoms per lane `apl` and mode `da`: 0 plain,
 // 1 delayed acceptance with the network per atom, 2 with its tables, 3 and 4
 // the same with the split groups' shared surrogate sums compiled in.
-const void *mc_kernel_fn(int apl, int da, bool tiled) {
+const void *mc_kernel_fn(int apl, int da, int rec) {
   switch (apl) {
-    case 1: return mc_kernel_handle<1>(da, tiled);
-    case 2: return mc_kernel_handle<2>(da, tiled);
-    case 3: return mc_kernel_handle<3>(da, tiled);
-    default: return mc_kernel_handle<4>(da, tiled);
+    case 1: return mc_kernel_handle<1>(da, rec);
+    case 2: return mc_kernel_handle<2>(da, rec);
+    case 3: return mc_kernel_handle<3>(da, rec);
+    default: return mc_kernel_handle<4>(da, rec);
   }
 }
 
@@ -1187,10 +1274,13 @@ hipError_t plan_classes(gd_ctx *ctx, const std::vector<LaunchClass> &classes, co
     ClassLaunch cl;
     cl.P = P0;
     KParams &P = cl.P;
-    apply_layout(P, lc.lay);
+    // the flat pair loop where every pack is split eight ways and the units
+    // fit; the direct network evaluation keeps the layout its scratch fits in
+    const bool flat = lc.lds_flat > 0 && !da_scratch;
+    apply_layout(P, flat ? lc.lay_flat : lc.lay);
     P.pack_base = lc.begin;
     cl.block = lc.block;
-    cl.lds = lc.lds;
+    cl.lds = flat ? lc.lds_flat : lc.lds;
     if (da && da_scratch) {
       P.off_da = (int)((cl.lds + 15) & ~(size_t)15);
       cl.lds = P.off_da + (size_t)(cl.block / 64) * 6208;
@@ -1214,7 +1304,7 @@ hipError_t plan_classes(gd_ctx *ctx, const std::vector<LaunchClass> &classes, co
       P.queue = queue + i;
       P.n_queue = n_pk;
     }
-    cl.f = mc_kernel_fn(lc.apl, da, lc.tile > 0);
+    cl.f = mc_kernel_fn(lc.apl, da, lc.tile > 0 ? REC_TILED : flat ? REC_FLAT : REC_CHUNKS);
     out.push_back(cl);
   }
   // the dynamic LDS limit of every instance used is the device's: classes

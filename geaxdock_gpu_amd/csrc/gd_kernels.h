@@ -25,6 +25,21 @@ enum { P_P1A = 0, P_P2A, P_PMF0, P_PMF1, P_HA, P_HB, P_HC, P_NR2, P_A0, P_A1, P_
 // pocket-specific potential (class 2).
 enum { KIND_PLAIN = 0, KIND_HPC = 1, KIND_PSP = 2 };
 
+// Units of the flat pair loop (gd_mc.h). Flag word: on the first unit of a
+// receptor type, that type and the number of unit pairs; on every unit the flags
+// and the mode (top two bits).
+constexpr int FLAT_F4 = 3;          // float4 per unit in LDS
+constexpr int FLAT_TYPE = 0x1f;
+constexpr int FLAT_PAIRS = 10, FLAT_PAIR_MASK = 0xfff;
+constexpr int FLAT_ONE = 1 << 23;   // the first point only
+constexpr int FLAT_END0 = 1 << 24;  // first, second point: last of its chunk's share
+constexpr int FLAT_END1 = 1 << 25;
+constexpr int FLAT_HPC = 1 << 26;   // a point of kind HPC or PSP
+constexpr int FLAT_EMPTY = 1 << 27; // no point (makes a type's units even)
+constexpr int FLAT_MODE = (int)0xc0000000u;
+constexpr int FLAT_SINGLES = 0, FLAT_BLOCK = 0x40000000, FLAT_FIRST = (int)0x80000000u,
+              FLAT_SECOND = (int)0xc0000000u;
+
 // One complex on the device. Receptor points are stored sorted by
 // (type, kind) so each chunk has one parameter record per ligand atom.
 struct DevComplex {
@@ -43,6 +58,9 @@ struct DevComplex {
   const float *prt_hpp;    // [pnp] hpp where c0_and_d12_or_c2, else 0
   const int *prt_psp;      // [pnp] seq3r where class 2, else -1
   const int4 *chunks;      // [n_chunks] start, length, type, kind
+  // units of the flat pair loop by lane group of a split of 8 (null: none)
+  const int4 *flat;        // [flat_off[8]] flag word, first point | second << 16, 0, 0
+  int flat_off[9];
   const float *params;     // [NPT * NLT * NPAR]
   const float *lig_orig;   // [n_lig][3][lna]
   const int *lig_t;        // [lna]
@@ -131,13 +149,15 @@ struct KParams {
 
 // Host handle of the MC kernel instance for `APL` ligand atoms per lane,
 // mode `da` (0 plain, 1 delayed acceptance with the network per atom, 2 with
-// its tabulated outputs) and receptor tiling; defined in gd_mc_inst.hip, one
-// object per APL.
+// its tabulated outputs) and receptor layout; defined in gd_mc_inst.hip, one
+// object per APL. REC_FLAT has instances for modes 0, 2 and 4 (null for the
+// others).
+enum { REC_CHUNKS = 0, REC_TILED = 1, REC_FLAT = 2 };
 template <int APL>
-const void *mc_kernel_handle(int da, bool tiled);
-template <> const void *mc_kernel_handle<1>(int da, bool tiled);
-template <> const void *mc_kernel_handle<2>(int da, bool tiled);
-template <> const void *mc_kernel_handle<3>(int da, bool tiled);
-template <> const void *mc_kernel_handle<4>(int da, bool tiled);
+const void *mc_kernel_handle(int da, int rec);
+template <> const void *mc_kernel_handle<1>(int da, int rec);
+template <> const void *mc_kernel_handle<2>(int da, int rec);
+template <> const void *mc_kernel_handle<3>(int da, int rec);
+template <> const void *mc_kernel_handle<4>(int da, int rec);
 
 }  // namespace gd

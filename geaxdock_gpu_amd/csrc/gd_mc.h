@@ -31,6 +31,7 @@ struct Lds {
   const float4 *kde;  // LDS, or HBM for tiled receptors
   const int2 *kr;
   const int4 *ch;
+  const float4 *fl;  // units of the flat pair loop
   float *xe;
   int *xi;
   int *xa;
@@ -46,6 +47,13 @@ struct Lds {
   int *tp;
   int tile;
 };
+
+// Pointers read from device structures are generic; their loads would count
+// as LDS accesses too and stall the LDS pipeline. Data in HBM is read through
+// global pointers.
+typedef const __attribute__((address_space(1))) float *gfloat_p;
+typedef const __attribute__((address_space(1))) f32x4_t *gfloat4_p;
+__device__ __forceinline__ gfloat_p glob(const float *p) { return (gfloat_p)p; }
 
 // Receptor split of one workgroup: lanes [h*half, (h+1)*half) form group h
 // of ns (1, 2, 4 or 8, per pack); every group holds the same replicas and
@@ -329,40 +337,347 @@ __device__ __forceinline__ void chunk_pairs(const Lds &S, int beg, int end, cons
   for (int k = 0; k < APL; ++k) pmf[k] = fmaf(cp[k].pmf1, pmfc[k], pmf[k]);
 }
 
+// ---- flat pair loop ---------------------------------------------------------
+// Under a receptor split of 8 a group's share of a chunk is a few points (2 of
+// a 1,200-point receptor, 1 of a 670-point one), and the chunk loop above
+// spends its time between them: chunk header, parameter records, loop set-up
+// and one of twelve code variants, each waiting out its LDS reads. Here a
+// group's points are listed as units of at most two (build_flat_units), by
+// receptor type, each unit's points and attributes together in LDS in the
+// order they are used. A type's records are read once for all its chunks and the
+// units one ahead. One variant serves all kinds: terms a unit
+// cannot have are skipped by its flags, and what runs without need adds exact
+// zeros (hpp is 0 at plain points, the H-bond factor of pairs without a record
+// is 0).
+//
+// Sums keep the bits of the chunk loop. Every accumulator adds the points in
+// the same order, and the near electrostatic corrections, which chunk_pairs
+// adds after the main terms of each group of NP points, follow the unit's mode:
+// FLAT_SINGLES (each point's correction after its own term), FLAT_BLOCK (a
+// group of two: both terms, then both corrections), FLAT_FIRST and FLAT_SECOND
+// (the halves of a group of four: the first half's corrections wait for the
+// second's terms).
+//
+// Bound: VALU issue of the CUs that hold a pack (71 % of it on one complex of
+// 8 replicas, 77 % on a coarse receptor; the rest is the two waves' latencies).
+// Measured per MC step, chunk loop -> units, together with the paired groups
+// of run_pack and the prefetched MCS templates: one complex of 8 replicas
+// (1,200 points) 48.9 -> 35 us, a coarse receptor of 672 points with 4,408 KDE
+// points and 196 MCS templates (408 replicas) 72 -> 50 us; scoring 16,384
+// poses on 2,400 points 5.1 -> 3.9 ms.
+template <int APL>
+struct FlatAcc {
+  float vdw[APL], ele[APL], pmf[APL], psp[APL], hdb[APL], hpc[APL];
+  float pmfc[APL];          // the current chunk's PMF sum, without pmf1
+  // the last PSP value read and its lanes' contact masks: added when the next
+  // one is read (or at the end), so no read is waited for
+  float pps[APL];
+  int ppm[APL];
+  float pv[2][APL], pw[2];  // corrections of a FLAT_FIRST unit, with its ele parameters
+  bool pend;
+  int cnt[APL];
+};
+
+struct FlatUnit {
+  float4 P[2];  // x, y, z, ele
+  int4 a;       // flags, hpp / 2 of both points, PSP columns (16 bits each, -1: none)
+};
+
+template <int APL>
+__device__ __forceinline__ void flat_psp_add(FlatAcc<APL> &A) {
+#pragma unroll
+  for (int k = 0; k < APL; ++k)
+    A.psp[k] += __int_as_float(__float_as_int(A.pps[k]) & A.ppm[k]);
+}
+
+// Keeps a rare wave-uniform branch a branch: if-converted, its instructions
+// and selects would run for every unit.
+__device__ __forceinline__ void keep_branch() { asm volatile("" ::: "memory"); }
+
+template <int APL, int N>
+__device__ __forceinline__ void flat_unit(int ux, bool hb, bool wide, const FlatUnit &U, const PairConst &K,
+                                          float nr2max, const float (&x)[APL],
+                                          const float (&y)[APL], const float (&z)[APL],
+                                          const ChunkPar (&cp)[APL],
+                                          gfloat_p const (&psprow)[APL], FlatAcc<APL> &A) {
+  const float pa = -0.5f * LOG2E;
+  float d2[N][APL], rd[N][APL], dd[N][APL], num[N][APL], den[N][APL];
+  bool near = false;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    float qmin = 0.0f;
+#pragma unroll
+    for (int k = 0; k < APL; ++k) {
+      const float q2 = pair_d2(x[k], y[k], z[k], U.P[j].x, U.P[j].y, U.P[j].z);
+      const float r = fast_rsq(q2);
+      const float d = q2 * r;
+      d2[j][k] = q2;
+      rd[j][k] = r;
+      dd[j][k] = d;
+      qmin = k == 0 ? q2 : fminf(qmin, q2);
+      const float d3 = q2 * d;
+      const float d6 = d3 * d3;
+      num[j][k] = fmaf(-cp[k].p2a, d3, cp[k].p1a);
+      den[j][k] = fmaf(d6, d3, fmaf(cp[k].a1, q2, cp[k].a0));
+    }
+    near |= qmin <= nr2max;
+  }
+  const bool any_near = __ballot(near) != 0;
+  float wv[N][APL], pt[N][APL];
+#pragma unroll
+  for (int j = 0; j < N; ++j)
+#pragma unroll
+    for (int k = 0; k < APL; ++k)
+      wv[j][k] = fmaf(pa, d2[j][k], fmaf(cp[k].pb, dd[j][k], cp[k].pc));
+  if (wide) {
+    keep_branch();
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+      for (int k = 0; k < APL; ++k) wv[j][k] = fminf(wv[j][k], 64.0f);
+  }
+#pragma unroll
+  for (int j = 0; j < N; ++j)
+#pragma unroll
+    for (int k = 0; k < APL; ++k) {
+      const float e = fast_exp2(wv[j][k]);
+      const float r = fast_rcp(fmaf(den[j][k], e, den[j][k]));
+      A.vdw[k] = fmaf(fmaf(num[j][k], e, num[j][k]), r, A.vdw[k]);
+      pt[j][k] = r;
+    }
+  auto end_chunk = [&] {
+#pragma unroll
+    for (int k = 0; k < APL; ++k) {
+      A.pmf[k] = fmaf(cp[k].pmf1, A.pmfc[k], A.pmf[k]);
+      A.pmfc[k] = 0.0f;
+    }
+  };
+#pragma unroll
+  for (int k = 0; k < APL; ++k) A.pmfc[k] = fmaf(den[0][k], pt[0][k], A.pmfc[k]);
+  if (ux & FLAT_END0) {  // the first point is its chunk's last
+    keep_branch();
+    end_chunk();
+  }
+  if constexpr (N == 2) {
+#pragma unroll
+    for (int k = 0; k < APL; ++k) A.pmfc[k] = fmaf(den[1][k], pt[1][k], A.pmfc[k]);
+    if (ux & FLAT_END1) {
+      keep_branch();
+      end_chunk();
+    }
+  }
+  if (hb) {
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+      for (int k = 0; k < APL; ++k) {
+        const float h = fmaf(dd[j][k], cp[k].ha, cp[k].hb);
+        A.hdb[k] = fmaf(cp[k].hc, fast_exp2(-(h * h)), A.hdb[k]);
+      }
+  }
+  if (ux & FLAT_HPC) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const float hp = __int_as_float(j == 0 ? U.a.y : U.a.z);
+#pragma unroll
+      for (int k = 0; k < APL; ++k) {
+        const float u = __builtin_amdgcn_fmed3f(fmaf(d2[j][k], -INV81, 1.0f), 0.0f, 1.0f);
+        const float u3 = u * u * u;
+        A.hpc[k] = fmaf(hp, fmaf(u3, u, u3), A.hpc[k]);
+      }
+    }
+  }
+  const int mode = ux & FLAT_MODE;
+  if (!any_near) {
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+      for (int k = 0; k < APL; ++k) A.ele[k] = fmaf(U.P[j].w, rd[j][k], A.ele[k]);
+    if constexpr (APL == 1 && N == 2) {
+      if (mode == FLAT_SECOND && A.pend) {
+        keep_branch();
+        A.pend = false;
+        A.ele[0] = fmaf(A.pw[1], A.pv[1][0], fmaf(A.pw[0], A.pv[0][0], A.ele[0]));
+      }
+    }
+    return;
+  }
+  // contacts, the pocket-specific potential and the near electrostatic form
+  // (the correction is 0 where that form does not hold)
+  const int pscol = __builtin_amdgcn_readfirstlane(U.a.w);
+  float v[N][APL];
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const int ps = j == 0 ? (pscol << 16) >> 16 : pscol >> 16;
+    const bool has_psp = ps >= 0;
+    if (has_psp) flat_psp_add(A);
+#pragma unroll
+    for (int k = 0; k < APL; ++k) {
+      const float d = dd[j][k];
+      const bool c = d <= cp[k].pmf0;
+      A.cnt[k] += c ? 1 : 0;
+      const float s = K.el1 * d;
+      const float gn = fmaf(s * s, fmaf(K.b1, s, K.a1), K.el0);
+      v[j][k] = s < 1.0f ? fmaf(K.el1, gn, -rd[j][k]) : 0.0f;
+      if (has_psp) {
+        A.pps[k] = psprow[k][ps];
+        A.ppm[k] = c ? -1 : 0;
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < APL; ++k) A.ele[k] = fmaf(U.P[0].w, rd[0][k], A.ele[k]);
+  if (N == 1 || mode == FLAT_SINGLES) {
+#pragma unroll
+    for (int k = 0; k < APL; ++k) A.ele[k] = fmaf(U.P[0].w, v[0][k], A.ele[k]);
+  }
+  if constexpr (N == 2) {
+#pragma unroll
+    for (int k = 0; k < APL; ++k) A.ele[k] = fmaf(U.P[1].w, rd[1][k], A.ele[k]);
+    if constexpr (APL == 1) {
+      if (mode == FLAT_FIRST) {
+        A.pend = true;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          A.pv[j][0] = v[j][0];
+          A.pw[j] = U.P[j].w;
+        }
+        return;
+      }
+      if (mode == FLAT_SECOND && A.pend) {
+        keep_branch();
+        A.pend = false;
+        A.ele[0] = fmaf(A.pw[1], A.pv[1][0], fmaf(A.pw[0], A.pv[0][0], A.ele[0]));
+      }
+    }
+    if (mode != FLAT_SINGLES) {
+#pragma unroll
+      for (int k = 0; k < APL; ++k) A.ele[k] = fmaf(U.P[0].w, v[0][k], A.ele[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < APL; ++k) A.ele[k] = fmaf(U.P[1].w, v[1][k], A.ele[k]);
+  }
+}
+
+// All units of lane group h. A receptor type's units come in an even number
+// (the last may be empty), two register sets in turn.
+template <int APL>
+__device__ __forceinline__ void flat_pairs(const DevComplex &C, const Lds &S, int h,
+                                           const PairConst &K, const float (&x)[APL],
+                                           const float (&y)[APL], const float (&z)[APL],
+                                           const int (&lt)[APL], gfloat_p const (&psprow)[APL],
+                                           FlatAcc<APL> &A) {
+  const int u0 = __builtin_amdgcn_readfirstlane(C.flat_off[h]);
+  int left = __builtin_amdgcn_readfirstlane(C.flat_off[h + 1]) - u0;
+  if (left <= 0) return;
+  const float *rec[APL];
+#pragma unroll
+  for (int k = 0; k < APL; ++k) rec[k] = S.par + lt[k] * NPAR;
+  const float4 *U = S.fl + (size_t)u0 * FLAT_F4;
+  auto read_unit = [&](FlatUnit &V) {
+    V.P[0] = U[0];
+    V.P[1] = U[1];
+    const float4 a = U[2];
+    V.a = make_int4(__float_as_int(a.x), __float_as_int(a.y), __float_as_int(a.z),
+                    __float_as_int(a.w));
+    U += FLAT_F4;
+  };
+  FlatUnit Va, Vb;
+  read_unit(Va);
+  int ua = __builtin_amdgcn_readfirstlane(Va.a.x);
+  while (left > 0) {
+    ChunkPar cp[APL];
+    float nr2max = 0.0f;
+    bool hbond = false, wide_l = false;
+    const int type = ua & FLAT_TYPE;
+#pragma unroll
+    for (int k = 0; k < APL; ++k) {
+      const float4 *r = reinterpret_cast<const float4 *>(rec[k] + type * (NLT * NPAR));
+      const float4 a = r[0], b = r[1], c = r[2];
+      cp[k].p1a = a.x;
+      cp[k].p2a = a.y;
+      cp[k].pmf0 = a.z;
+      cp[k].pmf1 = a.w;
+      cp[k].ha = b.x;
+      cp[k].hb = b.y;
+      cp[k].hc = b.z;
+      cp[k].nr2 = b.w;
+      cp[k].a0 = c.x;
+      cp[k].a1 = c.y;
+      cp[k].pb = c.z;
+      cp[k].pc = c.w;
+      const float t = cp[k].pmf0 - 12.0f;
+      wide_l |= !(0.125f * LOG2E * t * t <= 60.0f);  // as in pose_energy's chunks
+      hbond |= cp[k].hc != 0.0f;
+      nr2max = k == 0 ? cp[k].nr2 : fmaxf(nr2max, cp[k].nr2);
+    }
+    const bool hb = __ballot(hbond) != 0, wide = __ballot(wide_l) != 0;
+    int pairs = (ua >> FLAT_PAIRS) & FLAT_PAIR_MASK;
+    left -= 2 * pairs;
+    for (; pairs > 0; --pairs) {
+      read_unit(Vb);
+      if (ua & FLAT_ONE) flat_unit<APL, 1>(ua, hb, wide, Va, K, nr2max, x, y, z, cp, psprow, A);
+      else flat_unit<APL, 2>(ua, hb, wide, Va, K, nr2max, x, y, z, cp, psprow, A);
+      const int ub = __builtin_amdgcn_readfirstlane(Vb.a.x);
+      read_unit(Va);  // past the group's end: the next group's first unit, or the pad
+      if (!(ub & FLAT_EMPTY)) {
+        if (ub & FLAT_ONE) flat_unit<APL, 1>(ub, hb, wide, Vb, K, nr2max, x, y, z, cp, psprow, A);
+        else flat_unit<APL, 2>(ub, hb, wide, Vb, K, nr2max, x, y, z, cp, psprow, A);
+      }
+      ua = __builtin_amdgcn_readfirstlane(Va.a.x);
+    }
+  }
+  flat_psp_add(A);
+}
+
 // Sum over MCS templates [m_begin, m_end) of tcc_m * sqrt(mean squared
 // distance of the template's atoms), src/kernel_cuda_l2_calcenergy.cu:274-313. Templates go
-// four at a time: their loads are issued together and their lane sums share
-// each butterfly step, so the per-template latencies overlap. Per template
-// the additions are the same as one template at a time.
+// four at a time: their loads are issued together, one round ahead of their
+// use (a round waited out three dependent reads from L2 before: 196 templates
+// of a coarse receptor took 37,000 cycles of a step's 124,000 per wave), and
+// their lane sums share each butterfly step. Per template the additions are
+// the same as one template at a time.
 template <int APL>
 __device__ __forceinline__ float mcs_sum(const DevComplex &C, int lpr, const float (&x)[APL],
                                          const float (&y)[APL], const float (&z)[APL],
                                          const int (&li)[APL], const bool (&val)[APL],
                                          int m_begin, int m_end) {
   float elhm = 0.0f;
-  const int pos = m_end;
-  for (int m0 = m_begin; m0 < pos; m0 += 4) {
-    float s[4];
+  if (m_begin >= m_end) return elhm;
+  const gfloat4_p mcs = (gfloat4_p)C.mcs;
+  const gfloat_p cnt = glob(C.mcs_cnt), tcc = glob(C.mcs_tcc);
+  const int lna = C.lna;
+  f32x4_t M[4][APL];
+  float n[4], t[4];
+  auto read = [&](int m0) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int m = min(m0 + q, m_end - 1);
+#pragma unroll
+      for (int k = 0; k < APL; ++k) M[q][k] = mcs[(size_t)m * lna + li[k]];
+      n[q] = cnt[m];
+      t[q] = tcc[m];
+    }
+  };
+  read(m_begin);
+  for (int m0 = m_begin; m0 < m_end; m0 += 4) {
+    float s[4], nc[4], tc[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       s[q] = 0.0f;
-      const int m = m0 + q;
-      if (m >= pos) continue;
+      nc[q] = n[q];
+      tc[q] = t[q];
 #pragma unroll
       for (int k = 0; k < APL; ++k) {
         if (!val[k]) continue;
-        const float4 M = C.mcs[(size_t)m * C.lna + li[k]];
-        if (M.w != 0.0f) s[q] += pair_d2(x[k], y[k], z[k], M.x, M.y, M.z);
+        if (M[q][k][3] != 0.0f) s[q] += pair_d2(x[k], y[k], z[k], M[q][k][0], M[q][k][1], M[q][k][2]);
       }
     }
+    if (m0 + 4 < m_end) read(m0 + 4);
     seg_sums(lpr, s[0], s[1], s[2], s[3]);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int m = m0 + q;
-      if (m >= pos) break;
-      const float n = C.mcs_cnt[m];
-      if (n > 0.0f) elhm += C.mcs_tcc[m] * sqrtf(s[q] / n);
-    }
+    for (int q = 0; q < 4; ++q)
+      if (m0 + q < m_end && nc[q] > 0.0f) elhm += tc[q] * sqrtf(s[q] / nc[q]);
   }
   return elhm;
 }
@@ -384,7 +699,10 @@ __device__ __forceinline__ float mcs_sum(const DevComplex &C, int lpr, const flo
 // buffer; one workgroup barrier per tile.
 // Every thread runs the tile loop (waves without a pose only stage). Chunks
 // that cross a tile boundary are evaluated as one fragment per tile.
-template <int APL, bool TILE>
+//
+// FLAT: every pack of the launch has a split of 8 and a unit list in LDS; the
+// pair loop is flat_pairs.
+template <int APL, bool TILE, bool FLAT>
 __device__ __forceinline__ void pose_energy(const DevComplex &C, const Lds &S, int lpr, Split &sp,
                             bool live, const float (&x)[APL],
                             const float (&y)[APL], const float (&z)[APL],
@@ -475,7 +793,32 @@ __device__ __forceinline__ void pose_energy(const DevComplex &C, const Lds &S, i
     else by_clamp(std::integral_constant<int, KIND_PSP>{});
   };
 
-  if constexpr (!TILE) {
+  if constexpr (FLAT) {
+    if (live) {
+      FlatAcc<APL> A;
+      gfloat_p prow[APL];
+#pragma unroll
+      for (int k = 0; k < APL; ++k) {
+        A.vdw[k] = A.ele[k] = A.pmf[k] = A.psp[k] = A.hdb[k] = A.hpc[k] = A.pmfc[k] = 0.0f;
+        A.pps[k] = 0.0f;
+        A.ppm[k] = 0;
+        A.cnt[k] = 0;
+        prow[k] = glob(psprow[k]);
+      }
+      A.pend = false;
+      flat_pairs<APL>(C, S, sp.h, K, x, y, z, lt, prow, A);
+#pragma unroll
+      for (int k = 0; k < APL; ++k) {
+        vdw[k] = A.vdw[k];
+        ele[k] = A.ele[k];
+        pmf[k] = A.pmf[k];
+        psp[k] = A.psp[k];
+        hdb[k] = A.hdb[k];
+        hpc[k] = A.hpc[k];
+        cnt[k] = A.cnt[k];
+      }
+    }
+  } else if constexpr (!TILE) {
     for (int ci = 0; live && ci < n_chunks; ++ci) {
       const int4 ch = S.ch[ci];
       const int cb = __builtin_amdgcn_readfirstlane(ch.x);
@@ -570,7 +913,7 @@ __device__ __forceinline__ void pose_energy(const DevComplex &C, const Lds &S, i
 #pragma unroll
         for (int u = 0; u < 4; ++u) r[u] = rl[j + u];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) P[u] = TILE ? S.gx[r[u].x] : S.xyze[r[u].x];
+        for (int u = 0; u < 4; ++u) P[u] = TILE || FLAT ? S.gx[r[u].x] : S.xyze[r[u].x];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           const float d2 = pair_d2(x[k], y[k], z[k], P[u].x, P[u].y, P[u].z);
@@ -580,7 +923,7 @@ __device__ __forceinline__ void pose_energy(const DevComplex &C, const Lds &S, i
       }
       for (; j < re0; ++j) {
         const int2 r = rl[j];
-        const float4 P = TILE ? S.gx[r.x] : S.xyze[r.x];
+        const float4 P = TILE || FLAT ? S.gx[r.x] : S.xyze[r.x];
         const float d2 = pair_d2(x[k], y[k], z[k], P.x, P.y, P.z);
         const float d = d2 * fast_rsq(d2);
         t_tp += (d <= __int_as_float(r.y)) ? 1 : 0;
@@ -617,7 +960,7 @@ __device__ __forceinline__ void pose_energy(const DevComplex &C, const Lds &S, i
       float hg[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int k = 0; k < APL; ++k) hg[k] = hpc[k];
-      *reinterpret_cast<float4 *>(hb + (size_t)threadIdx.x * 4) = make_float4(hg[0], hg[1], hg[2], hg[3]);
+      *reinterpret_cast<float4 *>(hb + ((size_t)sp.h * sp.half + sp.ltid) * 4) = make_float4(hg[0], hg[1], hg[2], hg[3]);
       if ((sp.ltid - sp.slot * lpr) == 0) {
         float4 *r = reinterpret_cast<float4 *>(rb + ((size_t)sp.h * sp.slots + sp.slot) * 12);
         r[0] = make_float4(t_vdw, t_ele, t_pmf, t_psp);
@@ -928,7 +1271,7 @@ __device__ __forceinline__ void exchange_ladder(int n_tmp, int mode_t, const flo
 // DA: 0 plain Metropolis; delayed acceptance with the surrogate from the
 // network evaluated per atom (1) or from its tabulated outputs (2); 3 and 4
 // are 1 and 2 with the split groups' shared surrogate sums compiled in.
-template <int APL, int DA, bool TILE>
+template <int APL, int DA, bool TILE, bool FLAT>
 __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const DevComplex &C, const Lds &S,
                          int lpr, int step0) {
   constexpr int DAM = DA > 2 ? DA - 2 : DA;
@@ -937,9 +1280,13 @@ __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const
   Split sp;
   sp.ns = P.unsplit ? 1 : pk.ns;
   sp.half = P.unsplit ? (int)blockDim.x : pk.half;
-  // half is a multiple of 64, so the group index is wave-uniform
-  sp.h = __builtin_amdgcn_readfirstlane(tid / sp.half);
-  sp.ltid = tid - sp.h * sp.half;
+  // half is a multiple of 64, so the group index is wave-uniform. Shares of a
+  // chunk are rounded so that later groups hold more points; waves i and i + 4
+  // share a SIMD, so the second half of the waves takes the groups in reverse
+  // order and every SIMD gets a long and a short one.
+  const int hw = __builtin_amdgcn_readfirstlane(tid / sp.half);
+  sp.h = 2 * hw < sp.ns || hw >= sp.ns ? hw : sp.ns + sp.ns / 2 - 1 - hw;
+  sp.ltid = tid - hw * sp.half;
   sp.slots = sp.half / 8;
   sp.xp_floats = P.xp_floats;
   sp.par = 0;
@@ -1024,7 +1371,7 @@ __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const
   if (P.mode != MODE_MC) {
     place(mo);
     gd_energy E;
-    pose_energy<APL, TILE>(C, S, lpr, sp, true, x, y, z, ox, oy, oz, lt, q, li, val, mo, E);
+    pose_energy<APL, TILE, FLAT>(C, S, lpr, sp, true, x, y, z, ox, oy, oz, lt, q, li, val, mo, E);
     if (active && lead) {
       if (P.mode == MODE_EVAL) {
         P.ev_out[sv] = E;
@@ -1122,7 +1469,7 @@ __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const
         place(mn);
       }
       gd_energy E;
-      pose_energy<APL, TILE>(C, S, lpr, sp, wave_active, x, y, z, ox, oy, oz, lt, q, li, val, mn, E);
+      pose_energy<APL, TILE, FLAT>(C, S, lpr, sp, wave_active, x, y, z, ox, oy, oz, lt, q, li, val, mn, E);
       if (wave_active && metropolis(E.e[GD_MAXWEI - 1], eo.e[GD_MAXWEI - 1], mb, u[6])) {
 #pragma unroll
         for (int i = 0; i < 6; ++i) mo[i] = mn[i];
@@ -1181,7 +1528,7 @@ __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const
       const bool eval = wave_active && __ballot(moved) != 0;
       if (eval) place(yv);
       gd_energy E;
-      pose_energy<APL, TILE>(C, S, lpr, sp, eval, x, y, z, ox, oy, oz, lt, q, li, val, yv, E);
+      pose_energy<APL, TILE, FLAT>(C, S, lpr, sp, eval, x, y, z, ox, oy, oz, lt, q, li, val, yv, E);
       if (eval) {
         const float d1 = E.e[GD_MAXWEI - 1] - eo.e[GD_MAXWEI - 1];
         const float d2 = s_y - s_old;
@@ -1230,7 +1577,7 @@ __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const
   }
 }
 
-template <int APL, int DA, bool TILE>
+template <int APL, int DA, bool TILE, bool FLAT>
 __device__ __forceinline__ void mc_kernel_body(const KParams &P, int idx, int step0) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const Pack pk = P.packs[P.pack_base + idx];
@@ -1243,6 +1590,7 @@ __device__ __forceinline__ void mc_kernel_body(const KParams &P, int idx, int st
   S.kde = reinterpret_cast<const float4 *>(lds + P.off_kde);
   S.kr = reinterpret_cast<const int2 *>(lds + P.off_kr);
   S.ch = reinterpret_cast<const int4 *>(lds + P.off_ch);
+  S.fl = reinterpret_cast<const float4 *>(lds);
   S.xe = reinterpret_cast<float *>(lds + P.off_xe);
   S.xi = reinterpret_cast<int *>(lds + P.off_xi);
   S.xa = reinterpret_cast<int *>(lds + P.off_xa);
@@ -1269,14 +1617,28 @@ __device__ __forceinline__ void mc_kernel_body(const KParams &P, int idx, int st
     float4 *kde = reinterpret_cast<float4 *>(lds + P.off_kde);
     int2 *kr = reinterpret_cast<int2 *>(lds + P.off_kr);
     int4 *ch = reinterpret_cast<int4 *>(lds + P.off_ch);
-    if constexpr (!TILE) {
+    if constexpr (FLAT) {
+      // each unit: its two points of this conformer and its attributes
+      const int n_units = C.flat_off[8];
+      for (int i = threadIdx.x; i < n_units; i += nt) {
+        const int4 f = C.flat[i];
+        const int p0 = f.y & 0xffff, p1 = (unsigned)f.y >> 16;
+        int4 a = make_int4(f.x, __float_as_int(0.5f * C.prt_hpp[p0]),
+                           __float_as_int(0.5f * C.prt_hpp[p1]),
+                           (C.prt_psp[p0] & 0xffff) | (C.prt_psp[p1] << 16));
+        xyze[FLAT_F4 * i] = src[p0];
+        xyze[FLAT_F4 * i + 1] = src[p1];
+        *reinterpret_cast<int4 *>(xyze + FLAT_F4 * i + 2) = a;
+      }
+    } else if constexpr (!TILE) {
       for (int i = threadIdx.x; i < pnp; i += nt) {
         xyze[i] = src[i];
         hpp[i] = 0.5f * C.prt_hpp[i];
         psp[i] = C.prt_psp[i];
       }
-      for (int i = threadIdx.x; i < C.pnk; i += nt) kde[i] = C.kde[i];
     }
+    if constexpr (!TILE)
+      for (int i = threadIdx.x; i < C.pnk; i += nt) kde[i] = C.kde[i];
     for (int i = threadIdx.x; i < PAR_FLOATS; i += nt) par[i] = C.params[i];
     for (int i = threadIdx.x; i < NLT; i += nt) kr[i] = C.kde_range[i];
     for (int i = threadIdx.x; i < C.n_chunks; i += nt) ch[i] = C.chunks[i];
@@ -1290,14 +1652,14 @@ __device__ __forceinline__ void mc_kernel_body(const KParams &P, int idx, int st
   }
   __syncthreads();
 
-  run_pack<APL, DA, TILE>(P, pk, C, S, C.lpr, step0);
+  run_pack<APL, DA, TILE, FLAT>(P, pk, C, S, C.lpr, step0);
 }
 
 // MC kernel for packs whose complexes place APL ligand atoms on each lane:
 // plain MC, start-pose evaluation and pose evaluation (DA = false), or
 // delayed acceptance with surrogate sub-steps (DA = true). One instance per
 // APL keeps each variant's register allocation to what it needs.
-template <int APL, int DA, bool TILE>
+template <int APL, int DA, bool TILE, bool FLAT>
 __global__ void __launch_bounds__(512) gd_mc_kernel(KParams P) {
   const int step0 = P.step_dev ? *P.step_dev : P.step0;
   // persistent launches: each workgroup takes packs in LPT order from a
@@ -1314,7 +1676,7 @@ __global__ void __launch_bounds__(512) gd_mc_kernel(KParams P) {
       __syncthreads();  // every thread has read the index; the previous pack's LDS is free
       if (idx >= P.n_queue) break;
     }
-    mc_kernel_body<APL, DA, TILE>(P, idx, step0);
+    mc_kernel_body<APL, DA, TILE, FLAT>(P, idx, step0);
     if (!persistent) break;
   }
 }

@@ -6,28 +6,36 @@
 
 namespace gd {
 
-// Host handle of gd_mc_kernel<GD_MC_APL, da, tiled>: da 0 plain MC and pose
+// Host handle of gd_mc_kernel<GD_MC_APL, da, ...>: da 0 plain MC and pose
 // evaluation, 1 delayed acceptance with the network per atom, 2 with its
 // tabulated outputs, 3 and 4 the same with the receptor split's groups
-// sharing the surrogate's KDE and MCS sums; tiled: the receptor streams
-// through LDS tiles.
+// sharing the surrogate's KDE and MCS sums; rec: the receptor resident in LDS
+// by chunks, streamed through LDS tiles, or resident with unit lists.
 template <>
-const void *mc_kernel_handle<GD_MC_APL>(int da, bool tiled) {
-  if (tiled) {
+const void *mc_kernel_handle<GD_MC_APL>(int da, int rec) {
+  if (rec == REC_TILED) {
     switch (da) {
-      case 1: return (const void *)gd_mc_kernel<GD_MC_APL, 1, true>;
-      case 2: return (const void *)gd_mc_kernel<GD_MC_APL, 2, true>;
-      case 3: return (const void *)gd_mc_kernel<GD_MC_APL, 3, true>;
-      case 4: return (const void *)gd_mc_kernel<GD_MC_APL, 4, true>;
-      default: return (const void *)gd_mc_kernel<GD_MC_APL, 0, true>;
+      case 1: return (const void *)gd_mc_kernel<GD_MC_APL, 1, true, false>;
+      case 2: return (const void *)gd_mc_kernel<GD_MC_APL, 2, true, false>;
+      case 3: return (const void *)gd_mc_kernel<GD_MC_APL, 3, true, false>;
+      case 4: return (const void *)gd_mc_kernel<GD_MC_APL, 4, true, false>;
+      default: return (const void *)gd_mc_kernel<GD_MC_APL, 0, true, false>;
+    }
+  }
+  if (rec == REC_FLAT) {
+    switch (da) {
+      case 0: return (const void *)gd_mc_kernel<GD_MC_APL, 0, false, true>;
+      case 2: return (const void *)gd_mc_kernel<GD_MC_APL, 2, false, true>;
+      case 4: return (const void *)gd_mc_kernel<GD_MC_APL, 4, false, true>;
+      default: return nullptr;
     }
   }
   switch (da) {
-    case 1: return (const void *)gd_mc_kernel<GD_MC_APL, 1, false>;
-    case 2: return (const void *)gd_mc_kernel<GD_MC_APL, 2, false>;
-    case 3: return (const void *)gd_mc_kernel<GD_MC_APL, 3, false>;
-    case 4: return (const void *)gd_mc_kernel<GD_MC_APL, 4, false>;
-    default: return (const void *)gd_mc_kernel<GD_MC_APL, 0, false>;
+    case 1: return (const void *)gd_mc_kernel<GD_MC_APL, 1, false, false>;
+    case 2: return (const void *)gd_mc_kernel<GD_MC_APL, 2, false, false>;
+    case 3: return (const void *)gd_mc_kernel<GD_MC_APL, 3, false, false>;
+    case 4: return (const void *)gd_mc_kernel<GD_MC_APL, 4, false, false>;
+    default: return (const void *)gd_mc_kernel<GD_MC_APL, 0, false, false>;
   }
 }
 
