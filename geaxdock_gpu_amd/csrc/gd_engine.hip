@@ -124,6 +124,7 @@ struct gd_ctx {
     std::vector<float *> grid;  // per complex [n_prt][n^3][32]
     std::vector<SurGrid> g;
     std::vector<float *> tab;   // per complex [n_prt][NLT][n^3] network outputs
+    std::vector<size_t> grid_n, tab_n;  // floats held by each of them
     bool tab_valid = false;     // tab holds the current parameters' outputs
     float *p = nullptr, *m = nullptr, *v = nullptr, *grad = nullptr;  // FP32 master + Adam
     unsigned short *W1T = nullptr, *W2T = nullptr, *W2R = nullptr;    // bf16 layouts
@@ -2163,19 +2164,31 @@ gd_status gd_sur_build_grids(gd_ctx *ctx, float spacing, float half_width) {
   TRY(sync_complexes(ctx));
   auto &S = ctx->sur;
   const int n = (int)std::ceil(2.0f * half_width / spacing) + 1;
-  const size_t node_bytes = 32 * sizeof(float);
-  for (float *g : S.grid)
-    if (g) (void)hipFree(g);
-  for (float *g : S.tab)
-    if (g) (void)hipFree(g);
-  S.tab.assign(ctx->cx.size(), nullptr);
+  const size_t nodes = (size_t)n * n * n;
   S.tab_valid = false;
-  S.grid.assign(ctx->cx.size(), nullptr);
-  S.g.assign(ctx->cx.size(), SurGrid{});
-  for (size_t c = 0; c < ctx->cx.size(); ++c) {
+  // grids and tables of the sizes they had are kept, others replaced (the
+  // number of complexes only grows)
+  const size_t n_cx = ctx->cx.size();
+  S.grid.resize(n_cx, nullptr);
+  S.tab.resize(n_cx, nullptr);
+  S.grid_n.resize(n_cx, 0);
+  S.tab_n.resize(n_cx, 0);
+  S.g.assign(n_cx, SurGrid{});
+  for (size_t c = 0; c < n_cx; ++c) {
     const HostComplex &h = ctx->cx[c];
-    const size_t nodes = (size_t)n * n * n;
-    HIPCHK(hipMalloc(&S.grid[c], (size_t)h.d.n_prt * nodes * node_bytes));
+    const size_t need = (size_t)h.d.n_prt * nodes * 32;
+    if (S.tab_n[c] != (size_t)h.d.n_prt * NLT * nodes) {
+      if (S.tab[c]) (void)hipFree(S.tab[c]);
+      S.tab[c] = nullptr;
+      S.tab_n[c] = 0;
+    }
+    if (S.grid_n[c] != need) {
+      if (S.grid[c]) (void)hipFree(S.grid[c]);
+      S.grid[c] = nullptr;
+      S.grid_n[c] = 0;
+      HIPCHK(hipMalloc(&S.grid[c], need * sizeof(float)));
+      S.grid_n[c] = need;
+    }
     SurGrid G;
     G.grid = S.grid[c];
     G.ox = h.d.pocket_center[0] - half_width;
@@ -2192,12 +2205,12 @@ gd_status gd_sur_build_grids(gd_ctx *ctx, float spacing, float half_width) {
     ctx->cx[c].dev.sn = G.n;
     ctx->cx[c].dev.stab = nullptr;
     ctx->cx_dirty = true;
-    for (int p = 0; p < h.d.n_prt; ++p) {
-      hipLaunchKernelGGL(gd_sur_grid_kernel, dim3((unsigned)((nodes + 255) / 256)), dim3(256), 0,
-                         ctx->stream, h.dev.prt_xyze + (size_t)p * h.d.pnp, h.dev.prt_cls, h.d.pnp,
-                         G.ox, G.oy, G.oz, G.h, n, S.grid[c] + (size_t)p * nodes * 32);
-      HIPCHK(hipGetLastError());
-    }
+    const int64_t nb = (n + 3) / 4, bricks = nb * nb * nb;
+    hipLaunchKernelGGL(gd_sur_grid_kernel,
+                       dim3((unsigned)((bricks + 3) / 4), (unsigned)h.d.n_prt), dim3(256), 0,
+                       ctx->stream, h.dev.prt_xyze, h.dev.prt_cls, h.d.pnp, G.ox, G.oy, G.oz, G.h,
+                       n, S.grid[c]);
+    HIPCHK(hipGetLastError());
   }
   HIPCHK(hipStreamSynchronize(ctx->stream));
   TRY(sync_complexes(ctx));
@@ -2259,47 +2272,42 @@ gd_status gd_sur_tabulate(gd_ctx *ctx) {
   if (!S.have_params) return fail(ctx, GD_ERR_STATE, "no surrogate parameters");
   HIPCHK(hipSetDevice(ctx->device));
   SurW W{S.W1T, S.W2T, S.W2R, S.p + SP_B2, S.p + SP_W3, S.p + SP_B3};
+  const size_t n_cx = ctx->cx.size();
+  // only the ligands' atom types are evaluated: NLT slots per complex
+  std::vector<int> types(n_cx * NLT, 0), n_types(n_cx, 0);
+  for (size_t c = 0; c < n_cx; ++c) {
+    const HostComplex &h = ctx->cx[c];
+    for (int t = 0; t < NLT; ++t)
+      if (std::find(h.lig_t.begin(), h.lig_t.end(), t) != h.lig_t.end())
+        types[c * NLT + n_types[c]++] = t;
+    if (S.tab[c]) continue;
+    const size_t need = (size_t)h.d.n_prt * NLT * S.g[c].n * S.g[c].n * S.g[c].n;
+    if (hipMalloc(&S.tab[c], need * sizeof(float)) != hipSuccess) {
+      S.tab[c] = nullptr;
+      return fail(ctx, GD_ERR_NOMEM, "surrogate table of complex %zu", c);
+    }
+    S.tab_n[c] = need;
+  }
   int *d_types = nullptr;
-  HIPCHK(hipMalloc(&d_types, NLT * sizeof(int)));
-  gd_status st = GD_OK;
-  for (size_t c = 0; c < ctx->cx.size() && st == GD_OK; ++c) {
+  HIPCHK(hipMalloc(&d_types, std::max<size_t>(types.size(), 1) * sizeof(int)));
+  hipError_t e = hipMemcpyAsync(d_types, types.data(), types.size() * sizeof(int),
+                                hipMemcpyHostToDevice, ctx->stream);
+  for (size_t c = 0; c < n_cx && e == hipSuccess; ++c) {
     HostComplex &h = ctx->cx[c];
     const int n = S.g[c].n;
     const size_t n3 = (size_t)n * n * n;
-    if (!S.tab[c]) {
-      if (hipMalloc(&S.tab[c], (size_t)h.d.n_prt * NLT * n3 * sizeof(float)) != hipSuccess) {
-        S.tab[c] = nullptr;
-        st = fail(ctx, GD_ERR_NOMEM, "surrogate table of complex %zu", c);
-        break;
-      }
-    }
-    // only the ligand's atom types are evaluated
-    std::vector<int> types;
-    for (int t = 0; t < NLT; ++t)
-      for (int l = 0; l < h.d.lna; ++l)
-        if (h.lig_t[l] == t) {
-          types.push_back(t);
-          break;
-        }
-    if (hipMemcpy(d_types, types.data(), types.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess) {
-      st = fail(ctx, GD_ERR_HIP, "type list upload");
-      break;
-    }
-    const int64_t jobs = (int64_t)((n3 + 15) / 16) * (int64_t)types.size();
-    for (int p = 0; p < h.d.n_prt; ++p) {
-      hipLaunchKernelGGL(gd_sur_tab_kernel, dim3((unsigned)((jobs + 3) / 4)), dim3(256), 0,
-                         ctx->stream, S.grid[c] + (size_t)p * n3 * 32, (int)n3, d_types,
-                         (int)types.size(), W, S.tab[c] + (size_t)p * NLT * n3);
-    }
-    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(ctx->stream) != hipSuccess) {
-      st = fail(ctx, GD_ERR_HIP, "tabulation kernel");
-      break;
-    }
+    // two workgroups of four waves per CU, which walk the tiles of 16 points
+    const int64_t tiles = (int64_t)((n3 + 15) / 16) * h.d.n_prt;
+    const int64_t grid = std::min<int64_t>((tiles + 3) / 4, 2 * (int64_t)ctx->n_cu);
+    hipLaunchKernelGGL(gd_sur_tab_kernel, dim3((unsigned)grid), dim3(256), 0, ctx->stream,
+                       S.grid[c], (int)n3, h.d.n_prt, d_types + c * NLT, n_types[c], W, S.tab[c]);
+    e = hipGetLastError();
     h.dev.stab = S.tab[c];
     ctx->cx_dirty = true;
   }
+  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   (void)hipFree(d_types);
-  TRY(st);
+  if (e != hipSuccess) return fail(ctx, GD_ERR_HIP, "tabulation: %s", hipGetErrorString(e));
   TRY(sync_complexes(ctx));
   S.tab_valid = true;
   return GD_OK;

@@ -38,6 +38,14 @@ constexpr int SUR_NPARAM = SP_B3 + 1;
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
 
+// two floats rounded to bf16 (nearest even), the first in the low half
+__device__ inline unsigned int pk_bf16(float a, float b) {
+  typedef float f32x2_t __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+  const f32x2_t v = {a, b};
+  return __builtin_bit_cast(unsigned int, __builtin_convertvector(v, bf16x2_t));
+}
+
 __host__ __device__ inline unsigned short f2bf(float f) {
   unsigned int u;
   memcpy(&u, &f, 4);
@@ -61,29 +69,20 @@ __device__ inline bf16x8_t ld8(const unsigned short *p) {
 }
 
 // ---------------------------------------------------------------------------
-// Radial features of one position against a receptor conformer (sorted
-// points with per-point class).
+// Radial features of one position: receptor point (px, py, pz) of class C adds
+// to the class's eight features.
 // ---------------------------------------------------------------------------
-__device__ inline void radial32(float x, float y, float z, const float4 *xyze, const int *cls,
-                                int pnp, float (&f)[32]) {
+template <int C>
+__device__ inline void radial_add(float x, float y, float z, float px, float py, float pz,
+                                  float (&f)[32]) {
+  const float d2 = pair_d2(x, y, z, px, py, pz);
+  if (d2 < SUR_CUT * SUR_CUT) {
+    const float d = sqrtf(d2);
+    const float fc = 0.5f * (1.0f + cosf(3.14159265358979f * d / SUR_CUT));
 #pragma unroll
-  for (int i = 0; i < 32; ++i) f[i] = 0.0f;
-  const float c2 = SUR_CUT * SUR_CUT;
-  for (int p = 0; p < pnp; ++p) {
-    const float4 P = xyze[p];
-    const float d2 = pair_d2(x, y, z, P.x, P.y, P.z);
-    if (d2 < c2) {
-      const float d = sqrtf(d2);
-      const float fc = 0.5f * (1.0f + cosf(3.14159265358979f * d / SUR_CUT));
-      const int c = cls[p];
-#pragma unroll
-      for (int k = 0; k < SUR_NRBF; ++k) {
-        const float t = d - (float)(k + 1);
-        const float g = expf(-0.5f * t * t) * fc;
-#pragma unroll
-        for (int cc = 0; cc < SUR_NCLS; ++cc)
-          if (cc == c) f[cc * SUR_NRBF + k] += g;
-      }
+    for (int k = 0; k < SUR_NRBF; ++k) {
+      const float t = d - (float)(k + 1);
+      f[C * SUR_NRBF + k] += expf(-0.5f * t * t) * fc;
     }
   }
 }

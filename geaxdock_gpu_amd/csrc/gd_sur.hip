@@ -1,26 +1,81 @@
 // gd_sur.hip -- learned energy surrogate kernels: receptor feature grids,
 // feature rows, BF16 MFMA MLP forward/backward (FP32 accumulate), fixed-order
 // gradient sums, FP32 Adam. Building blocks and layouts: gd_sur.h.
+#include <type_traits>
+
 #include "gd_sur.h"
 
 namespace gd {
 
-// Feature grid of one protein conformer: n^3 nodes at origin + h*(i,j,k),
-// 32 floats per node, node index (i*n + j)*n + k.
-extern "C" __global__ void gd_sur_grid_kernel(const float4 *xyze, const int *cls, int pnp,
-                                              float ox, float oy, float oz, float h, int n,
-                                              float *grid) {
-  const int64_t node = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t total = (int64_t)n * n * n;
-  if (node >= total) return;
-  const int k = (int)(node % n);
-  const int j = (int)((node / n) % n);
-  const int i = (int)(node / ((int64_t)n * n));
+// Feature grids of all protein conformers (grid.y) of a complex: n^3 nodes at
+// origin + h*(i,j,k), 32 floats per node, node index (i*n + j)*n + k.
+//
+// A wave owns a brick of 4 x 4 x 4 nodes, so its lanes share most of the
+// receptor points within the cut-off. It tests 64 points at a time against
+// the brick (grown by the cut-off), one per lane, and takes the points that
+// pass, class by class, from the owning lane's registers as scalars: each class
+// then adds to its own eight registers without selects, in the point order of
+// a plain loop over the receptor (same bits). Bound: VALU, the eight expf of a
+// node-point pair. One wave per 64 nodes along z and a 32-way select per pair
+// took 744 us for 65^3 nodes and 2,400 points; this takes 182 us.
+extern "C" __global__ void __launch_bounds__(256) gd_sur_grid_kernel(
+    const float4 *xyze_all, const int *cls, int pnp, float ox, float oy, float oz, float h, int n,
+    float *grid_all) {
+  const int l = threadIdx.x & 63;
+  const int nb = (n + 3) / 4;
+  const int brick = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  if (brick >= nb * nb * nb) return;  // whole wave leaves; no block barrier
+  const float4 *xyze = xyze_all + (size_t)blockIdx.y * pnp;
+  const int bi = 4 * (brick / (nb * nb)), bj = 4 * ((brick / nb) % nb), bk = 4 * (brick % nb);
+  const int i = bi + (l >> 4), j = bj + ((l >> 2) & 3), k = bk + (l & 3);
+  const float x = ox + h * i, y = oy + h * j, z = oz + h * k;
+  // squared distance of a point to the brick; a margin covers its rounding
+  const float lx = ox + h * bi, ly = oy + h * bj, lz = oz + h * bk, w = 3.0f * h;
+  const float reach = SUR_CUT * SUR_CUT * 1.001f;
   float f[32];
-  radial32(ox + h * i, oy + h * j, oz + h * k, xyze, cls, pnp, f);
-  float4 *o = reinterpret_cast<float4 *>(grid + node * 32);
 #pragma unroll
-  for (int q = 0; q < 8; ++q) o[q] = make_float4(f[4 * q], f[4 * q + 1], f[4 * q + 2], f[4 * q + 3]);
+  for (int q = 0; q < 32; ++q) f[q] = 0.0f;
+  float4 P = make_float4(0.f, 0.f, 0.f, 0.f);
+  int c = -1;
+  if (l < pnp) {
+    P = xyze[l];
+    c = cls[l];
+  }
+  for (int p0 = 0; p0 < pnp; p0 += 64) {
+    const int pn = p0 + 64 + l;
+    float4 Pn = make_float4(0.f, 0.f, 0.f, 0.f);
+    int cn = -1;
+    if (pn < pnp) {
+      Pn = xyze[pn];
+      cn = cls[pn];
+    }
+    const float dx = fmaxf(fmaxf(lx - P.x, P.x - (lx + w)), 0.0f);
+    const float dy = fmaxf(fmaxf(ly - P.y, P.y - (ly + w)), 0.0f);
+    const float dz = fmaxf(fmaxf(lz - P.z, P.z - (lz + w)), 0.0f);
+    const bool in = dx * dx + dy * dy + dz * dz <= reach;
+    auto add = [&](auto cls_c) {
+      constexpr int C = decltype(cls_c)::value;
+      for (unsigned long long m = __ballot(in && c == C); m != 0; m &= m - 1) {
+        const int s = __builtin_ctzll(m);
+        radial_add<C>(x, y, z,
+                      __int_as_float(__builtin_amdgcn_readlane(__float_as_int(P.x), s)),
+                      __int_as_float(__builtin_amdgcn_readlane(__float_as_int(P.y), s)),
+                      __int_as_float(__builtin_amdgcn_readlane(__float_as_int(P.z), s)), f);
+      }
+    };
+    add(std::integral_constant<int, 0>{});
+    add(std::integral_constant<int, 1>{});
+    add(std::integral_constant<int, 2>{});
+    add(std::integral_constant<int, 3>{});
+    P = Pn;
+    c = cn;
+  }
+  if (i < n && j < n && k < n) {
+    float4 *o = reinterpret_cast<float4 *>(
+        grid_all + (((size_t)blockIdx.y * n + i) * n + j) * n * 32 + (size_t)k * 32);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) o[q] = make_float4(f[4 * q], f[4 * q + 1], f[4 * q + 2], f[4 * q + 3]);
+  }
 }
 
 // Feature rows of poses of one complex: one thread per ligand atom of each
@@ -252,51 +307,97 @@ extern "C" __global__ void __launch_bounds__(256) gd_mlp_fwd_kernel(const unsign
 }
 
 // Network output at every grid point for each listed ligand atom type:
-// Y[type][point] = MLP(onehot(type), features(point)), the features being
-// the grid's own values (no interpolation). One wave per 16 points of one
-// type; 4 waves per workgroup.
-extern "C" __global__ void __launch_bounds__(256) gd_sur_tab_kernel(const float *fgrid,
-                                                                    int n_pts,
-                                                                    const int *types,
-                                                                    int n_types, SurW W,
-                                                                    float *Y) {
-  __shared__ __attribute__((aligned(16))) unsigned short xs[4][16 * SUR_F];
-  __shared__ __attribute__((aligned(16))) unsigned short a1s[4][16 * SUR_H];
-  const int wv = threadIdx.x >> 6, l = threadIdx.x & 63;
-  const int tiles = (n_pts + 15) / 16;
-  const int64_t job = (int64_t)blockIdx.x * 4 + wv;
-  if (job >= (int64_t)tiles * n_types) return;  // whole wave leaves; no block barrier
-  const int ti = (int)(job / tiles);
-  const int p0 = (int)(job % tiles) * 16;
-  const int type = types[ti];
-  // lane l fills columns 16 (l % 4) .. +15 of row l / 4
-  {
-    const int r = l >> 2, c0 = 16 * (l & 3);
-    const int pt = min(p0 + r, n_pts - 1);
-    const float *f = fgrid + (size_t)pt * 32;
-    unsigned short *row = xs[wv] + r * SUR_F;
+// Y[conformer][type][point] = MLP(onehot(type), features(point)), the features
+// being the grid's own values (no interpolation).
+//
+// A wave keeps W1 and W2 in registers (192) and takes tiles of 16 points, each
+// through all the types: the points' features are read and rounded once per
+// tile, and only the one-hot half of the first K block changes. Both layers
+// are computed transposed (weights as the A operand, points as columns), so a
+// lane holds four consecutive hidden units of one point: A1 goes to LDS as
+// 8-byte rows instead of 32 two-byte stores, and the output's sum over units
+// needs two cross-lane steps instead of sixteen. Products, K order and the sum
+// tree are those of mlp_fwd16 and mlp_out16, so values have the same bits.
+// Bound: VALU (SiLU: 64 exp2 and 64 rcp per lane and tile), then MFMA. Reading
+// the weights from L2 for every tile took 2,217 us for 65^3 points and 20
+// types (122 TFLOP/s); this takes 520 us (520 TFLOP/s).
+constexpr int SUR_TAB_LD = SUR_H + 8;  // A1 row stride in LDS
+extern "C" __global__ void __launch_bounds__(256, 2) gd_sur_tab_kernel(
+    const float *fgrid, int n_pts, int n_prt, const int *types, int n_types, SurW W, float *Y) {
+  __shared__ __attribute__((aligned(16))) unsigned short a1s[4][16 * SUR_TAB_LD];
+  __shared__ __attribute__((aligned(16))) float b2s[SUR_H], w3s[SUR_H];
+  const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, lr = l & 15, lq = l >> 4;
+  for (int i = threadIdx.x; i < SUR_H; i += blockDim.x) {
+    b2s[i] = W.b2[i];
+    w3s[i] = W.w3[i];
+  }
+  __syncthreads();
+  bf16x8_t w1[8][2], w2[8][4];
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int c = c0 + q;
-      float v = 0.0f;
-      if (c < NLT) v = (c == type) ? 1.0f : 0.0f;
-      else if (c < NLT + 32) v = f[c - NLT];
-      else if (c == SUR_BIAS_COL) v = 1.0f;
-      row[c] = f2bf(v);
+  for (int t = 0; t < 8; ++t) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) w1[t][ks] = ld8(W.W1T + (16 * t + lr) * SUR_F + 32 * ks + 8 * lq);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) w2[t][ks] = ld8(W.W2T + (16 * t + lr) * SUR_H + 32 * ks + 8 * lq);
+  }
+  const float b3 = W.b3[0];
+  unsigned short *a1 = a1s[wv] + lr * SUR_TAB_LD;  // this lane's point
+  const int tiles = (n_pts + 15) / 16;
+  const int64_t n_tiles = (int64_t)tiles * n_prt;
+  for (int64_t job = (int64_t)blockIdx.x * 4 + wv; job < n_tiles; job += (int64_t)gridDim.x * 4) {
+    const int prt = (int)(job / tiles);
+    const int p0 = (int)(job % tiles) * 16;
+    // feature columns: K block 0 holds the one-hot (lq 0..2) and radial 0..7
+    // (lq 3), block 1 radial 8..31 (lq 0..2) and the bias column (lq 3)
+    const int pt = min(p0 + lr, n_pts - 1);
+    const float4 *f = reinterpret_cast<const float4 *>(
+        fgrid + ((size_t)prt * n_pts + pt) * 32 + (lq == 3 ? 0 : 8 + 8 * lq));
+    const float4 fa = f[0], fb = f[1];
+    const uint4 fx = make_uint4(pk_bf16(fa.x, fa.y), pk_bf16(fa.z, fa.w), pk_bf16(fb.x, fb.y),
+                                pk_bf16(fb.z, fb.w));
+    const uint4 x1 = lq == 3 ? make_uint4(0x3F80u, 0u, 0u, 0u) : fx;
+    for (int ti = 0; ti < n_types; ++ti) {
+      const int type = types[ti];
+      const int rel = type - 8 * lq;  // one-hot column within the lane's eight
+      auto hot = [&](int w) {
+        return rel == 2 * w ? 0x3F80u : (rel == 2 * w + 1 ? 0x3F800000u : 0u);
+      };
+      const uint4 x0 = lq == 3 ? fx : make_uint4(hot(0), hot(1), hot(2), hot(3));
+      const bf16x8_t xb0 = __builtin_bit_cast(bf16x8_t, x0);
+      const bf16x8_t xb1 = __builtin_bit_cast(bf16x8_t, x1);
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        f32x4_t c = {0.f, 0.f, 0.f, 0.f};
+        c = mfma32(w1[t][0], xb0, c);
+        c = mfma32(w1[t][1], xb1, c);
+        *reinterpret_cast<uint2 *>(a1 + 16 * t + 4 * lq) =
+            make_uint2(pk_bf16(silu(c[0]), silu(c[1])), pk_bf16(silu(c[2]), silu(c[3])));
+      }
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): A1 is in LDS
+      __builtin_amdgcn_wave_barrier();
+      bf16x8_t ab[4];
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) ab[ks] = ld8(a1 + 32 * ks + 8 * lq);
+      float y[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        f32x4_t c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) c = mfma32(w2[u][ks], ab[ks], c);
+        const float4 bb = *reinterpret_cast<const float4 *>(b2s + 16 * u + 4 * lq);
+        const float4 ww = *reinterpret_cast<const float4 *>(w3s + 16 * u + 4 * lq);
+        y[0] = fmaf(silu(c[0] + bb.x), ww.x, y[0]);
+        y[1] = fmaf(silu(c[1] + bb.y), ww.y, y[1]);
+        y[2] = fmaf(silu(c[2] + bb.z), ww.z, y[2]);
+        y[3] = fmaf(silu(c[3] + bb.w), ww.w, y[3]);
+      }
+      __builtin_amdgcn_wave_barrier();  // the next type's A1 goes to the same rows
+      float v = (y[0] + y[1]) + (y[2] + y[3]);
+      v += __shfl_xor(v, 16);
+      v += __shfl_xor(v, 32);
+      if (lq == 0 && p0 + lr < n_pts) Y[((size_t)prt * NLT + type) * n_pts + p0 + lr] = v + b3;
     }
   }
-  __builtin_amdgcn_s_waitcnt(0xc07f);
-  __builtin_amdgcn_wave_barrier();
-  f32x4_t h1[8], h2[8];
-  mlp_fwd16(xs[wv], 0, W, a1s[wv], h1, h2);
-  float yy[4];
-  mlp_out16(h2, W, yy);
-  if ((l & 15) == 0)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int pt = p0 + 4 * (l >> 4) + i;
-      if (pt < n_pts) Y[(size_t)type * n_pts + pt] = yy[i];
-    }
 }
 
 // Output gradient of each row of a batch: dyr[i] = dS of row i's pose when
