@@ -136,7 +136,6 @@ struct gd_ctx {
     std::vector<int64_t> off{0};  // pose row offsets
     std::vector<float> target;
     std::vector<int> pose_cx;
-    int *pose_of_row = nullptr;
     int64_t *d_off = nullptr;
     float *d_target = nullptr;
     bool dirty = true;
@@ -144,7 +143,8 @@ struct gd_ctx {
     float *y = nullptr, *dS = nullptr, *sq = nullptr, *S = nullptr;
     float *p1 = nullptr, *p2 = nullptr, *pb2 = nullptr, *pw3 = nullptr;
     float *dyr = nullptr;  // per-row output gradient of the current batch
-    int64_t work_rows = 0;
+    float *bl = nullptr;   // per-batch sums of squared residuals of an epoch
+    int64_t work_rows = 0, work_poses = 0, work_batches = 0;
     int last_groups = 0;  // backward workgroups (partials) of the last batch
   } sur;
 };
@@ -299,7 +299,7 @@ void gd_destroy(gd_ctx *ctx) {
       if (g) (void)hipFree(g);
     for (float *g : S.tab)
       if (g) (void)hipFree(g);
-    void *qs[] = {S.p, S.m, S.v, S.grad, S.W1T, S.W2T, S.W2R, S.X, S.pose_of_row,
+    void *qs[] = {S.p, S.m, S.v, S.grad, S.W1T, S.W2T, S.W2R, S.X, S.bl,
                   S.d_off, S.d_target, S.y, S.dS, S.sq, S.S, S.p1, S.p2, S.pb2, S.pw3,
                   S.dyr};
     for (void *p : qs)
@@ -2053,23 +2053,16 @@ gd_status sur_upload_index(gd_ctx *ctx) {
   const int64_t np = (int64_t)S.target.size();
   if (S.d_off) (void)hipFree(S.d_off);
   if (S.d_target) (void)hipFree(S.d_target);
-  if (S.pose_of_row) (void)hipFree(S.pose_of_row);
   S.d_off = nullptr;
   S.d_target = nullptr;
-  S.pose_of_row = nullptr;
   HIPCHK(hipMalloc(&S.d_off, (np + 1) * sizeof(int64_t)));
   HIPCHK(hipMalloc(&S.d_target, std::max<int64_t>(np, 1) * sizeof(float)));
-  HIPCHK(hipMalloc(&S.pose_of_row, (S.cap + 64) * sizeof(int)));
   // per-row outputs are indexed by absolute dataset row
   if (S.y) (void)hipFree(S.y);
   S.y = nullptr;
   HIPCHK(hipMalloc(&S.y, (S.cap + 64) * sizeof(float)));
-  std::vector<int> por(S.cap + 64, -1);
-  for (int64_t p = 0; p < np; ++p)
-    for (int64_t r = S.off[p]; r < S.off[p + 1]; ++r) por[r] = (int)p;
   HIPCHK(hipMemcpyAsync(S.d_off, S.off.data(), (np + 1) * sizeof(int64_t), hipMemcpyHostToDevice, ctx->stream));
   if (np) HIPCHK(hipMemcpyAsync(S.d_target, S.target.data(), np * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
-  HIPCHK(hipMemcpyAsync(S.pose_of_row, por.data(), por.size() * sizeof(int), hipMemcpyHostToDevice, ctx->stream));
   HIPCHK(hipStreamSynchronize(ctx->stream));
   S.dirty = false;
   return GD_OK;
@@ -2104,13 +2097,17 @@ gd_status sur_work(gd_ctx *ctx, int64_t rows, int64_t n_pose_total) {
                                hipFuncAttributeMaxDynamicSharedMemorySize, SUR_TRAIN_LDS));
     S.work_rows = rows;
   }
-  if (S.dS) (void)hipFree(S.dS);
-  if (S.sq) (void)hipFree(S.sq);
-  if (S.S) (void)hipFree(S.S);
   const int64_t np = std::max<int64_t>(n_pose_total, 1);
-  HIPCHK(hipMalloc(&S.dS, np * sizeof(float)));
-  HIPCHK(hipMalloc(&S.sq, np * sizeof(float)));
-  HIPCHK(hipMalloc(&S.S, np * sizeof(float)));
+  if (np > S.work_poses) {
+    float **qs[] = {&S.dS, &S.sq, &S.S};
+    S.work_poses = 0;
+    for (float **q : qs) {
+      if (*q) (void)hipFree(*q);
+      *q = nullptr;
+      HIPCHK(hipMalloc(q, np * sizeof(float)));
+    }
+    S.work_poses = np;
+  }
   return GD_OK;
 }
 
@@ -2127,18 +2124,17 @@ gd_status sur_batch(gd_ctx *ctx, int64_t p0, int64_t p1, bool grad, double *loss
   const unsigned short *X = S.X + r0 * SUR_F;
   hipLaunchKernelGGL(gd_mlp_fwd_kernel, dim3(sur_fwd_groups(ctx, nr)), dim3(256), 0, ctx->stream, X,
                      nr, W, S.y + r0);
-  hipLaunchKernelGGL(gd_mlp_pose_kernel, dim3((np + 255) / 256), dim3(256), 0, ctx->stream, S.y,
-                     S.d_off, (int)p0, (int)p1, S.d_target, S.dS, S.sq, S.S);
+  hipLaunchKernelGGL(gd_mlp_pose_kernel, dim3((np + 63) / 64), dim3(256), 0, ctx->stream, S.y,
+                     S.d_off, (int)p0, (int)p1, S.d_target, S.dS, S.sq, S.S,
+                     grad ? S.dyr : (float *)nullptr, nr);
   if (grad) {
     const int ng = sur_train_groups(ctx, nr);
-    hipLaunchKernelGGL(gd_mlp_dyrow_kernel, dim3((unsigned)((nr + 255) / 256)), dim3(256), 0,
-                       ctx->stream, S.pose_of_row + r0, nr, (int)p0, (int)p1, S.dS, S.dyr);
-    hipLaunchKernelGGL(gd_mlp_train_kernel, dim3(ng), dim3(256), SUR_TRAIN_LDS, ctx->stream, X,
+    hipLaunchKernelGGL(gd_mlp_train_kernel, dim3(ng), dim3(512), SUR_TRAIN_LDS, ctx->stream, X,
                        nr, S.dyr, W, S.p1, S.p2, S.pb2, S.pw3);
     S.last_groups = ng;
     if (!update)
-      hipLaunchKernelGGL(gd_mlp_gradsum_kernel, dim3((SUR_NPARAM + 255) / 256), dim3(256), 0,
-                         ctx->stream, S.p1, ng, S.p2, ng, S.pb2, S.pw3, (int64_t)ng, S.grad);
+      hipLaunchKernelGGL(gd_mlp_gradsum_kernel, dim3((SUR_NPARAM + 31) / 32), dim3(256), 0,
+                         ctx->stream, S.p1, S.p2, S.pb2, S.pw3, ng, S.grad);
   }
   HIPCHK(hipGetLastError());
   if (loss) {
@@ -2498,8 +2494,14 @@ gd_status gd_sur_train(gd_ctx *ctx, int pose_begin, int pose_end, int epochs, in
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   const int n_batch = (pose_end - pose_begin + batch_poses - 1) / batch_poses;
   // per-batch sums of squared residuals (before each batch's update)
-  float *d_bl = nullptr;
-  HIPCHK(hipMalloc(&d_bl, (size_t)n_batch * sizeof(float)));
+  if (n_batch > S.work_batches) {
+    if (S.bl) (void)hipFree(S.bl);
+    S.bl = nullptr;
+    S.work_batches = 0;
+    HIPCHK(hipMalloc(&S.bl, (size_t)n_batch * sizeof(float)));
+    S.work_batches = n_batch;
+  }
+  float *d_bl = S.bl;
   std::vector<float> bl(n_batch);
   const auto t0 = std::chrono::steady_clock::now();
   S.tab_valid = false;  // the parameters change
@@ -2510,14 +2512,13 @@ gd_status gd_sur_train(gd_ctx *ctx, int pose_begin, int pose_end, int epochs, in
       const int q = std::min(pose_end, p + batch_poses);
       st = sur_batch(ctx, p, q, true, nullptr, true);
       if (st != GD_OK) break;
-      hipLaunchKernelGGL(gd_mlp_sqsum_kernel, dim3(1), dim3(256), 0, ctx->stream, S.sq + p,
-                         q - p, d_bl + b);
       S.adam_t += 1;
       const float c1 = 1.0f - std::pow(b1, (float)S.adam_t);
       const float c2 = 1.0f - std::pow(b2, (float)S.adam_t);
-      hipLaunchKernelGGL(gd_mlp_update_kernel, dim3((SUR_NPARAM + 255) / 256), dim3(256), 0,
+      hipLaunchKernelGGL(gd_mlp_update_kernel, dim3((SUR_NPARAM + 31) / 32 + 1), dim3(256), 0,
                          ctx->stream, S.p1, S.p2, S.pb2, S.pw3, S.last_groups, S.p, S.m, S.v,
-                         S.grad, lr, b1, b2, eps, c1, c2, S.W1T, S.W2T, S.W2R);
+                         S.grad, lr, b1, b2, eps, c1, c2, S.W1T, S.W2T, S.W2R, S.sq + p, q - p,
+                         d_bl + b);
       if (hipGetLastError() != hipSuccess) st = fail(ctx, GD_ERR_HIP, "training launch failed");
     }
     if (st != GD_OK || !epoch_loss) continue;
@@ -2534,18 +2535,28 @@ gd_status gd_sur_train(gd_ctx *ctx, int pose_begin, int pose_end, int epochs, in
       epoch_loss[ep] = tot / (double)(pose_end - pose_begin);
     } else {
       // last epoch: the loss over the whole range with the final parameters
+      // (every batch's residuals in one copy)
       double tot = 0.0;
-      for (int p = pose_begin; p < pose_end && st == GD_OK; p += batch_poses) {
+      for (int p = pose_begin; p < pose_end && st == GD_OK; p += batch_poses)
+        st = sur_batch(ctx, p, std::min(pose_end, p + batch_poses), false, nullptr);
+      if (st != GD_OK) break;
+      std::vector<float> sq(pose_end - pose_begin);
+      if (hipMemcpyAsync(sq.data(), S.sq + pose_begin, sq.size() * sizeof(float),
+                         hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
+          hipStreamSynchronize(ctx->stream) != hipSuccess) {
+        st = fail(ctx, GD_ERR_HIP, "residual copy failed");
+        break;
+      }
+      for (int p = pose_begin; p < pose_end; p += batch_poses) {
         const int q = std::min(pose_end, p + batch_poses);
         double l = 0.0;
-        st = sur_batch(ctx, p, q, false, &l);
-        tot += l * (q - p);
+        for (int i = p; i < q; ++i) l += sq[i - pose_begin];
+        tot += l / (q - p) * (q - p);
       }
       epoch_loss[ep] = tot / (double)(pose_end - pose_begin);
     }
   }
   (void)hipStreamSynchronize(ctx->stream);
-  (void)hipFree(d_bl);
   TRY(st);
   HIPCHK(hipStreamSynchronize(ctx->stream));
   if (seconds) *seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();

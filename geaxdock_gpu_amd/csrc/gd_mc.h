@@ -66,46 +66,6 @@ struct Split {
   int par;
 };
 
-// One level of the xor butterfly over a replica's lanes: v + (v of lane ^ m).
-// Levels 1, 2, 4 and 8 are DPP operands of the add itself (4 and 8 as mirrors
-// of 8 and 16 lanes: after the levels below them every lane of a quad, or of
-// half a row, holds the same value, so the mirrored lane's value is lane ^ m's);
-// 16 and 32 are gfx950's row and half-wave swaps. The additions and their
-// bits are those of a butterfly of shuffles, but a level costs one to three
-// VALU slots where a shuffle is an LDS round trip. A step of one complex of 8
-// replicas went from 52.0 to 48.9 us, of a coarse receptor with 196 MCS
-// templates (408 replicas) from 79 to 72 us; a batch step gains 1.5 %.
-template <int CTRL>
-__device__ __forceinline__ int dpp_mov(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
-}
-constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_HALF_MIRROR = 0x141, DPP_MIRROR = 0x140;
-
-template <int CTRL>
-__device__ __forceinline__ void dpp_add(float &v) {
-  v += __int_as_float(dpp_mov<CTRL>(__float_as_int(v)));
-}
-template <int CTRL>
-__device__ __forceinline__ void dpp_add(int &v) {
-  v += dpp_mov<CTRL>(v);
-}
-__device__ __forceinline__ void swap16_add(float &v) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
-  v = __int_as_float(r[0]) + __int_as_float(r[1]);
-}
-__device__ __forceinline__ void swap16_add(int &v) {
-  const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-  v = (int)r[0] + (int)r[1];
-}
-__device__ __forceinline__ void swap32_add(float &v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
-  v = __int_as_float(r[0]) + __int_as_float(r[1]);
-}
-__device__ __forceinline__ void swap32_add(int &v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-  v = (int)r[0] + (int)r[1];
-}
-
 // Sums over the `lpr` lanes (8, 16, 32 or 64) of each replica, left in every
 // lane; several sums share the level tests and overlap.
 template <class... T>

@@ -72,6 +72,9 @@ __device__ inline bf16x8_t ld8(const unsigned short *p) {
 // Radial features of one position: receptor point (px, py, pz) of class C adds
 // to the class's eight features.
 // ---------------------------------------------------------------------------
+// The sums take one fused multiply-add each; the very last feature rounds its
+// product first, as the selects of a 32-way update did, so that grids keep
+// their bits.
 template <int C>
 __device__ inline void radial_add(float x, float y, float z, float px, float py, float pz,
                                   float (&f)[32]) {
@@ -82,7 +85,9 @@ __device__ inline void radial_add(float x, float y, float z, float px, float py,
 #pragma unroll
     for (int k = 0; k < SUR_NRBF; ++k) {
       const float t = d - (float)(k + 1);
-      f[C * SUR_NRBF + k] += expf(-0.5f * t * t) * fc;
+      const float g = expf(-0.5f * t * t);
+      float &s = f[C * SUR_NRBF + k];
+      s = C == 3 && k == 7 ? add_rn(s, mul_rn(g, fc)) : fmaf(g, fc, s);
     }
   }
 }
@@ -213,14 +218,7 @@ __device__ inline void mlp_out16(const f32x4_t (&h2)[8], const SurW &W, float (&
     for (int i = 0; i < 4; ++i) y[i] = fmaf(silu(h2[u][i]), w, y[i]);
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float v = y[i];
-    v += __shfl_xor(v, 1);
-    v += __shfl_xor(v, 2);
-    v += __shfl_xor(v, 4);
-    v += __shfl_xor(v, 8);
-    y[i] = v + W.b3[0];
-  }
+  for (int i = 0; i < 4; ++i) y[i] = row16_sum(y[i]) + W.b3[0];
 }
 
 }  // namespace gd

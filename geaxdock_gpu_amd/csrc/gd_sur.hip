@@ -124,53 +124,53 @@ constexpr int SUR_AS = SUR_H + 8;
 constexpr int SUR_TR = 72;    // transposed tiles: 64 rows + 8
 constexpr int SUR_STEP = 64;  // rows per step: 4 row tiles of 16
 
-// Column-split MLP of the batch kernels. A workgroup of 4 waves takes 64
-// rows at a time; wave w owns columns [32 w, 32 w + 32) of both 128-wide
-// layers for all 64 rows, so its slices of W1, W2 and W2^T stay in
-// registers for the whole kernel (B fragments: col tile c, K block kb), and
-// the rows' X and A1 tiles are shared through LDS.
+// Column-split MLP of the batch kernels. A workgroup takes 64 rows at a time;
+// each of its waves owns 16 NC columns of both 128-wide layers for all 64
+// rows, so its slices of W1, W2 and W2^T stay in registers for the whole
+// kernel (B fragments: col tile c, K block kb), and the rows' X and A1 tiles
+// are shared through LDS.
+template <int NC>
 struct ColW {
-  bf16x8_t w1[2][2];   // W1[:, 32w + 16c ..]: K = 64
-  bf16x8_t w2[2][4];   // W2[:, 32w + 16c ..]: K = 128
-  float b2[2], w3[2];  // per lane: column 32w + 16c + l % 16
+  bf16x8_t w1[NC][2];    // W1[:, 16 (NC w + c) ..]: K = 64
+  bf16x8_t w2[NC][4];    // W2[:, 16 (NC w + c) ..]: K = 128
+  float b2[NC], w3[NC];  // per lane: column 16 (NC w + c) + l % 16
 };
 
-__device__ inline void load_colw(const SurW &W, int wv, bool with_w2r, ColW &cw,
-                                 bf16x8_t (&w2r)[2][4]) {
+template <int NC>
+__device__ inline void load_colw(const SurW &W, int wv, ColW<NC> &cw) {
   const int l = threadIdx.x & 63, lr = l & 15, lq = l >> 4;
 #pragma unroll
-  for (int c = 0; c < 2; ++c) {
-    const int n = 32 * wv + 16 * c + lr;
+  for (int c = 0; c < NC; ++c) {
+    const int n = 16 * (NC * wv + c) + lr;
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) cw.w1[c][kb] = ld8(W.W1T + n * SUR_F + 32 * kb + 8 * lq);
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-      cw.w2[c][kb] = ld8(W.W2T + n * SUR_H + 32 * kb + 8 * lq);
-      if (with_w2r) w2r[c][kb] = ld8(W.W2R + n * SUR_H + 32 * kb + 8 * lq);
-    }
+    for (int kb = 0; kb < 4; ++kb) cw.w2[c][kb] = ld8(W.W2T + n * SUR_H + 32 * kb + 8 * lq);
     cw.b2[c] = W.b2[n];
     cw.w3[c] = W.w3[n];
   }
 }
 
-// X rows [r0, r0 + 64) as 512 pieces of 8 bf16, two per thread (all 256
+// X rows [r0, r0 + 64) as 512 pieces of 8 bf16, NV per thread (512 / NV
 // threads): read into registers, then written to xs (row-major) and, when xt
 // is given, xt (transposed, [64 features][SUR_TR]).
-__device__ inline void load_x(const unsigned short *X, int64_t r0, uint4 (&v)[2]) {
+template <int NV>
+__device__ inline void load_x(const unsigned short *X, int64_t r0, uint4 (&v)[NV]) {
   const int t = threadIdx.x;
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int e = t + 256 * h;
+  for (int h = 0; h < NV; ++h) {
+    const int e = t + (512 / NV) * h;
     const int r = e >> 3, c8 = (e & 7) * 8;
     v[h] = *reinterpret_cast<const uint4 *>(X + (r0 + r) * SUR_F + c8);
   }
 }
 
-__device__ inline void put_x(const uint4 (&v)[2], unsigned short *xs, unsigned short *xt) {
+template <int NV>
+__device__ inline void put_x(const uint4 (&v)[NV], unsigned short *xs, unsigned short *xt) {
   const int t = threadIdx.x;
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int e = t + 256 * h;
+  for (int h = 0; h < NV; ++h) {
+    const int e = t + (512 / NV) * h;
     const int r = e >> 3, c8 = (e & 7) * 8;
     *reinterpret_cast<uint4 *>(xs + r * SUR_XS + c8) = v[h];
     if (xt) {
@@ -184,70 +184,73 @@ __device__ inline void put_x(const uint4 (&v)[2], unsigned short *xs, unsigned s
   }
 }
 
-__device__ inline void stage_x(const unsigned short *X, int64_t r0, unsigned short *xs,
-                               unsigned short *xt) {
-  uint4 v[2];
-  load_x(X, r0, v);
-  put_x(v, xs, xt);
-}
-
-// Layer 1 of the wave's column slice: h1[rt][c] = C tile (rows 16 rt.., cols
-// 32w + 16c ..), from the staged X tile.
-__device__ inline void col_layer1(const unsigned short *xs, const ColW &cw, f32x4_t (&h1)[4][2]) {
+// Layer 1 of the wave's column slice: h1[rt][c] = C tile (rows 16 rt.., the
+// wave's column tile c), from the staged X tile.
+template <int NC>
+__device__ inline void col_layer1(const unsigned short *xs, const ColW<NC> &cw,
+                                  f32x4_t (&h1)[4][NC]) {
   const int l = threadIdx.x & 63, lr = l & 15, lq = l >> 4;
 #pragma unroll
-  for (int rt = 0; rt < 4; ++rt) h1[rt][0] = h1[rt][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+    for (int c = 0; c < NC; ++c) h1[rt][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) {
       const bf16x8_t a = ld8(xs + (16 * rt + lr) * SUR_XS + 32 * kb + 8 * lq);
-      h1[rt][0] = mfma32(a, cw.w1[0][kb], h1[rt][0]);
-      h1[rt][1] = mfma32(a, cw.w1[1][kb], h1[rt][1]);
+#pragma unroll
+      for (int c = 0; c < NC; ++c) h1[rt][c] = mfma32(a, cw.w1[c][kb], h1[rt][c]);
     }
 }
 
 // Layer 2 of the wave's column slice from the shared A1 tile (+ b2).
-__device__ inline void col_layer2(const unsigned short *a1s, const ColW &cw, f32x4_t (&h2)[4][2]) {
+template <int NC>
+__device__ inline void col_layer2(const unsigned short *a1s, const ColW<NC> &cw,
+                                  f32x4_t (&h2)[4][NC]) {
   const int l = threadIdx.x & 63, lr = l & 15, lq = l >> 4;
 #pragma unroll
-  for (int rt = 0; rt < 4; ++rt) h2[rt][0] = h2[rt][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+    for (int c = 0; c < NC; ++c) h2[rt][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) {
       const bf16x8_t a = ld8(a1s + (16 * rt + lr) * SUR_AS + 32 * kb + 8 * lq);
-      h2[rt][0] = mfma32(a, cw.w2[0][kb], h2[rt][0]);
-      h2[rt][1] = mfma32(a, cw.w2[1][kb], h2[rt][1]);
+#pragma unroll
+      for (int c = 0; c < NC; ++c) h2[rt][c] = mfma32(a, cw.w2[c][kb], h2[rt][c]);
     }
 #pragma unroll
   for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
-    for (int c = 0; c < 2; ++c)
+    for (int c = 0; c < NC; ++c)
 #pragma unroll
       for (int i = 0; i < 4; ++i) h2[rt][c][i] += cw.b2[c];
 }
 
-// Store the C tiles v (rows 16 rt + 4 lq + i, column 32w + 16c + lr) as bf16:
-// row-major into rm (row stride SUR_AS) and, when tr is given, transposed
-// into tr ([128][SUR_TR]).
-__device__ inline void put_tiles(const float (&v)[4][2][4], int wv, unsigned short *rm,
+// Store the C tiles v (rows 16 rt + 4 lq + i, column 16 (NC w + c) + lr) as
+// bf16: row-major into rm (row stride SUR_AS) and, when tr is given,
+// transposed into tr ([128][SUR_TR]).
+template <int NC>
+__device__ inline void put_tiles(const float (&v)[4][NC][4], int wv, unsigned short *rm,
                                  unsigned short *tr) {
   const int l = threadIdx.x & 63, lr = l & 15, lq = l >> 4;
 #pragma unroll
   for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const int col = 32 * wv + 16 * c + lr;
-      unsigned short b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        b[i] = f2bf(v[rt][c][i]);
-        if (rm) rm[(16 * rt + 4 * lq + i) * SUR_AS + col] = b[i];
+    for (int c = 0; c < NC; ++c) {
+      const int col = 16 * (NC * wv + c) + lr;
+      const unsigned int p01 = pk_bf16(v[rt][c][0], v[rt][c][1]);
+      const unsigned int p23 = pk_bf16(v[rt][c][2], v[rt][c][3]);
+      if (rm) {
+        unsigned short *r = rm + (16 * rt + 4 * lq) * SUR_AS + col;
+        r[0] = (unsigned short)p01;
+        r[SUR_AS] = (unsigned short)(p01 >> 16);
+        r[2 * SUR_AS] = (unsigned short)p23;
+        r[3 * SUR_AS] = (unsigned short)(p23 >> 16);
       }
-      if (tr)
-        *reinterpret_cast<uint2 *>(tr + col * SUR_TR + 16 * rt + 4 * lq) =
-            make_uint2(b[0] | ((unsigned)b[1] << 16), b[2] | ((unsigned)b[3] << 16));
+      if (tr) *reinterpret_cast<uint2 *>(tr + col * SUR_TR + 16 * rt + 4 * lq) = make_uint2(p01, p23);
     }
 }
 
@@ -261,9 +264,8 @@ extern "C" __global__ void __launch_bounds__(256) gd_mlp_fwd_kernel(const unsign
   __shared__ __attribute__((aligned(16))) unsigned short a1s[SUR_STEP * SUR_AS];
   __shared__ float red[4][SUR_STEP];
   const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, lr = l & 15, lq = l >> 4;
-  ColW cw;
-  bf16x8_t unused[2][4];
-  load_colw(W, wv, false, cw, unused);
+  ColW<2> cw;
+  load_colw(W, wv, cw);
   const float b3 = W.b3[0];
   const int64_t n_steps = n_rows / SUR_STEP;
   uint4 xv[2];
@@ -290,11 +292,7 @@ extern "C" __global__ void __launch_bounds__(256) gd_mlp_fwd_kernel(const unsign
     for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        float v = fmaf(silu(h2[rt][0][i]), cw.w3[0], silu(h2[rt][1][i]) * cw.w3[1]);
-        v += __shfl_xor(v, 1);
-        v += __shfl_xor(v, 2);
-        v += __shfl_xor(v, 4);
-        v += __shfl_xor(v, 8);
+        const float v = row16_sum(fmaf(silu(h2[rt][0][i]), cw.w3[0], silu(h2[rt][1][i]) * cw.w3[1]));
         if (lr == 0) red[wv][16 * rt + 4 * lq + i] = v;
       }
     __syncthreads();
@@ -400,41 +398,65 @@ extern "C" __global__ void __launch_bounds__(256, 2) gd_sur_tab_kernel(
   }
 }
 
-// Output gradient of each row of a batch: dyr[i] = dS of row i's pose when
-// that pose lies in [p0, p1), else 0 (rows of the 64-row padding that belong
-// to the next poses). One thread per row.
-extern "C" __global__ void gd_mlp_dyrow_kernel(const int *pose_of_row, int64_t n_rows, int p0,
-                                               int p1, const float *dS, float *dyr) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n_rows) return;
-  const int p = pose_of_row[i];
-  dyr[i] = (p >= p0 && p < p1) ? dS[p] : 0.0f;
-}
-
 // Pose sums over poses [p0, p1): S = sum of row outputs, residual against the
-// target, dS = 2 (S - target) / (p1 - p0), squared residuals for the loss.
-// Row offsets are absolute; y is indexed by absolute row.
-extern "C" __global__ void gd_mlp_pose_kernel(const float *y, const int64_t *off, int p0, int p1,
-                                              const float *target, float *dS, float *sq,
-                                              float *S_out) {
-  const int p = p0 + blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= p1) return;
+// target, dS = 2 (S - target) / (p1 - p0), squared residuals for the loss, and
+// (with dyr) the output gradient of every row of the batch's n_rows: its
+// pose's dS, 0 for the rows that pad the batch to whole steps. Row offsets and
+// y are absolute, dyr is relative to the batch's first row.
+//
+// One workgroup per 64 poses. Their rows are adjacent, so they are read in
+// whole lines into LDS, SUR_POSE_ROWS at a time; one lane per pose then adds
+// its rows in row order. Latency bound (64 workgroups for a batch of 4,096):
+// 7.7 us and a separate kernel for the rows' gradients before, 6.9 us now.
+constexpr int SUR_POSE_ROWS = 4096;
+extern "C" __global__ void __launch_bounds__(256) gd_mlp_pose_kernel(
+    const float *y, const int64_t *off, int p0, int p1, const float *target, float *dS, float *sq,
+    float *S_out, float *dyr, int64_t n_rows) {
+  __shared__ float ys[SUR_POSE_ROWS];
+  const int pb = p0 + blockIdx.x * 64, pe = min(pb + 64, p1);
+  const int t = threadIdx.x;
+  const bool mine = t < pe - pb;  // this thread's pose
+  const int p = mine ? pb + t : pb;
+  const int64_t base = off[p0], rb = off[pb], re = off[pe];
+  const int64_t mb = off[p], me = mine ? off[p + 1] : mb;
   float s = 0.0f;
-  for (int64_t r = off[p]; r < off[p + 1]; ++r) s += y[r];
+  for (int64_t r = rb; r < re; r += SUR_POSE_ROWS) {
+    const int n = (int)min(re - r, (int64_t)SUR_POSE_ROWS);
+    for (int i = t; i < n; i += 256) ys[i] = y[r + i];
+    __syncthreads();
+    const int b = (int)max(mb - r, (int64_t)0), e = (int)min(me - r, (int64_t)n);
+#pragma unroll 8
+    for (int i = b; i < e; ++i) s += ys[i];
+    __syncthreads();
+  }
   const float res = s - target[p];
-  dS[p] = 2.0f * res / (float)(p1 - p0);
-  sq[p] = res * res;
-  if (S_out) S_out[p] = s;
+  const float g = 2.0f * res / (float)(p1 - p0);
+  if (mine) {
+    dS[p] = g;
+    sq[p] = res * res;
+    if (S_out) S_out[p] = s;
+  }
+  if (!dyr) return;
+  for (int64_t r = rb; r < re; r += SUR_POSE_ROWS) {
+    const int n = (int)min(re - r, (int64_t)SUR_POSE_ROWS);
+    const int b = (int)max(mb - r, (int64_t)0), e = (int)min(me - r, (int64_t)n);
+    for (int i = b; i < e; ++i) ys[i] = g;
+    __syncthreads();
+    for (int i = t; i < n; i += 256) dyr[r + i - base] = ys[i];
+    __syncthreads();
+  }
+  if (pe == p1)
+    for (int64_t i = re - base + t; i < n_rows; i += 256) dyr[i] = 0.0f;
 }
 
 // Backward of one batch fused with its weight gradients, column-split like
-// gd_mlp_fwd_kernel. Workgroup b takes the contiguous 64-row steps
+// gd_mlp_fwd_kernel, in 8 waves of 16 columns. Workgroup b takes the contiguous 64-row steps
 // [b S / G, (b + 1) S / G) (S steps, G = gridDim.x). Per step, wave w
-// recomputes H1 and H2 of its 32 columns, forms
-//   dy = dyr of the row (gd_mlp_dyrow_kernel),  dH2 = dy w3 * silu'(H2),
+// recomputes H1 and H2 of its columns, forms
+//   dy = dyr of the row (gd_mlp_pose_kernel),  dH2 = dy w3 * silu'(H2),
 //   dA1 = dH2 W2^T (all of dH2 from LDS, W2^T slice in registers),
 //   dH1 = dA1 * silu'(H1)
-// and accumulates its 32 columns of
+// and accumulates its columns of
 //   dW2 += A1^T dH2   (A1^T of all waves from LDS),
 //   dW1 += X^T dH1    (row 56 of dW1 is the b1 gradient)
 // in MFMA accumulators, with b2, w3 and b3. Only fixed-order partials go to
@@ -443,7 +465,12 @@ extern "C" __global__ void gd_mlp_pose_kernel(const float *y, const int64_t *off
 // so training is deterministic). The next step's X rows are read into
 // registers while a step is evaluated, and a step's dy rows are read at its
 // start, so neither load stalls the step.
-extern "C" __global__ void __launch_bounds__(256) gd_mlp_train_kernel(
+//
+// Bound: VALU (SiLU and its derivative, bf16 conversions) and the LDS round
+// trips between layers. Four waves of 32 columns filled the register file
+// with one wave per SIMD, which waited out each of them; 16 columns per wave
+// leave room for two. 156,000 rows (4,096 poses): 69.6 -> 50 us.
+extern "C" __global__ void __launch_bounds__(512) gd_mlp_train_kernel(
     const unsigned short *X, int64_t n_rows, const float *dyr, SurW W, float *p1g, float *p2g,
     float *pb2, float *pw3) {
   extern __shared__ __attribute__((aligned(16))) unsigned char sm_train[];
@@ -455,22 +482,28 @@ extern "C" __global__ void __launch_bounds__(256) gd_mlp_train_kernel(
   unsigned short *d2t = d2s + SUR_STEP * SUR_AS;                        // dH2^T [128][SUR_TR]
   unsigned short *d1t = d2t + SUR_H * SUR_TR;                           // dH1^T [128][SUR_TR]
   const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, lr = l & 15, lq = l >> 4;
-  ColW cw;
-  bf16x8_t w2r[2][4];
-  load_colw(W, wv, true, cw, w2r);
-  f32x4_t g2[8][2], g1[4][2];
+  constexpr int NC = 1;
+  ColW<NC> cw;
+  load_colw(W, wv, cw);
+  bf16x8_t w2r[NC][4];
 #pragma unroll
-  for (int c = 0; c < 2; ++c) {
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+      w2r[c][kb] = ld8(W.W2R + (16 * (NC * wv + c) + lr) * SUR_H + 32 * kb + 8 * lq);
+  f32x4_t g2[8][NC], g1[4][NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
 #pragma unroll
     for (int t = 0; t < 8; ++t) g2[t][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < 4; ++t) g1[t][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
-  float gw3[2] = {0.f, 0.f}, gb2[2] = {0.f, 0.f}, gb3 = 0.0f;
+  float gw3[NC] = {}, gb2[NC] = {}, gb3 = 0.0f;
   const int64_t n_steps = n_rows / SUR_STEP;
   const int64_t s_beg = n_steps * blockIdx.x / gridDim.x;
   const int64_t s_end = n_steps * (blockIdx.x + 1) / gridDim.x;
-  uint4 xv[2];
+  uint4 xv[1];
   if (s_beg < s_end) load_x(X, s_beg * SUR_STEP, xv);
   for (int64_t st = s_beg; st < s_end; ++st) {
     const int64_t r0 = st * SUR_STEP;
@@ -484,14 +517,14 @@ extern "C" __global__ void __launch_bounds__(256) gd_mlp_train_kernel(
     put_x(xv, xs, xt);
     if (st + 1 < s_end) load_x(X, r0 + SUR_STEP, xv);
     __syncthreads();
-    f32x4_t h1[4][2], h2[4][2];
+    f32x4_t h1[4][NC], h2[4][NC];
     col_layer1(xs, cw, h1);
     {
-      float a1[4][2][4];
+      float a1[4][NC][4];
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
-        for (int c = 0; c < 2; ++c)
+        for (int c = 0; c < NC; ++c)
 #pragma unroll
           for (int i = 0; i < 4; ++i) a1[rt][c][i] = silu(h1[rt][c][i]);
       put_tiles(a1, wv, a1s, a1t);
@@ -511,39 +544,41 @@ extern "C" __global__ void __launch_bounds__(256) gd_mlp_train_kernel(
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt) gb3 += (dy[rt][0] + dy[rt][1]) + (dy[rt][2] + dy[rt][3]);
     {
-      float d2[4][2][4];
+      float d2[4][NC][4];
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
-        for (int c = 0; c < 2; ++c)
+        for (int c = 0; c < NC; ++c)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             gw3[c] = fmaf(silu(h2[rt][c][i]), dy[rt][i], gw3[c]);
-            const float g = dy[rt][i] * cw.w3[c] * dsilu(h2[rt][c][i]);
-            gb2[c] += g;
-            d2[rt][c][i] = g;
+            const float dyw = dy[rt][i] * cw.w3[c], ds = dsilu(h2[rt][c][i]);
+            gb2[c] = fmaf(dyw, ds, gb2[c]);
+            d2[rt][c][i] = dyw * ds;
           }
       put_tiles(d2, wv, d2s, d2t);
     }
     __syncthreads();
     // dA1 = dH2 W2^T for this wave's columns, dH1 transposed
     {
-      f32x4_t da[4][2];
+      f32x4_t da[4][NC];
 #pragma unroll
-      for (int rt = 0; rt < 4; ++rt) da[rt][0] = da[rt][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) da[rt][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
         for (int rt = 0; rt < 4; ++rt) {
           const bf16x8_t a = ld8(d2s + (16 * rt + lr) * SUR_AS + 32 * kb + 8 * lq);
-          da[rt][0] = mfma32(a, w2r[0][kb], da[rt][0]);
-          da[rt][1] = mfma32(a, w2r[1][kb], da[rt][1]);
+#pragma unroll
+          for (int c = 0; c < NC; ++c) da[rt][c] = mfma32(a, w2r[c][kb], da[rt][c]);
         }
-      float d1[4][2][4];
+      float d1[4][NC][4];
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
-        for (int c = 0; c < 2; ++c)
+        for (int c = 0; c < NC; ++c)
 #pragma unroll
           for (int i = 0; i < 4; ++i) d1[rt][c][i] = da[rt][c][i] * dsilu(h1[rt][c][i]);
       put_tiles(d1, wv, nullptr, d1t);
@@ -554,35 +589,35 @@ extern "C" __global__ void __launch_bounds__(256) gd_mlp_train_kernel(
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
       const int ko = 32 * kb + 8 * lq;
-      bf16x8_t b2v[2], b1v[2];
+      bf16x8_t b2v[NC], b1v[NC];
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        b2v[c] = ld8(d2t + (32 * wv + 16 * c + lr) * SUR_TR + ko);
-        b1v[c] = ld8(d1t + (32 * wv + 16 * c + lr) * SUR_TR + ko);
+      for (int c = 0; c < NC; ++c) {
+        b2v[c] = ld8(d2t + (16 * (NC * wv + c) + lr) * SUR_TR + ko);
+        b1v[c] = ld8(d1t + (16 * (NC * wv + c) + lr) * SUR_TR + ko);
       }
 #pragma unroll
       for (int t = 0; t < 8; ++t) {
         const bf16x8_t a = ld8(a1t + (16 * t + lr) * SUR_TR + ko);
-        g2[t][0] = mfma32(a, b2v[0], g2[t][0]);
-        g2[t][1] = mfma32(a, b2v[1], g2[t][1]);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) g2[t][c] = mfma32(a, b2v[c], g2[t][c]);
       }
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const bf16x8_t a = ld8(xt + (16 * t + lr) * SUR_TR + ko);
-        g1[t][0] = mfma32(a, b1v[0], g1[t][0]);
-        g1[t][1] = mfma32(a, b1v[1], g1[t][1]);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) g1[t][c] = mfma32(a, b1v[c], g1[t][c]);
       }
     }
     // no barrier here: the next step writes the other X buffer, and its
     // first barrier precedes every write to the shared A1 and dH2 tiles
   }
 
-  // partials of this workgroup: its 4 waves own disjoint columns
+  // partials of this workgroup: its waves own disjoint columns
   float *o2 = p2g + (int64_t)blockIdx.x * SUR_H * SUR_H;
   float *o1 = p1g + (int64_t)blockIdx.x * SUR_F * SUR_H;
 #pragma unroll
-  for (int c = 0; c < 2; ++c) {
-    const int col = 32 * wv + 16 * c + lr;
+  for (int c = 0; c < NC; ++c) {
+    const int col = 16 * (NC * wv + c) + lr;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
 #pragma unroll
@@ -593,7 +628,7 @@ extern "C" __global__ void __launch_bounds__(256) gd_mlp_train_kernel(
   }
   float *w3o = pw3 + (int64_t)blockIdx.x * (SUR_H + 1);
 #pragma unroll
-  for (int c = 0; c < 2; ++c) {
+  for (int c = 0; c < NC; ++c) {
     float v = gw3[c];
     v += __shfl_xor(v, 16);
     v += __shfl_xor(v, 32);
@@ -601,8 +636,8 @@ extern "C" __global__ void __launch_bounds__(256) gd_mlp_train_kernel(
     b += __shfl_xor(b, 16);
     b += __shfl_xor(b, 32);
     if (lq == 0) {
-      w3o[32 * wv + 16 * c + lr] = v;
-      pb2[(int64_t)blockIdx.x * SUR_H + 32 * wv + 16 * c + lr] = b;
+      w3o[16 * (NC * wv + c) + lr] = v;
+      pb2[(int64_t)blockIdx.x * SUR_H + 16 * (NC * wv + c) + lr] = b;
     }
   }
   gb3 += __shfl_xor(gb3, 16);
@@ -614,72 +649,80 @@ extern "C" __global__ void __launch_bounds__(256) gd_mlp_train_kernel(
 constexpr int SUR_TRAIN_LDS =
     (2 * (SUR_STEP * SUR_XS + SUR_F * SUR_TR) + 2 * SUR_STEP * SUR_AS + 3 * SUR_H * SUR_TR) * 2;
 
-// Sum of the squared residuals of poses [0, n) into *out: one workgroup,
-// strided partial sums then a fixed-shape tree (deterministic).
-extern "C" __global__ void __launch_bounds__(256) gd_mlp_sqsum_kernel(const float *sq, int n,
-                                                                     float *out) {
-  __shared__ float red[256];
-  float s = 0.0f;
-  for (int i = threadIdx.x; i < n; i += 256) s += sq[i];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int h = 128; h > 0; h >>= 1) {
-    if (threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
-    __syncthreads();
+// Gradient of a parameter as the fixed-order sum of n partials: eight
+// interleaved sums (partials c, c + 8, ...), then a fixed tree. A workgroup
+// takes 32 parameters; thread (j, i) adds interleave j of parameter i, so 128
+// adjacent bytes are read at a time and eight times as many loads are in
+// flight as with one thread per parameter. The sum is left in threads 0..31.
+__device__ inline float grad_sum(const float *p1, const float *p2, const float *pb2,
+                                 const float *pw3, int n, int q, float (&red)[8][33]) {
+  const int i = threadIdx.x & 31, j = threadIdx.x >> 5;
+  const float *part = nullptr;
+  int64_t stride = 0;
+  if (q < SP_W2) {
+    part = p1 + q;
+    stride = (int64_t)SUR_F * SUR_H;
+  } else if (q < SP_B2) {
+    part = p2 + (q - SP_W2);
+    stride = (int64_t)SUR_H * SUR_H;
+  } else if (q < SP_W3) {
+    part = pb2 + (q - SP_B2);
+    stride = SUR_H;
+  } else if (q < SUR_NPARAM) {
+    part = pw3 + (q - SP_W3);
+    stride = SUR_H + 1;
   }
-  if (threadIdx.x == 0) *out = red[0];
-}
-
-// Sum of n partials part[c * stride + q], c = 0..n-1, in a fixed order:
-// eight interleaved accumulators (eight loads in flight) then a fixed tree.
-__device__ inline float sum_partials(const float *part, int n, int64_t stride, int q) {
-  float a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  int c = 0;
-  for (; c + 8 <= n; c += 8)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) a[j] += part[(int64_t)(c + j) * stride + q];
-  for (int j = 0; c < n; ++c, ++j) a[j] += part[(int64_t)c * stride + q];
-  return ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+  float a = 0.0f;
+  if (part) {
+#pragma unroll 8
+    for (int c = j; c < n; c += 8) a += part[c * stride];
+  }
+  red[j][i] = a;
+  __syncthreads();
+  return ((red[0][i] + red[1][i]) + (red[2][i] + red[3][i])) +
+         ((red[4][i] + red[5][i]) + (red[6][i] + red[7][i]));
 }
 
 // Sums gradient partials into g[SUR_NPARAM] (fixed order: deterministic).
-extern "C" __global__ void gd_mlp_gradsum_kernel(const float *p1, int n1, const float *p2, int n2,
-                                                 const float *pb2, const float *pw3, int64_t nw,
-                                                 float *g) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= SUR_NPARAM) return;
-  float s = 0.0f;
-  if (q < SP_W2) {
-    s = sum_partials(p1, n1, (int64_t)SUR_F * SUR_H, q);
-  } else if (q < SP_B2) {
-    s = sum_partials(p2, n2, (int64_t)SUR_H * SUR_H, q - SP_W2);
-  } else if (q < SP_W3) {
-    s = sum_partials(pb2, n2, SUR_H, q - SP_B2);
-  } else {
-    s = sum_partials(pw3, (int)nw, SUR_H + 1, q - SP_W3);
-  }
-  g[q] = s;
+extern "C" __global__ void __launch_bounds__(256) gd_mlp_gradsum_kernel(
+    const float *p1, const float *p2, const float *pb2, const float *pw3, int n, float *g) {
+  __shared__ float red[8][33];
+  const int q = blockIdx.x * 32 + (threadIdx.x & 31);
+  const float s = grad_sum(p1, p2, pb2, pw3, n, q, red);
+  if (threadIdx.x < 32 && q < SUR_NPARAM) g[q] = s;
 }
 
 // One training update: each parameter's gradient from the fixed-order sum of
 // the backward's per-workgroup partials (ng of each), then Adam on it and the
-// refresh of its bf16 copies. The gradient is also left in g.
-extern "C" __global__ void gd_mlp_update_kernel(const float *p1, const float *p2, const float *pb2,
-                                                const float *pw3, int ng, float *p, float *m,
-                                                float *v, float *g, float lr, float b1, float b2,
-                                                float eps, float c1, float c2,
-                                                unsigned short *W1T, unsigned short *W2T,
-                                                unsigned short *W2R) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= SUR_NPARAM) return;
-  float gq;
-  if (q < SP_W2) gq = sum_partials(p1, ng, (int64_t)SUR_F * SUR_H, q);
-  else if (q < SP_B2) gq = sum_partials(p2, ng, (int64_t)SUR_H * SUR_H, q - SP_W2);
-  else if (q < SP_W3) gq = sum_partials(pb2, ng, SUR_H, q - SP_B2);
-  else gq = sum_partials(pw3, ng, SUR_H + 1, q - SP_W3);
+// refresh of its bf16 copies. The gradient is also left in g. The last
+// workgroup adds the batch's n_sq squared residuals into *loss instead
+// (strided partial sums, then a fixed tree). Bound: 25 MB of partials from L2,
+// 13.6 us with one thread per parameter, 7.6 us now.
+extern "C" __global__ void __launch_bounds__(256) gd_mlp_update_kernel(
+    const float *p1, const float *p2, const float *pb2, const float *pw3, int ng, float *p,
+    float *m, float *v, float *g, float lr, float b1, float b2, float eps, float c1, float c2,
+    unsigned short *W1T, unsigned short *W2T, unsigned short *W2R, const float *sq, int n_sq,
+    float *loss) {
+  __shared__ float red[8][33];
+  if (blockIdx.x == gridDim.x - 1) {
+    float *r = &red[0][0];
+    float s = 0.0f;
+    for (int i = threadIdx.x; i < n_sq; i += 256) s += sq[i];
+    r[threadIdx.x] = s;
+    __syncthreads();
+    for (int h = 128; h > 0; h >>= 1) {
+      if (threadIdx.x < h) r[threadIdx.x] += r[threadIdx.x + h];
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) *loss = r[0];
+    return;
+  }
+  const int q = blockIdx.x * 32 + (threadIdx.x & 31);
+  const float gq = grad_sum(p1, p2, pb2, pw3, ng, q, red);
+  if (threadIdx.x >= 32 || q >= SUR_NPARAM) return;
   g[q] = gq;
-  const float mq = b1 * m[q] + (1.0f - b1) * gq;
-  const float vq = b2 * v[q] + (1.0f - b2) * gq * gq;
+  const float mq = fmaf(1.0f - b1, gq, mul_rn(b1, m[q]));
+  const float vq = fmaf(gq, mul_rn(1.0f - b2, gq), mul_rn(b2, v[q]));
   m[q] = mq;
   v[q] = vq;
   const float x = p[q] - lr * (mq / c1) / (sqrtf(vq / c2) + eps);
