@@ -20,11 +20,13 @@
 //
 // Layout in HBM: features SoA [9][n] (coalesced per term), membership [n],
 // per group: centers [k][9] float, sums [k][9] int64, counts [k], pass count,
-// change count and a done flag. A pass is two launches over all groups at
-// once: assign (one workgroup per tile of 1,024 objects; centers and partial
-// sums in LDS, flushed with 64-bit atomics) and update (one workgroup per
-// group). The host checks the number of live groups every 8 passes; finished
-// groups cost one early return per tile.
+// change count and the pass that ended it. A pass is two launches over all
+// groups at once: assign (workgroups of a few waves over tiles of a group's
+// objects) and update (the centers). The sums live on between passes: an object
+// that changes cluster takes its terms from one sum to the other, which is
+// exact in integers, so a pass adds only what moved. The host checks the
+// number of live groups every 8 passes; finished groups cost one early return
+// per tile.
 
 #include <hip/hip_runtime.h>
 
@@ -39,7 +41,6 @@
 namespace gd {
 
 constexpr int KM_DIM = GD_MAXWEI - 1;  // vdw .. dst
-constexpr int KM_TILE = 1024;
 constexpr int KM_MAX_K = 512;
 constexpr int KM_MAX_GROUP = 1 << 19;  // objects per group (fixed-point sum range)
 constexpr float KM_CLAMP = 134217728.0f;  // 2^27
@@ -54,7 +55,8 @@ struct KmArgs {
   float *cent;         // [n_groups][k][KM_DIM]
   long long *sum;      // [n_groups][k][KM_DIM]
   int *cnt;            // [n_groups][k]
-  int *delta, *done, *pass;  // [n_groups]
+  int *delta, *pass;         // [n_groups]
+  int *done;                 // [n_groups]: the pass that ended the group (-1: never run)
   int *active;
   unsigned long long *best;  // [n_groups][k]: (distance bits << 32) | member
   int *size;                 // [n_groups][k]
@@ -82,125 +84,169 @@ __host__ __device__ inline float km_dist2(const float *a, const float *b) {
   return s;
 }
 
+// One assignment pass. A workgroup of 4 waves takes 64 O (4 / S) objects of a
+// group, O per lane; S waves share the same objects and take k / S centers
+// each, then the lowest distance in center order wins (ties to the lower
+// index, as in one loop over all centers). The rule (km_run) gives every CU
+// several waves: S = 4 for a group of few objects and many centers (22,000
+// objects and 500 centers ran on 22 CUs before: 190 us a pass, 29 us now),
+// O = 2 only when the objects alone fill the chip many times, where two
+// objects share each center's scalar loads.
+//
 // The centers are read-only here and wave-uniform: passed as their own
 // restrict pointer they are fetched with scalar loads and feed the distance
-// arithmetic as scalar operands (no LDS traffic for them).
-__global__ void __launch_bounds__(256) gd_km_assign_kernel(KmArgs A,
-                                                           const float *__restrict__ cent) {
+// arithmetic as scalar operands. Bound: VALU, 22 instructions per object and
+// center.
+//
+// FIRST (the first pass with S = 1): every object is new, so the sums are
+// gathered in LDS and flushed once per workgroup. Later passes move the
+// objects that changed with global atomics (a few percent of them; adding all
+// objects anew took 10 LDS atomics per object and pass).
+template <int O, int S, bool FIRST>
+__global__ void __launch_bounds__(256) gd_km_assign_kernel(KmArgs A, const float *__restrict__ cent,
+                                                           int pass) {
   const int g = A.tile_g[blockIdx.x];
-  if (A.done[g]) return;
+  if (A.done[g] < pass) return;
   const int k = A.k;
   extern __shared__ __align__(16) unsigned char km_lds[];
-  long long *sum = (long long *)km_lds;  // [k][KM_DIM]
-  int *cnt = (int *)(sum + (size_t)k * KM_DIM);  // [k]
-  int *dlt = cnt + k;
+  long long *lsum = (long long *)km_lds;              // FIRST: [k][KM_DIM]
+  int *lcnt = (int *)(lsum + (size_t)k * KM_DIM);     // FIRST: [k]
+  __shared__ float pd[S > 1 ? 4 : 1][O][64];
+  __shared__ int pb[S > 1 ? 4 : 1][O][64];
+  if constexpr (FIRST) {
+    for (int j = threadIdx.x; j < k * KM_DIM; j += 256) lsum[j] = 0;
+    for (int c = threadIdx.x; c < k; c += 256) lcnt[c] = 0;
+    __syncthreads();
+  }
   const float *cen = cent + (size_t)g * k * KM_DIM;
-  for (int j = threadIdx.x; j < k * KM_DIM; j += blockDim.x) sum[j] = 0;
-  for (int c = threadIdx.x; c < k; c += blockDim.x) cnt[c] = 0;
-  if (threadIdx.x == 0) *dlt = 0;
-  __syncthreads();
   const int64_t base = A.off[g];
   const int n = (int)(A.off[g + 1] - base);
-  const int s0 = A.tile_s[blockIdx.x];
-  const int s1 = min(n, s0 + KM_TILE);
-  int changed = 0;
-  // two objects per lane share each center's scalar loads
-  const int stride = 2 * (int)blockDim.x;
-  for (int i0 = s0 + (int)threadIdx.x; i0 < s1; i0 += stride) {
-    const int i1 = i0 + (int)blockDim.x;
-    const bool has1 = i1 < s1;
-    float f0[KM_DIM], f1[KM_DIM];
+  const int l = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int part = wv % S, og = wv / S;
+  const int i0 = A.tile_s[blockIdx.x] + og * 64 * O + l;
+  float f[O][KM_DIM], dist[O];
+  int best[O];
+  bool has[O];
 #pragma unroll
-    for (int d = 0; d < KM_DIM; ++d) {
-      f0[d] = A.feat[(size_t)d * A.n_total + base + i0];
-      f1[d] = has1 ? A.feat[(size_t)d * A.n_total + base + i1] : f0[d];
-    }
-    int b0 = 0, b1 = 0;
-    float d0 = km_dist2(f0, cen), d1 = km_dist2(f1, cen);
-#pragma unroll 2
-    for (int c = 1; c < k; ++c) {
-      const float *cc = cen + (size_t)c * KM_DIM;
-      const float e0 = km_dist2(f0, cc), e1 = km_dist2(f1, cc);
-      if (e0 < d0) {
-        d0 = e0;
-        b0 = c;
-      }
-      if (e1 < d1) {
-        d1 = e1;
-        b1 = c;
-      }
-    }
-    for (int h = 0; h < 2; ++h) {
-      if (h == 1 && !has1) break;
-      const int i = h ? i1 : i0, bc = h ? b1 : b0;
-      const float *f = h ? f1 : f0;
-      int *m = A.memb + base + i;
-      if (*m != bc) {
-        changed += 1;
-        *m = bc;
-      }
+  for (int o = 0; o < O; ++o) {
+    has[o] = i0 + 64 * o < n;
+    const int64_t i = base + (has[o] ? i0 + 64 * o : 0);
 #pragma unroll
-      for (int d = 0; d < KM_DIM; ++d)
-        atomicAdd((unsigned long long *)&sum[bc * KM_DIM + d], (unsigned long long)km_fixed(f[d]));
-      atomicAdd(&cnt[bc], 1);
+    for (int d = 0; d < KM_DIM; ++d) f[o][d] = A.feat[(size_t)d * A.n_total + i];
+    // the first center is taken whatever its distance; later parts start from
+    // nothing
+    best[o] = part == 0 ? 0 : -1;
+    dist[o] = part == 0 ? km_dist2(f[o], cen) : __builtin_inff();
+  }
+  const int c1 = (k * (part + 1)) / S;
+#pragma unroll 4
+  for (int c = part == 0 ? 1 : (k * part) / S; c < c1; ++c) {
+    const float *cc = cen + (size_t)c * KM_DIM;
+#pragma unroll
+    for (int o = 0; o < O; ++o) {
+      const float e = km_dist2(f[o], cc);
+      if (e < dist[o]) {
+        dist[o] = e;
+        best[o] = c;
+      }
     }
   }
-  if (changed) atomicAdd(dlt, changed);
-  __syncthreads();
+  if constexpr (S > 1) {
+#pragma unroll
+    for (int o = 0; o < O; ++o) {
+      pd[wv][o][l] = dist[o];
+      pb[wv][o][l] = best[o];
+    }
+    __syncthreads();
+    if (part != 0) return;
+#pragma unroll
+    for (int o = 0; o < O; ++o)
+      for (int q = 1; q < S; ++q)
+        if (pd[wv + q][o][l] < dist[o]) {
+          dist[o] = pd[wv + q][o][l];
+          best[o] = pb[wv + q][o][l];
+        }
+  }
   long long *gs = A.sum + (size_t)g * k * KM_DIM;
   int *gn = A.cnt + (size_t)g * k;
-  for (int c = threadIdx.x; c < k; c += blockDim.x) {
-    if (!cnt[c]) continue;
-    atomicAdd(gn + c, cnt[c]);
-    for (int d = 0; d < KM_DIM; ++d)
-      if (sum[c * KM_DIM + d])
-        atomicAdd((unsigned long long *)&gs[c * KM_DIM + d], (unsigned long long)sum[c * KM_DIM + d]);
+  int changed = 0;
+#pragma unroll
+  for (int o = 0; o < O; ++o) {
+    int *m = A.memb + base + i0 + 64 * o;
+    const int old = has[o] ? *m : 0, now = best[o];
+    const bool move = has[o] && old != now;
+    changed += __popcll(__ballot(move));
+    if (!move) continue;
+    *m = now;
+    if constexpr (FIRST) {
+#pragma unroll
+      for (int d = 0; d < KM_DIM; ++d)
+        atomicAdd((unsigned long long *)&lsum[now * KM_DIM + d], (unsigned long long)km_fixed(f[o][d]));
+      atomicAdd(&lcnt[now], 1);
+    } else {
+#pragma unroll
+      for (int d = 0; d < KM_DIM; ++d) {
+        const unsigned long long v = (unsigned long long)km_fixed(f[o][d]);
+        atomicAdd((unsigned long long *)&gs[now * KM_DIM + d], v);
+        if (old >= 0) atomicAdd((unsigned long long *)&gs[old * KM_DIM + d], 0ull - v);
+      }
+      atomicAdd(&gn[now], 1);
+      if (old >= 0) atomicAdd(&gn[old], -1);
+    }
   }
-  if (threadIdx.x == 0 && *dlt) atomicAdd(A.delta + g, *dlt);
+  if (l == 0 && changed) atomicAdd(A.delta + g, changed);
+  if constexpr (FIRST) {
+    __syncthreads();
+    for (int c = threadIdx.x; c < k; c += 256) {
+      if (!lcnt[c]) continue;
+      atomicAdd(gn + c, lcnt[c]);
+      for (int d = 0; d < KM_DIM; ++d)
+        if (lsum[c * KM_DIM + d])
+          atomicAdd((unsigned long long *)&gs[c * KM_DIM + d],
+                    (unsigned long long)lsum[c * KM_DIM + d]);
+    }
+  }
 }
 
 __host__ __device__ inline float km_mean(long long s, int n) {
   return (float)((double)s / (double)n / 65536.0);
 }
 
-__global__ void __launch_bounds__(256) gd_km_update_kernel(KmArgs A) {
+// Centers of pass `pass` (256 terms per workgroup, grid.y of them per group)
+// and each group's end: the group that ends now still gets its centers, so
+// workgroups look for earlier ends only.
+__global__ void __launch_bounds__(256) gd_km_update_kernel(KmArgs A, int pass) {
   const int g = blockIdx.x;
-  if (A.done[g]) return;
+  if (A.done[g] < pass) return;
   const int k = A.k;
-  float *gc = A.cent + (size_t)g * k * KM_DIM;
-  long long *gs = A.sum + (size_t)g * k * KM_DIM;
-  int *gn = A.cnt + (size_t)g * k;
-  for (int j = threadIdx.x; j < k * KM_DIM; j += blockDim.x) {
-    const int n = gn[j / KM_DIM];
-    if (n > 0) gc[j] = km_mean(gs[j], n);
-    gs[j] = 0;
+  const int j = blockIdx.y * 256 + threadIdx.x;
+  if (j < k * KM_DIM) {
+    const int n = A.cnt[(size_t)g * k + j / KM_DIM];
+    const size_t q = (size_t)g * k * KM_DIM + j;
+    if (n > 0) A.cent[q] = km_mean(A.sum[q], n);
   }
-  __syncthreads();
-  for (int c = threadIdx.x; c < k; c += blockDim.x) gn[c] = 0;
-  if (threadIdx.x == 0) {
+  if (j == 0) {
     const int n = (int)(A.off[g + 1] - A.off[g]);
     const float frac = (float)A.delta[g] / (float)n;
     A.delta[g] = 0;
-    const int p = A.pass[g] + 1;
-    A.pass[g] = p;
-    if (!(frac > A.threshold) || p >= A.max_pass) A.done[g] = 1;
+    A.pass[g] = pass + 1;
+    if (!(frac > A.threshold) || pass + 1 >= A.max_pass) A.done[g] = pass;
     else atomicAdd(A.active, 1);
   }
 }
 
-__global__ void __launch_bounds__(256) gd_km_medoid_kernel(KmArgs A) {
+// Per cluster, the member with the smallest (distance bits, index). One thread
+// per object of a tile of `tile` objects.
+__global__ void __launch_bounds__(256) gd_km_medoid_kernel(KmArgs A, int tile) {
   const int g = A.tile_g[blockIdx.x];
   const int k = A.k;
-  extern __shared__ __align__(16) unsigned char km_lds[];
-  float *cen = (float *)km_lds;
-  const float *gc = A.cent + (size_t)g * k * KM_DIM;
-  for (int j = threadIdx.x; j < k * KM_DIM; j += blockDim.x) cen[j] = gc[j];
-  __syncthreads();
+  const float *cen = A.cent + (size_t)g * k * KM_DIM;
   const int64_t base = A.off[g];
   const int n = (int)(A.off[g + 1] - base);
   const int s0 = A.tile_s[blockIdx.x];
-  const int s1 = min(n, s0 + KM_TILE);
-  for (int i = s0 + (int)threadIdx.x; i < s1; i += blockDim.x) {
+  const int s1 = min(n, s0 + tile);
+  for (int i = s0 + (int)threadIdx.x; i < s1; i += 256) {
     const int c = A.memb[base + i];
     if (c < 0 || c >= k) continue;
     float f[KM_DIM];
@@ -293,8 +339,9 @@ gd_status km_run(gd_ctx *ctx, int n_groups, const int64_t *off, const float *soa
   // groups with fewer than k objects: every object is its own medoid
   std::vector<int> tile_g, tile_s;
   std::vector<float> cent((size_t)n_groups * k * KM_DIM, 0.0f);
-  std::vector<int> done(n_groups, 1), init(k);
+  std::vector<int> done(n_groups, -1), init(k);
   std::vector<int> perm;
+  int64_t waves = 0;
   for (int g = 0; g < n_groups; ++g) {
     const int n = (int)(off[g + 1] - off[g]);
     if (passes) passes[g] = 0;
@@ -305,12 +352,23 @@ gd_status km_run(gd_ctx *ctx, int n_groups, const int64_t *off, const float *soa
       }
       continue;
     }
-    done[g] = 0;
+    done[g] = INT32_MAX;
+    waves += (n + 63) / 64;
     km_init_indices(n, k, g, level, seed, perm, init.data());
     for (int c = 0; c < k; ++c)
       for (int d = 0; d < KM_DIM; ++d)
         cent[((size_t)g * k + c) * KM_DIM + d] = soa_in[(size_t)d * n_total + off[g] + init[c]];
-    for (int s = 0; s < n; s += KM_TILE) {
+  }
+  // objects per lane and waves per object set (see the kernel): two objects per
+  // lane from 32 waves of objects per CU on, centers split four ways below two
+  // waves per CU (and not for a handful of centers)
+  const int o_lane = waves >= (int64_t)32 * ctx->n_cu ? 2 : 1;
+  const int c_split = waves < (int64_t)2 * ctx->n_cu && k >= 16 ? 4 : 1;
+  const int tile = 64 * o_lane * (4 / c_split);
+  for (int g = 0; g < n_groups; ++g) {
+    if (done[g] < 0) continue;
+    const int n = (int)(off[g + 1] - off[g]);
+    for (int s = 0; s < n; s += tile) {
       tile_g.push_back(g);
       tile_s.push_back(s);
     }
@@ -371,28 +429,39 @@ gd_status km_run(gd_ctx *ctx, int n_groups, const int64_t *off, const float *soa
   A.k = k;
   A.threshold = threshold;
   A.max_pass = max_pass;
-  const size_t lds_assign = (size_t)k * KM_DIM * 8 + (size_t)k * 4 + 16;
-  const size_t lds_medoid = (size_t)k * KM_DIM * 4;
-  HIPCHK(hipFuncSetAttribute((const void *)gd_km_assign_kernel,
-                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_assign));
+  // LDS sums of the first pass with unsplit centers
+  const size_t lds_first = (size_t)k * KM_DIM * 8 + (size_t)k * 4 + 16;
+  void (*assign)(KmArgs, const float *, int) = nullptr, (*first)(KmArgs, const float *, int) = nullptr;
+  if (c_split == 4) {
+    assign = first = gd_km_assign_kernel<1, 4, false>;
+  } else if (o_lane == 2) {
+    assign = gd_km_assign_kernel<2, 1, false>;
+    first = gd_km_assign_kernel<2, 1, true>;
+  } else {
+    assign = gd_km_assign_kernel<1, 1, false>;
+    first = gd_km_assign_kernel<1, 1, true>;
+  }
+  if (first != assign)
+    HIPCHK(hipFuncSetAttribute((const void *)first, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)lds_first));
+  const dim3 upd((unsigned)n_groups, (unsigned)((k * KM_DIM + 255) / 256));
   HIPCHK(hipEventRecord(ctx->ev0, st));
   for (int p = 0; p < max_pass;) {
     const int batch = std::min(8, max_pass - p);
-    for (int b = 0; b < batch; ++b) {
+    for (int b = 0; b < batch; ++b, ++p) {
       if (b == batch - 1) HIPCHK(hipMemsetAsync(A.active, 0, 4, st));
-      hipLaunchKernelGGL(gd_km_assign_kernel, dim3(n_tiles), dim3(256), lds_assign, st, A,
-                         (const float *)A.cent);
+      hipLaunchKernelGGL(p == 0 ? first : assign, dim3(n_tiles), dim3(256),
+                         p == 0 && first != assign ? lds_first : 0, st, A, (const float *)A.cent, p);
       HIPCHK(hipGetLastError());
-      hipLaunchKernelGGL(gd_km_update_kernel, dim3(n_groups), dim3(256), 0, st, A);
+      hipLaunchKernelGGL(gd_km_update_kernel, upd, dim3(256), 0, st, A, p);
       HIPCHK(hipGetLastError());
     }
-    p += batch;
     int live = 0;
     HIPCHK(hipMemcpyAsync(&live, A.active, 4, hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
     if (live == 0) break;
   }
-  hipLaunchKernelGGL(gd_km_medoid_kernel, dim3(n_tiles), dim3(256), lds_medoid, st, A);
+  hipLaunchKernelGGL(gd_km_medoid_kernel, dim3(n_tiles), dim3(256), 0, st, A, tile);
   HIPCHK(hipGetLastError());
   HIPCHK(hipEventRecord(ctx->ev1, st));
   std::vector<unsigned long long> best(gk);
