@@ -78,7 +78,7 @@ struct DevComplex {
   const float *psp;        // [NLT * n_res]
   int2 *ref;               // [lna * KMAX] sorted point index, pmf0 bits
   int *ref_cnt;            // [lna]
-  const int *prt_cls;      // [pnp] receptor class t mod 4 (sorted order), surrogate features
+  const int *prt_type;     // [pnp] receptor type (sorted order)
   // surrogate feature grid [n_prt][sn^3][32] at origin (sox, soy, soz), spacing sh
   const float *sgrid;
   float sox, soy, soz, sh;
@@ -94,9 +94,11 @@ struct DevComplex {
 // pack's receptor split: `ns` lane groups of `half` lanes (a multiple of 64)
 // each evaluate all of the pack's replicas over their share of every receptor
 // chunk.
+// A pack of poses may hold several rounds of `round` slots (flat pair loop
+// only; otherwise round = n_slots).
 struct Pack {
   int cx, prt, n_slots, n_groups, slot_off;
-  int ns, half;
+  int ns, half, round;
 };
 
 // MODE_SUREVAL: surrogate total of given poses (delayed-acceptance kernels)

@@ -1233,7 +1233,7 @@ __device__ __forceinline__ void exchange_ladder(int n_tmp, int mode_t, const flo
 // are 1 and 2 with the split groups' shared surrogate sums compiled in.
 template <int APL, int DA, bool TILE, bool FLAT>
 __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const DevComplex &C, const Lds &S,
-                         int lpr, int step0) {
+                         int lpr, int step0, int &par) {
   constexpr int DAM = DA > 2 ? DA - 2 : DA;
   constexpr bool SHARED = DA > 2;
   const int tid = threadIdx.x;
@@ -1249,7 +1249,7 @@ __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const
   sp.ltid = tid - hw * sp.half;
   sp.slots = sp.half / 8;
   sp.xp_floats = P.xp_floats;
-  sp.par = 0;
+  sp.par = par;
   const int slot = sp.ltid / lpr;
   sp.slot = slot;
   const int a = sp.ltid - slot * lpr;
@@ -1325,6 +1325,7 @@ __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const
                                           mo, Rp, a, ilig);
       }
       if (active && lead) P.ev_sur[sv] = sv_s;
+      par = sp.par;
       return;
     }
   }
@@ -1332,6 +1333,7 @@ __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const
     place(mo);
     gd_energy E;
     pose_energy<APL, TILE, FLAT>(C, S, lpr, sp, true, x, y, z, ox, oy, oz, lt, q, li, val, mo, E);
+    par = sp.par;
     if (active && lead) {
       if (P.mode == MODE_EVAL) {
         P.ev_out[sv] = E;
@@ -1612,7 +1614,20 @@ __device__ __forceinline__ void mc_kernel_body(const KParams &P, int idx, int st
   }
   __syncthreads();
 
-  run_pack<APL, DA, TILE, FLAT>(P, pk, C, S, C.lpr, step0);
+  int par = 0;
+  if constexpr (FLAT) {
+    // rounds of poses on the staged receptor (MC packs have one round); the
+    // exchange buffers' parity runs on, so a round's first exchange does not
+    // touch what the round before it may still be reading
+    Pack q = pk;
+    for (int b = 0; b < pk.n_slots; b += pk.round) {
+      q.slot_off = pk.slot_off + b;
+      q.n_slots = min(pk.round, pk.n_slots - b);
+      run_pack<APL, DA, TILE, FLAT>(P, q, C, S, C.lpr, step0, par);
+    }
+  } else {
+    run_pack<APL, DA, TILE, FLAT>(P, pk, C, S, C.lpr, step0, par);
+  }
 }
 
 // MC kernel for packs whose complexes place APL ligand atoms on each lane:

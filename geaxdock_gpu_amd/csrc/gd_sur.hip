@@ -19,7 +19,7 @@ namespace gd {
 // node-point pair. One wave per 64 nodes along z and a 32-way select per pair
 // took 744 us for 65^3 nodes and 2,400 points; this takes 182 us.
 extern "C" __global__ void __launch_bounds__(256) gd_sur_grid_kernel(
-    const float4 *xyze_all, const int *cls, int pnp, float ox, float oy, float oz, float h, int n,
+    const float4 *xyze_all, const int *type, int pnp, float ox, float oy, float oz, float h, int n,
     float *grid_all) {
   const int l = threadIdx.x & 63;
   const int nb = (n + 3) / 4;
@@ -39,7 +39,7 @@ extern "C" __global__ void __launch_bounds__(256) gd_sur_grid_kernel(
   int c = -1;
   if (l < pnp) {
     P = xyze[l];
-    c = cls[l];
+    c = type[l] % SUR_NCLS;
   }
   for (int p0 = 0; p0 < pnp; p0 += 64) {
     const int pn = p0 + 64 + l;
@@ -47,7 +47,7 @@ extern "C" __global__ void __launch_bounds__(256) gd_sur_grid_kernel(
     int cn = -1;
     if (pn < pnp) {
       Pn = xyze[pn];
-      cn = cls[pn];
+      cn = type[pn] % SUR_NCLS;
     }
     const float dx = fmaxf(fmaxf(lx - P.x, P.x - (lx + w)), 0.0f);
     const float dy = fmaxf(fmaxf(ly - P.y, P.y - (ly + w)), 0.0f);
