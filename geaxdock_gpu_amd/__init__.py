@@ -311,7 +311,7 @@ class Engine:
         ip = np.ascontiguousarray(idx_prt, np.int32)
         mm = np.ascontiguousarray(movematrix, np.float32).reshape(-1, 6)
         lna = self.complexes[cid].lna
-        out = np.zeros((len(mm), lna, 56), np.float32)
+        out = np.empty((len(mm), lna, 56), np.float32)
         self._check(self.lib.gd_sur_features(self._ctx, cid, len(mm), _i(il), _i(ip), _f(mm),
                                              _f(out)))
         return out
@@ -440,8 +440,11 @@ def run(cx, steps_total, steps_per_exchange=20, seed=0, steps_per_dump=2000, dev
     records = {}
 
     def sink(cid, recs):
-        for r in np.unique(recs["replica"][:, 0]):
-            records.setdefault(int(r), []).append(recs[recs["replica"][:, 0] == r])
+        # a window's records come by replica: cut where the replica changes
+        rep = recs["replica"][:, 0]
+        cuts = np.flatnonzero(rep[1:] != rep[:-1]) + 1
+        for b, e in zip([0, *cuts], [*cuts, len(recs)]):
+            records.setdefault(int(rep[b]), []).append(recs[b:e])
 
     with Engine(seed=seed, device=device, steps_per_dump=steps_per_dump) as eng:
         eng.add_complex(cx)

@@ -58,6 +58,14 @@ struct HostComplex {
   size_t lds_bytes = 0;
 };
 
+// A buffer that a context keeps between calls, grown to the largest need so
+// far and given back after a call that needed more than SCRATCH_KEEP bytes.
+struct Scratch {
+  unsigned char *p = nullptr;
+  size_t cap = 0;
+};
+constexpr size_t SCRATCH_KEEP = (size_t)256 << 20;
+
 }  // namespace
 
 struct gd_ctx {
@@ -72,6 +80,12 @@ struct gd_ctx {
   int n_cu = 0;
   size_t max_lds = 65536;
   unsigned char *scratch = nullptr;  // this device's copy of the file-scope scratch array
+  // staging of the calls that take or return host arrays: pinned host memory
+  // (also read and written by kernels directly for small calls) and device
+  // memory; `drain` is the record drains' own pinned staging (a drain runs
+  // beside a window)
+  Scratch pin, dev, drain_pin;
+  int64_t *h_counts = nullptr;  // pinned: accepted moves and exchanges before and after a run
   std::vector<HostComplex> cx;
   DevComplex *d_cx = nullptr;
   bool cx_dirty = true;
@@ -86,8 +100,6 @@ struct gd_ctx {
   // record rings: the MC kernels append accepted states to ring `ring`; with
   // a sink, windows alternate between two rings so one window's records are
   // drained while the next window runs (ring 1 is allocated on first use)
-  gd_record *d_rec = nullptr;  // ring 0
-  int *d_rec_cnt = nullptr;
   gd_record *d_ring[2] = {nullptr, nullptr};
   int *d_ring_cnt[2] = {nullptr, nullptr};
   int ring = 0;
@@ -184,6 +196,48 @@ gd_status dev_upload(gd_ctx *ctx, HostComplex &h, T **dst, const T *src, size_t 
     if (s_ != GD_OK) return s_;        \
   } while (0)
 
+void scratch_free(Scratch &s, bool pinned) {
+  if (s.p) (void)(pinned ? hipHostFree(s.p) : hipFree(s.p));
+  s = Scratch{};
+}
+
+// At least `bytes` in the scratch buffer (its contents are lost when it grows).
+gd_status scratch_need(gd_ctx *ctx, Scratch &s, size_t bytes, bool pinned) {
+  if (s.cap >= bytes) return GD_OK;
+  scratch_free(s, pinned);
+  const size_t cap = (bytes + bytes / 4 + 65535) & ~(size_t)65535;
+  void *p = nullptr;
+  if (pinned) HIPCHK(hipHostMalloc(&p, cap, hipHostMallocDefault));
+  else HIPCHK(hipMalloc(&p, cap));
+  s.p = static_cast<unsigned char *>(p);
+  s.cap = cap;
+  return GD_OK;
+}
+
+// Gives the context's scratch back at the end of a call if it is large.
+struct ScratchTrim {
+  gd_ctx *ctx;
+  ~ScratchTrim() {
+    if (ctx->pin.cap > SCRATCH_KEEP) scratch_free(ctx->pin, true);
+    if (ctx->dev.cap > SCRATCH_KEEP) scratch_free(ctx->dev, false);
+  }
+};
+
+// Regions of one scratch buffer, each 256-byte aligned.
+struct Regions {
+  size_t end = 0;
+  size_t add(size_t bytes) {
+    const size_t o = end;
+    end = (end + bytes + 255) & ~(size_t)255;
+    return o;
+  }
+};
+
+// Calls whose arrays stay below this go without copies: kernels read their
+// inputs from the pinned staging and write their results there. A copy costs
+// 5 to 10 us each way whatever its size; these reads cross the bus once.
+constexpr size_t ZERO_COPY_BYTES = 65536;
+
 // Lanes per replica and atoms per lane: the fewest lane slots lpr*apl that
 // hold lna atoms with apl <= 4, preferring 2..3 atoms per lane on ties (more
 // independent work per lane), with a whole ladder within 512 lanes.
@@ -261,14 +315,8 @@ gd_status gd_create(gd_ctx **out, const gd_opts *opts) {
             prop.gcnArchName, prop.multiProcessorCount, (size_t)prop.sharedMemPerBlock,
             (size_t)prop.maxSharedMemoryPerMultiProcessor, prop.regsPerBlock);
   HIPCHK(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
-  HIPCHK(hipStreamCreateWithFlags(&ctx->drain_stream, hipStreamNonBlocking));
   HIPCHK(hipEventCreate(&ctx->ev0));
   HIPCHK(hipEventCreate(&ctx->ev1));
-  HIPCHK(hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming));
-  for (int i = 0; i < 3; ++i) {
-    HIPCHK(hipStreamCreateWithFlags(&ctx->aux[i], hipStreamNonBlocking));
-    HIPCHK(hipEventCreateWithFlags(&ctx->ev_join[i], hipEventDisableTiming));
-  }
   HIPCHK(hipGetSymbolAddress((void **)&ctx->scratch, HIP_SYMBOL(scratch)));
   return GD_OK;
 }
@@ -282,11 +330,15 @@ void gd_destroy(gd_ctx *ctx) {
   for (auto &h : ctx->cx)
     for (void *p : h.bufs) (void)hipFree(p);
   void *ps[] = {ctx->d_cx, ctx->d_mm, ctx->d_eold, ctx->d_idx_tmp,
-                ctx->d_acs_mc, ctx->d_acs_x, ctx->d_rep_flat, ctx->d_rec, ctx->d_rec_cnt,
+                ctx->d_acs_mc, ctx->d_acs_x, ctx->d_rep_flat, ctx->d_ring[0], ctx->d_ring_cnt[0],
                 ctx->d_packs, ctx->d_slots, ctx->d_best_e, ctx->d_best_mm, ctx->d_ctrl,
                 ctx->d_drain_off, ctx->d_drain, ctx->d_ring[1], ctx->d_ring_cnt[1],
                 ctx->d_ladders};
   if (ctx->h_drain) (void)hipHostFree(ctx->h_drain);
+  if (ctx->h_counts) (void)hipHostFree(ctx->h_counts);
+  scratch_free(ctx->pin, true);
+  scratch_free(ctx->drain_pin, true);
+  scratch_free(ctx->dev, false);
   for (auto &g : ctx->gslot)
     if (g.exec) (void)hipGraphExecDestroy(g.exec);
   for (void *p : ps)
@@ -571,37 +623,52 @@ gd_status gd_add_complex(gd_ctx *ctx, const gd_complex_desc *d, int *complex_id)
     psp_zero.assign(psp_n, 0.0f);
     psp_src = psp_zero.data();
   }
-  TRY(dev_upload(ctx, h, (float4 **)&D.prt_xyze, xyze.data(), xyze.size()));
-  TRY(dev_upload(ctx, h, (float **)&D.prt_hpp, hpp.data(), hpp.size()));
-  TRY(dev_upload(ctx, h, (int **)&D.prt_psp, pspi.data(), pspi.size()));
+  // one device block and one copy for all arrays of the complex
+  std::vector<int> type(pnp);
+  for (int i = 0; i < pnp; ++i) type[i] = d->prt_t[perm[i]];
+  Regions R;
+  struct Part {
+    const void *src;
+    size_t bytes, at;
+    void **dst;
+  };
+  std::vector<Part> parts;
+  auto part = [&](auto **dst, const void *src, size_t n_items) {
+    const size_t bytes = n_items * sizeof(**dst);
+    parts.push_back({src, bytes, R.add(std::max<size_t>(bytes, 16)), (void **)dst});
+  };
+  part(&D.prt_xyze, xyze.data(), xyze.size());
+  part(&D.prt_hpp, hpp.data(), hpp.size());
+  part(&D.prt_psp, pspi.data(), pspi.size());
+  part(&D.prt_type, type.data(), type.size());
+  part(&D.chunks, chunks.data(), chunks.size());
+  part(&D.params, par.data(), par.size());
+  part(&D.lig_orig, orig.data(), orig.size());
+  part(&D.lig_t, d->lig_t, (size_t)lna);
+  part(&D.lig_c, d->lig_c, (size_t)lna);
+  part(&D.mcs, mcs.data(), mcs.size());
+  part(&D.mcs_tcc, tcc.data(), tcc.size());
+  part(&D.mcs_cnt, mcnt.data(), mcnt.size());
+  part(&D.mcsq, mcsq.data(), mcsq.size());
+  part(&D.kde, kde.data(), kde.size());
+  part(&D.kde_range, krange.data(), krange.size());
+  part(&D.psp, psp_src, psp_n);
+  const size_t up_bytes = R.end;
+  part(&D.ref, nullptr, (size_t)lna * KMAX);
+  part(&D.ref_cnt, nullptr, (size_t)lna);
+  void *block = nullptr;
+  HIPCHK(hipMalloc(&block, R.end));
+  h.bufs.push_back(block);
   {
-    std::vector<int> type(pnp);
-    for (int i = 0; i < pnp; ++i) type[i] = d->prt_t[perm[i]];
-    TRY(dev_upload(ctx, h, (int **)&D.prt_type, type.data(), type.size()));
+    const ScratchTrim trim{ctx};
+    TRY(scratch_need(ctx, ctx->pin, up_bytes, true));
+    for (const Part &q : parts) {
+      *q.dst = static_cast<unsigned char *>(block) + q.at;
+      if (q.src) memcpy(ctx->pin.p + q.at, q.src, q.bytes);
+    }
+    HIPCHK(hipMemcpyAsync(block, ctx->pin.p, up_bytes, hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
   }
-  TRY(dev_upload(ctx, h, (int4 **)&D.chunks, chunks.data(), chunks.size()));
-  TRY(dev_upload(ctx, h, (float **)&D.params, par.data(), par.size()));
-  TRY(dev_upload(ctx, h, (float **)&D.lig_orig, orig.data(), orig.size()));
-  TRY(dev_upload(ctx, h, (int **)&D.lig_t, d->lig_t, (size_t)lna));
-  TRY(dev_upload(ctx, h, (float **)&D.lig_c, d->lig_c, (size_t)lna));
-  TRY(dev_upload(ctx, h, (float4 **)&D.mcs, mcs.data(), mcs.size()));
-  TRY(dev_upload(ctx, h, (float **)&D.mcs_tcc, tcc.data(), tcc.size()));
-  TRY(dev_upload(ctx, h, (float **)&D.mcs_cnt, mcnt.data(), mcnt.size()));
-  TRY(dev_upload(ctx, h, (float4 **)&D.mcsq, mcsq.data(), mcsq.size()));
-  TRY(dev_upload(ctx, h, (float4 **)&D.kde, kde.data(), kde.size()));
-  TRY(dev_upload(ctx, h, (int2 **)&D.kde_range, krange.data(), krange.size()));
-  TRY(dev_upload(ctx, h, (float **)&D.psp, psp_src, psp_n));
-  TRY(dev_upload<int2>(ctx, h, &D.ref, nullptr, 0));
-  {
-    void *p = nullptr;
-    HIPCHK(hipMalloc(&p, (size_t)lna * KMAX * sizeof(int2)));
-    h.bufs.push_back(p);
-    D.ref = (int2 *)p;
-    HIPCHK(hipMalloc(&p, (size_t)lna * sizeof(int)));
-    h.bufs.push_back(p);
-    D.ref_cnt = (int *)p;
-  }
-  HIPCHK(hipStreamSynchronize(ctx->stream));
   h.lds_bytes = lds_need(h, 512 / h.lpr, 0);
   h.tiled = ctx->opts.receptor_tile > 0 || h.lds_bytes > ctx->max_lds;
   if (h.tiled) {
@@ -1135,8 +1202,7 @@ gd_status alloc_state(gd_ctx *ctx) {
   HIPCHK(hipMalloc(&ctx->d_acs_mc, (size_t)n * sizeof(int)));
   HIPCHK(hipMalloc(&ctx->d_acs_x, (size_t)n * sizeof(int)));
   HIPCHK(hipMalloc(&ctx->d_rep_flat, (size_t)n * sizeof(int)));
-  HIPCHK(hipMalloc(&ctx->d_rec_cnt, (size_t)n * sizeof(int)));
-  ctx->d_ring_cnt[0] = ctx->d_rec_cnt;
+  HIPCHK(hipMalloc(&ctx->d_ring_cnt[0], (size_t)n * sizeof(int)));
   std::vector<int> flat(n), itmp(n);
   for (auto &h : ctx->cx)
     for (int f = 0; f < h.n_rep; ++f) {
@@ -1149,12 +1215,7 @@ gd_status alloc_state(gd_ctx *ctx) {
   HIPCHK(hipMemsetAsync(ctx->d_eold, 0, (size_t)n * sizeof(gd_energy), ctx->stream));
   HIPCHK(hipMemsetAsync(ctx->d_acs_mc, 0, (size_t)n * sizeof(int), ctx->stream));
   HIPCHK(hipMemsetAsync(ctx->d_acs_x, 0, (size_t)n * sizeof(int), ctx->stream));
-  HIPCHK(hipMemsetAsync(ctx->d_rec_cnt, 0, (size_t)n * sizeof(int), ctx->stream));
-  if (ctx->opts.record) {
-    ctx->rec_cap = ctx->opts.steps_per_dump + 1;
-    HIPCHK(hipMalloc(&ctx->d_rec, (size_t)n * ctx->rec_cap * sizeof(gd_record)));
-    ctx->d_ring[0] = ctx->d_rec;
-  }
+  HIPCHK(hipMemsetAsync(ctx->d_ring_cnt[0], 0, (size_t)n * sizeof(int), ctx->stream));
   // receptor split: automatic (0, per pack) or fixed
   const int ns = ctx->opts.receptor_split;
   if (ns != 0 && ns != 1 && ns != 2 && ns != 4 && ns != 8)
@@ -1275,6 +1336,19 @@ struct ClassLaunch {
   size_t lds;
 };
 
+// Side streams and their events for a launch of n classes (made on first use:
+// a stream costs about 50 us and as much again to destroy).
+hipError_t side_streams(gd_ctx *ctx, int n) {
+  hipError_t e = hipSuccess;
+  if (n > 1 && !ctx->ev_fork) e = hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming);
+  for (int i = 0; i < std::min(n - 1, 3) && e == hipSuccess; ++i) {
+    if (!ctx->aux[i]) e = hipStreamCreateWithFlags(&ctx->aux[i], hipStreamNonBlocking);
+    if (e == hipSuccess && !ctx->ev_join[i])
+      e = hipEventCreateWithFlags(&ctx->ev_join[i], hipEventDisableTiming);
+  }
+  return e;
+}
+
 hipError_t plan_classes(gd_ctx *ctx, const std::vector<LaunchClass> &classes, const KParams &P0,
                         int da, bool da_scratch, int *queue, std::vector<ClassLaunch> &out) {
   out.clear();
@@ -1323,7 +1397,7 @@ hipError_t plan_classes(gd_ctx *ctx, const std::vector<LaunchClass> &classes, co
         hipFuncSetAttribute(cl.f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->max_lds);
     if (e != hipSuccess) return e;
   }
-  return hipSuccess;
+  return side_streams(ctx, (int)out.size());
 }
 
 // Enqueue planned class launches, the classes concurrently on side streams
@@ -1365,16 +1439,20 @@ hipError_t launch_classes(gd_ctx *ctx, const std::vector<LaunchClass> &classes, 
 // Drain record ring r: its accepted-state records, compacted on the device
 // into one window, copied to the pinned staging buffer and handed to the
 // sink per complex; then the ring's counts restart. All on `stream`, which
-// is synchronized before returning.
+// is synchronized before returning when there is a sink.
 gd_status drain_ring(gd_ctx *ctx, int r, gd_record_sink sink, void *user, hipStream_t stream) {
   if (!ctx->d_ring[r]) return GD_OK;
   const int n = ctx->n_rep;
   int *cnt_d = ctx->d_ring_cnt[r];
   if (sink) {
-    std::vector<int> cnt(n);
-    HIPCHK(hipMemcpyAsync(cnt.data(), cnt_d, n * sizeof(int), hipMemcpyDeviceToHost, stream));
+    Regions R;
+    const size_t o_off = R.add((n + 1) * sizeof(int64_t)), o_cnt = R.add(n * sizeof(int));
+    TRY(scratch_need(ctx, ctx->drain_pin, R.end, true));
+    int64_t *off = reinterpret_cast<int64_t *>(ctx->drain_pin.p + o_off);
+    int *cnt = reinterpret_cast<int *>(ctx->drain_pin.p + o_cnt);
+    HIPCHK(hipMemcpyAsync(cnt, cnt_d, n * sizeof(int), hipMemcpyDeviceToHost, stream));
     HIPCHK(hipStreamSynchronize(stream));
-    std::vector<int64_t> off(n + 1, 0);
+    off[0] = 0;
     for (int i = 0; i < n; ++i) off[i + 1] = off[i] + cnt[i];
     const int64_t tot = off[n];
     if (tot > 0) {
@@ -1390,23 +1468,24 @@ gd_status drain_ring(gd_ctx *ctx, int r, gd_record_sink sink, void *user, hipStr
         ctx->drain_cap = cap;
       }
       if (!ctx->d_drain_off) HIPCHK(hipMalloc(&ctx->d_drain_off, (n + 1) * sizeof(int64_t)));
-      HIPCHK(hipMemcpyAsync(ctx->d_drain_off, off.data(), (n + 1) * sizeof(int64_t),
+      HIPCHK(hipMemcpyAsync(ctx->d_drain_off, off, (n + 1) * sizeof(int64_t),
                             hipMemcpyHostToDevice, stream));
       hipLaunchKernelGGL(gd_compact_kernel, dim3(n), dim3(256), 0, stream, n, ctx->d_ring[r],
                          cnt_d, ctx->d_drain_off, ctx->rec_cap, ctx->d_drain);
       HIPCHK(hipGetLastError());
       HIPCHK(hipMemcpyAsync(ctx->h_drain, ctx->d_drain, tot * sizeof(gd_record),
                             hipMemcpyDeviceToHost, stream));
-      HIPCHK(hipStreamSynchronize(stream));
-      for (int c = 0; c < (int)ctx->cx.size(); ++c) {
-        const HostComplex &h = ctx->cx[c];
-        const int64_t b = off[h.rep_base], e = off[h.rep_base + h.n_rep];
-        if (e > b) sink(user, c, ctx->h_drain + b, e - b);
-      }
     }
+    HIPCHK(hipMemsetAsync(cnt_d, 0, n * sizeof(int), stream));
+    HIPCHK(hipStreamSynchronize(stream));
+    for (int c = 0; tot > 0 && c < (int)ctx->cx.size(); ++c) {
+      const HostComplex &h = ctx->cx[c];
+      const int64_t b = off[h.rep_base], e = off[h.rep_base + h.n_rep];
+      if (e > b) sink(user, c, ctx->h_drain + b, e - b);
+    }
+    return GD_OK;
   }
   HIPCHK(hipMemsetAsync(cnt_d, 0, n * sizeof(int), stream));
-  HIPCHK(hipStreamSynchronize(stream));
   return GD_OK;
 }
 
@@ -1414,28 +1493,45 @@ gd_status drain_records(gd_ctx *ctx, gd_record_sink sink, void *user) {
   return drain_ring(ctx, ctx->ring, sink, user, ctx->stream);
 }
 
-// Second record ring, allocated the first time a run drains to a sink.
-gd_status ensure_ring1(gd_ctx *ctx) {
-  if (ctx->d_ring[1] || !ctx->d_rec) return GD_OK;
-  const int n = ctx->n_rep;
-  HIPCHK(hipMalloc(&ctx->d_ring[1], (size_t)n * ctx->rec_cap * sizeof(gd_record)));
-  HIPCHK(hipMalloc(&ctx->d_ring_cnt[1], (size_t)n * sizeof(int)));
-  HIPCHK(hipMemsetAsync(ctx->d_ring_cnt[1], 0, (size_t)n * sizeof(int), ctx->stream));
+// Record rings for windows of up to `win` steps (and the start poses): ring 0,
+// and ring 1 when windows alternate. Called between runs, when they are empty.
+// They grow with the longest window asked for, not to steps_per_dump at once
+// (93 MB and 1 ms for a first run of 200 steps of 504 replicas).
+gd_status ensure_rings(gd_ctx *ctx, int win, bool both) {
+  if (!ctx->opts.record) return GD_OK;
+  const size_t n = ctx->n_rep;
+  if (win + 1 > ctx->rec_cap) {
+    for (int r = 0; r < 2; ++r) {
+      if (ctx->d_ring[r]) HIPCHK(hipFree(ctx->d_ring[r]));
+      ctx->d_ring[r] = nullptr;
+    }
+    for (int r = 0; r < 2; ++r)
+      if (ctx->d_ring_cnt[r]) HIPCHK(hipMemsetAsync(ctx->d_ring_cnt[r], 0, n * sizeof(int), ctx->stream));
+    for (auto &g : ctx->gslot) g.valid = false;  // captured launches hold the old rings
+    ctx->rec_cap = win + 1;
+  }
+  for (int r = 0; r < (both ? 2 : 1); ++r) {
+    if (!ctx->d_ring[r])
+      HIPCHK(hipMalloc(&ctx->d_ring[r], n * ctx->rec_cap * sizeof(gd_record)));
+    if (!ctx->d_ring_cnt[r]) {
+      HIPCHK(hipMalloc(&ctx->d_ring_cnt[r], n * sizeof(int)));
+      HIPCHK(hipMemsetAsync(ctx->d_ring_cnt[r], 0, n * sizeof(int), ctx->stream));
+    }
+  }
+  if (!ctx->d_ring[ctx->ring])  // ring 1 was current and is not kept
+    HIPCHK(hipMalloc(&ctx->d_ring[ctx->ring], n * ctx->rec_cap * sizeof(gd_record)));
+  if (both && !ctx->drain_stream)
+    HIPCHK(hipStreamCreateWithFlags(&ctx->drain_stream, hipStreamNonBlocking));
   HIPCHK(hipStreamSynchronize(ctx->stream));
   return GD_OK;
 }
 
-// Enqueue one MC launch (mode, window of n_steps from step0) on ctx->stream
-// between the timing events ev0 and ev1; launch_mc_wait waits for it.
-gd_status launch_mc_enqueue(gd_ctx *ctx, int mode, int step0, int n_steps, int nc, int da_k = 0,
-                            float sur_scale = 1.0f) {
+// Kernel arguments of an MC launch; with da_k > 0 of the delayed-acceptance
+// kernels.
+KParams mc_params(gd_ctx *ctx, int da_k, float sur_scale) {
   KParams P = base_params(ctx);
-  P.mode = mode;
-  P.step0 = step0;
-  P.n_steps = n_steps;
-  P.nc = nc;
-  bool scratch = false;
-  if (da_k > 0 && mode == MODE_MC) {
+  P.mode = MODE_MC;
+  if (da_k > 0) {
     auto &S = ctx->sur;
     P.da_k = da_k;
     P.sur_scale = sur_scale;
@@ -1445,8 +1541,21 @@ gd_status launch_mc_enqueue(gd_ctx *ctx, int mode, int step0, int n_steps, int n
     P.sw3 = S.p + SP_W3;
     P.sb3 = S.p + SP_B3;
     P.sur_tab = S.tab_valid ? 1 : 0;
-    scratch = !P.sur_tab;  // the direct network evaluation needs per-wave LDS scratch
   }
+  return P;
+}
+
+// Enqueue one MC launch (mode, window of n_steps from step0) on ctx->stream
+// between the timing events ev0 and ev1; launch_mc_wait waits for it.
+gd_status launch_mc_enqueue(gd_ctx *ctx, int mode, int step0, int n_steps, int nc, int da_k = 0,
+                            float sur_scale = 1.0f) {
+  KParams P = mc_params(ctx, mode == MODE_MC ? da_k : 0, sur_scale);
+  P.mode = mode;
+  P.step0 = step0;
+  P.n_steps = n_steps;
+  P.nc = nc;
+  // the direct network evaluation needs per-wave LDS scratch
+  const bool scratch = P.da_k > 0 && !P.sur_tab;
   const int da = P.da_k > 0 ? da_instance(ctx, P.sur_tab != 0) : 0;
   const bool persistent = (ctx->opts.launch & GD_LAUNCH_PERSISTENT) && mode == MODE_MC;
   const bool use_graph = !(ctx->opts.launch & GD_LAUNCH_NO_GRAPH) && mode == MODE_MC;
@@ -1517,31 +1626,45 @@ gd_status launch_mc(gd_ctx *ctx, int mode, int step0, int n_steps, int nc, float
 }
 
 // One window of spread packing: MC launches that end on exchange steps, each
-// followed by the ladder exchange kernel (timed with its launch). Advances
-// ctx->step by each launch's steps as it completes.
+// followed by the ladder exchange kernel, all enqueued at once and timed
+// together (waiting for each launch left the GPU idle for 60 to 90 us every
+// exchange interval). Advances ctx->step as launches are enqueued.
 gd_status spread_window(gd_ctx *ctx, int win, int nc, int da_k, float sur_scale, double *ms_sum,
                         int *launches) {
-  int done = 0;
-  while (done < win) {
+  KParams P = mc_params(ctx, da_k, sur_scale);
+  const int da = P.da_k > 0 ? da_instance(ctx, P.sur_tab != 0) : 0;
+  const bool persistent = (ctx->opts.launch & GD_LAUNCH_PERSISTENT) != 0;
+  int *queue = persistent ? ctx->d_ctrl + 1 : nullptr;
+  std::vector<ClassLaunch> cls;
+  const hipError_t pe =
+      plan_classes(ctx, ctx->mc_classes, P, da, P.da_k > 0 && !P.sur_tab, queue, cls);
+  if (pe == hipErrorInvalidValue)
+    return fail(ctx, GD_ERR_CAPACITY, "delayed acceptance scratch does not fit in LDS");
+  HIPCHK(pe);
+  HIPCHK(hipEventRecord(ctx->ev0, ctx->stream));
+  for (int done = 0; done < win;) {
     const int s = (int)ctx->step;
     int sub = win - done;
     if (nc > 0) sub = std::min(sub, nc - s % nc);
-    TRY(launch_mc_enqueue(ctx, MODE_MC, s, sub, 0, da_k, sur_scale));
+    for (ClassLaunch &cl : cls) {
+      cl.P.step0 = s;
+      cl.P.n_steps = sub;
+    }
+    HIPCHK(enqueue_classes(ctx, cls, queue, ctx->stream));
     if (nc > 0 && (s + sub) % nc == 0) {
-      const KParams P = base_params(ctx);
       hipLaunchKernelGGL(gd_ladder_exchange_kernel, dim3((ctx->n_ladders + 63) / 64), dim3(64),
                          0, ctx->stream, ctx->d_cx, ctx->d_ladders, ctx->n_ladders, s + sub, nc,
                          P.k0, P.k1, ctx->d_eold, ctx->d_idx_tmp, ctx->d_acs_x);
       HIPCHK(hipGetLastError());
-      HIPCHK(hipEventRecord(ctx->ev1, ctx->stream));
     }
-    float ms = 0.f;
-    TRY(launch_mc_wait(ctx, &ms));
-    *ms_sum += ms;
     *launches += 1;
     ctx->step += sub;
     done += sub;
   }
+  HIPCHK(hipEventRecord(ctx->ev1, ctx->stream));
+  float ms = 0.f;
+  TRY(launch_mc_wait(ctx, &ms));
+  *ms_sum += ms;
   return GD_OK;
 }
 
@@ -1580,9 +1703,18 @@ static gd_status run_impl(gd_ctx *ctx, int64_t n_steps, int steps_per_exchange,
   const auto t_start = std::chrono::steady_clock::now();
   TRY(alloc_state(ctx));
   gd_run_stats st{};
-  std::vector<int> acs0(ctx->n_rep), acx0(ctx->n_rep);
-  HIPCHK(hipMemcpyAsync(acs0.data(), ctx->d_acs_mc, ctx->n_rep * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(hipMemcpyAsync(acx0.data(), ctx->d_acs_x, ctx->n_rep * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+  const bool spread = spread_packing(ctx);
+  const bool overlap = sink && ctx->opts.record && n_steps > 0 && !spread;
+  const int win0 = (int)std::min<int64_t>(n_steps, ctx->opts.steps_per_dump);
+  TRY(ensure_rings(ctx, da_k > 0 ? std::max(da_k, win0) : win0, overlap));
+  // accepted moves and exchanges before and after, summed on the device
+  // (the sinks may call back: these words are not part of the scratch)
+  if (!ctx->h_counts)
+    HIPCHK(hipHostMalloc((void **)&ctx->h_counts, 4 * sizeof(int64_t), hipHostMallocDefault));
+  int64_t *counts = ctx->h_counts;
+  hipLaunchKernelGGL(gd_counts_kernel, dim3(1), dim3(1024), 0, ctx->stream, ctx->n_rep,
+                     ctx->d_acs_mc, ctx->d_acs_x, counts);
+  HIPCHK(hipGetLastError());
   if (!ctx->initialized) {
     float ms = 0.f;
     TRY(launch_mc(ctx, MODE_INIT, (int)ctx->step, 0, 0, &ms));
@@ -1593,9 +1725,6 @@ static gd_status run_impl(gd_ctx *ctx, int64_t n_steps, int steps_per_exchange,
   // with records and a sink, windows alternate between the two rings: the
   // previous window's records are drained (on the drain stream, sinks called
   // here) while the next window runs
-  const bool spread = spread_packing(ctx);
-  const bool overlap = sink && ctx->d_rec && n_steps > 0 && !spread;
-  if (overlap) TRY(ensure_ring1(ctx));
   int pending = -1;
   while (left > 0) {
     int win = (int)std::min<int64_t>(left, ctx->opts.steps_per_dump);
@@ -1626,20 +1755,51 @@ static gd_status run_impl(gd_ctx *ctx, int64_t n_steps, int steps_per_exchange,
   }
   if (pending >= 0) TRY(drain_ring(ctx, pending, sink, user, ctx->stream));
   if (n_steps == 0) TRY(drain_records(ctx, sink, user));
-  std::vector<int> acs1(ctx->n_rep), acx1(ctx->n_rep);
-  HIPCHK(hipMemcpyAsync(acs1.data(), ctx->d_acs_mc, ctx->n_rep * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(hipMemcpyAsync(acx1.data(), ctx->d_acs_x, ctx->n_rep * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+  hipLaunchKernelGGL(gd_counts_kernel, dim3(1), dim3(1024), 0, ctx->stream, ctx->n_rep,
+                     ctx->d_acs_mc, ctx->d_acs_x, counts + 2);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(ctx->stream));
-  for (int i = 0; i < ctx->n_rep; ++i) {
-    st.accepted += acs1[i] - acs0[i];
-    st.exchanges_accepted += acx1[i] - acx0[i];
-  }
+  st.accepted = counts[2] - counts[0];
+  st.exchanges_accepted = counts[3] - counts[1];
   st.t_compute = t_ms * 1e-3;
   st.steps = n_steps;
   st.replica_steps = n_steps * (int64_t)ctx->n_rep;
   st.kernel_ms_avg = st.kernel_launches ? t_ms / st.kernel_launches : 0.0;
   st.t_wall = std::chrono::duration<double>(std::chrono::steady_clock::now() - t_start).count();
   if (stats) *stats = st;
+  return GD_OK;
+}
+
+// Copies device arrays to host ones: one kernel gathers them into the pinned
+// staging (five copies of a few KB each took 100 us and more).
+struct HostCopy {
+  const void *src;
+  void *dst;  // null: left out
+  size_t bytes;
+};
+
+static gd_status copy_out(gd_ctx *ctx, std::initializer_list<HostCopy> parts) {
+  GatherArgs A{};
+  size_t words = 0;
+  for (const HostCopy &c : parts) {
+    if (!c.dst || c.bytes == 0) continue;
+    A.src[A.n] = static_cast<const int *>(c.src);
+    words += c.bytes / sizeof(int);
+    A.end[A.n++] = (long long)words;
+  }
+  if (A.n == 0) return GD_OK;
+  const ScratchTrim trim{ctx};
+  TRY(scratch_need(ctx, ctx->pin, words * sizeof(int), true));
+  hipLaunchKernelGGL(gd_gather_kernel, dim3((unsigned)std::min<size_t>((words + 255) / 256, 1024)),
+                     dim3(256), 0, ctx->stream, A, reinterpret_cast<int *>(ctx->pin.p));
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(ctx->stream));
+  const unsigned char *p = ctx->pin.p;
+  for (const HostCopy &c : parts) {
+    if (!c.dst || c.bytes == 0) continue;
+    memcpy(c.dst, p, c.bytes);
+    p += c.bytes;
+  }
   return GD_OK;
 }
 
@@ -1650,15 +1810,12 @@ gd_status gd_get_state(gd_ctx *ctx, int cid, float *movematrix, gd_energy *energ
   HIPCHK(hipSetDevice(ctx->device));
   const HostComplex &h = ctx->cx[cid];
   const size_t b = h.rep_base, n = h.n_rep;
-  if (movematrix)
-    HIPCHK(hipMemcpyAsync(movematrix, ctx->d_mm + b * 6, n * 6 * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-  if (energy_old)
-    HIPCHK(hipMemcpyAsync(energy_old, ctx->d_eold + b, n * sizeof(gd_energy), hipMemcpyDeviceToHost, ctx->stream));
-  if (acs_mc) HIPCHK(hipMemcpyAsync(acs_mc, ctx->d_acs_mc + b, n * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-  if (acs_x) HIPCHK(hipMemcpyAsync(acs_x, ctx->d_acs_x + b, n * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-  std::vector<int> it(n);
-  HIPCHK(hipMemcpyAsync(it.data(), ctx->d_idx_tmp + b, n * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(hipStreamSynchronize(ctx->stream));
+  std::vector<int> it(replica ? n : 0);
+  TRY(copy_out(ctx, {{ctx->d_mm + b * 6, movematrix, n * 6 * sizeof(float)},
+                     {ctx->d_eold + b, energy_old, n * sizeof(gd_energy)},
+                     {ctx->d_acs_mc + b, acs_mc, n * sizeof(int)},
+                     {ctx->d_acs_x + b, acs_x, n * sizeof(int)},
+                     {ctx->d_idx_tmp + b, replica ? it.data() : nullptr, n * sizeof(int)}}));
   if (replica) {
     for (size_t f = 0; f < n; ++f) {
       replica[f].idx_rep = (int)f;
@@ -1676,12 +1833,8 @@ gd_status gd_get_best(gd_ctx *ctx, int cid, float *best_e, float *best_mm) {
   HIPCHK(hipSetDevice(ctx->device));
   const HostComplex &h = ctx->cx[cid];
   const size_t b = h.rep_base, n = h.n_rep;
-  if (best_e)
-    HIPCHK(hipMemcpyAsync(best_e, ctx->d_best_e + b, n * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-  if (best_mm)
-    HIPCHK(hipMemcpyAsync(best_mm, ctx->d_best_mm + b * 6, n * 6 * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(hipStreamSynchronize(ctx->stream));
-  return GD_OK;
+  return copy_out(ctx, {{ctx->d_best_e + b, best_e, n * sizeof(float)},
+                        {ctx->d_best_mm + b * 6, best_mm, n * 6 * sizeof(float)}});
 }
 
 gd_status gd_reset_best(gd_ctx *ctx) {
@@ -1883,39 +2036,46 @@ static gd_status eval_poses(gd_ctx *ctx, int cid, int n, const int *idx_lig, con
     P.sw3 = S.p + SP_W3;
     P.sb3 = S.p + SP_B3;
   }
-  Pack *d_packs = nullptr;
-  int *d_slots = nullptr, *d_lig = nullptr;
-  float *d_mm = nullptr;
-  gd_energy *d_out = nullptr;
-  float *d_sur = nullptr;
+  // inputs (packs, slots, conformers, poses), then results
+  Regions R;
+  const size_t o_packs = R.add(ps.packs.size() * sizeof(Pack));
+  const size_t o_slots = R.add(ps.slots.size() * sizeof(int));
+  const size_t o_lig = R.add((size_t)n * sizeof(int));
+  const size_t o_mm = R.add((size_t)n * 6 * sizeof(float));
+  const size_t o_out = R.end;
+  const size_t res_bytes = (size_t)n * (sur ? sizeof(float) : sizeof(gd_energy));
+  R.add(res_bytes);
+  const ScratchTrim trim{ctx};
+  unsigned char *base = nullptr;  // where the kernel reads and writes
+  const bool direct = !no_alloc && R.end <= ZERO_COPY_BYTES;
   if (no_alloc) {
-    // regions of the scratch array, each 256-byte aligned
-    auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
-    const size_t o_slots = al(ps.packs.size() * sizeof(Pack));
-    const size_t o_lig = o_slots + al((size_t)n * sizeof(int));
-    const size_t o_mm = o_lig + al((size_t)n * sizeof(int));
-    const size_t o_out = o_mm + al((size_t)n * 6 * sizeof(float));
-    const size_t end = o_out + al((size_t)n * sizeof(gd_energy));
-    if (end > GD_NOALLOC_SCRATCH_BYTES)
+    if (R.end > GD_NOALLOC_SCRATCH_BYTES)
       return fail(ctx, GD_ERR_CAPACITY, "gd_calc_energy_noalloc: %zu scratch bytes needed, %d held",
-                  end, GD_NOALLOC_SCRATCH_BYTES);
-    d_packs = reinterpret_cast<Pack *>(ctx->scratch);
-    d_slots = reinterpret_cast<int *>(ctx->scratch + o_slots);
-    d_lig = reinterpret_cast<int *>(ctx->scratch + o_lig);
-    d_mm = reinterpret_cast<float *>(ctx->scratch + o_mm);
-    d_out = reinterpret_cast<gd_energy *>(ctx->scratch + o_out);
+                  R.end, GD_NOALLOC_SCRATCH_BYTES);
+    base = ctx->scratch;
+    HIPCHK(hipMemcpyAsync(base + o_packs, ps.packs.data(), ps.packs.size() * sizeof(Pack), hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(hipMemcpyAsync(base + o_slots, ps.slots.data(), ps.slots.size() * sizeof(int), hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(hipMemcpyAsync(base + o_lig, idx_lig, n * sizeof(int), hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(hipMemcpyAsync(base + o_mm, movematrix, (size_t)n * 6 * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
   } else {
-    HIPCHK(hipMalloc(&d_packs, ps.packs.size() * sizeof(Pack)));
-    HIPCHK(hipMalloc(&d_slots, ps.slots.size() * sizeof(int)));
-    HIPCHK(hipMalloc(&d_lig, n * sizeof(int)));
-    HIPCHK(hipMalloc(&d_mm, (size_t)n * 6 * sizeof(float)));
-    HIPCHK(hipMalloc(&d_out, (size_t)n * sizeof(gd_energy)));
-    HIPCHK(hipMalloc(&d_sur, (size_t)n * sizeof(float)));
+    TRY(scratch_need(ctx, ctx->pin, R.end, true));
+    memcpy(ctx->pin.p + o_packs, ps.packs.data(), ps.packs.size() * sizeof(Pack));
+    memcpy(ctx->pin.p + o_slots, ps.slots.data(), ps.slots.size() * sizeof(int));
+    memcpy(ctx->pin.p + o_lig, idx_lig, (size_t)n * sizeof(int));
+    memcpy(ctx->pin.p + o_mm, movematrix, (size_t)n * 6 * sizeof(float));
+    base = ctx->pin.p;
+    if (!direct) {
+      TRY(scratch_need(ctx, ctx->dev, R.end, false));
+      base = ctx->dev.p;
+      HIPCHK(hipMemcpyAsync(base, ctx->pin.p, o_out, hipMemcpyHostToDevice, ctx->stream));
+    }
   }
-  HIPCHK(hipMemcpyAsync(d_packs, ps.packs.data(), ps.packs.size() * sizeof(Pack), hipMemcpyHostToDevice, ctx->stream));
-  HIPCHK(hipMemcpyAsync(d_slots, ps.slots.data(), ps.slots.size() * sizeof(int), hipMemcpyHostToDevice, ctx->stream));
-  HIPCHK(hipMemcpyAsync(d_lig, idx_lig, n * sizeof(int), hipMemcpyHostToDevice, ctx->stream));
-  HIPCHK(hipMemcpyAsync(d_mm, movematrix, (size_t)n * 6 * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
+  Pack *d_packs = reinterpret_cast<Pack *>(base + o_packs);
+  int *d_slots = reinterpret_cast<int *>(base + o_slots);
+  int *d_lig = reinterpret_cast<int *>(base + o_lig);
+  float *d_mm = reinterpret_cast<float *>(base + o_mm);
+  gd_energy *d_out = reinterpret_cast<gd_energy *>(base + o_out);
+  float *d_sur = reinterpret_cast<float *>(base + o_out);
   P.cxs = ctx->d_cx;
   P.packs = d_packs;
   P.slots = d_slots;
@@ -1926,19 +2086,13 @@ static gd_status eval_poses(gd_ctx *ctx, int cid, int n, const int *idx_lig, con
   P.mode = sur ? MODE_SUREVAL : MODE_EVAL;
   hipError_t le = launch_classes(ctx, ps.classes, P, sur ? da_instance(ctx, P.sur_tab != 0) : 0,
                                  sur && !P.sur_tab, ctx->stream);
-  if (le == hipSuccess && out)
-    le = hipMemcpyAsync(out, d_out, (size_t)n * sizeof(gd_energy), hipMemcpyDeviceToHost, ctx->stream);
-  if (le == hipSuccess && sur)
-    le = hipMemcpyAsync(out_sur, d_sur, (size_t)n * sizeof(float), hipMemcpyDeviceToHost, ctx->stream);
+  void *res = sur ? static_cast<void *>(out_sur) : static_cast<void *>(out);
+  if (le == hipSuccess && no_alloc)
+    le = hipMemcpyAsync(res, base + o_out, res_bytes, hipMemcpyDeviceToHost, ctx->stream);
+  else if (le == hipSuccess && !direct)
+    le = hipMemcpyAsync(ctx->pin.p + o_out, base + o_out, res_bytes, hipMemcpyDeviceToHost, ctx->stream);
   if (le == hipSuccess) le = hipStreamSynchronize(ctx->stream);
-  if (!no_alloc) {
-    (void)hipFree(d_sur);
-    (void)hipFree(d_packs);
-    (void)hipFree(d_slots);
-    (void)hipFree(d_lig);
-    (void)hipFree(d_mm);
-    (void)hipFree(d_out);
-  }
+  if (le == hipSuccess && !no_alloc) memcpy(res, ctx->pin.p + o_out, res_bytes);
   if (le != hipSuccess) return fail(ctx, GD_ERR_HIP, "energy evaluation: %s", hipGetErrorString(le));
   return GD_OK;
 }
@@ -2250,6 +2404,43 @@ gd_status gd_sur_build_grids(gd_ctx *ctx, float spacing, float half_width) {
   return GD_OK;
 }
 
+// Pose arrays of a call on the device: one staged copy. `cid` and `row` may be
+// null; `extra_bytes` of device scratch follow them.
+struct PoseInputs {
+  int *cid = nullptr, *lig = nullptr, *prt = nullptr;
+  float *mm = nullptr;
+  int64_t *row = nullptr;
+  unsigned char *extra = nullptr;
+};
+
+static gd_status stage_poses(gd_ctx *ctx, int n, const int *cid, const int *idx_lig,
+                             const int *idx_prt, const float *movematrix, const int64_t *row,
+                             size_t extra_bytes, PoseInputs &in) {
+  Regions R;
+  const size_t o_row = R.add(row ? (size_t)n * sizeof(int64_t) : 0);
+  const size_t o_cid = R.add(cid ? (size_t)n * sizeof(int) : 0);
+  const size_t o_lig = R.add((size_t)n * sizeof(int));
+  const size_t o_prt = R.add((size_t)n * sizeof(int));
+  const size_t o_mm = R.add((size_t)n * 6 * sizeof(float));
+  const size_t o_extra = R.end;
+  TRY(scratch_need(ctx, ctx->pin, o_extra, true));
+  TRY(scratch_need(ctx, ctx->dev, o_extra + extra_bytes, false));
+  unsigned char *p = ctx->pin.p, *d = ctx->dev.p;
+  if (row) memcpy(p + o_row, row, (size_t)n * sizeof(int64_t));
+  if (cid) memcpy(p + o_cid, cid, (size_t)n * sizeof(int));
+  memcpy(p + o_lig, idx_lig, (size_t)n * sizeof(int));
+  memcpy(p + o_prt, idx_prt, (size_t)n * sizeof(int));
+  memcpy(p + o_mm, movematrix, (size_t)n * 6 * sizeof(float));
+  HIPCHK(hipMemcpyAsync(d, p, o_extra, hipMemcpyHostToDevice, ctx->stream));
+  in.row = reinterpret_cast<int64_t *>(d + o_row);
+  in.cid = reinterpret_cast<int *>(d + o_cid);
+  in.lig = reinterpret_cast<int *>(d + o_lig);
+  in.prt = reinterpret_cast<int *>(d + o_prt);
+  in.mm = reinterpret_cast<float *>(d + o_mm);
+  in.extra = d + o_extra;
+  return GD_OK;
+}
+
 gd_status gd_sur_features(gd_ctx *ctx, int cid, int n, const int *idx_lig, const int *idx_prt,
                           const float *movematrix, float *out) {
   if (!ctx || cid < 0 || cid >= (int)ctx->cx.size() || n < 0) return GD_ERR_INVALID;
@@ -2260,24 +2451,18 @@ gd_status gd_sur_features(gd_ctx *ctx, int cid, int n, const int *idx_lig, const
     if (idx_lig[i] < 0 || idx_lig[i] >= h.d.n_lig || idx_prt[i] < 0 || idx_prt[i] >= h.d.n_prt)
       return fail(ctx, GD_ERR_INVALID, "pose %d: conformer index out of range", i);
   HIPCHK(hipSetDevice(ctx->device));
-  std::vector<void *> keep;
-  int *dl, *dp;
-  float *dm, *dout;
-  gd_status s = GD_OK;
   const size_t rows = (size_t)n * h.d.lna;
-  if ((s = tmp_dev(ctx, keep, &dl, idx_lig, (size_t)n)) || (s = tmp_dev(ctx, keep, &dp, idx_prt, (size_t)n)) ||
-      (s = tmp_dev(ctx, keep, &dm, movematrix, (size_t)n * 6)) ||
-      (s = tmp_dev<float>(ctx, keep, &dout, nullptr, rows * SUR_NF))) {
-    free_all(keep);
-    return s;
-  }
+  const ScratchTrim trim{ctx};
+  PoseInputs in;
+  TRY(stage_poses(ctx, n, nullptr, idx_lig, idx_prt, movematrix, nullptr,
+                  rows * SUR_NF * sizeof(float), in));
+  float *dout = reinterpret_cast<float *>(in.extra);
   hipLaunchKernelGGL(gd_sur_feat_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0,
-                     ctx->stream, ctx->d_cx, cid, ctx->sur.g[cid], n, dl, dp, dm, (int64_t)0,
-                     (unsigned short *)nullptr, (unsigned short *)nullptr, (int64_t)0, dout);
+                     ctx->stream, ctx->d_cx, cid, ctx->sur.g[cid], n, in.lig, in.prt, in.mm,
+                     (int64_t)0, (unsigned short *)nullptr, dout);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipMemcpyAsync(out, dout, rows * SUR_NF * sizeof(float), hipMemcpyDeviceToHost, ctx->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-  free_all(keep);
   if (e != hipSuccess) return fail(ctx, GD_ERR_HIP, "gd_sur_features: %s", hipGetErrorString(e));
   return GD_OK;
 }
@@ -2399,21 +2584,14 @@ gd_status gd_sur_dataset_add(gd_ctx *ctx, int cid, int n, const int *idx_lig, co
   const int64_t add = (int64_t)n * h.d.lna;
   if (S.rows + add > S.cap) TRY(gd_sur_dataset_reserve(ctx, std::max<int64_t>(S.rows + add, 2 * S.cap)));
   HIPCHK(hipSetDevice(ctx->device));
-  std::vector<void *> keep;
-  int *dl, *dp;
-  float *dm;
-  gd_status s = GD_OK;
-  if ((s = tmp_dev(ctx, keep, &dl, idx_lig, (size_t)n)) || (s = tmp_dev(ctx, keep, &dp, idx_prt, (size_t)n)) ||
-      (s = tmp_dev(ctx, keep, &dm, movematrix, (size_t)n * 6))) {
-    free_all(keep);
-    return s;
-  }
+  const ScratchTrim trim{ctx};
+  PoseInputs in;
+  TRY(stage_poses(ctx, n, nullptr, idx_lig, idx_prt, movematrix, nullptr, 0, in));
   hipLaunchKernelGGL(gd_sur_feat_kernel, dim3((unsigned)((add + 255) / 256)), dim3(256), 0,
-                     ctx->stream, ctx->d_cx, cid, S.g[cid], n, dl, dp, dm, S.rows, S.X, nullptr,
-                     S.cap + 64, (float *)nullptr);
+                     ctx->stream, ctx->d_cx, cid, S.g[cid], n, in.lig, in.prt, in.mm, S.rows, S.X,
+                     (float *)nullptr);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-  free_all(keep);
   if (e != hipSuccess) return fail(ctx, GD_ERR_HIP, "gd_sur_dataset_add: %s", hipGetErrorString(e));
   for (int i = 0; i < n; ++i) {
     S.off.push_back(S.off.back() + h.d.lna);
@@ -2447,23 +2625,13 @@ gd_status gd_sur_dataset_add_multi(gd_ctx *ctx, int n, const int *cid, const int
   if (S.rows + add > S.cap) TRY(gd_sur_dataset_reserve(ctx, std::max<int64_t>(S.rows + add, 2 * S.cap)));
   HIPCHK(hipSetDevice(ctx->device));
   TRY(sync_complexes(ctx));
-  std::vector<void *> keep;
-  int *dc, *dl, *dp;
-  float *dm;
-  int64_t *dr;
-  gd_status s = GD_OK;
-  if ((s = tmp_dev(ctx, keep, &dc, cid, (size_t)n)) || (s = tmp_dev(ctx, keep, &dl, idx_lig, (size_t)n)) ||
-      (s = tmp_dev(ctx, keep, &dp, idx_prt, (size_t)n)) ||
-      (s = tmp_dev(ctx, keep, &dm, movematrix, (size_t)n * 6)) ||
-      (s = tmp_dev(ctx, keep, &dr, row_of.data(), (size_t)n))) {
-    free_all(keep);
-    return s;
-  }
+  const ScratchTrim trim{ctx};
+  PoseInputs in;
+  TRY(stage_poses(ctx, n, cid, idx_lig, idx_prt, movematrix, row_of.data(), 0, in));
   hipLaunchKernelGGL(gd_sur_feat_multi_kernel, dim3((unsigned)n), dim3(64), 0, ctx->stream,
-                     ctx->d_cx, n, dc, dl, dp, dm, dr, S.X, nullptr, S.cap + 64);
+                     ctx->d_cx, n, in.cid, in.lig, in.prt, in.mm, in.row, S.X);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-  free_all(keep);
   if (e != hipSuccess) return fail(ctx, GD_ERR_HIP, "gd_sur_dataset_add_multi: %s", hipGetErrorString(e));
   for (int i = 0; i < n; ++i) {
     S.off.push_back(S.off.back() + ctx->cx[cid[i]].d.lna);

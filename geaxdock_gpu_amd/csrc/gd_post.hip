@@ -290,7 +290,7 @@ namespace {
 template <class F>
 void par_for(int64_t n, F f) {
   const int64_t hw = std::max(1u, std::thread::hardware_concurrency());
-  const int nt = (int)std::min<int64_t>(std::min<int64_t>(hw, 16), std::max<int64_t>(1, n / 65536));
+  const int nt = (int)std::min<int64_t>(std::min<int64_t>(hw, 16), std::max<int64_t>(1, n / 32768));
   if (nt <= 1) {
     f(0, (int64_t)0, n);
     return;
@@ -308,7 +308,7 @@ std::unique_ptr<T[]> uninit(size_t n) {
 
 inline int par_threads(int64_t n) {
   const int64_t hw = std::max(1u, std::thread::hardware_concurrency());
-  return (int)std::min<int64_t>(std::min<int64_t>(hw, 16), std::max<int64_t>(1, n / 65536));
+  return (int)std::min<int64_t>(std::min<int64_t>(hw, 16), std::max<int64_t>(1, n / 32768));
 }
 
 // Device k-means of n_groups groups of objects whose features are given as
@@ -377,36 +377,34 @@ gd_status km_run(gd_ctx *ctx, int n_groups, const int64_t *off, const float *soa
   if (n_tiles == 0) return GD_OK;
   HIPCHK(hipSetDevice(ctx->device));
   const size_t gk = (size_t)n_groups * k;
-  std::vector<void *> bufs;
-  auto alloc = [&](void **p, size_t bytes) -> hipError_t {
-    const hipError_t e = hipMalloc(p, std::max<size_t>(bytes, 16));
-    if (e == hipSuccess) bufs.push_back(*p);
-    return e;
-  };
-  struct Free {
-    std::vector<void *> &b;
-    ~Free() {
-      for (void *p : b) (void)hipFree(p);
-    }
-  } free_all{bufs};
+  const ScratchTrim trim{ctx};
+  Regions R;
+  const size_t o_feat = R.add((size_t)KM_DIM * n_total * 4);
+  const size_t o_off = R.add((size_t)(n_groups + 1) * 8);
+  const size_t o_tg = R.add((size_t)n_tiles * 4), o_ts = R.add((size_t)n_tiles * 4);
+  const size_t o_cent = R.add(gk * KM_DIM * 4), o_done = R.add((size_t)n_groups * 4);
+  const size_t o_zero = R.end;  // cleared: sums, counts, changes, passes, sizes
+  const size_t o_sum = R.add(gk * KM_DIM * 8), o_cnt = R.add(gk * 4);
+  const size_t o_delta = R.add((size_t)n_groups * 4), o_pass = R.add((size_t)n_groups * 4);
+  const size_t o_size = R.add(gk * 4), o_active = R.add(4);
+  const size_t o_ones = R.end;  // set to all ones: memberships, medoid keys
+  const size_t o_memb = R.add((size_t)n_total * 4), o_best = R.add(gk * 8);
+  TRY(scratch_need(ctx, ctx->dev, R.end, false));
+  unsigned char *base = ctx->dev.p;
   KmArgs A{};
-  float *d_feat;
-  int64_t *d_off;
-  int *d_tg, *d_ts;
-  HIPCHK(alloc((void **)&d_feat, (size_t)KM_DIM * n_total * 4));
-  HIPCHK(alloc((void **)&d_off, (size_t)(n_groups + 1) * 8));
-  HIPCHK(alloc((void **)&d_tg, (size_t)n_tiles * 4));
-  HIPCHK(alloc((void **)&d_ts, (size_t)n_tiles * 4));
-  HIPCHK(alloc((void **)&A.memb, (size_t)n_total * 4));
-  HIPCHK(alloc((void **)&A.cent, gk * KM_DIM * 4));
-  HIPCHK(alloc((void **)&A.sum, gk * KM_DIM * 8));
-  HIPCHK(alloc((void **)&A.cnt, gk * 4));
-  HIPCHK(alloc((void **)&A.delta, (size_t)n_groups * 4));
-  HIPCHK(alloc((void **)&A.done, (size_t)n_groups * 4));
-  HIPCHK(alloc((void **)&A.pass, (size_t)n_groups * 4));
-  HIPCHK(alloc((void **)&A.active, 4));
-  HIPCHK(alloc((void **)&A.best, gk * 8));
-  HIPCHK(alloc((void **)&A.size, gk * 4));
+  float *d_feat = (float *)(base + o_feat);
+  int64_t *d_off = (int64_t *)(base + o_off);
+  int *d_tg = (int *)(base + o_tg), *d_ts = (int *)(base + o_ts);
+  A.cent = (float *)(base + o_cent);
+  A.done = (int *)(base + o_done);
+  A.sum = (long long *)(base + o_sum);
+  A.cnt = (int *)(base + o_cnt);
+  A.delta = (int *)(base + o_delta);
+  A.pass = (int *)(base + o_pass);
+  A.size = (int *)(base + o_size);
+  A.active = (int *)(base + o_active);
+  A.memb = (int *)(base + o_memb);
+  A.best = (unsigned long long *)(base + o_best);
   hipStream_t st = ctx->stream;
   HIPCHK(hipMemcpyAsync(d_feat, soa_in, (size_t)KM_DIM * n_total * 4, hipMemcpyHostToDevice, st));
   HIPCHK(hipMemcpyAsync(d_off, off, (size_t)(n_groups + 1) * 8, hipMemcpyHostToDevice, st));
@@ -414,13 +412,8 @@ gd_status km_run(gd_ctx *ctx, int n_groups, const int64_t *off, const float *soa
   HIPCHK(hipMemcpyAsync(d_ts, tile_s.data(), (size_t)n_tiles * 4, hipMemcpyHostToDevice, st));
   HIPCHK(hipMemcpyAsync(A.cent, cent.data(), gk * KM_DIM * 4, hipMemcpyHostToDevice, st));
   HIPCHK(hipMemcpyAsync(A.done, done.data(), (size_t)n_groups * 4, hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemsetAsync(A.memb, 0xFF, (size_t)n_total * 4, st));
-  HIPCHK(hipMemsetAsync(A.sum, 0, gk * KM_DIM * 8, st));
-  HIPCHK(hipMemsetAsync(A.cnt, 0, gk * 4, st));
-  HIPCHK(hipMemsetAsync(A.delta, 0, (size_t)n_groups * 4, st));
-  HIPCHK(hipMemsetAsync(A.pass, 0, (size_t)n_groups * 4, st));
-  HIPCHK(hipMemsetAsync(A.best, 0xFF, gk * 8, st));
-  HIPCHK(hipMemsetAsync(A.size, 0, gk * 4, st));
+  HIPCHK(hipMemsetAsync(base + o_zero, 0, o_ones - o_zero, st));
+  HIPCHK(hipMemsetAsync(base + o_ones, 0xFF, R.end - o_ones, st));
   A.feat = d_feat;
   A.n_total = n_total;
   A.off = d_off;
@@ -557,8 +550,11 @@ gd_status post_mc_impl(gd_ctx *ctx, const gd_record *recs, int64_t n, int k_repl
   *n_medoids = 0;
   if (n == 0) return GD_OK;
   // records grouped by replica (ascending replica, each in the given order):
-  // a stable counting sort, chunk-parallel
+  // a stable counting sort, chunk-parallel, over the replica indices (read from
+  // the records once)
   const int nt = par_threads(n);
+  auto rep_v = uninit<int>((size_t)n);
+  int *rep = rep_v.get();
   std::vector<int> tmax(nt, -1), tbad(nt, -1);
   par_for(n, [&](int t, int64_t a, int64_t b) {
     int mx = -1;
@@ -566,6 +562,7 @@ gd_status post_mc_impl(gd_ctx *ctx, const gd_record *recs, int64_t n, int k_repl
       const int r = recs[i].replica.idx_rep;
       if (r < 0 && tbad[t] < 0) tbad[t] = (int)std::min<int64_t>(i, INT32_MAX);
       mx = std::max(mx, r);
+      rep[i] = r;
     }
     tmax[t] = mx;
   });
@@ -578,7 +575,7 @@ gd_status post_mc_impl(gd_ctx *ctx, const gd_record *recs, int64_t n, int k_repl
   std::vector<int64_t> tcnt((size_t)nt * nr, 0);
   par_for(n, [&](int t, int64_t a, int64_t b) {
     int64_t *c = tcnt.data() + (size_t)t * nr;
-    for (int64_t i = a; i < b; ++i) c[recs[i].replica.idx_rep] += 1;
+    for (int64_t i = a; i < b; ++i) c[rep[i]] += 1;
   });
   std::vector<int64_t> cnt(nr + 1, 0);
   for (size_t r = 0; r < nr; ++r) {
@@ -590,23 +587,33 @@ gd_status post_mc_impl(gd_ctx *ctx, const gd_record *recs, int64_t n, int k_repl
     }
     cnt[r + 1] = s0;
   }
-  auto order = uninit<int64_t>((size_t)n);
-  par_for(n, [&](int t, int64_t a, int64_t b) {
-    int64_t *pos = tcnt.data() + (size_t)t * nr;
-    for (int64_t i = a; i < b; ++i) order[(size_t)pos[recs[i].replica.idx_rep]++] = i;
-  });
   // groups: replicas that have records
   std::vector<int64_t> off{0};
   for (size_t r = 0; r < nr; ++r)
     if (cnt[r + 1] > cnt[r]) off.push_back(cnt[r + 1]);
   const int n_groups = (int)off.size() - 1;
-  // features of the grouped records as SoA terms
-  auto feat_v = uninit<float>((size_t)KM_DIM * n);
-  float *feat = feat_v.get();
-  par_for(n, [&](int, int64_t a, int64_t b) {
+  // order and features (SoA terms) of the grouped records, the features in
+  // the context's pinned staging unless they are more than it keeps
+  HIPCHK(hipSetDevice(ctx->device));
+  const ScratchTrim trim{ctx};
+  auto order = uninit<int64_t>((size_t)n);
+  std::unique_ptr<float[]> feat_v;
+  float *feat = nullptr;
+  const size_t feat_bytes = (size_t)KM_DIM * n * sizeof(float);
+  if (feat_bytes <= SCRATCH_KEEP / 2) {
+    TRY(scratch_need(ctx, ctx->pin, feat_bytes, true));
+    feat = reinterpret_cast<float *>(ctx->pin.p);
+  } else {
+    feat_v = uninit<float>((size_t)KM_DIM * n);
+    feat = feat_v.get();
+  }
+  par_for(n, [&](int t, int64_t a, int64_t b) {
+    int64_t *pos = tcnt.data() + (size_t)t * nr;
     for (int64_t i = a; i < b; ++i) {
-      const float *e = recs[order[i]].energy.e;
-      for (int d = 0; d < KM_DIM; ++d) feat[(size_t)d * n + i] = e[d];
+      const int64_t at = pos[rep[i]]++;
+      order[(size_t)at] = i;
+      const float *e = recs[i].energy.e;
+      for (int d = 0; d < KM_DIM; ++d) feat[(size_t)d * n + at] = e[d];
     }
   });
   std::vector<int> med((size_t)n_groups * k_replica), sz((size_t)n_groups * k_replica);

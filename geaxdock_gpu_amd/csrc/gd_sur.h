@@ -129,11 +129,10 @@ __device__ inline void grid_radial(const SurGrid &G, int prt, float x, float y, 
 }
 
 // Feature row of ligand atom l of one pose (movematrix m, ligand conformer
-// il, protein conformer ip): bf16 into X [row][64] and, when xt != null, the
-// transpose XT [64][ld]; FP32 features into xf when given.
+// il, protein conformer ip): bf16 into X [row][64] (whole 128-byte rows), FP32
+// features into xf, each when given.
 __device__ inline void feat_row(const DevComplex &C, const SurGrid &G, const float *m, int il,
-                                int ip, int l, int64_t row, unsigned short *X,
-                                unsigned short *XT, int64_t ld, float *xf) {
+                                int ip, int l, int64_t row, unsigned short *X, float *xf) {
   const int lna = C.lna;
   const Rot R = euler(m[3], m[4], m[5]);
   const float *orig = C.lig_orig + (size_t)il * 3 * lna;
@@ -152,12 +151,13 @@ __device__ inline void feat_row(const DevComplex &C, const SurGrid &G, const flo
 #pragma unroll
   for (int q = 0; q < 32; ++q) v[NLT + q] = f[q];
   v[SUR_BIAS_COL] = 1.0f;
-  if (X)
+  if (X) {
+    uint4 *o = reinterpret_cast<uint4 *>(X + row * SUR_F);
 #pragma unroll
-    for (int q = 0; q < SUR_F; ++q) X[row * SUR_F + q] = f2bf(v[q]);
-  if (XT)
-#pragma unroll
-    for (int q = 0; q < SUR_F; ++q) XT[(int64_t)q * ld + row] = f2bf(v[q]);
+    for (int q = 0; q < 8; ++q)
+      o[q] = make_uint4(pk_bf16(v[8 * q], v[8 * q + 1]), pk_bf16(v[8 * q + 2], v[8 * q + 3]),
+                        pk_bf16(v[8 * q + 4], v[8 * q + 5]), pk_bf16(v[8 * q + 6], v[8 * q + 7]));
+  }
   if (xf)
 #pragma unroll
     for (int q = 0; q < SUR_NF; ++q) xf[q] = v[q];

@@ -83,14 +83,13 @@ extern "C" __global__ void __launch_bounds__(256) gd_sur_grid_kernel(
 extern "C" __global__ void gd_sur_feat_kernel(const DevComplex *cxs, int cxi, SurGrid G, int n,
                                               const int *idx_lig, const int *idx_prt,
                                               const float *mm, int64_t row0,
-                                              unsigned short *X, unsigned short *XT,
-                                              int64_t ld, float *xf) {
+                                              unsigned short *X, float *xf) {
   const DevComplex &C = cxs[cxi];
   const int lna = C.lna;
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (int64_t)n * lna) return;
   const int pose = (int)(t / lna), l = (int)(t % lna);
-  feat_row(C, G, mm + (size_t)pose * 6, idx_lig[pose], idx_prt[pose], l, row0 + t, X, XT, ld,
+  feat_row(C, G, mm + (size_t)pose * 6, idx_lig[pose], idx_prt[pose], l, row0 + t, X,
            xf ? xf + (size_t)t * SUR_NF : nullptr);
 }
 
@@ -99,8 +98,7 @@ extern "C" __global__ void gd_sur_feat_kernel(const DevComplex *cxs, int cxi, Su
 extern "C" __global__ void gd_sur_feat_multi_kernel(const DevComplex *cxs, int n, const int *cid,
                                                     const int *idx_lig, const int *idx_prt,
                                                     const float *mm, const int64_t *row_of,
-                                                    unsigned short *X, unsigned short *XT,
-                                                    int64_t ld) {
+                                                    unsigned short *X) {
   const int pose = blockIdx.x;
   if (pose >= n) return;
   const DevComplex &C = cxs[cid[pose]];
@@ -112,8 +110,8 @@ extern "C" __global__ void gd_sur_feat_multi_kernel(const DevComplex *cxs, int n
   G.h = C.sh;
   G.n = C.sn;
   for (int l = threadIdx.x; l < C.lna; l += blockDim.x)
-    feat_row(C, G, mm + (size_t)pose * 6, idx_lig[pose], idx_prt[pose], l, row_of[pose] + l, X, XT,
-             ld, nullptr);
+    feat_row(C, G, mm + (size_t)pose * 6, idx_lig[pose], idx_prt[pose], l, row_of[pose] + l, X,
+             nullptr);
 }
 
 // Row strides (bf16) of the LDS tiles of the batch kernels: 64 + 8 and

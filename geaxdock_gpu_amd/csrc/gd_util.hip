@@ -12,6 +12,49 @@ extern "C" __global__ void gd_queue_reset_kernel(int *queue, int n) {
   if (i < n) queue[i] = 0;
 }
 
+// Accepted moves and exchanges of all replicas: out[0], out[1] (one workgroup).
+extern "C" __global__ void __launch_bounds__(1024) gd_counts_kernel(int n, const int *mc,
+                                                                   const int *x, int64_t *out) {
+  __shared__ long long red[2][16];
+  long long a = 0, b = 0;
+  for (int i = threadIdx.x; i < n; i += 1024) {
+    a += mc[i];
+    b += x[i];
+  }
+  for (int m = 32; m > 0; m >>= 1) {
+    a += __shfl_xor(a, m);
+    b += __shfl_xor(b, m);
+  }
+  const int w = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) {
+    red[0][w] = a;
+    red[1][w] = b;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    long long s = 0;
+    for (int i = 0; i < 16; ++i) s += red[threadIdx.x][i];
+    out[threadIdx.x] = s;
+  }
+}
+
+// Word copies of up to five arrays, one after the other, into dst.
+struct GatherArgs {
+  const int *src[5];
+  long long end[5];  // words up to and with each array
+  int n;
+};
+
+extern "C" __global__ void __launch_bounds__(256) gd_gather_kernel(GatherArgs A, int *dst) {
+  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < A.end[A.n - 1];
+       i += (long long)gridDim.x * 256) {
+    int q = 0;
+    long long b = 0;
+    while (i >= A.end[q]) b = A.end[q++];
+    dst[i] = A.src[q][i - b];
+  }
+}
+
 // Best-so-far := current state, for every replica.
 extern "C" __global__ void gd_reset_best_kernel(int n, const gd_energy *e_old, const float *mm,
                                                 float *best_e, float *best_mm) {
