@@ -48,7 +48,7 @@ struct HostComplex {
   int lpr = 0, apl = 0, n_chunks = 0;
   bool tiled = false;  // receptor streamed through LDS tiles
   bool ref_built = false;
-  int flat_n = 0;      // units of the flat pair loop (0: no list)
+  int flat_n[4] = {0, 0, 0, 0};  // units of the flat pair loop by split (0: no list)
   bool shape_final = false;  // lane shape fixed (the complex's energies have bits)
   std::vector<int4> chunks;  // receptor chunks (host copy)
   std::vector<int> lig_t;  // ligand atom types (host copy)
@@ -87,6 +87,8 @@ struct gd_ctx {
   Scratch pin, dev, drain_pin;
   int64_t *h_counts = nullptr;  // pinned: accepted moves and exchanges before and after a run
   std::vector<HostComplex> cx;
+  std::vector<void *> flat_bufs;  // unit lists of the flat pair loop
+  bool flat = false;              // packs with unit lists use them
   DevComplex *d_cx = nullptr;
   bool cx_dirty = true;
   // replica state
@@ -262,6 +264,17 @@ void choose_shape(int lna, int n_tmp, int force_lpr, int force_apl, int *lpr, in
   *apl = best_a;
 }
 
+// Without spread packing, packs of the automatic split take the flat pair loop
+// where a lane group's share of a receptor chunk is at most this many points on
+// average (a split that the caller fixed keeps the chunk loop, with the block
+// sizes it brings): short shares spend their time on a chunk's ends, which units do not have. Batches
+// of 40 to 100 complexes of 600 to 3,300 points, whose packs are split 2, 4 and
+// 8 ways (9 to 10 points a share): 38.7 ms by chunks, 36.1 by units at 64
+// complexes, 26.8 and 25.8 at 40, 55.1 and 52.1 at 100. Unsplit packs (20 to
+// 22 points): 77.3 ms by chunks, 104 by units at 150 complexes, 145.8 and
+// 149.6 at 300, 21.7 and 22.0 for one complex of 220 ladders.
+constexpr int FLAT_SHARE = 14;
+
 // Default tile length of receptors that do not fit in LDS.
 constexpr int DEFAULT_TILE = 256;
 
@@ -329,6 +342,7 @@ void gd_destroy(gd_ctx *ctx) {
   }
   for (auto &h : ctx->cx)
     for (void *p : h.bufs) (void)hipFree(p);
+  for (void *p : ctx->flat_bufs) (void)hipFree(p);
   void *ps[] = {ctx->d_cx, ctx->d_mm, ctx->d_eold, ctx->d_idx_tmp,
                 ctx->d_acs_mc, ctx->d_acs_x, ctx->d_rep_flat, ctx->d_ring[0], ctx->d_ring_cnt[0],
                 ctx->d_packs, ctx->d_slots, ctx->d_best_e, ctx->d_best_mm, ctx->d_ctrl,
@@ -687,6 +701,8 @@ gd_status gd_add_complex(gd_ctx *ctx, const gd_complex_desc *d, int *complex_id)
 namespace {
 
 bool spread_packing(const gd_ctx *ctx);
+int auto_gmax(const gd_ctx *ctx);
+std::vector<int> lig_splits(const gd_ctx *ctx, const HostComplex &h, int gmax);
 
 // Packs of one wave of replicas (spread packing) for a complex at lpr lanes
 // per replica.
@@ -745,15 +761,18 @@ gd_status widen_shapes(gd_ctx *ctx) {
   return GD_OK;
 }
 
-// Unit list of the flat pair loop (gd_mc.h) for lane groups of a split of 8:
+int flat_index(int ns) { return ns >= 8 ? 3 : ns >= 4 ? 2 : ns >= 2 ? 1 : 0; }
+
+// Unit list of the flat pair loop (gd_mc.h) for lane groups of a split of ns:
 // group g's share of every chunk, in chunk order, cut into units of one
 // receptor type, an even number for each type. `apl` sets the groups of NP
 // points that chunk_pairs forms (4, 2 and 1 for 1, 2 and more atoms per lane),
 // which the units' modes keep.
-std::vector<int4> build_flat_units(const std::vector<int4> &chunks, int apl, int (&off)[9]) {
+std::vector<int4> build_flat_units(const std::vector<int4> &chunks, int apl, int ns,
+                                   int (&off)[9]) {
   std::vector<int4> U;
   const int np = apl >= 3 ? 1 : (apl == 2 ? 2 : 4);
-  for (int g = 0; g < 8; ++g) {
+  for (int g = 0; g < ns; ++g) {
     off[g] = (int)U.size();
     std::vector<int> first, types;  // each type's first unit
     int lone = -1;                  // a unit of one point that may take a second
@@ -762,7 +781,7 @@ std::vector<int4> build_flat_units(const std::vector<int4> &chunks, int apl, int
         U.push_back(make_int4(FLAT_EMPTY, U.back().y, 0, 0));
     };
     for (const int4 &ch : chunks) {
-      const int fb = ch.x + (ch.y * g) / 8, fe = ch.x + (ch.y * (g + 1)) / 8;
+      const int fb = ch.x + (ch.y * g) / ns, fe = ch.x + (ch.y * (g + 1)) / ns;
       if (fb >= fe) continue;
       if (types.empty() || types.back() != ch.z) {
         even();
@@ -803,24 +822,61 @@ std::vector<int4> build_flat_units(const std::vector<int4> &chunks, int apl, int
       U[first[i]].x |= types[i] | (((end - first[i]) / 2) << FLAT_PAIRS);
     }
   }
-  off[8] = (int)U.size();
+  off[ns] = (int)U.size();
   return U;
+}
+
+// Unit lists of the complexes that lack one for a split their packs have, in
+// one device block (points and PSP columns are 16-bit in a unit and a type has
+// at most FLAT_PAIR_MASK unit pairs in a group).
+gd_status build_flat(gd_ctx *ctx) {
+  const bool spread = spread_packing(ctx);
+  const int gmax = spread ? 0 : auto_gmax(ctx);
+  std::vector<int> want(ctx->cx.size(), 0);  // bit f: packs of split 1 << f
+  int64_t points = 0, shares = 0;
+  for (size_t c = 0; c < ctx->cx.size(); ++c) {
+    const HostComplex &h = ctx->cx[c];
+    if (h.tiled) continue;
+    for (int ns : lig_splits(ctx, h, gmax)) {
+      points += (int64_t)h.d.n_prt * h.d.pnp;
+      shares += (int64_t)h.d.n_prt * h.n_chunks * ns;
+      want[c] |= 1 << flat_index(ns);
+    }
+  }
+  ctx->flat = spread || (ctx->opts.receptor_split == 0 && points <= FLAT_SHARE * shares);
+  if (!ctx->flat) return GD_OK;
+  struct Todo {
+    HostComplex *h;
+    int f;
+    size_t at;
+  };
+  std::vector<Todo> todo;
+  std::vector<int4> all;
+  for (size_t c = 0; c < ctx->cx.size(); ++c) {
+    HostComplex &h = ctx->cx[c];
+    if (h.d.pnp > 4 * FLAT_PAIR_MASK || h.d.n_res > 0x7fff) continue;
+    for (int f = 0; f < 4; ++f) {
+      if (!(want[c] >> f & 1) || h.flat_n[f] > 0) continue;
+      const std::vector<int4> U = build_flat_units(h.chunks, h.apl, 1 << f, h.dev.flat_off[f]);
+      h.flat_n[f] = (int)U.size();
+      todo.push_back({&h, f, all.size()});
+      all.insert(all.end(), U.begin(), U.end());
+    }
+  }
+  if (todo.empty()) return GD_OK;
+  void *p = nullptr;
+  HIPCHK(hipMalloc(&p, all.size() * sizeof(int4)));
+  ctx->flat_bufs.push_back(p);
+  HIPCHK(hipMemcpyAsync(p, all.data(), all.size() * sizeof(int4), hipMemcpyHostToDevice, ctx->stream));
+  HIPCHK(hipStreamSynchronize(ctx->stream));
+  for (const Todo &t : todo) t.h->dev.flat[t.f] = static_cast<int4 *>(p) + t.at;
+  return GD_OK;
 }
 
 gd_status sync_complexes(gd_ctx *ctx) {
   if (!ctx->cx_dirty) return GD_OK;
   TRY(widen_shapes(ctx));
-  // spread packing splits every receptor eight ways: its complexes get unit
-  // lists (points and PSP columns are 16-bit there, a type has at most
-  // FLAT_PAIR_MASK unit pairs in a group; receptors in LDS are far below that)
-  if (spread_packing(ctx))
-    for (HostComplex &h : ctx->cx) {
-      if (h.tiled || h.flat_n > 0 || h.d.pnp > 4096 * 4 || h.d.n_res > 0x7fff) continue;
-      const std::vector<int4> U = build_flat_units(h.chunks, h.apl, h.dev.flat_off);
-      TRY(dev_upload(ctx, h, (int4 **)&h.dev.flat, U.data(), U.size()));
-      HIPCHK(hipStreamSynchronize(ctx->stream));
-      h.flat_n = (int)U.size();
-    }
+  TRY(build_flat(ctx));
   if (ctx->d_cx) HIPCHK(hipFree(ctx->d_cx));
   ctx->d_cx = nullptr;
   for (auto &g : ctx->gslot) g.valid = false;  // captured launches hold the old pointer
@@ -960,7 +1016,7 @@ void apply_layout(KParams &P, const KParams &L) {
 // file alone (two waves per SIMD), so LDS does not split their classes.
 void pack_finish(const gd_ctx *ctx, PackSet &ps) {
   const size_t n_pk = ps.packs.size();
-  std::vector<int> res(n_pk), block(n_pk), apl(n_pk), tile(n_pk);
+  std::vector<int> res(n_pk), block(n_pk), apl(n_pk), tile(n_pk), units(n_pk);
   std::vector<double> cost(n_pk);
   for (size_t i = 0; i < n_pk; ++i) {
     Pack &p = ps.packs[i];
@@ -974,6 +1030,12 @@ void pack_finish(const gd_ctx *ctx, PackSet &ps) {
     cost[i] = (double)h.d.pnp * (double)p.half * h.apl;
     KParams L{};
     size_t need = 0;
+    // units of the flat pair loop, where they fit
+    units[i] = ctx->flat && tile[i] == 0 && block[i] == 512 ? h.flat_n[flat_index(p.ns)] : 0;
+    if (units[i] > 0) {
+      layout(L, &need, 0, h.d.pnk, h.n_chunks, p.round, block[i], p.ns > 1, 0, units[i]);
+      if (need > ctx->max_lds) units[i] = 0;
+    }
     layout(L, &need, (h.d.pnp + 3) & ~3, h.d.pnk, h.n_chunks, p.round, block[i], p.ns > 1,
            tile[i]);
     res[i] = block[i] >= 512
@@ -987,6 +1049,7 @@ void pack_finish(const gd_ctx *ctx, PackSet &ps) {
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
     if (apl[a] != apl[b]) return apl[a] < apl[b];
     if (tile[a] != tile[b]) return tile[a] < tile[b];
+    if ((units[a] > 0) != (units[b] > 0)) return units[a] > 0;
     if (block[a] != block[b]) return block[a] > block[b];
     if (res[a] != res[b]) return res[a] < res[b];
     return cost[a] > cost[b];
@@ -1003,11 +1066,13 @@ void pack_finish(const gd_ctx *ctx, PackSet &ps) {
     lc.block = block[o0];
     lc.tile = tile[o0];
     int pnp_max = 0, pnk_max = 0, nch_max = 0, slots_max = 1, half_max = 64, flat_max = 0;
-    bool split = false, flat = lc.tile == 0;
+    bool split = false;
+    const bool flat = units[o0] > 0;
     size_t e = b;
     for (; e < n_pk; ++e) {
       const int oe = order[e];
-      if (apl[oe] != lc.apl || tile[oe] != lc.tile || block[oe] != lc.block || res[oe] != res[o0])
+      if (apl[oe] != lc.apl || tile[oe] != lc.tile || block[oe] != lc.block ||
+          res[oe] != res[o0] || (units[oe] > 0) != flat)
         break;
       const Pack &p = ps.packs[e];
       const HostComplex &h = ctx->cx[p.cx];
@@ -1019,14 +1084,18 @@ void pack_finish(const gd_ctx *ctx, PackSet &ps) {
       layout(L, &need, (np + 3) & ~3, nk, nc, ns, lc.block, sp, lc.tile);
       const size_t fit = ctx->max_lds / std::max<size_t>(need, 1);
       if (e > b && (fit < 1 || (res[o0] > 1 && fit < (size_t)res[o0]))) break;
+      const int nu = std::max(flat_max, units[oe]);
+      if (flat) {
+        layout(L, &need, 0, nk, nc, ns, lc.block, sp, 0, nu);
+        if (e > b && need > ctx->max_lds) break;
+      }
+      flat_max = nu;
       pnp_max = np;
       pnk_max = nk;
       nch_max = nc;
       slots_max = ns;
       split = sp;
       half_max = std::max(half_max, p.half);
-      flat_max = std::max(flat_max, h.flat_n);
-      flat = flat && p.ns == 8 && h.flat_n > 0;
     }
     lc.end = (int)e;
     lc.half_max = half_max;
@@ -1035,7 +1104,6 @@ void pack_finish(const gd_ctx *ctx, PackSet &ps) {
     if (flat) {
       layout(lc.lay_flat, &lc.lds_flat, 0, pnk_max, nch_max, slots_max, lc.block, split, 0,
              flat_max);
-      if (lc.lds_flat > ctx->max_lds) lc.lds_flat = 0;
     }
     ps.classes.push_back(lc);
     b = e;
@@ -1115,10 +1183,11 @@ bool spread_packing(const gd_ctx *ctx) {
 
 // Receptor split of each ligand conformer's MC packs. The split sets the
 // summation order, so a pose's energy bits follow it; gd_calc_energy uses it.
-std::vector<int> lig_splits(const gd_ctx *ctx, const HostComplex &h) {
+// `gmax`: auto_gmax(ctx) (unused under spread packing).
+std::vector<int> lig_splits(const gd_ctx *ctx, const HostComplex &h, int gmax) {
   std::vector<int> ns(h.d.n_lig, spread_packing(ctx) ? 8 : 1);
   if (spread_packing(ctx)) return ns;
-  for (const LadderGroup &lg : ladder_groups(ctx, h, auto_gmax(ctx)))
+  for (const LadderGroup &lg : ladder_groups(ctx, h, gmax))
     for (int g = 0; g < lg.ng; ++g) ns[lg.l0 + g] = lg.ns;
   return ns;
 }
@@ -1357,8 +1426,8 @@ hipError_t plan_classes(gd_ctx *ctx, const std::vector<LaunchClass> &classes, co
     ClassLaunch cl;
     cl.P = P0;
     KParams &P = cl.P;
-    // the flat pair loop where every pack is split eight ways and the units
-    // fit; the direct network evaluation keeps the layout its scratch fits in
+    // the flat pair loop where the packs have unit lists; the direct network
+    // evaluation keeps the layout its scratch fits in
     const bool flat = lc.lds_flat > 0 && !da_scratch;
     apply_layout(P, flat ? lc.lay_flat : lc.lay);
     P.pack_base = lc.begin;
@@ -1972,7 +2041,7 @@ static gd_status eval_poses(gd_ctx *ctx, int cid, int n, const int *idx_lig, con
   // each pose is evaluated with the receptor split of its ligand conformer's
   // MC packs, so a pose's energy has the bits an MC step gives it
   std::vector<int> lig_ns = h.lig_ns;
-  if (lig_ns.size() != (size_t)h.d.n_lig) lig_ns = lig_splits(ctx, h);
+  if (lig_ns.size() != (size_t)h.d.n_lig) lig_ns = lig_splits(ctx, h, auto_gmax(ctx));
   // poses by protein conformer and split
   std::vector<int> key(n), start(h.d.n_prt * 4 + 1, 0), order(n);
   for (int i = 0; i < n; ++i) {
@@ -1987,11 +2056,11 @@ static gd_status eval_poses(gd_ctx *ctx, int cid, int n, const int *idx_lig, con
   }
   // the launch takes the flat pair loop (plan_classes): a list that fits, and
   // no scratch of the direct network evaluation
-  bool flat = h.flat_n > 0 && !(out_sur && !ctx->sur.tab_valid);
+  bool flat = ctx->flat && h.flat_n[3] > 0 && !(out_sur && !ctx->sur.tab_valid);
   if (flat) {
     KParams L{};
     size_t need = 0;
-    layout(L, &need, 0, h.d.pnk, h.n_chunks, std::max(1, 64 / h.lpr), 512, true, 0, h.flat_n);
+    layout(L, &need, 0, h.d.pnk, h.n_chunks, std::max(1, 64 / h.lpr), 512, true, 0, h.flat_n[3]);
     flat = need <= ctx->max_lds;
   }
   PackSet ps;

@@ -58,9 +58,10 @@ struct DevComplex {
   const float *prt_hpp;    // [pnp] hpp where c0_and_d12_or_c2, else 0
   const int *prt_psp;      // [pnp] seq3r where class 2, else -1
   const int4 *chunks;      // [n_chunks] start, length, type, kind
-  // units of the flat pair loop by lane group of a split of 8 (null: none)
-  const int4 *flat;        // [flat_off[8]] flag word, first point | second << 16, 0, 0
-  int flat_off[9];
+  // units of the flat pair loop for receptor splits of 1, 2, 4 and 8 (null:
+  // none), group g of split 1 << f: [flat_off[f][g], flat_off[f][g + 1])
+  const int4 *flat[4];     // flag word, first point | second << 16, 0, 0
+  int flat_off[4][9];
   const float *params;     // [NPT * NLT * NPAR]
   const float *lig_orig;   // [n_lig][3][lna]
   const int *lig_t;        // [lna]

@@ -519,16 +519,19 @@ __device__ __forceinline__ void flat_unit(int ux, bool hb, bool wide, const Flat
   }
 }
 
-// All units of lane group h. A receptor type's units come in an even number
-// (the last may be empty), two register sets in turn.
+// Unit list of a receptor split (1, 2, 4 or 8).
+__device__ __forceinline__ int flat_index(int ns) { return 31 - __builtin_clz(ns); }
+
+// All units of lane group h (list bounds `off`). A receptor type's units come in
+// an even number (the last may be empty), two register sets in turn.
 template <int APL>
-__device__ __forceinline__ void flat_pairs(const DevComplex &C, const Lds &S, int h,
+__device__ __forceinline__ void flat_pairs(const int *off, const Lds &S, int h,
                                            const PairConst &K, const float (&x)[APL],
                                            const float (&y)[APL], const float (&z)[APL],
                                            const int (&lt)[APL], gfloat_p const (&psprow)[APL],
                                            FlatAcc<APL> &A) {
-  const int u0 = __builtin_amdgcn_readfirstlane(C.flat_off[h]);
-  int left = __builtin_amdgcn_readfirstlane(C.flat_off[h + 1]) - u0;
+  const int u0 = __builtin_amdgcn_readfirstlane(off[h]);
+  int left = __builtin_amdgcn_readfirstlane(off[h + 1]) - u0;
   if (left <= 0) return;
   const float *rec[APL];
 #pragma unroll
@@ -660,7 +663,7 @@ __device__ __forceinline__ float mcs_sum(const DevComplex &C, int lpr, const flo
 // Every thread runs the tile loop (waves without a pose only stage). Chunks
 // that cross a tile boundary are evaluated as one fragment per tile.
 //
-// FLAT: every pack of the launch has a split of 8 and a unit list in LDS; the
+// FLAT: every pack of the launch has the unit list of its split in LDS; the
 // pair loop is flat_pairs.
 template <int APL, bool TILE, bool FLAT>
 __device__ __forceinline__ void pose_energy(const DevComplex &C, const Lds &S, int lpr, Split &sp,
@@ -766,7 +769,7 @@ __device__ __forceinline__ void pose_energy(const DevComplex &C, const Lds &S, i
         prow[k] = glob(psprow[k]);
       }
       A.pend = false;
-      flat_pairs<APL>(C, S, sp.h, K, x, y, z, lt, prow, A);
+      flat_pairs<APL>(C.flat_off[flat_index(sp.ns)], S, sp.h, K, x, y, z, lt, prow, A);
 #pragma unroll
       for (int k = 0; k < APL; ++k) {
         vdw[k] = A.vdw[k];
@@ -1581,9 +1584,11 @@ __device__ __forceinline__ void mc_kernel_body(const KParams &P, int idx, int st
     int4 *ch = reinterpret_cast<int4 *>(lds + P.off_ch);
     if constexpr (FLAT) {
       // each unit: its two points of this conformer and its attributes
-      const int n_units = C.flat_off[8];
+      const int fi = flat_index(pk.ns);
+      const int n_units = C.flat_off[fi][pk.ns];
+      const int4 *units = C.flat[fi];
       for (int i = threadIdx.x; i < n_units; i += nt) {
-        const int4 f = C.flat[i];
+        const int4 f = units[i];
         const int p0 = f.y & 0xffff, p1 = (unsigned)f.y >> 16;
         int4 a = make_int4(f.x, __float_as_int(0.5f * C.prt_hpp[p0]),
                            __float_as_int(0.5f * C.prt_hpp[p1]),
