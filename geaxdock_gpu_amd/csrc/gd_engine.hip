@@ -12,6 +12,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <limits>
 #include <string>
 #include <vector>
 
@@ -239,6 +240,40 @@ struct Regions {
 // inputs from the pinned staging and write their results there. A copy costs
 // 5 to 10 us each way whatever its size; these reads cross the bus once.
 constexpr size_t ZERO_COPY_BYTES = 65536;
+
+// Squared distance beyond which every pair of the complex can go without the
+// PMF's exponential, HPC and the contact terms, with the same bits: there
+// e <= 2^-26, so den + den e and num + num e round to den and num; u is 0; no
+// contact or near electrostatic form holds. The PMF exponent's upper root of
+// (d - 12)(d - pmf0) = 2 * 26 / log2(e). Infinite (nothing is skipped) for
+// values with which a skipped term could be other than an exact zero: those
+// not finite, or so large that a distance's ninth power overflows.
+float skip_range2(const gd_complex_desc &d, const std::vector<float> &par) {
+  const float none = std::numeric_limits<float>::infinity();
+  for (size_t i = 0; i < (size_t)d.n_prt * d.pnp; ++i)
+    if (!(std::fabs(d.prt_x[i]) < FAR_COORD && std::fabs(d.prt_y[i]) < FAR_COORD &&
+          std::fabs(d.prt_z[i]) < FAR_COORD))
+      return none;
+  bool lt[NLT] = {}, pt[NPT] = {};
+  for (int l = 0; l < d.lna; ++l) lt[d.lig_t[l]] = true;
+  for (int p = 0; p < d.pnp; ++p) {
+    pt[d.prt_t[p]] = true;
+    if (!std::isfinite(d.prt_hpp[p])) return none;
+  }
+  double r2 = 82.0;
+  for (int j = 0; j < NPT; ++j)
+    for (int i = 0; i < NLT; ++i) {
+      if (!pt[j] || !lt[i]) continue;
+      const float *r = &par[(j * NLT + i) * NPAR];
+      for (int q : {P_P1A, P_P2A, P_A0, P_A1, P_HA, P_HB, P_HC})
+        if (!(std::fabs(r[q]) < 1e20f)) return none;
+      if (!(std::fabs(r[P_PMF0]) < 1e4f) || !(r[P_HA] >= 0.0f)) return none;
+      const double p = r[P_PMF0], D = (12.0 - p) * (12.0 - p) + 8.0 * 26.0 / 1.4426950408889634;
+      const double F = 0.5 * (12.0 + p + std::sqrt(D));
+      r2 = std::max({r2, F * F, (double)r[P_NR2]});
+    }
+  return (float)(r2 * 1.002);
+}
 
 // Lanes per replica and atoms per lane: the fewest lane slots lpr*apl that
 // hold lna atoms with apl <= 4, preferring 2..3 atoms per lane on ties (more
@@ -618,6 +653,7 @@ gd_status gd_add_complex(gd_ctx *ctx, const gd_complex_desc *d, int *complex_id)
   D.b1 = ep.b1;
   D.kde2l = ep.kde2 * 1.44269504088896340736f;
   D.kde3 = ep.kde3;
+  D.far2 = skip_range2(*d, par);
   for (int i = 0; i < GD_MAXWEI; ++i) {
     D.w[i] = ep.w[i];
     D.a_para[i] = ep.a_para[i];

@@ -25,6 +25,9 @@ enum { P_P1A = 0, P_P2A, P_PMF0, P_PMF1, P_HA, P_HB, P_HC, P_NR2, P_A0, P_A1, P_
 // pocket-specific potential (class 2).
 enum { KIND_PLAIN = 0, KIND_HPC = 1, KIND_PSP = 2 };
 
+// Ligand and receptor coordinates within which terms are skipped by distance.
+constexpr float FAR_COORD = 4000.0f;
+
 // Units of the flat pair loop (gd_mc.h). Flag word: on the first unit of a
 // receptor type, that type and the number of unit pairs; on every unit the flags
 // and the mode (top two bits).
@@ -51,6 +54,7 @@ struct DevComplex {
   float pocket[3];
   float move_scale[6];
   float el0, el1, a1, b1, kde2l, kde3;
+  float far2;     // skip_range2 (gd_engine.hip)
   float w[GD_MAXWEI], a_para[GD_MAXWEI], b_para[GD_MAXWEI];
   float hpl0[NLT], hpl1[NLT], hpl2[NLT];
   float minus_beta[GD_MAX_NTMP];

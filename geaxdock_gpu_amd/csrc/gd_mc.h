@@ -130,6 +130,27 @@ struct ChunkPar {
   float nr2;  // contacts and the near electrostatic form lie within sqrt(nr2)
 };
 
+// Squared distances that let a group of pairs skip terms without a change of
+// bits, per lane for one receptor type.
+struct Range {
+  float nr2;   // contacts, the near electrostatic form and PSP lie within
+  float far2;  // beyond: the PMF's exponential does not change 1 + e, HPC is 0
+  float hb2;   // beyond: every H-bond term is exactly 0
+};
+
+// Largest squared distance at which an H-bond term of these records is not 0:
+// exp2(-h^2) is 0 below 2^-126 (the hardware's exp2 has no denormals), h = 11.3
+// lies beyond it. `all` (a pose or a complex outside the range that the skips
+// are proven for): every distance.
+template <int APL>
+__device__ __forceinline__ float hb_range2(const ChunkPar (&cp)[APL], bool all) {
+  float r = 0.0f;
+#pragma unroll
+  for (int k = 0; k < APL; ++k)
+    if (cp[k].hc != 0.0f) r = fmaxf(r, (11.3f - cp[k].hb) * fast_rcp(cp[k].ha));
+  return all ? __builtin_huge_valf() : r * r * 1.001f;
+}
+
 // Receptor points [p, p + NP) of one chunk against the lane's APL atoms.
 // All terms of src/kernel_cuda_l2_calcenergy.cu:105-184 plus the contact
 // count of CalcMcc_d:
@@ -147,16 +168,27 @@ struct ChunkPar {
 //   psp  psp[lig_t][seq3r] when class 2 and d <= pmf0 (KIND == 2);
 //   contacts  d <= pmf0.
 // Every pair takes the full form of every term, so a pair's contribution is
-// a function of that pair alone. One wave-uniform branch skips work no lane
-// needs: contacts, the near electrostatic form and PSP run only when some lane
-// is within contact range (the terms inside test each pair exactly, so pairs
-// outside add exact zeros). Two chunk-uniform choices are template parameters:
-// CLAMP keeps the PMF exponent finite where the chunk's pmf0 lets it grow
-// past 60, HB evaluates the H-bond term where some lane's atom has an H-bond
-// record with the chunk's receptor type.
+// a function of that pair alone. Wave-uniform branches skip only what leaves
+// every lane's sums as they are, bit for bit (Range): where all lanes are
+// beyond far2 (about 15.5 A) the PMF's exponential is below 2^-26, so den + den e
+// and num + num e round to den and num, and HPC and contacts are exact zeros;
+// beyond a lane's hb2 its H-bond terms are exact zeros; contacts, the near
+// electrostatic form and PSP run only when some lane is within contact range
+// (the terms inside test each pair exactly). Two chunk-uniform choices are
+// template parameters: CLAMP keeps the PMF exponent finite where the chunk's
+// pmf0 lets it grow past 60, HB evaluates the H-bond term where some lane's
+// atom has an H-bond record with the chunk's receptor type.
+// Bound: VALU issue (95 % on the CUs that hold a pack). The two distance tests
+// cost a compare each per group of points; in the ensemble of 3,520 replicas
+// (3,000 points) they take 12 % of the transcendentals and 6 % of the VALU
+// instructions away, 21.6 -> 20.5 ms a kernel of 40 steps; 2,000 poses on 8,000
+// points 1,624 -> 1,535 us a call. With kind, clamp and H-bond as run-time
+// branches instead (one variant of the loop) the ensemble took 5 % longer. The flat
+// loop below goes without the tests: its units hold points of smaller receptors,
+// few of them far, and they cost 3 % there.
 template <int APL, int KIND, int NP, bool CLAMP, bool HB>
 __device__ __forceinline__ void pair_group(const Lds &S, int p, const float4 (&P)[NP],
-                                           const PairConst &K, float nr2max,
+                                           const PairConst &K, const Range &G,
                                            const float (&x)[APL], const float (&y)[APL],
                                            const float (&z)[APL], const ChunkPar (&cp)[APL],
                                            const float *const (&psprow)[APL],
@@ -172,14 +204,10 @@ __device__ __forceinline__ void pair_group(const Lds &S, int p, const float4 (&P
     hp[j] = (KIND >= KIND_HPC) ? S.hpp[p + j] : 0.0f;
     ps[j] = (KIND == KIND_PSP) ? S.psp[p + j] : 0;
   }
-  float d2[NP][APL], rd[NP][APL], dd[NP][APL], num[NP][APL], den[NP][APL];
-  bool near = false;
+  float d2[NP][APL], rd[NP][APL], dd[NP][APL], num[NP][APL], den[NP][APL], dn[NP][APL];
+  float qmin = 0.0f;  // the lane's nearest atom to any of the points
 #pragma unroll
   for (int j = 0; j < NP; ++j) {
-    // contact range: the lane's nearest atom against the largest of its
-    // atoms' near radii (a superset of the pairs the branch needs; the terms
-    // inside test each pair exactly)
-    float qmin = 0.0f;
 #pragma unroll
     for (int k = 0; k < APL; ++k) {
       const float q2 = pair_d2(x[k], y[k], z[k], P[j].x, P[j].y, P[j].z);
@@ -188,66 +216,83 @@ __device__ __forceinline__ void pair_group(const Lds &S, int p, const float4 (&P
       d2[j][k] = q2;
       rd[j][k] = r;
       dd[j][k] = d;
-      qmin = k == 0 ? q2 : fminf(qmin, q2);
+      qmin = j == 0 && k == 0 ? q2 : fminf(qmin, q2);
       const float d3 = q2 * d;
       const float d6 = d3 * d3;
       num[j][k] = fmaf(-cp[k].p2a, d3, cp[k].p1a);
-      den[j][k] = fmaf(d6, d3, fmaf(cp[k].a1, q2, cp[k].a0));
+      den[j][k] = dn[j][k] = fmaf(d6, d3, fmaf(cp[k].a1, q2, cp[k].a0));
       ele[k] = fmaf(P[j].w, r, ele[k]);
     }
-    near |= qmin <= nr2max;
+  }
+  if (__ballot(!(qmin > G.far2)) != 0) {
+#pragma unroll
+    for (int j = 0; j < NP; ++j)
+#pragma unroll
+      for (int k = 0; k < APL; ++k) {
+        const float q2 = d2[j][k];
+        // the exponent is clamped at 64 (exp2 must stay finite) only in chunks
+        // whose parameters let it reach 60; elsewhere the clamp is a no-op
+        const float wv0 = fmaf(pa, q2, fmaf(cp[k].pb, dd[j][k], cp[k].pc));
+        const float wv = CLAMP ? fminf(wv0, 64.0f) : wv0;
+        // den (1 + e) and num (1 + e) as den + den e and num + num e: one
+        // fma each, one rounding each
+        const float e = fast_exp2(wv);
+        dn[j][k] = fmaf(den[j][k], e, den[j][k]);
+        num[j][k] = fmaf(num[j][k], e, num[j][k]);
+        if (KIND >= KIND_HPC) {
+          // u <= 1, so clamping to [0, 1] is max(u, 0): the fma's own clamp
+          const float u = __builtin_amdgcn_fmed3f(fmaf(q2, -INV81, 1.0f), 0.0f, 1.0f);
+          const float u3 = u * u * u;
+          hpc[k] = fmaf(hp[j], fmaf(u3, u, u3), hpc[k]);
+        }
+      }
+    // contact range: the lane's nearest atom against the largest of its
+    // atoms' near radii (a superset of the pairs the branch needs; the terms
+    // inside test each pair exactly)
+    if (__ballot(qmin <= G.nr2) != 0) {
+#pragma unroll
+      for (int j = 0; j < NP; ++j)
+#pragma unroll
+        for (int k = 0; k < APL; ++k) {
+          const float d = dd[j][k];
+          const bool c = d <= cp[k].pmf0;
+          cnt[k] += c ? 1 : 0;
+          const float s = K.el1 * d;
+          if (s < 1.0f) {
+            const float gn = fmaf(s * s, fmaf(K.b1, s, K.a1), K.el0);
+            ele[k] = fmaf(P[j].w, fmaf(K.el1, gn, -rd[j][k]), ele[k]);
+          }
+          if (KIND == KIND_PSP) {
+            if (c) psp[k] += psprow[k][ps[j]];
+          }
+        }
+    }
+  }
+  // H-bond: only in chunks where some lane's atom has an H-bond record with
+  // this receptor type (elsewhere every term would be 0 * exp2), and there
+  // only where such a lane is within its records' range
+  if (HB && __ballot(!(qmin > G.hb2)) != 0) {
+#pragma unroll
+    for (int j = 0; j < NP; ++j)
+#pragma unroll
+      for (int k = 0; k < APL; ++k) {
+        const float h = fmaf(dd[j][k], cp[k].ha, cp[k].hb);
+        hdb[k] = fmaf(cp[k].hc, fast_exp2(-(h * h)), hdb[k]);
+      }
   }
 #pragma unroll
   for (int j = 0; j < NP; ++j)
 #pragma unroll
     for (int k = 0; k < APL; ++k) {
-      const float q2 = d2[j][k], d = dd[j][k];
-      // the exponent is clamped at 64 (exp2 must stay finite) only in chunks
-      // whose parameters let it reach 60; elsewhere the clamp is a no-op
-      const float wv0 = fmaf(pa, q2, fmaf(cp[k].pb, d, cp[k].pc));
-      const float wv = CLAMP ? fminf(wv0, 64.0f) : wv0;
-      // den (1 + e) and num (1 + e) as den + den e and num + num e: one
-      // fma each, one rounding each
-      const float e = fast_exp2(wv);
-      const float r = fast_rcp(fmaf(den[j][k], e, den[j][k]));
-      vdw[k] = fmaf(fmaf(num[j][k], e, num[j][k]), r, vdw[k]);
+      const float r = fast_rcp(dn[j][k]);
+      vdw[k] = fmaf(num[j][k], r, vdw[k]);
       pmf[k] = fmaf(den[j][k], r, pmf[k]);
-      // H-bond: only in chunks where some lane's atom has an H-bond record
-      // with this receptor type (elsewhere every term would be 0 * exp2)
-      if (HB) {
-        const float h = fmaf(d, cp[k].ha, cp[k].hb);
-        hdb[k] = fmaf(cp[k].hc, fast_exp2(-(h * h)), hdb[k]);
-      }
-      if (KIND >= KIND_HPC) {
-        // u <= 1, so clamping to [0, 1] is max(u, 0): the fma's own clamp
-        const float u = __builtin_amdgcn_fmed3f(fmaf(q2, -INV81, 1.0f), 0.0f, 1.0f);
-        const float u3 = u * u * u;
-        hpc[k] = fmaf(hp[j], fmaf(u3, u, u3), hpc[k]);
-      }
     }
-  if (__ballot(near) != 0) {
-#pragma unroll
-    for (int j = 0; j < NP; ++j)
-#pragma unroll
-      for (int k = 0; k < APL; ++k) {
-        const float d = dd[j][k];
-        const bool c = d <= cp[k].pmf0;
-        cnt[k] += c ? 1 : 0;
-        const float s = K.el1 * d;
-        if (s < 1.0f) {
-          const float gn = fmaf(s * s, fmaf(K.b1, s, K.a1), K.el0);
-          ele[k] = fmaf(P[j].w, fmaf(K.el1, gn, -rd[j][k]), ele[k]);
-        }
-        if (KIND == KIND_PSP) {
-          if (c) psp[k] += psprow[k][ps[j]];
-        }
-      }
-  }
 }
 
 template <int APL, int KIND, bool CLAMP, bool HB>
 __device__ __forceinline__ void chunk_pairs(const Lds &S, int beg, int end, const PairConst &K,
-                                            float nr2max,
+                                            const Range &G,
                                             const float (&x)[APL], const float (&y)[APL],
                                             const float (&z)[APL], const ChunkPar (&cp)[APL],
                                             const float *const (&psprow)[APL],
@@ -275,22 +320,22 @@ __device__ __forceinline__ void chunk_pairs(const Lds &S, int beg, int end, cons
     for (; p + 2 * NP <= end; p += 2 * NP) {
 #pragma unroll
       for (int j = 0; j < NP; ++j) Pb[j] = S.xyze[p + NP + j];
-      pair_group<APL, KIND, NP, CLAMP, HB>(S, p, Pa, K, nr2max, x, y, z, cp, psprow, vdw, ele,
+      pair_group<APL, KIND, NP, CLAMP, HB>(S, p, Pa, K, G, x, y, z, cp, psprow, vdw, ele,
                                            pmfc, psp, hdb, hpc, cnt);
 #pragma unroll
       for (int j = 0; j < NP; ++j) Pa[j] = S.xyze[min(p + 2 * NP + j, end - 1)];
-      pair_group<APL, KIND, NP, CLAMP, HB>(S, p + NP, Pb, K, nr2max, x, y, z, cp, psprow, vdw,
+      pair_group<APL, KIND, NP, CLAMP, HB>(S, p + NP, Pb, K, G, x, y, z, cp, psprow, vdw,
                                            ele, pmfc, psp, hdb, hpc, cnt);
     }
     if (p + NP <= end) {
-      pair_group<APL, KIND, NP, CLAMP, HB>(S, p, Pa, K, nr2max, x, y, z, cp, psprow, vdw, ele,
+      pair_group<APL, KIND, NP, CLAMP, HB>(S, p, Pa, K, G, x, y, z, cp, psprow, vdw, ele,
                                            pmfc, psp, hdb, hpc, cnt);
       p += NP;
     }
   }
   for (; p < end; ++p) {
     const float4 P1[1] = {S.xyze[p]};
-    pair_group<APL, KIND, 1, CLAMP, HB>(S, p, P1, K, nr2max, x, y, z, cp, psprow, vdw, ele, pmfc,
+    pair_group<APL, KIND, 1, CLAMP, HB>(S, p, P1, K, G, x, y, z, cp, psprow, vdw, ele, pmfc,
                                         psp, hdb, hpc, cnt);
   }
 #pragma unroll
@@ -690,6 +735,20 @@ __device__ __forceinline__ void pose_energy(const DevComplex &C, const Lds &S, i
     psprow[k] = C.psp + (size_t)lt[k] * C.n_res;
   }
 
+  // A pose of ordinary coordinates (so that no power of a distance overflows)
+  // on a complex of ordinary parameters may skip terms by distance.
+  float far2 = C.far2;
+  bool odd;
+  {
+    bool o = false;
+#pragma unroll
+    for (int k = 0; k < APL; ++k)
+      o |= !(fabsf(x[k]) < FAR_COORD && fabsf(y[k]) < FAR_COORD && fabsf(z[k]) < FAR_COORD);
+    odd = live && __ballot(o) != 0;
+  }
+  odd |= !(far2 < __builtin_huge_valf());
+  if (odd) far2 = __builtin_huge_valf();
+
   // fragment [fb, fe) of chunk ci, indices into T's point arrays; each lane
   // group of a receptor split takes its share
   auto fragment = [&](const Lds &T, int ci, int fb, int fe) {
@@ -728,19 +787,22 @@ __device__ __forceinline__ void pose_energy(const DevComplex &C, const Lds &S, i
     // the PMF exponent (6 - d/2)(d - pmf0) log2(e) peaks at (pmf0 - 12)^2 / 8
     // log2(e); only a chunk where some lane's peak passes 60 needs the clamp
     bool wide = false, hbond = false;
-    float nr2max = cp[0].nr2;
+    Range G;
+    G.nr2 = cp[0].nr2;
+    G.far2 = far2;
+    G.hb2 = hb_range2<APL>(cp, odd);
 #pragma unroll
     for (int k = 0; k < APL; ++k) {
       const float t = cp[k].pmf0 - 12.0f;
       wide |= !(0.125f * LOG2E * t * t <= 60.0f);
       hbond |= cp[k].hc != 0.0f;
-      nr2max = fmaxf(nr2max, cp[k].nr2);
+      G.nr2 = fmaxf(G.nr2, cp[k].nr2);
     }
     const bool clamp = __ballot(wide) != 0;
     const bool hb = __ballot(hbond) != 0;
     auto pairs = [&](auto kind_c, auto clamp_c, auto hb_c) {
       chunk_pairs<APL, decltype(kind_c)::value, decltype(clamp_c)::value,
-                  decltype(hb_c)::value>(T, beg, end, K, nr2max, x, y, z, cp, psprow, vdw, ele,
+                  decltype(hb_c)::value>(T, beg, end, K, G, x, y, z, cp, psprow, vdw, ele,
                                          pmf, psp, hdb, hpc, cnt);
     };
     auto by_hb = [&](auto kind_c, auto clamp_c) {
