@@ -85,7 +85,7 @@ struct gd_ctx {
   // (also read and written by kernels directly for small calls) and device
   // memory; `drain` is the record drains' own pinned staging (a drain runs
   // beside a window)
-  Scratch pin, dev, drain_pin;
+  Scratch pin, dev, drain_pin, tree;
   int64_t *h_counts = nullptr;  // pinned: accepted moves and exchanges before and after a run
   std::vector<HostComplex> cx;
   std::vector<void *> flat_bufs;  // unit lists of the flat pair loop
@@ -388,6 +388,7 @@ void gd_destroy(gd_ctx *ctx) {
   scratch_free(ctx->pin, true);
   scratch_free(ctx->drain_pin, true);
   scratch_free(ctx->dev, false);
+  scratch_free(ctx->tree, false);
   for (auto &g : ctx->gslot)
     if (g.exec) (void)hipGraphExecDestroy(g.exec);
   for (void *p : ps)
@@ -1437,7 +1438,7 @@ int da_instance(const gd_ctx *ctx, bool tab) {
 struct ClassLaunch {
   const void *f;
   KParams P;
-  int grid, block;
+  int grid, block, packs;
   size_t lds;
 };
 
@@ -1482,7 +1483,7 @@ hipError_t plan_classes(gd_ctx *ctx, const std::vector<LaunchClass> &classes, co
       P.off_da = (int)((cl.lds + 15) & ~(size_t)15);
     }
     const int n_pk = lc.end - lc.begin;
-    cl.grid = n_pk;
+    cl.grid = cl.packs = n_pk;
     if (queue) {
       // resident workgroups: LDS-limited, and at most 8 waves per CU (the
       // kernels' register use allows two waves per SIMD)
@@ -1730,6 +1731,35 @@ gd_status launch_mc(gd_ctx *ctx, int mode, int step0, int n_steps, int nc, float
   return launch_mc_wait(ctx, ms);
 }
 
+// Steps that one launch of a small context takes through a tree of energies
+// (MODE_TREE in gd_mc.h): the deepest tree whose nodes, one workgroup each per
+// pack, still run side by side, one workgroup per CU. 1: plain MC launches.
+// A launch of two steps already pays at the line (85 packs, small receptors
+// of 300 points: 2.4 -> 2.25 ms for 100 steps; 2,000 points: 5.5 -> 2.9 ms at
+// 32 packs); beyond it the nodes would queue.
+int tree_depth(const gd_ctx *ctx) {
+  int64_t packs = 0;
+  for (const LaunchClass &lc : ctx->mc_classes) packs += lc.end - lc.begin;
+  int d = 1;
+  while (d < TREE_DEPTH && packs * ((2 << d) - 1) <= ctx->n_cu) ++d;
+  return d;
+}
+
+// The packs' counts of finished nodes (zero between launches), then the
+// energies of the tree's nodes for every replica.
+gd_status tree_buffers(gd_ctx *ctx, int depth, int **cnt, gd_energy **e) {
+  size_t packs = 0;
+  for (const LaunchClass &lc : ctx->mc_classes) packs = std::max(packs, (size_t)lc.end);
+  Regions R;
+  const size_t o_cnt = R.add(packs * sizeof(int));
+  const size_t o_e = R.add((size_t)ctx->n_rep * ((1 << depth) - 1) * sizeof(gd_energy));
+  TRY(scratch_need(ctx, ctx->tree, R.end, false));
+  *cnt = reinterpret_cast<int *>(ctx->tree.p + o_cnt);
+  *e = reinterpret_cast<gd_energy *>(ctx->tree.p + o_e);
+  HIPCHK(hipMemsetAsync(*cnt, 0, packs * sizeof(int), ctx->stream));
+  return GD_OK;
+}
+
 // One window of spread packing: MC launches that end on exchange steps, each
 // followed by the ladder exchange kernel, all enqueued at once and timed
 // together (waiting for each launch left the GPU idle for 60 to 90 us every
@@ -1737,8 +1767,9 @@ gd_status launch_mc(gd_ctx *ctx, int mode, int step0, int n_steps, int nc, float
 gd_status spread_window(gd_ctx *ctx, int win, int nc, int da_k, float sur_scale, double *ms_sum,
                         int *launches) {
   KParams P = mc_params(ctx, da_k, sur_scale);
-  const int da = P.da_k > 0 ? da_instance(ctx, P.sur_tab != 0) : 0;
   const bool persistent = (ctx->opts.launch & GD_LAUNCH_PERSISTENT) != 0;
+  const int depth = da_k > 0 || persistent ? 1 : tree_depth(ctx);
+  const int da = P.da_k > 0 ? da_instance(ctx, P.sur_tab != 0) : depth > 1 ? DA_TREE : 0;
   int *queue = persistent ? ctx->d_ctrl + 1 : nullptr;
   std::vector<ClassLaunch> cls;
   const hipError_t pe =
@@ -1746,16 +1777,40 @@ gd_status spread_window(gd_ctx *ctx, int win, int nc, int da_k, float sur_scale,
   if (pe == hipErrorInvalidValue)
     return fail(ctx, GD_ERR_CAPACITY, "delayed acceptance scratch does not fit in LDS");
   HIPCHK(pe);
+  int *tree_cnt = nullptr;
+  gd_energy *tree_e = nullptr;
+  if (depth > 1) TRY(tree_buffers(ctx, depth, &tree_cnt, &tree_e));
   HIPCHK(hipEventRecord(ctx->ev0, ctx->stream));
   for (int done = 0; done < win;) {
     const int s = (int)ctx->step;
     int sub = win - done;
     if (nc > 0) sub = std::min(sub, nc - s % nc);
-    for (ClassLaunch &cl : cls) {
-      cl.P.step0 = s;
-      cl.P.n_steps = sub;
+    if (depth > 1) {
+      // even shares of the interval, none deeper than `depth`
+      const int rounds = (sub + depth - 1) / depth;
+      for (int r = 0, at = s; r < rounds; ++r) {
+        const int d = (s + sub - at) / (rounds - r);
+        for (ClassLaunch &cl : cls) {
+          cl.P.mode = MODE_TREE;
+          cl.P.tree_cnt = tree_cnt;
+          cl.P.ev_out = tree_e;
+          cl.P.step0 = at;
+          cl.P.n_steps = d;
+          cl.P.tree_nodes = (1 << d) - 1;
+          cl.P.tree_packs = cl.packs;
+          cl.grid = cl.packs * cl.P.tree_nodes;
+        }
+        HIPCHK(enqueue_classes(ctx, cls, nullptr, ctx->stream));
+        at += d;
+      }
+      *launches += rounds - 1;
+    } else {
+      for (ClassLaunch &cl : cls) {
+        cl.P.step0 = s;
+        cl.P.n_steps = sub;
+      }
+      HIPCHK(enqueue_classes(ctx, cls, queue, ctx->stream));
     }
-    HIPCHK(enqueue_classes(ctx, cls, queue, ctx->stream));
     if (nc > 0 && (s + sub) % nc == 0) {
       hipLaunchKernelGGL(gd_ladder_exchange_kernel, dim3((ctx->n_ladders + 63) / 64), dim3(64),
                          0, ctx->stream, ctx->d_cx, ctx->d_ladders, ctx->n_ladders, s + sub, nc,

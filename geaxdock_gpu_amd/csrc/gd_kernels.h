@@ -107,7 +107,10 @@ struct Pack {
 };
 
 // MODE_SUREVAL: surrogate total of given poses (delayed-acceptance kernels)
-enum { MODE_MC = 0, MODE_INIT = 1, MODE_EVAL = 2, MODE_SUREVAL = 3 };
+// MODE_TREE: the next n_steps MC steps by a tree of energies (gd_mc.h)
+enum { MODE_MC = 0, MODE_INIT = 1, MODE_EVAL = 2, MODE_SUREVAL = 3, MODE_TREE = 4 };
+constexpr int DA_TREE = 5;     // its kernel instances (see mc_kernel_handle)
+constexpr int TREE_DEPTH = 6;  // a wave's lanes hold the 2^depth - 1 energies
 
 struct KParams {
   const DevComplex *cxs;
@@ -130,6 +133,10 @@ struct KParams {
   const float *ev_mm;
   const int *ev_lig;
   gd_energy *ev_out;
+  // MODE_TREE: workgroups (node, pack) of tree_packs packs; ev_out holds
+  // [slot value][tree_nodes] energies, tree_cnt[pack] counts finished nodes
+  int tree_nodes, tree_packs;
+  int *tree_cnt;
   int mode;
   int step0, n_steps, nc;
   const int *step_dev;  // when set, the first step is read here (graph replays)
@@ -157,8 +164,8 @@ struct KParams {
 // Host handle of the MC kernel instance for `APL` ligand atoms per lane,
 // mode `da` (0 plain, 1 delayed acceptance with the network per atom, 2 with
 // its tabulated outputs) and receptor layout; defined in gd_mc_inst.hip, one
-// object per APL. REC_FLAT has instances for modes 0, 2 and 4 (null for the
-// others).
+// object per APL. REC_FLAT has instances for modes 0, 2, 4 and DA_TREE
+// (null for the others).
 enum { REC_CHUNKS = 0, REC_TILED = 1, REC_FLAT = 2 };
 template <int APL>
 const void *mc_kernel_handle(int da, int rec);

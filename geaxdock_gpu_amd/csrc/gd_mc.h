@@ -1293,14 +1293,128 @@ __device__ __forceinline__ void exchange_ladder(int n_tmp, int mode_t, const flo
   }
 }
 
-// DA: 0 plain Metropolis; delayed acceptance with the surrogate from the
+// ---- MC steps by a tree of energies -----------------------------------------
+// A context with few packs leaves most CUs idle, and one MC step waits for the
+// one before it. But a step's proposal needs only the random numbers of its
+// step and the state it starts from, and that state is known up to the outcomes
+// of the steps between: from one known state, the 2^D - 1 poses that the next D
+// steps can propose are the nodes of a binary tree (node v's children: 2v after
+// a rejection, 2v + 1 after an acceptance). MODE_TREE evaluates them all at once,
+// one workgroup per pack and node; the last workgroup of a pack to finish then
+// takes the D decisions in order along the tree and leaves the state, records
+// and counts as D single steps do. Every energy and decision is the same
+// expression of the same numbers, so results keep their bits.
+//
+// Bound: one evaluation and its launch, 50 us for 5 steps of 1,200 points
+// against 35 us for each step in turn. One complex of 8 replicas (4 packs), 200
+// steps: 7.3 -> 2.3 ms; 96 replicas of 40 atoms and 1,311 points (20 packs),
+// 159 steps 6.5 -> 4.7 ms; 8 replicas of 120 atoms and 6,000 points, 100 steps
+// 21.4 -> 4.9 ms. The count needs no wait: whichever workgroup is last decides.
+//
+// The pose `from` moved by the offsets that wave lane `src` holds.
+__device__ __forceinline__ void tree_move(const float from[6], const float dm[6], int src,
+                                          float to[6]) {
+  float d[6];
+#pragma unroll
+  for (int i = 0; i < 6; ++i) d[i] = __shfl(dm[i], src);
+  apply_move(from, d, to);
+}
+
+// The pose of tree node v (1-based) of a replica: `a` its lane, `base` the
+// wave lane of its lane 0. Called by whole waves with a uniform v.
+__device__ __forceinline__ void tree_pose(const KParams &P, const DevComplex &C, int flat, int a,
+                                          int base, int step0, int v, float mo[6]) {
+  const int depth = 31 - __builtin_clz(v);
+  float u[8], dm[6], scale[6], mn[6];
+#pragma unroll
+  for (int i = 0; i < 6; ++i) scale[i] = C.move_scale[i];
+  mc_uniforms(P.k0, P.k1, C.cid, flat, step0 + min(a, depth), u);
+  move_offsets(u, scale, C.move_kind, dm);
+  for (int i = 0; i < depth; ++i)
+    if (v >> (depth - 1 - i) & 1) {
+      tree_move(mo, dm, base + i, mn);
+#pragma unroll
+      for (int q = 0; q < 6; ++q) mo[q] = mn[q];
+    }
+  tree_move(mo, dm, base + depth, mn);
+#pragma unroll
+  for (int q = 0; q < 6; ++q) mo[q] = mn[q];
+}
+
+// Decisions of replica sv's steps [step0, step0 + n_steps) by one wave, whose
+// lane l holds the energy of node l + 1 and the random numbers of step l.
+__device__ __forceinline__ void tree_decide(const KParams &P, const DevComplex &C, int prt,
+                                            int sv, int step0) {
+  const int l = threadIdx.x & 63;
+  const int flat = P.rep_flat[sv];
+  const int ilig = flat % C.n_lig, itmp = P.idx_tmp[sv];
+  const float mb = C.minus_beta[itmp];
+  gd_energy E = P.ev_out[(size_t)sv * P.tree_nodes + min(l, P.tree_nodes - 1)];
+  float mo[6], scale[6], u[8], dm[6], mn[6];
+#pragma unroll
+  for (int i = 0; i < 6; ++i) {
+    mo[i] = P.mm[(size_t)sv * 6 + i];
+    scale[i] = C.move_scale[i];
+  }
+  mc_uniforms(P.k0, P.k1, C.cid, flat, step0 + min(l, P.n_steps - 1), u);
+  move_offsets(u, scale, C.move_kind, dm);
+  float e = P.e_old[sv].e[GD_MAXWEI - 1];
+  float best = P.best_e[sv];
+  int rc = P.rec ? P.rec_cnt[sv] : 0;
+  int acs = 0, kept = 0, v = 1;
+  for (int i = 0; i < P.n_steps; ++i) {
+    const float en = __shfl(E.e[GD_MAXWEI - 1], v - 1);
+    const bool yes = metropolis(en, e, mb, __shfl(u[6], i));
+    if (yes) {
+      tree_move(mo, dm, i, mn);
+#pragma unroll
+      for (int q = 0; q < 6; ++q) mo[q] = mn[q];
+      e = en;
+      acs += 1;
+      kept = v;
+      if (P.rec) {
+        if (l == v - 1 && rc < P.rec_cap) {
+          gd_record &r = P.rec[(size_t)sv * P.rec_cap + rc];
+          r.replica.idx_rep = flat;
+          r.replica.idx_prt = prt;
+          r.replica.idx_tmp = itmp;
+          r.replica.idx_lig = ilig;
+          r.energy = E;
+#pragma unroll
+          for (int q = 0; q < 6; ++q) r.movematrix[q] = mo[q];
+          r.step = step0 + i;
+        }
+        rc += 1;
+      }
+      if (e < best) {
+        best = e;
+        if (l == 0)
+#pragma unroll
+          for (int q = 0; q < 6; ++q) P.best_mm[(size_t)sv * 6 + q] = mo[q];
+      }
+    }
+    v = 2 * v + (yes ? 1 : 0);
+  }
+  if (kept > 0 && l == kept - 1) P.e_old[sv] = E;
+  if (l == 0) {
+#pragma unroll
+    for (int q = 0; q < 6; ++q) P.mm[(size_t)sv * 6 + q] = mo[q];
+    P.best_e[sv] = best;
+    P.acs_mc[sv] += acs;
+    if (P.rec) P.rec_cnt[sv] = rc < P.rec_cap ? rc : P.rec_cap;
+  }
+}
+
+// DA: 0 plain Metropolis (DA_TREE: by a tree of energies, in instances of its
+// own, so that the step loop's registers stay as they are); delayed acceptance with the surrogate from the
 // network evaluated per atom (1) or from its tabulated outputs (2); 3 and 4
 // are 1 and 2 with the split groups' shared surrogate sums compiled in.
 template <int APL, int DA, bool TILE, bool FLAT>
 __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const DevComplex &C, const Lds &S,
-                         int lpr, int step0, int &par) {
-  constexpr int DAM = DA > 2 ? DA - 2 : DA;
-  constexpr bool SHARED = DA > 2;
+                         int lpr, int step0, int idx, int node, int &par) {
+  constexpr bool TREE = DA == DA_TREE;
+  constexpr int DAM = TREE ? 0 : DA > 2 ? DA - 2 : DA;
+  constexpr bool SHARED = DAM != 0 && DA > 2;
   const int tid = threadIdx.x;
   Split sp;
   sp.ns = P.unsplit ? 1 : pk.ns;
@@ -1372,7 +1486,7 @@ __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const
     }
   };
 
-  if constexpr (DA) {
+  if constexpr (DAM) {
     if (P.mode == MODE_SUREVAL) {
       extern __shared__ __attribute__((aligned(16))) unsigned char lds_se[];
       unsigned char *dse = lds_se + P.off_da + (threadIdx.x >> 6) * 6208;
@@ -1394,11 +1508,28 @@ __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const
       return;
     }
   }
-  if (P.mode != MODE_MC) {
+  if (TREE || P.mode != MODE_MC) {
+    if constexpr (TREE) tree_pose(P, C, flat, a, (threadIdx.x & 63) - a, step0, node + 1, mo);
     place(mo);
     gd_energy E;
     pose_energy<APL, TILE, FLAT>(C, S, lpr, sp, true, x, y, z, ox, oy, oz, lt, q, li, val, mo, E);
     par = sp.par;
+    if constexpr (TREE) {
+      // the wave of group 0 writes: its energies are visible on the device
+      // before the node is counted, and are read after the last count
+      if (active && lead) P.ev_out[(size_t)sv * P.tree_nodes + node] = E;
+      if (sp.h == 0) __threadfence();
+      __syncthreads();
+      if (tid == 0) S.xo[0] = atomicAdd(P.tree_cnt + P.pack_base + idx, 1);
+      __syncthreads();
+      if (S.xo[0] != P.tree_nodes - 1) return;
+      __threadfence();
+      if (tid == 0) P.tree_cnt[P.pack_base + idx] = 0;
+      for (int i = __builtin_amdgcn_readfirstlane(tid >> 6); i < n_slots;
+           i += (int)(blockDim.x >> 6))
+        tree_decide(P, C, pk.prt, P.slots[pk.slot_off + i], step0);
+      return;
+    }
     if (active && lead) {
       if (P.mode == MODE_EVAL) {
         P.ev_out[sv] = E;
@@ -1464,14 +1595,14 @@ __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const
   // delayed acceptance (surrogate transition): K surrogate Metropolis
   // sub-steps, then one exact test of the composite move with
   // min(1, exp(-beta [(E(y) - E(x)) - (S(y) - S(x))]))
-  const int K = DA ? P.da_k : 1;
+  const int K = DAM ? P.da_k : 1;
   unsigned char *da = nullptr;
   float s_old = 0.0f;
   // the split's groups share the surrogate's KDE and MCS sums for complexes
   // with large KDE or MCS sets (one exchange per surrogate evaluation, so
   // every thread evaluates it together)
   const bool share = SHARED && sp.ns > 1 && C.da_share != 0;
-  if constexpr (DA) {
+  if constexpr (DAM) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_da[];
     da = lds_da + P.off_da + (threadIdx.x >> 6) * 6208;
     if (wave_active) place(mo);
@@ -1486,7 +1617,7 @@ __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const
   }
 
   for (int s = step0; s < step0 + P.n_steps; s += K) {
-    if constexpr (!DA) {
+    if constexpr (!DAM) {
       float u[8], mn[6];
       if (wave_active) {
         float dm[6];
@@ -1606,6 +1737,11 @@ __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const
 
 template <int APL, int DA, bool TILE, bool FLAT>
 __device__ __forceinline__ void mc_kernel_body(const KParams &P, int idx, int step0) {
+  int node = 0;
+  if constexpr (DA == DA_TREE) {
+    node = idx / P.tree_packs;
+    idx -= node * P.tree_packs;
+  }
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const Pack pk = P.packs[P.pack_base + idx];
   const DevComplex &C = P.cxs[pk.cx];
@@ -1690,16 +1826,16 @@ __device__ __forceinline__ void mc_kernel_body(const KParams &P, int idx, int st
     for (int b = 0; b < pk.n_slots; b += pk.round) {
       q.slot_off = pk.slot_off + b;
       q.n_slots = min(pk.round, pk.n_slots - b);
-      run_pack<APL, DA, TILE, FLAT>(P, q, C, S, C.lpr, step0, par);
+      run_pack<APL, DA, TILE, FLAT>(P, q, C, S, C.lpr, step0, idx, node, par);
     }
   } else {
-    run_pack<APL, DA, TILE, FLAT>(P, pk, C, S, C.lpr, step0, par);
+    run_pack<APL, DA, TILE, FLAT>(P, pk, C, S, C.lpr, step0, idx, node, par);
   }
 }
 
 // MC kernel for packs whose complexes place APL ligand atoms on each lane:
-// plain MC, start-pose evaluation and pose evaluation (DA = false), or
-// delayed acceptance with surrogate sub-steps (DA = true). One instance per
+// plain MC, start-pose evaluation and pose evaluation (DA = 0), plain MC by a
+// tree of energies (DA_TREE), or delayed acceptance with surrogate sub-steps. One instance per
 // APL keeps each variant's register allocation to what it needs.
 template <int APL, int DA, bool TILE, bool FLAT>
 __global__ void __launch_bounds__(512) gd_mc_kernel(KParams P) {

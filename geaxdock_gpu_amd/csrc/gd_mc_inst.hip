@@ -9,7 +9,8 @@ namespace gd {
 // Host handle of gd_mc_kernel<GD_MC_APL, da, ...>: da 0 plain MC and pose
 // evaluation, 1 delayed acceptance with the network per atom, 2 with its
 // tabulated outputs, 3 and 4 the same with the receptor split's groups
-// sharing the surrogate's KDE and MCS sums; rec: the receptor resident in LDS
+// sharing the surrogate's KDE and MCS sums, DA_TREE plain MC by a tree of
+// energies; rec: the receptor resident in LDS
 // by chunks, streamed through LDS tiles, or resident with unit lists.
 template <>
 const void *mc_kernel_handle<GD_MC_APL>(int da, int rec) {
@@ -19,6 +20,7 @@ const void *mc_kernel_handle<GD_MC_APL>(int da, int rec) {
       case 2: return (const void *)gd_mc_kernel<GD_MC_APL, 2, true, false>;
       case 3: return (const void *)gd_mc_kernel<GD_MC_APL, 3, true, false>;
       case 4: return (const void *)gd_mc_kernel<GD_MC_APL, 4, true, false>;
+      case DA_TREE: return (const void *)gd_mc_kernel<GD_MC_APL, DA_TREE, true, false>;
       default: return (const void *)gd_mc_kernel<GD_MC_APL, 0, true, false>;
     }
   }
@@ -27,6 +29,7 @@ const void *mc_kernel_handle<GD_MC_APL>(int da, int rec) {
       case 0: return (const void *)gd_mc_kernel<GD_MC_APL, 0, false, true>;
       case 2: return (const void *)gd_mc_kernel<GD_MC_APL, 2, false, true>;
       case 4: return (const void *)gd_mc_kernel<GD_MC_APL, 4, false, true>;
+      case DA_TREE: return (const void *)gd_mc_kernel<GD_MC_APL, DA_TREE, false, true>;
       default: return nullptr;
     }
   }
@@ -35,6 +38,7 @@ const void *mc_kernel_handle<GD_MC_APL>(int da, int rec) {
     case 2: return (const void *)gd_mc_kernel<GD_MC_APL, 2, false, false>;
     case 3: return (const void *)gd_mc_kernel<GD_MC_APL, 3, false, false>;
     case 4: return (const void *)gd_mc_kernel<GD_MC_APL, 4, false, false>;
+    case DA_TREE: return (const void *)gd_mc_kernel<GD_MC_APL, DA_TREE, false, false>;
     default: return (const void *)gd_mc_kernel<GD_MC_APL, 0, false, false>;
   }
 }
