@@ -47,6 +47,7 @@ struct HostComplex {
   gd_complex_desc d;  // sizes, scalars (pointers are not kept)
   int n_rep = 0, rep_base = 0;
   int lpr = 0, apl = 0, n_chunks = 0;
+  int lpr0 = 0, apl0 = 0;  // the shape of fewest lane slots (lpr and apl may be widened)
   bool tiled = false;  // receptor streamed through LDS tiles
   bool ref_built = false;
   int flat_n[4] = {0, 0, 0, 0};  // units of the flat pair loop by split (0: no list)
@@ -482,6 +483,8 @@ gd_status gd_add_complex(gd_ctx *ctx, const gd_complex_desc *d, int *complex_id)
                &h.apl);
   if (h.lpr * h.apl < lna || h.apl < 1 || h.apl > 4)
     return fail(ctx, GD_ERR_INVALID, "no lane shape for lna %d (lpr %d apl %d)", lna, h.lpr, h.apl);
+  h.lpr0 = h.lpr;
+  h.apl0 = h.apl;
 
   // receptor sorted by (type, kind); kind: 2 = class 2, 1 = hydrophobic flag
   std::vector<int> kind(pnp), perm(pnp);
@@ -1051,20 +1054,20 @@ void apply_layout(KParams &P, const KParams &L) {
 // among its packs: a class closes when the next pack would lower the
 // workgroups per CU it allows. Workgroups of 512 lanes take a CU's register
 // file alone (two waves per SIMD), so LDS does not split their classes.
-void pack_finish(const gd_ctx *ctx, PackSet &ps) {
+void pack_finish(const gd_ctx *ctx, PackSet &ps, int lpr = 0, int apl_of_lpr = 0) {
   const size_t n_pk = ps.packs.size();
   std::vector<int> res(n_pk), block(n_pk), apl(n_pk), tile(n_pk), units(n_pk);
   std::vector<double> cost(n_pk);
   for (size_t i = 0; i < n_pk; ++i) {
     Pack &p = ps.packs[i];
     const HostComplex &h = ctx->cx[p.cx];
-    p.half = ((p.round * h.lpr + 63) / 64) * 64;
+    p.half = ((p.round * (lpr > 0 ? lpr : h.lpr) + 63) / 64) * 64;
     block[i] = p.half * p.ns;
-    apl[i] = h.apl;
+    apl[i] = lpr > 0 ? apl_of_lpr : h.apl;
     // the tile length depends on the options only (not on the pack's block),
     // so every launch of a complex sums its chunks in the same order
     tile[i] = complex_tile(ctx, h);
-    cost[i] = (double)h.d.pnp * (double)p.half * h.apl;
+    cost[i] = (double)h.d.pnp * (double)p.half * apl[i];
     KParams L{};
     size_t need = 0;
     // units of the flat pair loop, where they fit
@@ -2147,18 +2150,34 @@ static gd_status eval_poses(gd_ctx *ctx, int cid, int n, const int *idx_lig, con
   }
   // the launch takes the flat pair loop (plan_classes): a list that fits, and
   // no scratch of the direct network evaluation
-  bool flat = ctx->flat && h.flat_n[3] > 0 && !(out_sur && !ctx->sur.tab_valid);
-  if (flat) {
+  auto flat_fits = [&](int lpr) {
     KParams L{};
     size_t need = 0;
-    layout(L, &need, 0, h.d.pnk, h.n_chunks, std::max(1, 64 / h.lpr), 512, true, 0, h.flat_n[3]);
-    flat = need <= ctx->max_lds;
+    layout(L, &need, 0, h.d.pnk, h.n_chunks, std::max(1, 64 / lpr), 512, true, 0, h.flat_n[3]);
+    return need <= ctx->max_lds;
+  };
+  const bool flat = ctx->flat && h.flat_n[3] > 0 && !(out_sur && !ctx->sur.tab_valid) &&
+                    flat_fits(h.lpr);
+  // Spread packing widens the lane shape of complexes with few packs, at the
+  // cost of lanes without an atom and of independent work per lane. Where
+  // poses at the shape of fewest lane slots still make a pack for every CU, they
+  // are evaluated with it, in the wide shape's order of additions (J in
+  // gd_mc.h): 16,384 poses of 38 atoms (64 lanes of one atom, 16 of three) on
+  // 2,400 points 3.77 -> 2.38 ms, 14,221 of 19 atoms on 839 points 1.22 -> 0.61,
+  // 791 of 63 atoms on 2,073 points (396 packs instead of 791) 0.29 -> 0.24. Fewer
+  // packs than CUs would leave some idle.
+  int lpr = h.lpr, apl = h.apl, da_poses = 0;
+  if (flat && !out_sur && spread_packing(ctx) && h.lpr0 < h.lpr && h.apl0 > 1 &&
+      flat_fits(h.lpr0) && (int64_t)n * h.lpr0 >= (int64_t)64 * ctx->n_cu) {
+    lpr = h.lpr0;
+    apl = h.apl0;
+    da_poses = apl > 2 && h.lpr == 2 * lpr ? DA_POSES2 : DA_POSES;
   }
   PackSet ps;
   ps.slots = order;
   for (int k = 0; k < h.d.n_prt * 4; ++k) {
     const int cnt = start[k + 1] - start[k], ns = 1 << (k & 3);
-    const int per = std::max(1, (512 / ns) / h.lpr);
+    const int per = std::max(1, (512 / ns) / lpr);
     // With the flat pair loop (a split of 8: a few poses at a time) a workgroup
     // stages the receptor once for several rounds of poses, as long as that
     // leaves four workgroups per CU: 16,384 poses on 2,400 points staged about
@@ -2177,11 +2196,12 @@ static gd_status eval_poses(gd_ctx *ctx, int cid, int n, const int *idx_lig, con
       ps.packs.push_back(pk);
     }
   }
-  pack_finish(ctx, ps);
+  if (da_poses) pack_finish(ctx, ps, lpr, apl);
+  else pack_finish(ctx, ps);
   for (const LaunchClass &lc : ps.classes)
     for (int i = lc.begin; i < lc.end; ++i)
-      if (ps.packs[i].round < ps.packs[i].n_slots && lc.lds_flat == 0)
-        return fail(ctx, GD_ERR_STATE, "rounds of poses without the flat pair loop");
+      if ((da_poses || ps.packs[i].round < ps.packs[i].n_slots) && lc.lds_flat == 0)
+        return fail(ctx, GD_ERR_STATE, "pose packs without the flat pair loop");
   for (const LaunchClass &lc : ps.classes)
     if (lc.lds > ctx->max_lds && lc.lds_flat == 0) return fail(ctx, GD_ERR_CAPACITY, "LDS %zu > %zu", lc.lds, ctx->max_lds);
   KParams P{};
@@ -2244,7 +2264,8 @@ static gd_status eval_poses(gd_ctx *ctx, int cid, int n, const int *idx_lig, con
   P.ev_out = d_out;
   P.ev_sur = d_sur;
   P.mode = sur ? MODE_SUREVAL : MODE_EVAL;
-  hipError_t le = launch_classes(ctx, ps.classes, P, sur ? da_instance(ctx, P.sur_tab != 0) : 0,
+  P.ev_lpr = lpr;
+  hipError_t le = launch_classes(ctx, ps.classes, P, sur ? da_instance(ctx, P.sur_tab != 0) : da_poses,
                                  sur && !P.sur_tab, ctx->stream);
   void *res = sur ? static_cast<void *>(out_sur) : static_cast<void *>(out);
   if (le == hipSuccess && no_alloc)

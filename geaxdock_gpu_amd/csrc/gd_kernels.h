@@ -109,7 +109,8 @@ struct Pack {
 // MODE_SUREVAL: surrogate total of given poses (delayed-acceptance kernels)
 // MODE_TREE: the next n_steps MC steps by a tree of energies (gd_mc.h)
 enum { MODE_MC = 0, MODE_INIT = 1, MODE_EVAL = 2, MODE_SUREVAL = 3, MODE_TREE = 4 };
-constexpr int DA_TREE = 5;     // its kernel instances (see mc_kernel_handle)
+// kernel instances besides the modes of delayed acceptance (see mc_kernel_handle)
+constexpr int DA_TREE = 5, DA_POSES = 6, DA_POSES2 = 7;
 constexpr int TREE_DEPTH = 6;  // a wave's lanes hold the 2^depth - 1 energies
 
 struct KParams {
@@ -132,6 +133,7 @@ struct KParams {
   // poses (MODE_EVAL), indexed by slot value
   const float *ev_mm;
   const int *ev_lig;
+  int ev_lpr;  // DA_POSES: lanes per pose
   gd_energy *ev_out;
   // MODE_TREE: workgroups (node, pack) of tree_packs packs; ev_out holds
   // [slot value][tree_nodes] energies, tree_cnt[pack] counts finished nodes
@@ -164,8 +166,8 @@ struct KParams {
 // Host handle of the MC kernel instance for `APL` ligand atoms per lane,
 // mode `da` (0 plain, 1 delayed acceptance with the network per atom, 2 with
 // its tabulated outputs) and receptor layout; defined in gd_mc_inst.hip, one
-// object per APL. REC_FLAT has instances for modes 0, 2, 4 and DA_TREE
-// (null for the others).
+// object per APL. REC_FLAT has instances for modes 0, 2, 4, DA_TREE and
+// (2 to 4 atoms per lane) DA_POSES (null for the others).
 enum { REC_CHUNKS = 0, REC_TILED = 1, REC_FLAT = 2 };
 template <int APL>
 const void *mc_kernel_handle(int da, int rec);

@@ -107,6 +107,19 @@ __device__ __forceinline__ float seg_sum(float v, int lpr) {
   return v;
 }
 
+// Poses evaluated with fewer lanes than the complex's lane shape has (J > 1,
+// see eval_poses in gd_engine.hip): slot k of a lane belongs to block k % J of
+// the wider shape's lanes. Each block's sum over its lanes is a subtree of the
+// wider shape's butterfly; its last levels add the blocks in pairs (blocks
+// without an atom would add zeros).
+template <int J>
+__device__ __forceinline__ float block_total(const float (&t)[J]) {
+  if constexpr (J == 1) return t[0];
+  else if constexpr (J == 2) return t[0] + t[1];
+  else if constexpr (J == 3) return (t[0] + t[1]) + t[2];
+  else return (t[0] + t[1]) + (t[2] + t[3]);
+}
+
 // KDE sum of one atom over points [b, e) of its type's range:
 // sum_j exp2(kde2l |x - q_j|^2) (src/kernel_cuda_l2_calcenergy.cu:232-246).
 // Four points are read and exponentiated ahead of their additions, which stay
@@ -424,7 +437,7 @@ __device__ __forceinline__ void flat_psp_add(FlatAcc<APL> &A) {
 // and selects would run for every unit.
 __device__ __forceinline__ void keep_branch() { asm volatile("" ::: "memory"); }
 
-template <int APL, int N>
+template <int APL, int N, bool PEND>
 __device__ __forceinline__ void flat_unit(int ux, bool hb, bool wide, const FlatUnit &U, const PairConst &K,
                                           float nr2max, const float (&x)[APL],
                                           const float (&y)[APL], const float (&z)[APL],
@@ -523,11 +536,13 @@ __device__ __forceinline__ void flat_unit(int ux, bool hb, bool wide, const Flat
     for (int j = 0; j < N; ++j)
 #pragma unroll
       for (int k = 0; k < APL; ++k) A.ele[k] = fmaf(U.P[j].w, rd[j][k], A.ele[k]);
-    if constexpr (APL == 1 && N == 2) {
+    if constexpr (PEND && N == 2) {
       if (mode == FLAT_SECOND && A.pend) {
         keep_branch();
         A.pend = false;
-        A.ele[0] = fmaf(A.pw[1], A.pv[1][0], fmaf(A.pw[0], A.pv[0][0], A.ele[0]));
+#pragma unroll
+        for (int k = 0; k < APL; ++k)
+          A.ele[k] = fmaf(A.pw[1], A.pv[1][k], fmaf(A.pw[0], A.pv[0][k], A.ele[k]));
       }
     }
     return;
@@ -564,12 +579,13 @@ __device__ __forceinline__ void flat_unit(int ux, bool hb, bool wide, const Flat
   if constexpr (N == 2) {
 #pragma unroll
     for (int k = 0; k < APL; ++k) A.ele[k] = fmaf(U.P[1].w, rd[1][k], A.ele[k]);
-    if constexpr (APL == 1) {
+    if constexpr (PEND) {
       if (mode == FLAT_FIRST) {
         A.pend = true;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-          A.pv[j][0] = v[j][0];
+#pragma unroll
+          for (int k = 0; k < APL; ++k) A.pv[j][k] = v[j][k];
           A.pw[j] = U.P[j].w;
         }
         return;
@@ -577,7 +593,9 @@ __device__ __forceinline__ void flat_unit(int ux, bool hb, bool wide, const Flat
       if (mode == FLAT_SECOND && A.pend) {
         keep_branch();
         A.pend = false;
-        A.ele[0] = fmaf(A.pw[1], A.pv[1][0], fmaf(A.pw[0], A.pv[0][0], A.ele[0]));
+#pragma unroll
+        for (int k = 0; k < APL; ++k)
+          A.ele[k] = fmaf(A.pw[1], A.pv[1][k], fmaf(A.pw[0], A.pv[0][k], A.ele[k]));
       }
     }
     if (mode != FLAT_SINGLES) {
@@ -594,7 +612,7 @@ __device__ __forceinline__ int flat_index(int ns) { return 31 - __builtin_clz(ns
 
 // All units of lane group h (list bounds `off`). A receptor type's units come in
 // an even number (the last may be empty), two register sets in turn.
-template <int APL>
+template <int APL, bool PEND>
 __device__ __forceinline__ void flat_pairs(const int *off, const Lds &S, int h,
                                            const PairConst &K, const float (&x)[APL],
                                            const float (&y)[APL], const float (&z)[APL],
@@ -649,13 +667,13 @@ __device__ __forceinline__ void flat_pairs(const int *off, const Lds &S, int h,
     left -= 2 * pairs;
     for (; pairs > 0; --pairs) {
       read_unit(Vb);
-      if (ua & FLAT_ONE) flat_unit<APL, 1>(ua, hb, wide, Va, K, nr2max, x, y, z, cp, psprow, A);
-      else flat_unit<APL, 2>(ua, hb, wide, Va, K, nr2max, x, y, z, cp, psprow, A);
+      if (ua & FLAT_ONE) flat_unit<APL, 1, PEND>(ua, hb, wide, Va, K, nr2max, x, y, z, cp, psprow, A);
+      else flat_unit<APL, 2, PEND>(ua, hb, wide, Va, K, nr2max, x, y, z, cp, psprow, A);
       const int ub = __builtin_amdgcn_readfirstlane(Vb.a.x);
       read_unit(Va);  // past the group's end: the next group's first unit, or the pad
       if (!(ub & FLAT_EMPTY)) {
-        if (ub & FLAT_ONE) flat_unit<APL, 1>(ub, hb, wide, Vb, K, nr2max, x, y, z, cp, psprow, A);
-        else flat_unit<APL, 2>(ub, hb, wide, Vb, K, nr2max, x, y, z, cp, psprow, A);
+        if (ub & FLAT_ONE) flat_unit<APL, 1, PEND>(ub, hb, wide, Vb, K, nr2max, x, y, z, cp, psprow, A);
+        else flat_unit<APL, 2, PEND>(ub, hb, wide, Vb, K, nr2max, x, y, z, cp, psprow, A);
       }
       ua = __builtin_amdgcn_readfirstlane(Va.a.x);
     }
@@ -670,7 +688,7 @@ __device__ __forceinline__ void flat_pairs(const int *off, const Lds &S, int h,
 // of a coarse receptor took 37,000 cycles of a step's 124,000 per wave), and
 // their lane sums share each butterfly step. Per template the additions are
 // the same as one template at a time.
-template <int APL>
+template <int APL, int J>
 __device__ __forceinline__ float mcs_sum(const DevComplex &C, int lpr, const float (&x)[APL],
                                          const float (&y)[APL], const float (&z)[APL],
                                          const int (&li)[APL], const bool (&val)[APL],
@@ -694,23 +712,25 @@ __device__ __forceinline__ float mcs_sum(const DevComplex &C, int lpr, const flo
   };
   read(m_begin);
   for (int m0 = m_begin; m0 < m_end; m0 += 4) {
-    float s[4], nc[4], tc[4];
+    float s[4][J], nc[4], tc[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      s[q] = 0.0f;
+#pragma unroll
+      for (int j = 0; j < J; ++j) s[q][j] = 0.0f;
       nc[q] = n[q];
       tc[q] = t[q];
 #pragma unroll
       for (int k = 0; k < APL; ++k) {
         if (!val[k]) continue;
-        if (M[q][k][3] != 0.0f) s[q] += pair_d2(x[k], y[k], z[k], M[q][k][0], M[q][k][1], M[q][k][2]);
+        if (M[q][k][3] != 0.0f) s[q][k % J] += pair_d2(x[k], y[k], z[k], M[q][k][0], M[q][k][1], M[q][k][2]);
       }
     }
     if (m0 + 4 < m_end) read(m0 + 4);
-    seg_sums(lpr, s[0], s[1], s[2], s[3]);
+#pragma unroll
+    for (int j = 0; j < J; ++j) seg_sums(lpr, s[0][j], s[1][j], s[2][j], s[3][j]);
 #pragma unroll
     for (int q = 0; q < 4; ++q)
-      if (m0 + q < m_end && nc[q] > 0.0f) elhm += tc[q] * sqrtf(s[q] / nc[q]);
+      if (m0 + q < m_end && nc[q] > 0.0f) elhm += tc[q] * sqrtf(block_total(s[q]) / nc[q]);
   }
   return elhm;
 }
@@ -735,7 +755,7 @@ __device__ __forceinline__ float mcs_sum(const DevComplex &C, int lpr, const flo
 //
 // FLAT: every pack of the launch has the unit list of its split in LDS; the
 // pair loop is flat_pairs.
-template <int APL, bool TILE, bool FLAT>
+template <int APL, bool TILE, bool FLAT, int J = 1>
 __device__ __forceinline__ void pose_energy(const DevComplex &C, const Lds &S, int lpr, Split &sp,
                             bool live, const float (&x)[APL],
                             const float (&y)[APL], const float (&z)[APL],
@@ -856,7 +876,7 @@ __device__ __forceinline__ void pose_energy(const DevComplex &C, const Lds &S, i
         prow[k] = glob(psprow[k]);
       }
       A.pend = false;
-      flat_pairs<APL>(C.flat_off[flat_index(sp.ns)], S, sp.h, K, x, y, z, lt, prow, A);
+      flat_pairs<APL, (APL == 1 || J > 1)>(C.flat_off[flat_index(sp.ns)], S, sp.h, K, x, y, z, lt, prow, A);
 #pragma unroll
       for (int k = 0; k < APL; ++k) {
         vdw[k] = A.vdw[k];
@@ -938,7 +958,7 @@ __device__ __forceinline__ void pose_energy(const DevComplex &C, const Lds &S, i
   // templates, and the partial sums join the exchange below. With one group
   // the parts are the whole lists.
   const float kde2l = C.kde2l;
-  float t_kde = 0.f, elhm = 0.f;
+  float b_kde[J] = {}, elhm = 0.f;
   int t_tp = 0;
   if (live) {
 #pragma unroll
@@ -949,7 +969,7 @@ __device__ __forceinline__ void pose_energy(const DevComplex &C, const Lds &S, i
       const int kl = kr.y - kr.x;
       const int kb = kr.x + (kl * sp.h) / sp.ns, ke = kr.x + (kl * (sp.h + 1)) / sp.ns;
       const float ks = kde_sum(S.kde, kde2l, x[k], y[k], z[k], kb, ke);
-      if (kl > 0) t_kde += ks / (float)kl;
+      if (kl > 0) b_kde[k % J] += ks / (float)kl;
       // true positives against the reference contact list
       const int nr = C.ref_cnt[li[k]];
       const int2 *rl = C.ref + (size_t)li[k] * KMAX;
@@ -980,25 +1000,29 @@ __device__ __forceinline__ void pose_energy(const DevComplex &C, const Lds &S, i
       }
     }
     // MCS restraints, src/kernel_cuda_l2_calcenergy.cu:274-313
-    elhm = mcs_sum<APL>(C, lpr, x, y, z, li, val, (C.pos * sp.h) / sp.ns,
+    elhm = mcs_sum<APL, J>(C, lpr, x, y, z, li, val, (C.pos * sp.h) / sp.ns,
                         (C.pos * (sp.h + 1)) / sp.ns);
   }
 
   // pair sums that are linear in the receptor points
-  float t_vdw = 0.f, t_ele = 0.f, t_pmf = 0.f, t_psp = 0.f, t_hdb = 0.f, t_hpc = 0.f;
-  float t_rms = 0.f;
+  float b_vdw[J] = {}, b_ele[J] = {}, b_pmf[J] = {}, b_psp[J] = {}, b_hdb[J] = {};
   int t_cnt = 0;
 #pragma unroll
   for (int k = 0; k < APL; ++k) {
     if (!val[k]) continue;
-    t_vdw += vdw[k];
-    t_ele += q[k] * ele[k];
-    t_pmf += pmf[k];
-    t_psp += psp[k];
-    t_hdb += hdb[k];
+    b_vdw[k % J] += vdw[k];
+    b_ele[k % J] += q[k] * ele[k];
+    b_pmf[k % J] += pmf[k];
+    b_psp[k % J] += psp[k];
+    b_hdb[k % J] += hdb[k];
     t_cnt += cnt[k];
   }
-  seg_sums(lpr, t_vdw, t_ele, t_pmf, t_psp, t_hdb, t_cnt, t_kde, t_tp);
+  seg_sums(lpr, b_vdw[0], b_ele[0], b_pmf[0], b_psp[0], b_hdb[0], t_cnt, b_kde[0], t_tp);
+#pragma unroll
+  for (int j = 1; j < J; ++j)
+    seg_sums(lpr, b_vdw[j], b_ele[j], b_pmf[j], b_psp[j], b_hdb[j], b_kde[j]);
+  float t_vdw = block_total(b_vdw), t_ele = block_total(b_ele), t_pmf = block_total(b_pmf);
+  float t_psp = block_total(b_psp), t_hdb = block_total(b_hdb), t_kde = block_total(b_kde);
   if (sp.ns > 1) {
     // exchange: per-atom HPC sums (the restraint is nonlinear in them) and
     // the replica's linear sums. Every group adds the ns partials in group
@@ -1057,21 +1081,24 @@ __device__ __forceinline__ void pose_energy(const DevComplex &C, const Lds &S, i
   if (!live) return;
 
   // per-atom terms
+  float b_hpc[J] = {}, b_rms[J] = {};
 #pragma unroll
   for (int k = 0; k < APL; ++k) {
     if (!val[k]) continue;
     // hydrophobic restraint, src/kernel_cuda_l2_calcenergy.cu:200-205
     const float h2 = (hpc[k] - C.hpl0[lt[k]]) / C.hpl1[lt[k]];
-    t_hpc += 0.5f * h2 * h2 - C.hpl2[lt[k]];
+    b_hpc[k % J] += 0.5f * h2 * h2 - C.hpl2[lt[k]];
     // RMSD against the start pose
     const float dx = x[k] - (ox[k] + C.pocket[0]);
     const float dy = y[k] - (oy[k] + C.pocket[1]);
     const float dz = z[k] - (oz[k] + C.pocket[2]);
-    t_rms += dx * dx + dy * dy + dz * dz;
+    b_rms[k % J] += dx * dx + dy * dy + dz * dz;
   }
   const int pos = C.pos;
 
-  seg_sums(lpr, t_hpc, t_rms);
+#pragma unroll
+  for (int j = 0; j < J; ++j) seg_sums(lpr, b_hpc[j], b_rms[j]);
+  const float t_hpc = block_total(b_hpc), t_rms = block_total(b_rms);
 
   // src/kernel_cuda_l2_calcenergy.cu:334-359, src/kernel_cuda_l3_combineenergy.cu:28-37
   const float lna = (float)C.lna;
@@ -1431,14 +1458,17 @@ __device__ __forceinline__ void tree_decide(const KParams &P, const DevComplex &
 }
 
 // DA: 0 plain Metropolis (DA_TREE: by a tree of energies, in instances of its
-// own, so that the step loop's registers stay as they are); delayed acceptance with the surrogate from the
-// network evaluated per atom (1) or from its tabulated outputs (2); 3 and 4
+// own, so that the step loop's registers stay as they are; DA_POSES and
+// DA_POSES2: poses with fewer lanes than the complex's shape has, slot k in
+// block k or k % 2 of block_total); delayed acceptance with the surrogate from
+// the network evaluated per atom (1) or from its tabulated outputs (2); 3 and 4
 // are 1 and 2 with the split groups' shared surrogate sums compiled in.
 template <int APL, int DA, bool TILE, bool FLAT>
 __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const DevComplex &C, const Lds &S,
                          int lpr, int step0, int idx, int node, int &par) {
-  constexpr bool TREE = DA == DA_TREE;
-  constexpr int DAM = TREE ? 0 : DA > 2 ? DA - 2 : DA;
+  constexpr bool TREE = DA == DA_TREE, POSES = DA == DA_POSES || DA == DA_POSES2;
+  constexpr int DAM = TREE || POSES ? 0 : DA > 2 ? DA - 2 : DA;
+  constexpr int J = !POSES ? 1 : DA == DA_POSES2 ? 2 : APL;
   constexpr bool SHARED = DAM != 0 && DA > 2;
   const int tid = threadIdx.x;
   Split sp;
@@ -1468,7 +1498,7 @@ __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const
   int flat = 0, ilig;
   float mo[6];
   gd_energy eo;
-  if (P.mode == MODE_EVAL || P.mode == MODE_SUREVAL) {
+  if (POSES || P.mode == MODE_EVAL || P.mode == MODE_SUREVAL) {
     ilig = P.ev_lig[sv];
 #pragma unroll
     for (int i = 0; i < 6; ++i) mo[i] = P.ev_mm[(size_t)sv * 6 + i];
@@ -1533,11 +1563,11 @@ __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const
       return;
     }
   }
-  if (TREE || P.mode != MODE_MC) {
+  if (TREE || POSES || P.mode != MODE_MC) {
     if constexpr (TREE) tree_pose(P, C, flat, a, (threadIdx.x & 63) - a, step0, node + 1, mo);
     place(mo);
     gd_energy E;
-    pose_energy<APL, TILE, FLAT>(C, S, lpr, sp, true, x, y, z, ox, oy, oz, lt, q, li, val, mo, E);
+    pose_energy<APL, TILE, FLAT, J>(C, S, lpr, sp, true, x, y, z, ox, oy, oz, lt, q, li, val, mo, E);
     par = sp.par;
     if constexpr (TREE) {
       // the wave of group 0 writes: its energies are visible on the device
@@ -1556,7 +1586,7 @@ __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const
       return;
     }
     if (active && lead) {
-      if (P.mode == MODE_EVAL) {
+      if (POSES || P.mode == MODE_EVAL) {
         P.ev_out[sv] = E;
       } else {
         P.e_old[sv] = E;
@@ -1860,6 +1890,7 @@ __device__ __forceinline__ void mc_kernel_body(const KParams &P, int idx, int st
   __syncthreads();
 
   int par = 0;
+  const int lpr = DA == DA_POSES || DA == DA_POSES2 ? P.ev_lpr : C.lpr;
   if constexpr (FLAT) {
     // rounds of poses on the staged receptor (MC packs have one round); the
     // exchange buffers' parity runs on, so a round's first exchange does not
@@ -1868,10 +1899,10 @@ __device__ __forceinline__ void mc_kernel_body(const KParams &P, int idx, int st
     for (int b = 0; b < pk.n_slots; b += pk.round) {
       q.slot_off = pk.slot_off + b;
       q.n_slots = min(pk.round, pk.n_slots - b);
-      run_pack<APL, DA, TILE, FLAT>(P, q, C, S, C.lpr, step0, idx, node, par);
+      run_pack<APL, DA, TILE, FLAT>(P, q, C, S, lpr, step0, idx, node, par);
     }
   } else {
-    run_pack<APL, DA, TILE, FLAT>(P, pk, C, S, C.lpr, step0, idx, node, par);
+    run_pack<APL, DA, TILE, FLAT>(P, pk, C, S, lpr, step0, idx, node, par);
   }
 }
 

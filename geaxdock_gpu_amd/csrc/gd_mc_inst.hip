@@ -10,7 +10,7 @@ namespace gd {
 // evaluation, 1 delayed acceptance with the network per atom, 2 with its
 // tabulated outputs, 3 and 4 the same with the receptor split's groups
 // sharing the surrogate's KDE and MCS sums, DA_TREE plain MC by a tree of
-// energies; rec: the receptor resident in LDS
+// energies, DA_POSES poses with fewer lanes than the complex's shape; rec: the receptor resident in LDS
 // by chunks, streamed through LDS tiles, or resident with unit lists.
 template <>
 const void *mc_kernel_handle<GD_MC_APL>(int da, int rec) {
@@ -30,6 +30,12 @@ const void *mc_kernel_handle<GD_MC_APL>(int da, int rec) {
       case 2: return (const void *)gd_mc_kernel<GD_MC_APL, 2, false, true>;
       case 4: return (const void *)gd_mc_kernel<GD_MC_APL, 4, false, true>;
       case DA_TREE: return (const void *)gd_mc_kernel<GD_MC_APL, DA_TREE, false, true>;
+#if GD_MC_APL > 1
+      case DA_POSES: return (const void *)gd_mc_kernel<GD_MC_APL, DA_POSES, false, true>;
+#endif
+#if GD_MC_APL > 2
+      case DA_POSES2: return (const void *)gd_mc_kernel<GD_MC_APL, DA_POSES2, false, true>;
+#endif
       default: return nullptr;
     }
   }
