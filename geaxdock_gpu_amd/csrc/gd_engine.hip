@@ -2159,19 +2159,26 @@ static gd_status eval_poses(gd_ctx *ctx, int cid, int n, const int *idx_lig, con
   const bool flat = ctx->flat && h.flat_n[3] > 0 && !(out_sur && !ctx->sur.tab_valid) &&
                     flat_fits(h.lpr);
   // Spread packing widens the lane shape of complexes with few packs, at the
-  // cost of lanes without an atom and of independent work per lane. Where
-  // poses at the shape of fewest lane slots still make a pack for every CU, they
-  // are evaluated with it, in the wide shape's order of additions (J in
-  // gd_mc.h): 16,384 poses of 38 atoms (64 lanes of one atom, 16 of three) on
-  // 2,400 points 3.77 -> 2.38 ms, 14,221 of 19 atoms on 839 points 1.22 -> 0.61,
-  // 791 of 63 atoms on 2,073 points (396 packs instead of 791) 0.29 -> 0.24. Fewer
-  // packs than CUs would leave some idle.
+  // cost of lanes without an atom and of independent work per lane. Larger
+  // pose sets take the shape of fewest lane slots, in the wide shape's order of
+  // additions (J in gd_mc.h), where its rounds of packs over the CUs cost
+  // less: per atom of a lane 0.65 of the wide shape's time with unit lists,
+  // 0.75 with tiles. 16,384 poses of 38 atoms (64 lanes of one atom, 16 of
+  // three) on 2,400 points 3.77 -> 2.38 ms; 2,000 of 61 atoms on 8,000 points
+  // (tiles) 1.54 -> 1.30; 1,100 of 45 atoms on 6,000 points, near the line, 0.79
+  // -> 0.74.
   int lpr = h.lpr, apl = h.apl, da_poses = 0;
-  if (flat && !out_sur && spread_packing(ctx) && h.lpr0 < h.lpr && h.apl0 > 1 &&
-      flat_fits(h.lpr0) && (int64_t)n * h.lpr0 >= (int64_t)64 * ctx->n_cu) {
-    lpr = h.lpr0;
-    apl = h.apl0;
-    da_poses = apl > 2 && h.lpr == 2 * lpr ? DA_POSES2 : DA_POSES;
+  if ((h.tiled || (flat && flat_fits(h.lpr0))) && !out_sur && spread_packing(ctx) &&
+      h.lpr0 < h.lpr && h.apl0 > 1 && h.apl0 < 4) {
+    auto cost = [&](int l, int a) {
+      const int64_t packs = ((int64_t)n * l + 63) / 64;
+      return (double)((packs + ctx->n_cu - 1) / ctx->n_cu) * a;
+    };
+    if (cost(h.lpr0, h.apl0) * (h.tiled ? 0.75 : 0.65) < 0.95 * cost(h.lpr, h.apl)) {
+      lpr = h.lpr0;
+      apl = h.apl0;
+      da_poses = h.apl == 2 ? DA_POSES2 : DA_POSES;
+    }
   }
   PackSet ps;
   ps.slots = order;
@@ -2200,7 +2207,7 @@ static gd_status eval_poses(gd_ctx *ctx, int cid, int n, const int *idx_lig, con
   else pack_finish(ctx, ps);
   for (const LaunchClass &lc : ps.classes)
     for (int i = lc.begin; i < lc.end; ++i)
-      if ((da_poses || ps.packs[i].round < ps.packs[i].n_slots) && lc.lds_flat == 0)
+      if (lc.lds_flat == 0 && ((da_poses && lc.tile == 0) || ps.packs[i].round < ps.packs[i].n_slots))
         return fail(ctx, GD_ERR_STATE, "pose packs without the flat pair loop");
   for (const LaunchClass &lc : ps.classes)
     if (lc.lds > ctx->max_lds && lc.lds_flat == 0) return fail(ctx, GD_ERR_CAPACITY, "LDS %zu > %zu", lc.lds, ctx->max_lds);

@@ -166,8 +166,8 @@ struct KParams {
 // Host handle of the MC kernel instance for `APL` ligand atoms per lane,
 // mode `da` (0 plain, 1 delayed acceptance with the network per atom, 2 with
 // its tabulated outputs) and receptor layout; defined in gd_mc_inst.hip, one
-// object per APL. REC_FLAT has instances for modes 0, 2, 4, DA_TREE and
-// (2 to 4 atoms per lane) DA_POSES (null for the others).
+// object per APL. DA_POSES (2 or 3 atoms per lane) and DA_POSES2 (3) have
+// instances for REC_TILED and REC_FLAT, REC_FLAT none for modes 1 and 3.
 enum { REC_CHUNKS = 0, REC_TILED = 1, REC_FLAT = 2 };
 template <int APL>
 const void *mc_kernel_handle(int da, int rec);

@@ -328,7 +328,11 @@ __device__ __forceinline__ void pair_group(const Lds &S, int p, const float4 (&P
     }
 }
 
-template <int APL, int KIND, bool CLAMP, bool HB>
+// Points per group of a lane shape: enough independent pairs per lane to cover
+// latency.
+__host__ __device__ constexpr int group_points(int apl) { return apl >= 3 ? 1 : (apl == 2 ? 2 : 4); }
+
+template <int APL, int NP, int KIND, bool CLAMP, bool HB>
 __device__ __forceinline__ void chunk_pairs(const Lds &S, int beg, int end, const PairConst &K,
                                             const Range &G,
                                             const float (&x)[APL], const float (&y)[APL],
@@ -338,8 +342,6 @@ __device__ __forceinline__ void chunk_pairs(const Lds &S, int beg, int end, cons
                                             float (&pmf)[APL], float (&psp)[APL],
                                             float (&hdb)[APL], float (&hpc)[APL],
                                             int (&cnt)[APL]) {
-  // points per group: enough independent pairs per lane to cover latency
-  constexpr int NP = APL >= 3 ? 1 : (APL == 2 ? 2 : 4);
   int p = beg;
   // the chunk's PMF sum is taken without pmf1, which multiplies it once at
   // the end
@@ -755,7 +757,7 @@ __device__ __forceinline__ float mcs_sum(const DevComplex &C, int lpr, const flo
 //
 // FLAT: every pack of the launch has the unit list of its split in LDS; the
 // pair loop is flat_pairs.
-template <int APL, bool TILE, bool FLAT, int J = 1>
+template <int APL, bool TILE, bool FLAT, int J = 1, int NP = group_points(APL)>
 __device__ __forceinline__ void pose_energy(const DevComplex &C, const Lds &S, int lpr, Split &sp,
                             bool live, const float (&x)[APL],
                             const float (&y)[APL], const float (&z)[APL],
@@ -846,7 +848,7 @@ __device__ __forceinline__ void pose_energy(const DevComplex &C, const Lds &S, i
     const bool clamp = __ballot(wide) != 0;
     const bool hb = __ballot(hbond) != 0;
     auto pairs = [&](auto kind_c, auto clamp_c, auto hb_c) {
-      chunk_pairs<APL, decltype(kind_c)::value, decltype(clamp_c)::value,
+      chunk_pairs<APL, NP, decltype(kind_c)::value, decltype(clamp_c)::value,
                   decltype(hb_c)::value>(T, beg, end, K, G, x, y, z, cp, psprow, vdw, ele,
                                          pmf, psp, hdb, hpc, cnt);
     };
@@ -1469,6 +1471,8 @@ __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const
   constexpr bool TREE = DA == DA_TREE, POSES = DA == DA_POSES || DA == DA_POSES2;
   constexpr int DAM = TREE || POSES ? 0 : DA > 2 ? DA - 2 : DA;
   constexpr int J = !POSES ? 1 : DA == DA_POSES2 ? 2 : APL;
+  // the wide shape has one atom per lane (DA_POSES) or two
+  constexpr int NP = group_points(DA == DA_POSES ? 1 : DA == DA_POSES2 ? 2 : APL);
   constexpr bool SHARED = DAM != 0 && DA > 2;
   const int tid = threadIdx.x;
   Split sp;
@@ -1567,7 +1571,7 @@ __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const
     if constexpr (TREE) tree_pose(P, C, flat, a, (threadIdx.x & 63) - a, step0, node + 1, mo);
     place(mo);
     gd_energy E;
-    pose_energy<APL, TILE, FLAT, J>(C, S, lpr, sp, true, x, y, z, ox, oy, oz, lt, q, li, val, mo, E);
+    pose_energy<APL, TILE, FLAT, J, NP>(C, S, lpr, sp, true, x, y, z, ox, oy, oz, lt, q, li, val, mo, E);
     par = sp.par;
     if constexpr (TREE) {
       // the wave of group 0 writes: its energies are visible on the device

@@ -21,6 +21,12 @@ const void *mc_kernel_handle<GD_MC_APL>(int da, int rec) {
       case 3: return (const void *)gd_mc_kernel<GD_MC_APL, 3, true, false>;
       case 4: return (const void *)gd_mc_kernel<GD_MC_APL, 4, true, false>;
       case DA_TREE: return (const void *)gd_mc_kernel<GD_MC_APL, DA_TREE, true, false>;
+#if GD_MC_APL == 2 || GD_MC_APL == 3
+      case DA_POSES: return (const void *)gd_mc_kernel<GD_MC_APL, DA_POSES, true, false>;
+#endif
+#if GD_MC_APL == 3
+      case DA_POSES2: return (const void *)gd_mc_kernel<GD_MC_APL, DA_POSES2, true, false>;
+#endif
       default: return (const void *)gd_mc_kernel<GD_MC_APL, 0, true, false>;
     }
   }
@@ -30,10 +36,10 @@ const void *mc_kernel_handle<GD_MC_APL>(int da, int rec) {
       case 2: return (const void *)gd_mc_kernel<GD_MC_APL, 2, false, true>;
       case 4: return (const void *)gd_mc_kernel<GD_MC_APL, 4, false, true>;
       case DA_TREE: return (const void *)gd_mc_kernel<GD_MC_APL, DA_TREE, false, true>;
-#if GD_MC_APL > 1
+#if GD_MC_APL == 2 || GD_MC_APL == 3
       case DA_POSES: return (const void *)gd_mc_kernel<GD_MC_APL, DA_POSES, false, true>;
 #endif
-#if GD_MC_APL > 2
+#if GD_MC_APL == 3
       case DA_POSES2: return (const void *)gd_mc_kernel<GD_MC_APL, DA_POSES2, false, true>;
 #endif
       default: return nullptr;
