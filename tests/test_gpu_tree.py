@@ -3,7 +3,8 @@
 Persistent launches step one at a time, so both must leave the same bits:
 states, best poses, records and counts. The packs of a context set the depth
 (6 steps for 4 packs or fewer, 2 for 85, none beyond), exchange intervals and
-run lengths that it does not divide leave shorter trees.
+run lengths that it does not divide leave shorter trees, and trees span
+exchanges.
 """
 import numpy as np
 import pytest
@@ -37,10 +38,12 @@ def _result(gd, cxs, persistent, runs, record, **kw):
 
 
 # (lna, receptor points, ligand and receptor conformers, temperatures, lanes,
-# atoms per lane): packs 1, 4, 8, 9, 17, 36, 37, 85, 86
+# atoms per lane): packs 1, 4, 8, 9, 17, 36, 37, 85, 86, then ladders of more
+# replicas than a workgroup has waves
 SHAPES = [(8, 40, 1, 1, 1, 8, 1), (30, 300, 1, 1, 8, 32, 1), (60, 700, 1, 1, 8, 64, 1),
           (29, 500, 3, 3, 4, 16, 2), (48, 2501, 17, 1, 3, 16, 3), (61, 900, 6, 3, 8, 16, 4),
-          (20, 130, 37, 1, 2, 32, 1), (16, 60, 17, 5, 2, 16, 1), (16, 60, 43, 2, 2, 16, 1)]
+          (20, 130, 37, 1, 2, 32, 1), (16, 60, 17, 5, 2, 16, 1), (16, 60, 43, 2, 2, 16, 1),
+          (30, 300, 1, 1, 13, 32, 1), (15, 60, 2, 1, 40, 8, 2)]
 
 
 @pytest.mark.parametrize("record", [True, False])
@@ -49,7 +52,7 @@ def test_tree_equals_single_steps(gd, lna, pnp, n_lig, n_prt, n_tmp, lpr, apl, r
     cx = synth.make_complex(lna, lna=lna, pnp=pnp, pnk=30, pos=2, mcs_atoms=5, n_lig=n_lig,
                             n_prt=n_prt, n_tmp=n_tmp, void_radius=3.0)
     kw = dict(lanes_per_replica=lpr, atoms_per_lane=apl, steps_per_dump=31)
-    runs = [(47, 20), (1, 7), (13, 0), (9, 1)]
+    runs = [(47, 20), (1, 7), (13, 0), (9, 1), (17, 3)]
     assert (_result(gd, [cx], False, runs, record, **kw)
             == _result(gd, [cx], True, runs, record, **kw))
 
