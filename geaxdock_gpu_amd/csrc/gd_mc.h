@@ -243,7 +243,11 @@ __device__ __forceinline__ void pair_group(const Lds &S, int p, const float4 (&P
     ps[j] = (KIND == KIND_PSP) ? S.psp[p + j] : 0;
   }
   float d2[NP][APL], rd[NP][APL], dd[NP][APL], num[NP][APL], den[NP][APL], dn[NP][APL];
-  float qmin = 0.0f;  // the lane's nearest atom to any of the points
+  // the distance tests go by blocks of two points: four at once are seldom far
+  // from every atom of a wave (2,000 poses of 61 atoms on 8,000 points in tiles
+  // 1.30 -> 1.22 ms, of 45 atoms on 6,000 points 0.76 -> 0.69)
+  constexpr int NB = NP < 2 ? NP : 2;
+  float qm[NP];  // the lane's nearest atom to each point
 #pragma unroll
   for (int j = 0; j < NP; ++j) {
 #pragma unroll
@@ -254,7 +258,7 @@ __device__ __forceinline__ void pair_group(const Lds &S, int p, const float4 (&P
       d2[j][k] = q2;
       rd[j][k] = r;
       dd[j][k] = d;
-      qmin = j == 0 && k == 0 ? q2 : fminf(qmin, q2);
+      qm[j] = k == 0 ? q2 : fminf(qm[j], q2);
       const float d3 = q2 * d;
       const float d6 = d3 * d3;
       num[j][k] = fmaf(-cp[k].p2a, d3, cp[k].p1a);
@@ -262,61 +266,67 @@ __device__ __forceinline__ void pair_group(const Lds &S, int p, const float4 (&P
       ele[k] = fmaf(P[j].w, r, ele[k]);
     }
   }
-  if (__ballot(!(qmin > G.far2)) != 0) {
 #pragma unroll
-    for (int j = 0; j < NP; ++j)
+  for (int j0 = 0; j0 < NP; j0 += NB) {
+    float qmin = qm[j0];
 #pragma unroll
-      for (int k = 0; k < APL; ++k) {
-        const float q2 = d2[j][k];
-        // the exponent is clamped at 64 (exp2 must stay finite) only in chunks
-        // whose parameters let it reach 60; elsewhere the clamp is a no-op
-        const float wv0 = fmaf(pa, q2, fmaf(cp[k].pb, dd[j][k], cp[k].pc));
-        const float wv = CLAMP ? fminf(wv0, 64.0f) : wv0;
-        // den (1 + e) and num (1 + e) as den + den e and num + num e: one
-        // fma each, one rounding each
-        const float e = fast_exp2(wv);
-        dn[j][k] = fmaf(den[j][k], e, den[j][k]);
-        num[j][k] = fmaf(num[j][k], e, num[j][k]);
-        if (KIND >= KIND_HPC) {
-          // u <= 1, so clamping to [0, 1] is max(u, 0): the fma's own clamp
-          const float u = __builtin_amdgcn_fmed3f(fmaf(q2, -INV81, 1.0f), 0.0f, 1.0f);
-          const float u3 = u * u * u;
-          hpc[k] = fmaf(hp[j], fmaf(u3, u, u3), hpc[k]);
-        }
-      }
-    // contact range: the lane's nearest atom against the largest of its
-    // atoms' near radii (a superset of the pairs the branch needs; the terms
-    // inside test each pair exactly)
-    if (__ballot(qmin <= G.nr2) != 0) {
+    for (int j = j0 + 1; j < j0 + NB; ++j) qmin = fminf(qmin, qm[j]);
+    if (__ballot(!(qmin > G.far2)) != 0) {
 #pragma unroll
-      for (int j = 0; j < NP; ++j)
+      for (int j = j0; j < j0 + NB; ++j)
 #pragma unroll
         for (int k = 0; k < APL; ++k) {
-          const float d = dd[j][k];
-          const bool c = d <= cp[k].pmf0;
-          cnt[k] += c ? 1 : 0;
-          const float s = K.el1 * d;
-          if (s < 1.0f) {
-            const float gn = fmaf(s * s, fmaf(K.b1, s, K.a1), K.el0);
-            ele[k] = fmaf(P[j].w, fmaf(K.el1, gn, -rd[j][k]), ele[k]);
-          }
-          if (KIND == KIND_PSP) {
-            if (c) psp[k] += psprow[k][ps[j]];
+          const float q2 = d2[j][k];
+          // the exponent is clamped at 64 (exp2 must stay finite) only in chunks
+          // whose parameters let it reach 60; elsewhere the clamp is a no-op
+          const float wv0 = fmaf(pa, q2, fmaf(cp[k].pb, dd[j][k], cp[k].pc));
+          const float wv = CLAMP ? fminf(wv0, 64.0f) : wv0;
+          // den (1 + e) and num (1 + e) as den + den e and num + num e: one
+          // fma each, one rounding each
+          const float e = fast_exp2(wv);
+          dn[j][k] = fmaf(den[j][k], e, den[j][k]);
+          num[j][k] = fmaf(num[j][k], e, num[j][k]);
+          if (KIND >= KIND_HPC) {
+            // u <= 1, so clamping to [0, 1] is max(u, 0): the fma's own clamp
+            const float u = __builtin_amdgcn_fmed3f(fmaf(q2, -INV81, 1.0f), 0.0f, 1.0f);
+            const float u3 = u * u * u;
+            hpc[k] = fmaf(hp[j], fmaf(u3, u, u3), hpc[k]);
           }
         }
-    }
-  }
-  // H-bond: only in chunks where some lane's atom has an H-bond record with
-  // this receptor type (elsewhere every term would be 0 * exp2), and there
-  // only where such a lane is within its records' range
-  if (HB && __ballot(!(qmin > G.hb2)) != 0) {
+      // contact range: the lane's nearest atom against the largest of its
+      // atoms' near radii (a superset of the pairs the branch needs; the terms
+      // inside test each pair exactly)
+      if (__ballot(qmin <= G.nr2) != 0) {
 #pragma unroll
-    for (int j = 0; j < NP; ++j)
+        for (int j = j0; j < j0 + NB; ++j)
 #pragma unroll
-      for (int k = 0; k < APL; ++k) {
-        const float h = fmaf(dd[j][k], cp[k].ha, cp[k].hb);
-        hdb[k] = fmaf(cp[k].hc, fast_exp2(-(h * h)), hdb[k]);
+          for (int k = 0; k < APL; ++k) {
+            const float d = dd[j][k];
+            const bool c = d <= cp[k].pmf0;
+            cnt[k] += c ? 1 : 0;
+            const float s = K.el1 * d;
+            if (s < 1.0f) {
+              const float gn = fmaf(s * s, fmaf(K.b1, s, K.a1), K.el0);
+              ele[k] = fmaf(P[j].w, fmaf(K.el1, gn, -rd[j][k]), ele[k]);
+            }
+            if (KIND == KIND_PSP) {
+              if (c) psp[k] += psprow[k][ps[j]];
+            }
+          }
       }
+    }
+    // H-bond: only in chunks where some lane's atom has an H-bond record with
+    // this receptor type (elsewhere every term would be 0 * exp2), and there
+    // only where such a lane is within its records' range
+    if (HB && __ballot(!(qmin > G.hb2)) != 0) {
+#pragma unroll
+      for (int j = j0; j < j0 + NB; ++j)
+#pragma unroll
+        for (int k = 0; k < APL; ++k) {
+          const float h = fmaf(dd[j][k], cp[k].ha, cp[k].hb);
+          hdb[k] = fmaf(cp[k].hc, fast_exp2(-(h * h)), hdb[k]);
+        }
+    }
   }
 #pragma unroll
   for (int j = 0; j < NP; ++j)
