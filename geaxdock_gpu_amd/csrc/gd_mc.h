@@ -243,10 +243,12 @@ __device__ __forceinline__ void pair_group(const Lds &S, int p, const float4 (&P
     ps[j] = (KIND == KIND_PSP) ? S.psp[p + j] : 0;
   }
   float d2[NP][APL], rd[NP][APL], dd[NP][APL], num[NP][APL], den[NP][APL], dn[NP][APL];
-  // the distance tests go by blocks of two points: four at once are seldom far
-  // from every atom of a wave (2,000 poses of 61 atoms on 8,000 points in tiles
-  // 1.30 -> 1.22 ms, of 45 atoms on 6,000 points 0.76 -> 0.69)
-  constexpr int NB = NP < 2 ? NP : 2;
+  // the distance tests go by blocks of points, of one where a lane has several
+  // atoms (independent work enough), else of two: four at once are seldom far
+  // from every atom of a wave (four -> two -> this, in tiles: 2,000 poses of 61
+  // atoms on 8,000 points 1.30 -> 1.22 -> 1.21 ms, of 45 atoms on 6,000 points 0.76
+  // -> 0.70 -> 0.66)
+  constexpr int NB = NP < 2 || APL >= 2 ? 1 : 2;
   float qm[NP];  // the lane's nearest atom to each point
 #pragma unroll
   for (int j = 0; j < NP; ++j) {
