@@ -889,6 +889,7 @@ gd_status build_flat(gd_ctx *ctx) {
     HostComplex *h;
     int f;
     size_t at;
+    int n;
   };
   std::vector<Todo> todo;
   std::vector<int4> all;
@@ -898,8 +899,7 @@ gd_status build_flat(gd_ctx *ctx) {
     for (int f = 0; f < 4; ++f) {
       if (!(want[c] >> f & 1) || h.flat_n[f] > 0) continue;
       const std::vector<int4> U = build_flat_units(h.chunks, h.apl, 1 << f, h.dev.flat_off[f]);
-      h.flat_n[f] = (int)U.size();
-      todo.push_back({&h, f, all.size()});
+      todo.push_back({&h, f, all.size(), (int)U.size()});
       all.insert(all.end(), U.begin(), U.end());
     }
   }
@@ -909,7 +909,11 @@ gd_status build_flat(gd_ctx *ctx) {
   ctx->flat_bufs.push_back(p);
   HIPCHK(hipMemcpyAsync(p, all.data(), all.size() * sizeof(int4), hipMemcpyHostToDevice, ctx->stream));
   HIPCHK(hipStreamSynchronize(ctx->stream));
-  for (const Todo &t : todo) t.h->dev.flat[t.f] = static_cast<int4 *>(p) + t.at;
+  // a list counts (flat_n) from here on, when the device holds it
+  for (const Todo &t : todo) {
+    t.h->dev.flat[t.f] = static_cast<int4 *>(p) + t.at;
+    t.h->flat_n[t.f] = t.n;
+  }
   return GD_OK;
 }
 

@@ -1,0 +1,118 @@
+"""Host code of the engine when a device call fails: allocations and launches
+fail where a case says so, on a HIP runtime of host memory that runs no kernel
+(tests/cpp/host_hip.cpp). A failed call is an error; what the context does
+afterwards must not use memory that is not there.
+
+Each case runs in a process of its own, since the library binds its runtime once.
+"""
+import ctypes as C
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+
+class HostHip:
+    """The controls and records of host_hip.cpp."""
+
+    def __init__(self, path):
+        # global: the engine's library, loaded later, binds to these symbols
+        self.lib = C.CDLL(path, mode=C.RTLD_GLOBAL)
+        self.lib.host_hip_alloc_size.restype = C.c_size_t
+        self.lib.host_hip_kernel.restype = C.c_char_p
+        self.lib.host_hip_grid.restype = C.c_uint
+        for f in ("num_allocs", "num_live", "num_made", "num_launches"):
+            getattr(self.lib, "host_hip_" + f).restype = C.c_long
+
+    def fail_alloc(self, n=0):
+        self.lib.host_hip_fail_alloc(C.c_long(n))
+
+    def fail_launch(self, n=0):
+        self.lib.host_hip_fail_launch(C.c_long(n))
+
+    def fail_above(self, size):
+        self.lib.host_hip_fail_above(C.c_size_t(size))
+
+    def count(self, what):
+        return getattr(self.lib, "host_hip_num_" + what)()
+
+    def allocs(self, begin=0):
+        return [self.lib.host_hip_alloc_size(C.c_long(i))
+                for i in range(begin, self.count("allocs"))]
+
+    def launches(self, name="", begin=0):
+        out = []
+        for i in range(begin, self.count("launches")):
+            k = self.lib.host_hip_kernel(C.c_long(i)).decode()
+            if name in k:
+                out.append((k, [self.lib.host_hip_grid(C.c_long(i), a) for a in range(3)],
+                            bool(self.lib.host_hip_table(C.c_long(i)))))
+        return out
+
+
+def complex_(seed=1, **kw):
+    from geaxdock_gpu_amd import synth
+    return synth.make_complex(seed, **{**dict(lna=20, pnp=300, pnk=30, pos=3, mcs_atoms=5,
+                                              n_lig=2, n_prt=1, n_tmp=4, void_radius=3.0), **kw})
+
+
+def poses(n, n_lig=2):
+    return (np.arange(n, dtype=np.int32) % n_lig, np.zeros(n, np.int32),
+            np.zeros((n, 6), np.float32))
+
+
+def fails(call, *status):
+    """The call ends with one of these statuses."""
+    import geaxdock_gpu_amd as gd
+    from geaxdock_gpu_amd import abi
+    with pytest.raises(gd.GeauxDockError) as e:
+        call()
+    assert abi.STATUS[e.value.status] in status, str(e.value)
+
+
+def unit_lists(hip):
+    """A unit list that found no memory is built by the next call; before, the
+    launches of that call read the list through a null pointer."""
+    import geaxdock_gpu_amd as gd
+    with gd.Engine(seed=1) as eng:
+        eng.add_complex(complex_())
+        # the first allocation of the call is the list's
+        begin = hip.count("allocs")
+        hip.fail_alloc(0)
+        fails(lambda: eng.calc_energy(0, *poses(3)), "GD_ERR_HIP")
+        size = hip.allocs(begin)[0]
+        assert size >= 16 * 8  # at least a unit for each of eight groups
+        begin, first = hip.count("allocs"), hip.count("launches")
+        eng.calc_energy(0, *poses(3))
+        assert hip.allocs(begin)[0] == size
+        # the units' instance: <1, 0, false, true>
+        assert any("Lb0ELb1E" in k for k, _, _ in hip.launches("gd_mc_kernel", first))
+
+
+CASES = [unit_lists]
+
+
+@pytest.fixture(scope="module")
+def runtime(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("host_hip") / "libhost_hip.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__",
+                    "-I/opt/rocm/include", os.path.join(HERE, "cpp", "host_hip.cpp"), "-o", so],
+                   check=True)
+    return so
+
+
+@pytest.mark.parametrize("case", [c.__name__ for c in CASES])
+def test_host_failures(runtime, case):
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), runtime, case], cwd=ROOT,
+                       capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+if __name__ == "__main__":
+    sys.path.insert(0, ROOT)
+    {c.__name__: c for c in CASES}[sys.argv[2]](HostHip(sys.argv[1]))
