@@ -921,15 +921,22 @@ gd_status sync_complexes(gd_ctx *ctx) {
   if (!ctx->cx_dirty) return GD_OK;
   TRY(widen_shapes(ctx));
   TRY(build_flat(ctx));
-  if (ctx->d_cx) HIPCHK(hipFree(ctx->d_cx));
-  ctx->d_cx = nullptr;
-  for (auto &g : ctx->gslot) g.valid = false;  // captured launches hold the old pointer
+  // runs and feature kernels do not come through here: the table they use stays
+  // until the new one is on the device
   std::vector<DevComplex> v;
   for (auto &h : ctx->cx) v.push_back(h.dev);
-  HIPCHK(hipMalloc(&ctx->d_cx, std::max<size_t>(v.size(), 1) * sizeof(DevComplex)));
-  HIPCHK(hipMemcpyAsync(ctx->d_cx, v.data(), v.size() * sizeof(DevComplex), hipMemcpyHostToDevice,
-                        ctx->stream));
-  HIPCHK(hipStreamSynchronize(ctx->stream));
+  DevComplex *table = nullptr;
+  HIPCHK(hipMalloc(&table, std::max<size_t>(v.size(), 1) * sizeof(DevComplex)));
+  hipError_t e = hipMemcpyAsync(table, v.data(), v.size() * sizeof(DevComplex),
+                                hipMemcpyHostToDevice, ctx->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+  if (e != hipSuccess) {
+    (void)hipFree(table);
+    return fail(ctx, GD_ERR_HIP, "complex table: %s", hipGetErrorString(e));
+  }
+  if (ctx->d_cx) (void)hipFree(ctx->d_cx);
+  ctx->d_cx = table;
+  for (auto &g : ctx->gslot) g.valid = false;  // captured launches hold the old pointer
   ctx->cx_dirty = false;
   return GD_OK;
 }

@@ -94,7 +94,25 @@ def unit_lists(hip):
         assert any("Lb0ELb1E" in k for k, _, _ in hip.launches("gd_mc_kernel", first))
 
 
-CASES = [unit_lists]
+def complex_table(hip):
+    """The complex table on the device is replaced only when the new one is
+    there: runs after a failed upload read the table they had."""
+    import geaxdock_gpu_amd as gd
+    with gd.Engine(seed=1, launch=gd.abi.LAUNCH_NO_GRAPH | gd.abi.LAUNCH_NO_SPREAD) as eng:
+        eng.add_complex(complex_())
+        eng.run(4, 2)
+        begin = hip.count("allocs")
+        eng.sur_build_grids(1.0, 4.0)
+        n = hip.count("allocs") - begin  # the table's is the last
+        hip.fail_alloc(n - 2)  # the grid keeps its memory this time
+        fails(lambda: eng.sur_build_grids(1.0, 4.0), "GD_ERR_HIP")
+        first = hip.count("launches")
+        eng.run(4, 2)
+        runs = hip.launches("gd_mc_kernel", first)
+        assert runs and all(table for _, _, table in runs)
+
+
+CASES = [unit_lists, complex_table]
 
 
 @pytest.fixture(scope="module")
