@@ -2551,7 +2551,15 @@ gd_status gd_sur_build_grids(gd_ctx *ctx, float spacing, float half_width) {
   auto &S = ctx->sur;
   const int n = (int)std::ceil(2.0f * half_width / spacing) + 1;
   const size_t nodes = (size_t)n * n * n;
+  // no grids (S.g is what calls ask) until all of them are there and in the
+  // complex table: a failure below leaves some replaced, some freed
   S.tab_valid = false;
+  S.g.clear();
+  for (HostComplex &h : ctx->cx) {
+    h.dev.sgrid = nullptr;
+    h.dev.stab = nullptr;
+  }
+  ctx->cx_dirty = true;
   // grids and tables of the sizes they had are kept, others replaced (the
   // number of complexes only grows)
   const size_t n_cx = ctx->cx.size();
@@ -2559,7 +2567,7 @@ gd_status gd_sur_build_grids(gd_ctx *ctx, float spacing, float half_width) {
   S.tab.resize(n_cx, nullptr);
   S.grid_n.resize(n_cx, 0);
   S.tab_n.resize(n_cx, 0);
-  S.g.assign(n_cx, SurGrid{});
+  std::vector<SurGrid> grids(n_cx);
   for (size_t c = 0; c < n_cx; ++c) {
     const HostComplex &h = ctx->cx[c];
     const size_t need = (size_t)h.d.n_prt * nodes * 32;
@@ -2582,15 +2590,13 @@ gd_status gd_sur_build_grids(gd_ctx *ctx, float spacing, float half_width) {
     G.oz = h.d.pocket_center[2] - half_width;
     G.h = spacing;
     G.n = n;
-    S.g[c] = G;
+    grids[c] = G;
     ctx->cx[c].dev.sgrid = G.grid;
     ctx->cx[c].dev.sox = G.ox;
     ctx->cx[c].dev.soy = G.oy;
     ctx->cx[c].dev.soz = G.oz;
     ctx->cx[c].dev.sh = G.h;
     ctx->cx[c].dev.sn = G.n;
-    ctx->cx[c].dev.stab = nullptr;
-    ctx->cx_dirty = true;
     const int64_t nb = (n + 3) / 4, bricks = nb * nb * nb;
     hipLaunchKernelGGL(gd_sur_grid_kernel,
                        dim3((unsigned)((bricks + 3) / 4), (unsigned)h.d.n_prt), dim3(256), 0,
@@ -2600,6 +2606,7 @@ gd_status gd_sur_build_grids(gd_ctx *ctx, float spacing, float half_width) {
   }
   HIPCHK(hipStreamSynchronize(ctx->stream));
   TRY(sync_complexes(ctx));
+  S.g = std::move(grids);
   return GD_OK;
 }
 

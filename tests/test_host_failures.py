@@ -112,7 +112,39 @@ def complex_table(hip):
         assert runs and all(table for _, _, table in runs)
 
 
-CASES = [unit_lists, complex_table]
+def feature_grids(hip):
+    """Grids that found no memory, or never reached the complex table, are no
+    grids: the calls that read them refuse until they are built again."""
+    import geaxdock_gpu_amd as gd
+    target = np.zeros(3, np.float32)
+    for failing in range(4):  # grid 0, grid 1, the table; then none
+        with gd.Engine(seed=1) as eng:
+            for seed in (1, 2):
+                eng.add_complex(complex_(seed))
+            eng.sur_set_params(np.zeros(eng.sur_num_params, np.float32))
+            eng.sur_build_grids(1.0, 4.0)
+            eng.sur_tabulate()
+            first = hip.count("launches")
+            if failing < 3:
+                hip.fail_alloc(failing)
+                fails(lambda: eng.sur_build_grids(1.0, 5.0), "GD_ERR_HIP")
+                uses = [lambda c=c: eng.sur_features(c, *poses(3)) for c in (0, 1)]
+                uses += [lambda c=c: eng.sur_dataset_add(c, *poses(3), target) for c in (0, 1)]
+                uses += [lambda: eng.sur_dataset_add_multi(np.zeros(3, np.int32), *poses(3), target),
+                         lambda: eng.sur_surrogate(0, *poses(3), 1.0), eng.sur_tabulate,
+                         lambda: eng.run_da(4, 0, 2, 1.0)]
+                for use in uses:
+                    fails(use, "GD_ERR_STATE")
+                assert not hip.launches("gd_sur_feat", first) and not hip.launches("gd_mc", first)
+                eng.calc_energy(0, *poses(3))  # needs no grids
+                eng.sur_build_grids(1.0, 5.0)
+            for c in (0, 1):
+                eng.sur_features(c, *poses(3))
+            eng.sur_tabulate()
+            eng.run_da(4, 0, 2, 1.0)
+
+
+CASES = [unit_lists, complex_table, feature_grids]
 
 
 @pytest.fixture(scope="module")
