@@ -430,8 +430,21 @@ int gd_num_replicas(const gd_ctx *ctx, int cid) {
   return ctx->cx[cid].n_rep;
 }
 
+static gd_status add_complex(gd_ctx *ctx, const gd_complex_desc *d, int *complex_id);
+
 gd_status gd_add_complex(gd_ctx *ctx, const gd_complex_desc *d, int *complex_id) {
   if (!ctx || !d) return GD_ERR_INVALID;
+  const size_t n = ctx->cx.size();
+  const gd_status st = add_complex(ctx, d, complex_id);
+  // a complex that failed half-way has arrays missing: it leaves the context
+  if (st != GD_OK && ctx->cx.size() > n) {
+    for (void *p : ctx->cx.back().bufs) (void)hipFree(p);
+    ctx->cx.pop_back();
+  }
+  return st;
+}
+
+static gd_status add_complex(gd_ctx *ctx, const gd_complex_desc *d, int *complex_id) {
   if (ctx->state_alloc) return fail(ctx, GD_ERR_STATE, "complexes must be added before gd_run");
   if (d->n_lig <= 0 || d->n_prt <= 0 || d->n_tmp <= 0 || d->lna <= 0 || d->pnp <= 0 ||
       d->pnk < 0 || d->pos < 0)

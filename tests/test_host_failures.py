@@ -144,7 +144,28 @@ def feature_grids(hip):
             eng.run_da(4, 0, 2, 1.0)
 
 
-CASES = [unit_lists, complex_table, feature_grids]
+def refused_complex(hip):
+    """A complex that could not be added is not in the context: the next one
+    takes its id, and kernels get no record without arrays."""
+    import geaxdock_gpu_amd as gd
+    # no memory for the device block, for the staging; tiles beyond LDS
+    for kw, failing, status in [({}, 0, "GD_ERR_HIP"), ({}, 1, "GD_ERR_HIP"),
+                                (dict(receptor_tile=4000), -1, "GD_ERR_CAPACITY")]:
+        with gd.Engine(seed=1, **kw) as eng:
+            live = hip.count("live")
+            hip.fail_alloc(failing)
+            fails(lambda: eng.add_complex(complex_()), status)
+            assert eng.num_replicas(0) == -1
+            assert hip.count("live") <= live + 1  # at most the staging stays
+            if kw:
+                continue
+            assert eng.add_complex(complex_()) == 0
+            first = hip.count("launches")
+            eng.calc_energy(0, *poses(3))
+            assert hip.launches("gd_ref_kernel", first)[0][1] == [20, 1, 1]  # one complex
+
+
+CASES = [unit_lists, complex_table, feature_grids, refused_complex]
 
 
 @pytest.fixture(scope="module")
