@@ -2487,9 +2487,12 @@ gd_status sur_work(gd_ctx *ctx, int64_t rows, int64_t n_pose_total) {
   auto &S = ctx->sur;
   rows = (rows + 63) / 64 * 64 + 64;
   if (rows > S.work_rows) {
-    void *qs[] = {S.p1, S.p2, S.pb2, S.pw3, S.dyr};
-    for (void *p : qs)
-      if (p) (void)hipFree(p);
+    float **qs[] = {&S.p1, &S.p2, &S.pb2, &S.pw3, &S.dyr};
+    S.work_rows = 0;
+    for (float **q : qs) {
+      if (*q) (void)hipFree(*q);
+      *q = nullptr;
+    }
     const int64_t ng = std::max(1, ctx->n_cu);
     HIPCHK(hipMalloc(&S.dyr, (size_t)rows * sizeof(float)));
     HIPCHK(hipMalloc(&S.p1, (size_t)ng * SUR_F * SUR_H * sizeof(float)));

@@ -165,7 +165,26 @@ def refused_complex(hip):
             assert hip.launches("gd_ref_kernel", first)[0][1] == [20, 1, 1]  # one complex
 
 
-CASES = [unit_lists, complex_table, feature_grids, refused_complex]
+def training_buffers(hip):
+    """Work buffers that could not grow are gone, not in use after their end:
+    every buffer is given back once (host_hip.cpp aborts on a second time)."""
+    import geaxdock_gpu_amd as gd
+    for failing in range(5):  # rows' gradients, then the four gradient partials
+        with gd.Engine(seed=1) as eng:
+            eng.add_complex(complex_())
+            eng.sur_set_params(np.zeros(eng.sur_num_params, np.float32))
+            eng.sur_build_grids(1.0, 4.0)
+            eng.sur_dataset_add(0, *poses(40), np.zeros(40, np.float32))
+            eng.sur_loss_grad(0, 2)
+            hip.fail_alloc(failing)
+            fails(lambda: eng.sur_loss_grad(0, 40), "GD_ERR_HIP")
+            begin = hip.count("allocs")
+            eng.sur_loss_grad(0, 2)
+            assert hip.count("allocs") - begin == 5
+            eng.sur_loss_grad(0, 40)
+
+
+CASES = [unit_lists, complex_table, feature_grids, refused_complex, training_buffers]
 
 
 @pytest.fixture(scope="module")
