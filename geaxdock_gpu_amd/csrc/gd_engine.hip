@@ -2418,14 +2418,14 @@ namespace {
 
 gd_status sur_alloc_params(gd_ctx *ctx) {
   auto &S = ctx->sur;
-  if (S.p) return GD_OK;
-  HIPCHK(hipMalloc(&S.p, SUR_NPARAM * sizeof(float)));
-  HIPCHK(hipMalloc(&S.m, SUR_NPARAM * sizeof(float)));
-  HIPCHK(hipMalloc(&S.v, SUR_NPARAM * sizeof(float)));
-  HIPCHK(hipMalloc(&S.grad, SUR_NPARAM * sizeof(float)));
-  HIPCHK(hipMalloc(&S.W1T, SUR_F * SUR_H * 2));
-  HIPCHK(hipMalloc(&S.W2T, SUR_H * SUR_H * 2));
-  HIPCHK(hipMalloc(&S.W2R, SUR_H * SUR_H * 2));
+  // each that is missing: an earlier call may have failed half-way
+  auto need = [](auto **p, size_t n) {
+    return *p ? hipSuccess : hipMalloc(p, n * sizeof(**p));
+  };
+  for (float **p : {&S.p, &S.m, &S.v, &S.grad}) HIPCHK(need(p, SUR_NPARAM));
+  HIPCHK(need(&S.W1T, SUR_F * SUR_H));
+  HIPCHK(need(&S.W2T, SUR_H * SUR_H));
+  HIPCHK(need(&S.W2R, SUR_H * SUR_H));
   return GD_OK;
 }
 

@@ -184,7 +184,22 @@ def training_buffers(hip):
             eng.sur_loss_grad(0, 40)
 
 
-CASES = [unit_lists, complex_table, feature_grids, refused_complex, training_buffers]
+def parameter_buffers(hip):
+    """Parameters whose buffers were not all allocated get the missing ones in
+    the next call; before, it wrote the weights' layouts to null pointers."""
+    import geaxdock_gpu_amd as gd
+    for failing in range(7):
+        with gd.Engine(seed=1) as eng:
+            p = np.zeros(eng.sur_num_params, np.float32)
+            live = hip.count("live")
+            hip.fail_alloc(failing)
+            fails(lambda: eng.sur_set_params(p), "GD_ERR_HIP")
+            eng.sur_set_params(p)
+            assert hip.count("live") == live + 7
+
+
+CASES = [unit_lists, complex_table, feature_grids, refused_complex, training_buffers,
+         parameter_buffers]
 
 
 @pytest.fixture(scope="module")
