@@ -173,6 +173,9 @@ gd_status fail(gd_ctx *c, gd_status s, const char *fmt, ...) {
   vsnprintf(buf, sizeof buf, fmt, ap);
   va_end(ap);
   if (c) c->err = buf;
+  // the runtime keeps a failed call's error until it is asked for: it is
+  // reported here and must not be found by the next call's launch check
+  if (s == GD_ERR_HIP || s == GD_ERR_NOMEM) (void)hipGetLastError();
   return s;
 }
 

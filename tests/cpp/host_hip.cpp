@@ -33,13 +33,15 @@ struct {
   hipStream_t stream;
 } config;
 
+hipError_t last = hipSuccess;  // of any call, until it is asked for
+
 hipError_t allocate(void **p, size_t bytes) {
   allocs.push_back(bytes);
   *p = nullptr;
-  if (fail_alloc >= 0 && fail_alloc-- == 0) return hipErrorOutOfMemory;
-  if (fail_above > 0 && bytes > fail_above) return hipErrorOutOfMemory;
+  if (fail_alloc >= 0 && fail_alloc-- == 0) return last = hipErrorOutOfMemory;
+  if (fail_above > 0 && bytes > fail_above) return last = hipErrorOutOfMemory;
   *p = std::calloc(1, bytes);
-  if (!*p) return hipErrorOutOfMemory;
+  if (!*p) return last = hipErrorOutOfMemory;
   live[*p] = bytes;
   return hipSuccess;
 }
@@ -103,7 +105,6 @@ hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *lds, hipSt
   return hipSuccess;
 }
 
-static hipError_t last = hipSuccess;
 hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3, void **args, size_t, hipStream_t) {
   if (!f) std::abort();
   if (fail_launch >= 0 && fail_launch-- == 0) return last = hipErrorLaunchFailure;
