@@ -1632,30 +1632,42 @@ gd_status drain_records(gd_ctx *ctx, gd_record_sink sink, void *user) {
 // Record rings for windows of up to `win` steps (and the start poses): ring 0,
 // and ring 1 when windows alternate. Called between runs, when they are empty.
 // They grow with the longest window asked for, not to steps_per_dump at once
-// (93 MB and 1 ms for a first run of 200 steps of 504 replicas).
+// (93 MB and 1 ms for a first run of 200 steps of 504 replicas). Rings that do
+// not fit are all given back, so a run of shorter windows sizes its own.
 gd_status ensure_rings(gd_ctx *ctx, int win, bool both) {
   if (!ctx->opts.record) return GD_OK;
   const size_t n = ctx->n_rep;
-  if (win + 1 > ctx->rec_cap) {
+  auto drop = [&] {
     for (int r = 0; r < 2; ++r) {
-      if (ctx->d_ring[r]) HIPCHK(hipFree(ctx->d_ring[r]));
+      if (ctx->d_ring[r]) (void)hipFree(ctx->d_ring[r]);
       ctx->d_ring[r] = nullptr;
     }
+    for (auto &g : ctx->gslot) g.valid = false;  // captured launches hold the old rings
+    ctx->rec_cap = 0;
+  };
+  if (win + 1 > ctx->rec_cap) {
+    drop();
     for (int r = 0; r < 2; ++r)
       if (ctx->d_ring_cnt[r]) HIPCHK(hipMemsetAsync(ctx->d_ring_cnt[r], 0, n * sizeof(int), ctx->stream));
-    for (auto &g : ctx->gslot) g.valid = false;  // captured launches hold the old rings
     ctx->rec_cap = win + 1;
   }
-  for (int r = 0; r < (both ? 2 : 1); ++r) {
-    if (!ctx->d_ring[r])
-      HIPCHK(hipMalloc(&ctx->d_ring[r], n * ctx->rec_cap * sizeof(gd_record)));
-    if (!ctx->d_ring_cnt[r]) {
+  for (int r = 0; r < 2; ++r) {
+    // the ring in use may be the second, left current by windows that alternated
+    const bool used = r == 0 || both || r == ctx->ring;
+    if (used && !ctx->d_ring[r]) {
+      const hipError_t e = hipMalloc(&ctx->d_ring[r], n * ctx->rec_cap * sizeof(gd_record));
+      if (e != hipSuccess) {
+        ctx->d_ring[r] = nullptr;
+        const int cap = ctx->rec_cap;
+        drop();
+        return fail(ctx, GD_ERR_HIP, "record rings of %d steps: %s", cap, hipGetErrorString(e));
+      }
+    }
+    if (used && !ctx->d_ring_cnt[r]) {
       HIPCHK(hipMalloc(&ctx->d_ring_cnt[r], n * sizeof(int)));
       HIPCHK(hipMemsetAsync(ctx->d_ring_cnt[r], 0, n * sizeof(int), ctx->stream));
     }
   }
-  if (!ctx->d_ring[ctx->ring])  // ring 1 was current and is not kept
-    HIPCHK(hipMalloc(&ctx->d_ring[ctx->ring], n * ctx->rec_cap * sizeof(gd_record)));
   if (both && !ctx->drain_stream)
     HIPCHK(hipStreamCreateWithFlags(&ctx->drain_stream, hipStreamNonBlocking));
   HIPCHK(hipStreamSynchronize(ctx->stream));

@@ -198,8 +198,28 @@ def parameter_buffers(hip):
             assert hip.count("live") == live + 7
 
 
+def record_rings(hip):
+    """After a window whose record rings do not fit, runs of windows that do fit
+    go on, with one ring (no sink) or two."""
+    import geaxdock_gpu_amd as gd
+    record, n_rep = 92, 8
+    fit = record * n_rep * 101  # a window of 100 steps
+    for sink in (None, lambda c, r: None):
+        for launch in (0, gd.abi.LAUNCH_NO_SPREAD):
+            with gd.Engine(seed=1, launch=launch, steps_per_dump=1 << 20) as eng:
+                eng.add_complex(complex_())
+                assert eng.num_replicas(0) == n_rep
+                eng.run(10, 0, sink)
+                hip.fail_above(fit)
+                fails(lambda: eng.run(1 << 20, 0, sink), "GD_ERR_HIP")
+                eng.run(100, 0, sink)
+                eng.run(10, 0, sink)
+                hip.fail_above(0)
+                eng.run(200, 0, sink)
+
+
 CASES = [unit_lists, complex_table, feature_grids, refused_complex, training_buffers,
-         parameter_buffers]
+         parameter_buffers, record_rings]
 
 
 @pytest.fixture(scope="module")
