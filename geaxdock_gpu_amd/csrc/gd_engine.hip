@@ -1805,7 +1805,8 @@ gd_status tree_buffers(gd_ctx *ctx, int depth, int **cnt, gd_energy **e) {
 // One window of spread packing: MC launches that end on exchange steps, each
 // followed by the ladder exchange kernel, all enqueued at once and timed
 // together (waiting for each launch left the GPU idle for 60 to 90 us every
-// exchange interval). Advances ctx->step as launches are enqueued.
+// exchange interval). ctx->step follows each launch as it is enqueued, so a window
+// that ends in an error does not take the same random numbers again.
 gd_status spread_window(gd_ctx *ctx, int win, int nc, int da_k, float sur_scale, double *ms_sum,
                         int *launches) {
   KParams P = mc_params(ctx, da_k, sur_scale);
@@ -1843,6 +1844,7 @@ gd_status spread_window(gd_ctx *ctx, int win, int nc, int da_k, float sur_scale,
           cl.grid = cl.packs * cl.P.tree_nodes;
         }
         HIPCHK(enqueue_classes(ctx, cls, nullptr, ctx->stream));
+        ctx->step += d;
         at += d;
       }
       *launches += rounds - 1;
@@ -1852,6 +1854,7 @@ gd_status spread_window(gd_ctx *ctx, int win, int nc, int da_k, float sur_scale,
         cl.P.n_steps = sub;
       }
       HIPCHK(enqueue_classes(ctx, cls, queue, ctx->stream));
+      ctx->step += sub;
     }
     if (nc > 0 && (s + sub) % nc == 0) {
       hipLaunchKernelGGL(gd_ladder_exchange_kernel, dim3((ctx->n_ladders + 63) / 64), dim3(64),
@@ -1860,7 +1863,6 @@ gd_status spread_window(gd_ctx *ctx, int win, int nc, int da_k, float sur_scale,
       HIPCHK(hipGetLastError());
     }
     *launches += 1;
-    ctx->step += sub;
     done += sub;
   }
   HIPCHK(hipEventRecord(ctx->ev1, ctx->stream));

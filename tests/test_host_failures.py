@@ -7,6 +7,7 @@ Each case runs in a process of its own, since the library binds its runtime once
 """
 import ctypes as C
 import os
+import struct
 import subprocess
 import sys
 
@@ -218,8 +219,28 @@ def record_rings(hip):
                 eng.run(200, 0, sink)
 
 
+def window_steps(hip):
+    """A window of several launches that ends in an error has taken the steps
+    of the launches before it: its random numbers are not used again."""
+    import geaxdock_gpu_amd as gd
+    with gd.Engine(seed=1, launch=gd.abi.LAUNCH_SPREAD) as eng:
+        eng.add_complex(complex_())  # eight packs: trees of five steps
+        eng.run(0, 10)
+        step = 0
+        # launches of a run: the counts, two trees, an exchange, two trees, an exchange
+        for failing, taken in ((1, 0), (2, 5), (3, 10), (4, 10), (5, 15), (6, 20)):
+            hip.fail_launch(failing)
+            fails(lambda: eng.run(20, 10), "GD_ERR_HIP")
+            step += taken
+            assert struct.unpack_from("<8I", eng.checkpoint())[4] == step, failing
+            rest = -step % 10
+            if rest:
+                eng.run(rest, 10)
+                step += rest
+
+
 CASES = [unit_lists, complex_table, feature_grids, refused_complex, training_buffers,
-         parameter_buffers, record_rings]
+         parameter_buffers, record_rings, window_steps]
 
 
 @pytest.fixture(scope="module")
