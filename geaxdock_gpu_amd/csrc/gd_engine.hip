@@ -68,6 +68,8 @@ struct Scratch {
 };
 constexpr size_t SCRATCH_KEEP = (size_t)256 << 20;
 
+constexpr int SIDE_STREAMS = 3;  // streams beside the main one for launch classes
+
 }  // namespace
 
 struct gd_ctx {
@@ -76,8 +78,8 @@ struct gd_ctx {
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   // side streams for concurrent launches of the per-APL kernel classes
-  hipStream_t aux[3] = {nullptr, nullptr, nullptr};
-  hipEvent_t ev_fork = nullptr, ev_join[3] = {nullptr, nullptr, nullptr};
+  hipStream_t aux[SIDE_STREAMS] = {};
+  hipEvent_t ev_fork = nullptr, ev_join[SIDE_STREAMS] = {};
   std::string err;
   int n_cu = 0;
   size_t max_lds = 65536;
@@ -412,7 +414,7 @@ void gd_destroy(gd_ctx *ctx) {
   if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
   if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
   if (ctx->ev_fork) (void)hipEventDestroy(ctx->ev_fork);
-  for (int i = 0; i < 3; ++i) {
+  for (int i = 0; i < SIDE_STREAMS; ++i) {
     if (ctx->ev_join[i]) (void)hipEventDestroy(ctx->ev_join[i]);
     if (ctx->aux[i]) (void)hipStreamDestroy(ctx->aux[i]);
   }
@@ -756,6 +758,19 @@ static gd_status add_complex(gd_ctx *ctx, const gd_complex_desc *d, int *complex
 
 namespace {
 
+// Side streams and their events for a launch of n classes (made on first use:
+// a stream costs about 50 us and as much again to destroy).
+hipError_t side_streams(gd_ctx *ctx, int n) {
+  hipError_t e = hipSuccess;
+  if (n > 1 && !ctx->ev_fork) e = hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming);
+  for (int i = 0; i < std::min(n - 1, SIDE_STREAMS) && e == hipSuccess; ++i) {
+    if (!ctx->aux[i]) e = hipStreamCreateWithFlags(&ctx->aux[i], hipStreamNonBlocking);
+    if (e == hipSuccess && !ctx->ev_join[i])
+      e = hipEventCreateWithFlags(&ctx->ev_join[i], hipEventDisableTiming);
+  }
+  return e;
+}
+
 bool spread_packing(const gd_ctx *ctx);
 int auto_gmax(const gd_ctx *ctx);
 std::vector<int> lig_splits(const gd_ctx *ctx, const HostComplex &h, int gmax);
@@ -969,6 +984,9 @@ gd_status ensure_ref(gd_ctx *ctx) {
       lna_max = std::max(lna_max, ctx->cx[c].d.lna);
     }
   if (todo.empty()) return GD_OK;
+  // pose calls without allocations come after this call and may need a launch
+  // for each block size (packs of a split below 8)
+  if (!spread_packing(ctx)) HIPCHK(side_streams(ctx, SIDE_STREAMS + 1));
   const size_t n = todo.size();
   int2 *d_out = nullptr;  // per complex: contacts, atoms beyond the limit; then the list
   HIPCHK(hipMalloc(&d_out, n * (sizeof(int2) + sizeof(int))));
@@ -1472,19 +1490,6 @@ struct ClassLaunch {
   size_t lds;
 };
 
-// Side streams and their events for a launch of n classes (made on first use:
-// a stream costs about 50 us and as much again to destroy).
-hipError_t side_streams(gd_ctx *ctx, int n) {
-  hipError_t e = hipSuccess;
-  if (n > 1 && !ctx->ev_fork) e = hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming);
-  for (int i = 0; i < std::min(n - 1, 3) && e == hipSuccess; ++i) {
-    if (!ctx->aux[i]) e = hipStreamCreateWithFlags(&ctx->aux[i], hipStreamNonBlocking);
-    if (e == hipSuccess && !ctx->ev_join[i])
-      e = hipEventCreateWithFlags(&ctx->ev_join[i], hipEventDisableTiming);
-  }
-  return e;
-}
-
 hipError_t plan_classes(gd_ctx *ctx, const std::vector<LaunchClass> &classes, const KParams &P0,
                         int da, bool da_scratch, int *queue, std::vector<ClassLaunch> &out) {
   out.clear();
@@ -1546,14 +1551,14 @@ hipError_t enqueue_classes(gd_ctx *ctx, std::vector<ClassLaunch> &cls, int *queu
     hipLaunchKernelGGL(gd_queue_reset_kernel, dim3((n + 63) / 64), dim3(64), 0, stream, queue, n);
     e = hipGetLastError();
   }
-  const int n_side = std::min(n - 1, 3);
+  const int n_side = std::min(n - 1, SIDE_STREAMS);
   if (e == hipSuccess && n_side > 0) {
     e = hipEventRecord(ctx->ev_fork, stream);
     for (int i = 0; i < n_side && e == hipSuccess; ++i) e = hipStreamWaitEvent(ctx->aux[i], ctx->ev_fork, 0);
   }
   for (int i = 0; i < n && e == hipSuccess; ++i) {
     void *args[] = {&cls[i].P};
-    const int side = i % 4;  // 0: the main stream
+    const int side = i % (SIDE_STREAMS + 1);  // 0: the main stream
     hipStream_t s = side == 0 ? stream : ctx->aux[side - 1];
     e = hipLaunchKernel(cls[i].f, dim3(cls[i].grid), dim3(cls[i].block), args, cls[i].lds, s);
   }

@@ -239,8 +239,25 @@ def window_steps(hip):
                 step += rest
 
 
+def pose_calls_without_allocations(hip):
+    """gd_calc_energy_noalloc allocates and creates nothing, whatever its
+    launches, after a gd_calc_energy of one pose or a gd_run."""
+    import geaxdock_gpu_amd as gd
+    for prepare in (lambda e: e.calc_energy(0, *poses(1)), lambda e: e.run(0)):
+        with gd.Engine(seed=1, ladders_per_pack=2) as eng:
+            eng.add_complex(complex_(n_lig=3, n_tmp=8))  # conformers of splits of 4 and 8
+            prepare(eng)
+            for n in (1, 5, 340):  # the last pack of a split may be small
+                made, allocs = hip.count("made"), hip.count("allocs")
+                first = hip.count("launches")
+                eng.calc_energy_noalloc(0, *poses(n, 3))
+                assert n == 1 or len(hip.launches("gd_mc_kernel", first)) > 1
+                assert (hip.count("made"), hip.count("allocs")) == (made, allocs), n
+
+
 CASES = [unit_lists, complex_table, feature_grids, refused_complex, training_buffers,
-         parameter_buffers, record_rings, window_steps]
+         parameter_buffers, record_rings, window_steps,
+         pose_calls_without_allocations]
 
 
 @pytest.fixture(scope="module")
