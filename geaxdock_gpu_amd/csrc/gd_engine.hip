@@ -68,6 +68,7 @@ struct Scratch {
 };
 constexpr size_t SCRATCH_KEEP = (size_t)256 << 20;
 
+constexpr int GRID_ROWS = 32768;  // rows (grid.y, 16 bits) of a launch
 constexpr int SIDE_STREAMS = 3;  // streams beside the main one for launch classes
 
 }  // namespace
@@ -994,9 +995,9 @@ gd_status ensure_ref(gd_ctx *ctx) {
   std::vector<int2> out(n);
   hipError_t e = hipMemcpyAsync(d_todo, todo.data(), n * sizeof(int), hipMemcpyHostToDevice, ctx->stream);
   if (e == hipSuccess) e = hipMemsetAsync(d_out, 0, n * sizeof(int2), ctx->stream);
-  for (size_t b = 0; b < n && e == hipSuccess; b += 32768) {  // grid.y is 16 bits
+  for (size_t b = 0; b < n && e == hipSuccess; b += GRID_ROWS) {
     hipLaunchKernelGGL(gd_ref_kernel,
-                       dim3((unsigned)lna_max, (unsigned)std::min<size_t>(32768, n - b)), dim3(64),
+                       dim3((unsigned)lna_max, (unsigned)std::min<size_t>(GRID_ROWS, n - b)), dim3(64),
                        0, ctx->stream, ctx->d_cx, d_todo + b, d_out + b);
     e = hipGetLastError();
   }
@@ -2636,11 +2637,15 @@ gd_status gd_sur_build_grids(gd_ctx *ctx, float spacing, float half_width) {
     ctx->cx[c].dev.sh = G.h;
     ctx->cx[c].dev.sn = G.n;
     const int64_t nb = (n + 3) / 4, bricks = nb * nb * nb;
-    hipLaunchKernelGGL(gd_sur_grid_kernel,
-                       dim3((unsigned)((bricks + 3) / 4), (unsigned)h.d.n_prt), dim3(256), 0,
-                       ctx->stream, h.dev.prt_xyze, h.dev.prt_type, h.d.pnp, G.ox, G.oy, G.oz, G.h,
-                       n, S.grid[c]);
-    HIPCHK(hipGetLastError());
+    for (int p = 0; p < h.d.n_prt; p += GRID_ROWS) {
+      hipLaunchKernelGGL(gd_sur_grid_kernel,
+                         dim3((unsigned)((bricks + 3) / 4),
+                              (unsigned)std::min(GRID_ROWS, h.d.n_prt - p)),
+                         dim3(256), 0, ctx->stream, h.dev.prt_xyze + (size_t)p * h.d.pnp,
+                         h.dev.prt_type, h.d.pnp, G.ox, G.oy, G.oz, G.h, n,
+                         S.grid[c] + (size_t)p * nodes * 32);
+      HIPCHK(hipGetLastError());
+    }
   }
   HIPCHK(hipStreamSynchronize(ctx->stream));
   TRY(sync_complexes(ctx));

@@ -255,9 +255,20 @@ def pose_calls_without_allocations(hip):
                 assert (hip.count("made"), hip.count("allocs")) == (made, allocs), n
 
 
+def many_conformers(hip):
+    """Feature grids of more receptor conformers than a launch has rows for."""
+    import geaxdock_gpu_amd as gd
+    n_prt = 70000
+    with gd.Engine(seed=1) as eng:
+        eng.add_complex(complex_(pnp=2, n_lig=1, n_prt=n_prt, n_tmp=1))
+        first = hip.count("launches")
+        eng.sur_build_grids(1.0, 1.01)
+        assert sum(g[1] for _, g, _ in hip.launches("gd_sur_grid", first)) == n_prt
+
+
 CASES = [unit_lists, complex_table, feature_grids, refused_complex, training_buffers,
          parameter_buffers, record_rings, window_steps,
-         pose_calls_without_allocations]
+         pose_calls_without_allocations, many_conformers]
 
 
 @pytest.fixture(scope="module")
