@@ -197,14 +197,17 @@ typedef struct gd_opts {
 #define GD_LAUNCH_NO_SPREAD 8
 
 typedef struct gd_run_stats {
-  double t_compute; /* seconds in MC kernels (HIP events), the reference's McLog.t0 */
+  double t_compute; /* device seconds of the MC windows (HIP events around each: its MC
+                       launches and, under spread packing, the exchange kernels between
+                       them), the reference's McLog.t0 */
   double t_wall;    /* seconds including record transfer, McLog.t1 */
   int64_t steps;    /* MC steps this call */
   int64_t replica_steps;
   int64_t accepted;          /* accepted MC moves this call */
   int64_t exchanges_accepted;
-  int kernel_launches;
-  double kernel_ms_avg;      /* mean MC-kernel duration (HIP events) */
+  int kernel_launches;       /* MC launches: one a window; under spread packing one or
+                                more an exchange interval */
+  double kernel_ms_avg;      /* t_compute per launch, in ms */
 } gd_run_stats;
 
 /* Record sink: called once per dump window and complex with that window's
