@@ -189,17 +189,6 @@ gd_status fail(gd_ctx *c, gd_status s, const char *fmt, ...) {
       return fail(ctx, GD_ERR_HIP, "%s failed: %s", #expr, hipGetErrorString(e_));    \
   } while (0)
 
-template <class T>
-gd_status dev_upload(gd_ctx *ctx, HostComplex &h, T **dst, const T *src, size_t n) {
-  void *p = nullptr;
-  const size_t bytes = std::max<size_t>(n, 1) * sizeof(T);
-  HIPCHK(hipMalloc(&p, bytes));
-  h.bufs.push_back(p);
-  if (n) HIPCHK(hipMemcpyAsync(p, src, n * sizeof(T), hipMemcpyHostToDevice, ctx->stream));
-  *dst = static_cast<T *>(p);
-  return GD_OK;
-}
-
 #define TRY(expr)                      \
   do {                                 \
     gd_status s_ = (expr);             \
@@ -759,8 +748,8 @@ static gd_status add_complex(gd_ctx *ctx, const gd_complex_desc *d, int *complex
 
 namespace {
 
-// Side streams and their events for a launch of n classes (made on first use:
-// a stream costs about 50 us and as much again to destroy).
+// Side streams and their events for a launch of n classes (made when a context
+// first may need them: a stream costs about 50 us and as much again to destroy).
 hipError_t side_streams(gd_ctx *ctx, int n) {
   hipError_t e = hipSuccess;
   if (n > 1 && !ctx->ev_fork) e = hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming);
@@ -2169,7 +2158,8 @@ gd_status gd_sur_surrogate(gd_ctx *ctx, int cid, int n, const int *idx_lig, cons
 // Energies (or surrogate totals) of n poses of one complex. With no_alloc the
 // pose tables and outputs live in the device scratch array (the caller has
 // checked n and that the complex table and contact map are on the device);
-// otherwise they are allocated for the call.
+// otherwise in the context's staging: pinned memory that the kernel reads and
+// writes itself for small calls, else device memory with a copy each way.
 static gd_status eval_poses(gd_ctx *ctx, int cid, int n, const int *idx_lig, const int *idx_prt,
                             const float *movematrix, gd_energy *out, float *out_sur,
                             float sur_scale, bool no_alloc) {
