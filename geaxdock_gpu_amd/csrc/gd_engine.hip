@@ -112,11 +112,13 @@ struct gd_ctx {
   int ring = 0;
   int rec_cap = 0;
   hipStream_t drain_stream = nullptr;
+  hipEvent_t ev_compact = nullptr;  // the pending window is compacted
   // record drains: device offsets and compacted window, and the pinned host
   // staging buffer the sink reads, grown as needed and reused across windows
   int64_t *d_drain_off = nullptr;
   gd_record *d_drain = nullptr, *h_drain = nullptr;
-  int64_t drain_cap = 0;
+  int64_t d_drain_cap = 0, h_drain_cap = 0;
+  int64_t drain_total = 0;  // records of the compacted window (their offsets: drain_pin)
   // packs of the MC launch
   Pack *d_packs = nullptr;
   int *d_slots = nullptr;
@@ -408,6 +410,7 @@ void gd_destroy(gd_ctx *ctx) {
     if (ctx->ev_join[i]) (void)hipEventDestroy(ctx->ev_join[i]);
     if (ctx->aux[i]) (void)hipStreamDestroy(ctx->aux[i]);
   }
+  if (ctx->ev_compact) (void)hipEventDestroy(ctx->ev_compact);
   if (ctx->drain_stream) (void)hipStreamDestroy(ctx->drain_stream);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
   delete ctx;
@@ -1567,61 +1570,84 @@ hipError_t launch_classes(gd_ctx *ctx, const std::vector<LaunchClass> &classes, 
   return e;
 }
 
-// Drain record ring r: its accepted-state records, compacted on the device
-// into one window, copied to the pinned staging buffer and handed to the
-// sink per complex; then the ring's counts restart. All on `stream`, which
-// is synchronized before returning when there is a sink.
-gd_status drain_ring(gd_ctx *ctx, int r, gd_record_sink sink, void *user, hipStream_t stream) {
+// A drain of record ring r hands its accepted-state records to the sink in two
+// halves. compact_ring gathers them on the device into one window and restarts
+// the ring's counts, before the next window begins: MC workgroups may leave no
+// registers to its kernels, which then waited for that window's end (1,024
+// complexes with records 7.9M replica-steps/s, 9.7M now). deliver_records
+// copies the window to the pinned staging buffer and hands it out per complex:
+// copy engines work beside the next window.
+gd_status compact_ring(gd_ctx *ctx, int r, hipStream_t stream) {
+  ctx->drain_total = 0;
   if (!ctx->d_ring[r]) return GD_OK;
   const int n = ctx->n_rep;
   int *cnt_d = ctx->d_ring_cnt[r];
-  if (sink) {
-    Regions R;
-    const size_t o_off = R.add((n + 1) * sizeof(int64_t)), o_cnt = R.add(n * sizeof(int));
-    TRY(scratch_need(ctx, ctx->drain_pin, R.end, true));
-    int64_t *off = reinterpret_cast<int64_t *>(ctx->drain_pin.p + o_off);
-    int *cnt = reinterpret_cast<int *>(ctx->drain_pin.p + o_cnt);
-    HIPCHK(hipMemcpyAsync(cnt, cnt_d, n * sizeof(int), hipMemcpyDeviceToHost, stream));
-    HIPCHK(hipStreamSynchronize(stream));
-    off[0] = 0;
-    for (int i = 0; i < n; ++i) off[i + 1] = off[i] + cnt[i];
-    const int64_t tot = off[n];
-    if (tot > 0) {
-      if (tot > ctx->drain_cap) {
-        if (ctx->d_drain) (void)hipFree(ctx->d_drain);
-        if (ctx->h_drain) (void)hipHostFree(ctx->h_drain);
-        ctx->d_drain = nullptr;
-        ctx->h_drain = nullptr;
-        ctx->drain_cap = 0;
-        const int64_t cap = tot + tot / 8;
-        HIPCHK(hipMalloc(&ctx->d_drain, cap * sizeof(gd_record)));
-        HIPCHK(hipHostMalloc(&ctx->h_drain, cap * sizeof(gd_record), hipHostMallocDefault));
-        ctx->drain_cap = cap;
-      }
-      if (!ctx->d_drain_off) HIPCHK(hipMalloc(&ctx->d_drain_off, (n + 1) * sizeof(int64_t)));
-      HIPCHK(hipMemcpyAsync(ctx->d_drain_off, off, (n + 1) * sizeof(int64_t),
-                            hipMemcpyHostToDevice, stream));
-      hipLaunchKernelGGL(gd_compact_kernel, dim3(n), dim3(256), 0, stream, n, ctx->d_ring[r],
-                         cnt_d, ctx->d_drain_off, ctx->rec_cap, ctx->d_drain);
-      HIPCHK(hipGetLastError());
-      HIPCHK(hipMemcpyAsync(ctx->h_drain, ctx->d_drain, tot * sizeof(gd_record),
-                            hipMemcpyDeviceToHost, stream));
+  Regions R;
+  const size_t o_off = R.add((n + 1) * sizeof(int64_t)), o_cnt = R.add(n * sizeof(int));
+  TRY(scratch_need(ctx, ctx->drain_pin, R.end, true));
+  int64_t *off = reinterpret_cast<int64_t *>(ctx->drain_pin.p + o_off);
+  int *cnt = reinterpret_cast<int *>(ctx->drain_pin.p + o_cnt);
+  HIPCHK(hipMemcpyAsync(cnt, cnt_d, n * sizeof(int), hipMemcpyDeviceToHost, stream));
+  HIPCHK(hipStreamSynchronize(stream));
+  off[0] = 0;
+  for (int i = 0; i < n; ++i) off[i + 1] = off[i] + cnt[i];
+  const int64_t tot = off[n];
+  if (tot > 0) {
+    if (tot > ctx->d_drain_cap) {
+      if (ctx->d_drain) (void)hipFree(ctx->d_drain);
+      ctx->d_drain = nullptr;
+      ctx->d_drain_cap = 0;
+      const int64_t cap = tot + tot / 8;
+      HIPCHK(hipMalloc(&ctx->d_drain, cap * sizeof(gd_record)));
+      ctx->d_drain_cap = cap;
     }
-    HIPCHK(hipMemsetAsync(cnt_d, 0, n * sizeof(int), stream));
-    HIPCHK(hipStreamSynchronize(stream));
-    for (int c = 0; tot > 0 && c < (int)ctx->cx.size(); ++c) {
-      const HostComplex &h = ctx->cx[c];
-      const int64_t b = off[h.rep_base], e = off[h.rep_base + h.n_rep];
-      if (e > b) sink(user, c, ctx->h_drain + b, e - b);
-    }
-    return GD_OK;
+    if (!ctx->d_drain_off) HIPCHK(hipMalloc(&ctx->d_drain_off, (n + 1) * sizeof(int64_t)));
+    HIPCHK(hipMemcpyAsync(ctx->d_drain_off, off, (n + 1) * sizeof(int64_t),
+                          hipMemcpyHostToDevice, stream));
+    hipLaunchKernelGGL(gd_compact_kernel, dim3(n), dim3(256), 0, stream, n, ctx->d_ring[r],
+                       cnt_d, ctx->d_drain_off, ctx->rec_cap, ctx->d_drain);
+    HIPCHK(hipGetLastError());
   }
   HIPCHK(hipMemsetAsync(cnt_d, 0, n * sizeof(int), stream));
+  ctx->drain_total = tot;
   return GD_OK;
 }
 
+// The compacted window to the sink; `stream` (compact_ring's) is synchronized
+// before.
+gd_status deliver_records(gd_ctx *ctx, gd_record_sink sink, void *user, hipStream_t stream) {
+  const int64_t tot = ctx->drain_total;
+  ctx->drain_total = 0;
+  if (tot == 0) return GD_OK;
+  if (tot > ctx->h_drain_cap) {
+    if (ctx->h_drain) (void)hipHostFree(ctx->h_drain);
+    ctx->h_drain = nullptr;
+    ctx->h_drain_cap = 0;
+    HIPCHK(hipHostMalloc(&ctx->h_drain, ctx->d_drain_cap * sizeof(gd_record),
+                         hipHostMallocDefault));
+    ctx->h_drain_cap = ctx->d_drain_cap;
+  }
+  HIPCHK(hipMemcpyAsync(ctx->h_drain, ctx->d_drain, tot * sizeof(gd_record),
+                        hipMemcpyDeviceToHost, stream));
+  HIPCHK(hipStreamSynchronize(stream));
+  const int64_t *off = reinterpret_cast<const int64_t *>(ctx->drain_pin.p);
+  for (int c = 0; c < (int)ctx->cx.size(); ++c) {
+    const HostComplex &h = ctx->cx[c];
+    const int64_t b = off[h.rep_base], e = off[h.rep_base + h.n_rep];
+    if (e > b) sink(user, c, ctx->h_drain + b, e - b);
+  }
+  return GD_OK;
+}
+
+// Drains the current ring on the main stream; without a sink its records go.
 gd_status drain_records(gd_ctx *ctx, gd_record_sink sink, void *user) {
-  return drain_ring(ctx, ctx->ring, sink, user, ctx->stream);
+  if (!ctx->d_ring[ctx->ring]) return GD_OK;
+  if (!sink) {
+    HIPCHK(hipMemsetAsync(ctx->d_ring_cnt[ctx->ring], 0, ctx->n_rep * sizeof(int), ctx->stream));
+    return GD_OK;
+  }
+  TRY(compact_ring(ctx, ctx->ring, ctx->stream));
+  return deliver_records(ctx, sink, user, ctx->stream);
 }
 
 // Record rings for windows of up to `win` steps (and the start poses): ring 0,
@@ -1665,6 +1691,8 @@ gd_status ensure_rings(gd_ctx *ctx, int win, bool both) {
   }
   if (both && !ctx->drain_stream)
     HIPCHK(hipStreamCreateWithFlags(&ctx->drain_stream, hipStreamNonBlocking));
+  if (both && !ctx->ev_compact)
+    HIPCHK(hipEventCreateWithFlags(&ctx->ev_compact, hipEventDisableTiming));
   HIPCHK(hipStreamSynchronize(ctx->stream));
   return GD_OK;
 }
@@ -1922,9 +1950,9 @@ static gd_status run_impl(gd_ctx *ctx, int64_t n_steps, int steps_per_exchange,
   int64_t left = n_steps;
   double t_ms = 0.0;
   // with records and a sink, windows alternate between the two rings: the
-  // previous window's records are drained (on the drain stream, sinks called
-  // here) while the next window runs
-  int pending = -1;
+  // previous window's records, compacted between the windows, are delivered (on
+  // the drain stream, sinks called here) while the next window runs
+  bool pending = false;
   while (left > 0) {
     int win = (int)std::min<int64_t>(left, ctx->opts.steps_per_dump);
     if (da_k > 0) win = std::max(da_k, win / da_k * da_k);
@@ -1938,7 +1966,7 @@ static gd_status run_impl(gd_ctx *ctx, int64_t n_steps, int steps_per_exchange,
     TRY(launch_mc_enqueue(ctx, MODE_MC, (int)ctx->step, win, steps_per_exchange, da_k, sur_scale));
     // a failed drain is reported after the window in flight has finished
     const gd_status ds =
-        pending >= 0 ? drain_ring(ctx, pending, sink, user, ctx->drain_stream) : GD_OK;
+        pending ? deliver_records(ctx, sink, user, ctx->drain_stream) : GD_OK;
     TRY(launch_mc_wait(ctx, &ms));
     t_ms += ms;
     st.kernel_launches += 1;
@@ -1946,13 +1974,18 @@ static gd_status run_impl(gd_ctx *ctx, int64_t n_steps, int steps_per_exchange,
     left -= win;
     if (ds != GD_OK) return ds;
     if (overlap) {
-      pending = ctx->ring;
+      TRY(compact_ring(ctx, ctx->ring, left > 0 ? ctx->drain_stream : ctx->stream));
+      if (left > 0) {
+        HIPCHK(hipEventRecord(ctx->ev_compact, ctx->drain_stream));
+        HIPCHK(hipStreamWaitEvent(ctx->stream, ctx->ev_compact, 0));
+      }
+      pending = true;
       ctx->ring ^= 1;
     } else {
       TRY(drain_records(ctx, sink, user));
     }
   }
-  if (pending >= 0) TRY(drain_ring(ctx, pending, sink, user, ctx->stream));
+  if (pending) TRY(deliver_records(ctx, sink, user, ctx->stream));
   if (n_steps == 0) TRY(drain_records(ctx, sink, user));
   hipLaunchKernelGGL(gd_counts_kernel, dim3(1), dim3(1024), 0, ctx->stream, ctx->n_rep,
                      ctx->d_acs_mc, ctx->d_acs_x, counts + 2);

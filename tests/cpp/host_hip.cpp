@@ -25,6 +25,7 @@ std::map<const void *, std::string> kernels;
 std::vector<Launch> launches;
 long made = 0;                           // streams and events created
 long fail_alloc = -1, fail_launch = -1;  // calls until the failing one
+int fill = 0;                            // what a word cleared to 0 becomes
 size_t fail_above = 0;                   // every allocation above this fails (0: none)
 unsigned char symbol[4 << 20];
 struct {
@@ -73,6 +74,7 @@ extern "C" {
 void host_hip_fail_alloc(long n) { fail_alloc = n; }    // the n-th from now, once
 void host_hip_fail_launch(long n) { fail_launch = n; }
 void host_hip_fail_above(size_t bytes) { fail_above = bytes; }
+void host_hip_fill(int value) { fill = value; }
 long host_hip_num_allocs() { return (long)allocs.size(); }
 size_t host_hip_alloc_size(long i) { return allocs[i]; }
 long host_hip_num_live() { return (long)live.size(); }
@@ -159,6 +161,8 @@ hipError_t hipMemcpyAsync(void *dst, const void *src, size_t bytes, hipMemcpyKin
 }
 hipError_t hipMemsetAsync(void *dst, int value, size_t bytes, hipStream_t) {
   std::memset(dst, value, bytes);
+  if (value == 0 && fill != 0)
+    for (size_t i = 0; i < bytes / sizeof(int); ++i) static_cast<int *>(dst)[i] = fill;
   return hipSuccess;
 }
 

@@ -266,9 +266,32 @@ def many_conformers(hip):
         assert sum(g[1] for _, g, _ in hip.launches("gd_sur_grid", first)) == n_prt
 
 
+def window_drains(hip):
+    """Records of a window go to the sink beside the next window by copy engines
+    alone: they are compacted before it starts, since a kernel beside it would
+    wait for registers until its end."""
+    import geaxdock_gpu_amd as gd
+    launch = gd.abi.LAUNCH_NO_GRAPH | gd.abi.LAUNCH_NO_SPREAD
+    with gd.Engine(seed=1, launch=launch, steps_per_dump=10) as eng:
+        eng.add_complex(complex_())
+        eng.run(0)
+        hip.lib.host_hip_fill(C.c_int(1))  # a cleared count is 1: a record for each replica
+        first, got = hip.count("launches"), []
+        eng.run(30, 0, sink=lambda c, r: got.append((hip.count("launches"), len(r))))
+        hip.lib.host_hip_fill(C.c_int(0))
+        kernels = [("C" if "compact" in k else "M") for k, _, _ in hip.launches("", first)
+                   if "compact" in k or "gd_mc_kernel" in k]
+        assert kernels == list("MCMCMC")
+        # the first two windows' records arrive with the next window's launch made
+        assert [n for _, n in got] == [eng.num_replicas(0)] * 3
+        made = [i for i in range(first, hip.count("launches"))
+                if "gd_mc_kernel" in hip.lib.host_hip_kernel(C.c_long(i)).decode()]
+        assert got[0][0] > made[1] and got[1][0] > made[2]
+
+
 CASES = [unit_lists, complex_table, feature_grids, refused_complex, training_buffers,
          parameter_buffers, record_rings, window_steps,
-         pose_calls_without_allocations, many_conformers]
+         pose_calls_without_allocations, many_conformers, window_drains]
 
 
 @pytest.fixture(scope="module")
