@@ -41,6 +41,7 @@ struct LaunchClass {
   KParams lay{};     // LDS offsets and exchange-buffer fields
   size_t lds_flat = 0;  // the same with the receptor as units of the flat
   KParams lay_flat{};   // pair loop (0: none)
+  bool near = false;  // plain chunk loop without distance tests (DA_NEAR)
 };
 
 struct HostComplex {
@@ -50,6 +51,7 @@ struct HostComplex {
   int lpr0 = 0, apl0 = 0;  // the shape of fewest lane slots (lpr and apl may be widened)
   bool tiled = false;  // receptor streamed through LDS tiles
   bool ref_built = false;
+  float far_share = 0.0f;  // share of receptor points far from the start pose
   int flat_n[4] = {0, 0, 0, 0};  // units of the flat pair loop by split (0: no list)
   bool shape_final = false;  // lane shape fixed (the complex's energies have bits)
   std::vector<int4> chunks;  // receptor chunks (host copy)
@@ -272,6 +274,38 @@ float skip_range2(const gd_complex_desc &d, const std::vector<float> &par) {
     }
   return (float)(r2 * 1.002);
 }
+
+// Share of the receptor's points (first conformer) whose pairs the distance
+// tests can skip around the start pose: points beyond far2 of a sphere of half
+// the ligand's radius (which counts within 0.08 of the points that are that
+// far from every atom).
+float far_share(const gd_complex_desc &d, float far2) {
+  if (!std::isfinite(far2)) return 0.0f;
+  float r2 = 0.0f;
+  for (int l = 0; l < d.lna; ++l)
+    r2 = std::max(r2, d.lig_x[l] * d.lig_x[l] + d.lig_y[l] * d.lig_y[l] + d.lig_z[l] * d.lig_z[l]);
+  const float reach = std::sqrt(far2) + 0.5f * std::sqrt(r2);
+  int n = 0;
+  for (int p = 0; p < d.pnp; ++p) {
+    const float x = d.prt_x[p] - d.pocket_center[0], y = d.prt_y[p] - d.pocket_center[1],
+                z = d.prt_z[p] - d.pocket_center[2];
+    n += x * x + y * y + z * z > reach * reach ? 1 : 0;
+  }
+  return (float)n / (float)d.pnp;
+}
+
+// Launches of the chunk loop go without its distance tests (DA_NEAR, same bits)
+// where these cost more than they skip. At a wave per SIMD (blocks of at most
+// 256 lanes) nothing hides the tests' branches: 64 ladders of 4 replicas of 30
+// atoms, split 1, 2,000 points, 14.2 ms with tests and 12.1 without, 3,500 points
+// 22.8 and 20.4; one pose on 1,200 points 116 us and 106. At two waves per SIMD
+// the tests pay from a share of far points on that falls with the atoms per
+// lane (batches and ladders, tests first): 1 atom, 2,000 points (share 0.6) 5.8 ms
+// and 5.5, 3,500 (0.77) 8.4 and 8.7; 2 atoms, 1,000 points (0.13) 65.8 and 63.1,
+// 2,000 (0.44) 10.6 and 10.4, 2,500 (0.52) 139.9 and 142.9; 3 atoms, 1,000 (0.14)
+// 43.2 and 43.1, 2,000 (0.46) 78.0 and 81.4.
+constexpr int NEAR_BLOCK = 256;
+constexpr float NEAR_SHARE[4] = {0.65f, 0.45f, 0.3f, 0.3f};
 
 // Lanes per replica and atoms per lane: the fewest lane slots lpr*apl that
 // hold lna atoms with apl <= 4, preferring 2..3 atoms per lane on ties (more
@@ -669,6 +703,7 @@ static gd_status add_complex(gd_ctx *ctx, const gd_complex_desc *d, int *complex
   D.kde2l = ep.kde2 * 1.44269504088896340736f;
   D.kde3 = ep.kde3;
   D.far2 = skip_range2(*d, par);
+  h.far_share = far_share(*d, D.far2);
   for (int i = 0; i < GD_MAXWEI; ++i) {
     D.w[i] = ep.w[i];
     D.a_para[i] = ep.a_para[i];
@@ -1145,6 +1180,7 @@ void pack_finish(const gd_ctx *ctx, PackSet &ps, int lpr = 0, int apl_of_lpr = 0
     lc.tile = tile[o0];
     int pnp_max = 0, pnk_max = 0, nch_max = 0, slots_max = 1, half_max = 64, flat_max = 0;
     bool split = false;
+    double far = 0.0, all = 0.0;
     const bool flat = units[o0] > 0;
     size_t e = b;
     for (; e < n_pk; ++e) {
@@ -1174,8 +1210,11 @@ void pack_finish(const gd_ctx *ctx, PackSet &ps, int lpr = 0, int apl_of_lpr = 0
       slots_max = ns;
       split = sp;
       half_max = std::max(half_max, p.half);
+      far += cost[oe] * h.far_share;
+      all += cost[oe];
     }
     lc.end = (int)e;
+    lc.near = lc.block <= NEAR_BLOCK || far < NEAR_SHARE[lc.apl - 1] * all;
     lc.half_max = half_max;
     layout(lc.lay, &lc.lds, (pnp_max + 3) & ~3, pnk_max, nch_max, slots_max, lc.block, split,
            lc.tile);
@@ -1450,7 +1489,8 @@ KParams base_params(gd_ctx *ctx) {
 
 // Kernel instance for atoms per lane `apl` and mode `da`: 0 plain,
 // 1 delayed acceptance with the network per atom, 2 with its tables, 3 and 4
-// the same with the split groups' shared surrogate sums compiled in.
+// the same with the split groups' shared surrogate sums compiled in; and the
+// other modes of gd_kernels.h.
 const void *mc_kernel_fn(int apl, int da, int rec) {
   switch (apl) {
     case 1: return mc_kernel_handle<1>(da, rec);
@@ -1521,7 +1561,8 @@ hipError_t plan_classes(gd_ctx *ctx, const std::vector<LaunchClass> &classes, co
       P.queue = queue + i;
       P.n_queue = n_pk;
     }
-    cl.f = mc_kernel_fn(lc.apl, da, lc.tile > 0 ? REC_TILED : flat ? REC_FLAT : REC_CHUNKS);
+    const int rec = lc.tile > 0 ? REC_TILED : flat ? REC_FLAT : REC_CHUNKS;
+    cl.f = mc_kernel_fn(lc.apl, da == 0 && rec == REC_CHUNKS && lc.near ? DA_NEAR : da, rec);
     out.push_back(cl);
   }
   // the dynamic LDS limit of every instance used is the device's: classes

@@ -110,7 +110,7 @@ struct Pack {
 // MODE_TREE: the next n_steps MC steps by a tree of energies (gd_mc.h)
 enum { MODE_MC = 0, MODE_INIT = 1, MODE_EVAL = 2, MODE_SUREVAL = 3, MODE_TREE = 4 };
 // kernel instances besides the modes of delayed acceptance (see mc_kernel_handle)
-constexpr int DA_TREE = 5, DA_POSES = 6, DA_POSES2 = 7;
+constexpr int DA_TREE = 5, DA_POSES = 6, DA_POSES2 = 7, DA_NEAR = 8;
 constexpr int TREE_DEPTH = 6;  // a wave's lanes hold the 2^depth - 1 energies
 
 struct KParams {
@@ -167,7 +167,8 @@ struct KParams {
 // mode `da` (0 plain, 1 delayed acceptance with the network per atom, 2 with
 // its tabulated outputs) and receptor layout; defined in gd_mc_inst.hip, one
 // object per APL. DA_POSES (2 or 3 atoms per lane) and DA_POSES2 (3) have
-// instances for REC_TILED and REC_FLAT, REC_FLAT none for modes 1 and 3.
+// instances for REC_TILED and REC_FLAT, DA_NEAR for REC_CHUNKS, REC_FLAT none for
+// modes 1 and 3.
 enum { REC_CHUNKS = 0, REC_TILED = 1, REC_FLAT = 2 };
 template <int APL>
 const void *mc_kernel_handle(int da, int rec);

@@ -221,10 +221,12 @@ __device__ __forceinline__ float hb_range2(const ChunkPar (&cp)[APL], bool all) 
 // (3,000 points) they take 12 % of the transcendentals and 6 % of the VALU
 // instructions away, 21.6 -> 20.5 ms a kernel of 40 steps; 2,000 poses on 8,000
 // points 1,624 -> 1,535 us a call. With kind, clamp and H-bond as run-time
-// branches instead (one variant of the loop) the ensemble took 5 % longer. The flat
-// loop below goes without the tests: its units hold points of smaller receptors,
-// few of them far, and they cost 3 % there.
-template <int APL, int KIND, int NP, bool CLAMP, bool HB>
+// branches instead (one variant of the loop) the ensemble took 5 % longer. Without
+// SKIP every pair takes all terms: where few points are far, or a SIMD holds one
+// wave, the tests cost more than they save (rule and figures: NEAR_SHARE in
+// gd_engine.hip). The flat loop below goes without them too: its units hold
+// points of smaller receptors, and they cost 3 % there.
+template <int APL, int KIND, int NP, bool CLAMP, bool HB, bool SKIP>
 __device__ __forceinline__ void pair_group(const Lds &S, int p, const float4 (&P)[NP],
                                            const PairConst &K, const Range &G,
                                            const float (&x)[APL], const float (&y)[APL],
@@ -248,7 +250,7 @@ __device__ __forceinline__ void pair_group(const Lds &S, int p, const float4 (&P
   // from every atom of a wave (four -> two -> this, in tiles: 2,000 poses of 61
   // atoms on 8,000 points 1.30 -> 1.22 -> 1.21 ms, of 45 atoms on 6,000 points 0.76
   // -> 0.70 -> 0.66)
-  constexpr int NB = NP < 2 || APL >= 2 ? 1 : 2;
+  constexpr int NB = !SKIP ? NP : NP < 2 || APL >= 2 ? 1 : 2;
   float qm[NP];  // the lane's nearest atom to each point
 #pragma unroll
   for (int j = 0; j < NP; ++j) {
@@ -273,7 +275,7 @@ __device__ __forceinline__ void pair_group(const Lds &S, int p, const float4 (&P
     float qmin = qm[j0];
 #pragma unroll
     for (int j = j0 + 1; j < j0 + NB; ++j) qmin = fminf(qmin, qm[j]);
-    if (__ballot(!(qmin > G.far2)) != 0) {
+    if (!SKIP || __ballot(!(qmin > G.far2)) != 0) {
 #pragma unroll
       for (int j = j0; j < j0 + NB; ++j)
 #pragma unroll
@@ -320,7 +322,7 @@ __device__ __forceinline__ void pair_group(const Lds &S, int p, const float4 (&P
     // H-bond: only in chunks where some lane's atom has an H-bond record with
     // this receptor type (elsewhere every term would be 0 * exp2), and there
     // only where such a lane is within its records' range
-    if (HB && __ballot(!(qmin > G.hb2)) != 0) {
+    if (HB && (!SKIP || __ballot(!(qmin > G.hb2)) != 0)) {
 #pragma unroll
       for (int j = j0; j < j0 + NB; ++j)
 #pragma unroll
@@ -344,7 +346,7 @@ __device__ __forceinline__ void pair_group(const Lds &S, int p, const float4 (&P
 // latency.
 __host__ __device__ constexpr int group_points(int apl) { return apl >= 3 ? 1 : (apl == 2 ? 2 : 4); }
 
-template <int APL, int NP, int KIND, bool CLAMP, bool HB>
+template <int APL, int NP, int KIND, bool CLAMP, bool HB, bool SKIP>
 __device__ __forceinline__ void chunk_pairs(const Lds &S, int beg, int end, const PairConst &K,
                                             const Range &G,
                                             const float (&x)[APL], const float (&y)[APL],
@@ -372,22 +374,22 @@ __device__ __forceinline__ void chunk_pairs(const Lds &S, int beg, int end, cons
     for (; p + 2 * NP <= end; p += 2 * NP) {
 #pragma unroll
       for (int j = 0; j < NP; ++j) Pb[j] = S.xyze[p + NP + j];
-      pair_group<APL, KIND, NP, CLAMP, HB>(S, p, Pa, K, G, x, y, z, cp, psprow, vdw, ele,
+      pair_group<APL, KIND, NP, CLAMP, HB, SKIP>(S, p, Pa, K, G, x, y, z, cp, psprow, vdw, ele,
                                            pmfc, psp, hdb, hpc, cnt);
 #pragma unroll
       for (int j = 0; j < NP; ++j) Pa[j] = S.xyze[min(p + 2 * NP + j, end - 1)];
-      pair_group<APL, KIND, NP, CLAMP, HB>(S, p + NP, Pb, K, G, x, y, z, cp, psprow, vdw,
+      pair_group<APL, KIND, NP, CLAMP, HB, SKIP>(S, p + NP, Pb, K, G, x, y, z, cp, psprow, vdw,
                                            ele, pmfc, psp, hdb, hpc, cnt);
     }
     if (p + NP <= end) {
-      pair_group<APL, KIND, NP, CLAMP, HB>(S, p, Pa, K, G, x, y, z, cp, psprow, vdw, ele,
+      pair_group<APL, KIND, NP, CLAMP, HB, SKIP>(S, p, Pa, K, G, x, y, z, cp, psprow, vdw, ele,
                                            pmfc, psp, hdb, hpc, cnt);
       p += NP;
     }
   }
   for (; p < end; ++p) {
     const float4 P1[1] = {S.xyze[p]};
-    pair_group<APL, KIND, 1, CLAMP, HB>(S, p, P1, K, G, x, y, z, cp, psprow, vdw, ele, pmfc,
+    pair_group<APL, KIND, 1, CLAMP, HB, SKIP>(S, p, P1, K, G, x, y, z, cp, psprow, vdw, ele, pmfc,
                                         psp, hdb, hpc, cnt);
   }
 #pragma unroll
@@ -769,7 +771,7 @@ __device__ __forceinline__ float mcs_sum(const DevComplex &C, int lpr, const flo
 //
 // FLAT: every pack of the launch has the unit list of its split in LDS; the
 // pair loop is flat_pairs.
-template <int APL, bool TILE, bool FLAT, int J = 1, int NP = group_points(APL)>
+template <int APL, bool TILE, bool FLAT, int J = 1, int NP = group_points(APL), bool SKIP = true>
 __device__ __forceinline__ void pose_energy(const DevComplex &C, const Lds &S, int lpr, Split &sp,
                             bool live, const float (&x)[APL],
                             const float (&y)[APL], const float (&z)[APL],
@@ -861,7 +863,7 @@ __device__ __forceinline__ void pose_energy(const DevComplex &C, const Lds &S, i
     const bool hb = __ballot(hbond) != 0;
     auto pairs = [&](auto kind_c, auto clamp_c, auto hb_c) {
       chunk_pairs<APL, NP, decltype(kind_c)::value, decltype(clamp_c)::value,
-                  decltype(hb_c)::value>(T, beg, end, K, G, x, y, z, cp, psprow, vdw, ele,
+                  decltype(hb_c)::value, SKIP>(T, beg, end, K, G, x, y, z, cp, psprow, vdw, ele,
                                          pmf, psp, hdb, hpc, cnt);
     };
     auto by_hb = [&](auto kind_c, auto clamp_c) {
@@ -1472,7 +1474,8 @@ __device__ __forceinline__ void tree_decide(const KParams &P, const DevComplex &
 }
 
 // DA: 0 plain Metropolis (DA_TREE: by a tree of energies, in instances of its
-// own, so that the step loop's registers stay as they are; DA_POSES and
+// own, so that the step loop's registers stay as they are; DA_NEAR: without
+// distance tests; DA_POSES and
 // DA_POSES2: poses with fewer lanes than the complex's shape has, slot k in
 // block k or k % 2 of block_total); delayed acceptance with the surrogate from
 // the network evaluated per atom (1) or from its tabulated outputs (2); 3 and 4
@@ -1481,7 +1484,8 @@ template <int APL, int DA, bool TILE, bool FLAT>
 __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const DevComplex &C, const Lds &S,
                          int lpr, int step0, int idx, int node, int &par) {
   constexpr bool TREE = DA == DA_TREE, POSES = DA == DA_POSES || DA == DA_POSES2;
-  constexpr int DAM = TREE || POSES ? 0 : DA > 2 ? DA - 2 : DA;
+  constexpr bool SKIP = DA != DA_NEAR;
+  constexpr int DAM = TREE || POSES || !SKIP ? 0 : DA > 2 ? DA - 2 : DA;
   constexpr int J = !POSES ? 1 : DA == DA_POSES2 ? 2 : APL;
   // the wide shape has one atom per lane (DA_POSES) or two
   constexpr int NP = group_points(DA == DA_POSES ? 1 : DA == DA_POSES2 ? 2 : APL);
@@ -1583,7 +1587,7 @@ __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const
     if constexpr (TREE) tree_pose(P, C, flat, a, (threadIdx.x & 63) - a, step0, node + 1, mo);
     place(mo);
     gd_energy E;
-    pose_energy<APL, TILE, FLAT, J, NP>(C, S, lpr, sp, true, x, y, z, ox, oy, oz, lt, q, li, val, mo, E);
+    pose_energy<APL, TILE, FLAT, J, NP, SKIP>(C, S, lpr, sp, true, x, y, z, ox, oy, oz, lt, q, li, val, mo, E);
     par = sp.par;
     if constexpr (TREE) {
       // the wave of group 0 writes: its energies are visible on the device
@@ -1698,7 +1702,7 @@ __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const
         place(mn);
       }
       gd_energy E;
-      pose_energy<APL, TILE, FLAT>(C, S, lpr, sp, wave_active, x, y, z, ox, oy, oz, lt, q, li, val, mn, E);
+      pose_energy<APL, TILE, FLAT, J, NP, SKIP>(C, S, lpr, sp, wave_active, x, y, z, ox, oy, oz, lt, q, li, val, mn, E);
       if (wave_active && metropolis(E.e[GD_MAXWEI - 1], eo.e[GD_MAXWEI - 1], mb, u[6])) {
 #pragma unroll
         for (int i = 0; i < 6; ++i) mo[i] = mn[i];

@@ -10,8 +10,9 @@ namespace gd {
 // evaluation, 1 delayed acceptance with the network per atom, 2 with its
 // tabulated outputs, 3 and 4 the same with the receptor split's groups
 // sharing the surrogate's KDE and MCS sums, DA_TREE plain MC by a tree of
-// energies, DA_POSES poses with fewer lanes than the complex's shape; rec: the receptor resident in LDS
-// by chunks, streamed through LDS tiles, or resident with unit lists.
+// energies, DA_POSES poses with fewer lanes than the complex's shape, DA_NEAR 0
+// without the distance tests; rec: the receptor resident in LDS by chunks,
+// streamed through LDS tiles, or resident with unit lists.
 template <>
 const void *mc_kernel_handle<GD_MC_APL>(int da, int rec) {
   if (rec == REC_TILED) {
@@ -51,6 +52,7 @@ const void *mc_kernel_handle<GD_MC_APL>(int da, int rec) {
     case 3: return (const void *)gd_mc_kernel<GD_MC_APL, 3, false, false>;
     case 4: return (const void *)gd_mc_kernel<GD_MC_APL, 4, false, false>;
     case DA_TREE: return (const void *)gd_mc_kernel<GD_MC_APL, DA_TREE, false, false>;
+    case DA_NEAR: return (const void *)gd_mc_kernel<GD_MC_APL, DA_NEAR, false, false>;
     default: return (const void *)gd_mc_kernel<GD_MC_APL, 0, false, false>;
   }
 }
