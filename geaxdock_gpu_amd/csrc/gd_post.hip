@@ -42,6 +42,8 @@ namespace gd {
 
 constexpr int KM_DIM = GD_MAXWEI - 1;  // vdw .. dst
 constexpr int KM_MAX_K = 512;
+constexpr int KM_GATHER_K = 128;  // all passes gather in LDS up to this many centers
+constexpr int KM_ROUNDS_K = 15;   // fewer than are ever split over waves
 constexpr int KM_MAX_GROUP = 1 << 19;  // objects per group (fixed-point sum range)
 constexpr float KM_CLAMP = 134217728.0f;  // 2^27
 
@@ -58,6 +60,7 @@ struct KmArgs {
   int *delta, *pass;         // [n_groups]
   int *done;                 // [n_groups]: the pass that ended the group (-1: never run)
   int *active;
+  int rounds;  // tiles of a gathering workgroup
   unsigned long long *best;  // [n_groups][k]: (distance bits << 32) | member
   int *size;                 // [n_groups][k]
   int k;
@@ -98,22 +101,25 @@ __host__ __device__ inline float km_dist2(const float *a, const float *b) {
 // arithmetic as scalar operands. Bound: VALU, 22 instructions per object and
 // center.
 //
-// FIRST (the first pass with S = 1): every object is new, so the sums are
-// gathered in LDS and flushed once per workgroup. Later passes move the
-// objects that changed with global atomics (a few percent of them; adding all
-// objects anew took 10 LDS atomics per object and pass).
-template <int O, int S, bool FIRST>
+// GATHER (S = 1): a workgroup's changes to the sums are gathered in LDS and
+// flushed once. It serves the first pass, where every object is new, and all
+// passes of up to KM_GATHER_K centers, whose few sums the objects' atomics
+// would all meet on: 400,000 objects, 3 centers, 159 us a pass with global
+// atomics, 35 so; 24 centers 51 and 32 us, 100 centers 42 and 41. With more
+// centers later passes move the objects that changed with global atomics (500
+// centers 110 us, 126 by LDS: few objects of a workgroup share a center).
+template <int O, int S, bool GATHER>
 __global__ void __launch_bounds__(256) gd_km_assign_kernel(KmArgs A, const float *__restrict__ cent,
                                                            int pass) {
   const int g = A.tile_g[blockIdx.x];
   if (A.done[g] < pass) return;
   const int k = A.k;
   extern __shared__ __align__(16) unsigned char km_lds[];
-  long long *lsum = (long long *)km_lds;              // FIRST: [k][KM_DIM]
-  int *lcnt = (int *)(lsum + (size_t)k * KM_DIM);     // FIRST: [k]
+  long long *lsum = (long long *)km_lds;              // GATHER: [k][KM_DIM]
+  int *lcnt = (int *)(lsum + (size_t)k * KM_DIM);     // GATHER: [k]
   __shared__ float pd[S > 1 ? 4 : 1][O][64];
   __shared__ int pb[S > 1 ? 4 : 1][O][64];
-  if constexpr (FIRST) {
+  if constexpr (GATHER) {
     for (int j = threadIdx.x; j < k * KM_DIM; j += 256) lsum[j] = 0;
     for (int c = threadIdx.x; c < k; c += 256) lcnt[c] = 0;
     __syncthreads();
@@ -124,88 +130,94 @@ __global__ void __launch_bounds__(256) gd_km_assign_kernel(KmArgs A, const float
   const int l = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int part = wv % S, og = wv / S;
-  const int i0 = A.tile_s[blockIdx.x] + og * 64 * O + l;
-  float f[O][KM_DIM], dist[O];
-  int best[O];
-  bool has[O];
-#pragma unroll
-  for (int o = 0; o < O; ++o) {
-    has[o] = i0 + 64 * o < n;
-    const int64_t i = base + (has[o] ? i0 + 64 * o : 0);
-#pragma unroll
-    for (int d = 0; d < KM_DIM; ++d) f[o][d] = A.feat[(size_t)d * A.n_total + i];
-    // the first center is taken whatever its distance; later parts start from
-    // nothing
-    best[o] = part == 0 ? 0 : -1;
-    dist[o] = part == 0 ? km_dist2(f[o], cen) : __builtin_inff();
-  }
-  const int c1 = (k * (part + 1)) / S;
-#pragma unroll 4
-  for (int c = part == 0 ? 1 : (k * part) / S; c < c1; ++c) {
-    const float *cc = cen + (size_t)c * KM_DIM;
-#pragma unroll
-    for (int o = 0; o < O; ++o) {
-      const float e = km_dist2(f[o], cc);
-      if (e < dist[o]) {
-        dist[o] = e;
-        best[o] = c;
-      }
-    }
-  }
-  if constexpr (S > 1) {
-#pragma unroll
-    for (int o = 0; o < O; ++o) {
-      pd[wv][o][l] = dist[o];
-      pb[wv][o][l] = best[o];
-    }
-    __syncthreads();
-    if (part != 0) return;
-#pragma unroll
-    for (int o = 0; o < O; ++o)
-      for (int q = 1; q < S; ++q)
-        if (pd[wv + q][o][l] < dist[o]) {
-          dist[o] = pd[wv + q][o][l];
-          best[o] = pb[wv + q][o][l];
-        }
-  }
   long long *gs = A.sum + (size_t)g * k * KM_DIM;
   int *gn = A.cnt + (size_t)g * k;
   int changed = 0;
+  // a gathering workgroup takes `rounds` tiles
+  const int t1 = GATHER ? min(n, A.tile_s[blockIdx.x] + A.rounds * 256 * O) : n;
+  for (int t0 = A.tile_s[blockIdx.x];;) {
+    const int i0 = t0 + og * 64 * O + l;
+    float f[O][KM_DIM], dist[O];
+    int best[O];
+    bool has[O];
 #pragma unroll
-  for (int o = 0; o < O; ++o) {
-    int *m = A.memb + base + i0 + 64 * o;
-    const int old = has[o] ? *m : 0, now = best[o];
-    const bool move = has[o] && old != now;
-    changed += __popcll(__ballot(move));
-    if (!move) continue;
-    *m = now;
-    if constexpr (FIRST) {
+    for (int o = 0; o < O; ++o) {
+      has[o] = i0 + 64 * o < n;
+      const int64_t i = base + (has[o] ? i0 + 64 * o : 0);
 #pragma unroll
-      for (int d = 0; d < KM_DIM; ++d)
-        atomicAdd((unsigned long long *)&lsum[now * KM_DIM + d], (unsigned long long)km_fixed(f[o][d]));
-      atomicAdd(&lcnt[now], 1);
-    } else {
-#pragma unroll
-      for (int d = 0; d < KM_DIM; ++d) {
-        const unsigned long long v = (unsigned long long)km_fixed(f[o][d]);
-        atomicAdd((unsigned long long *)&gs[now * KM_DIM + d], v);
-        if (old >= 0) atomicAdd((unsigned long long *)&gs[old * KM_DIM + d], 0ull - v);
-      }
-      atomicAdd(&gn[now], 1);
-      if (old >= 0) atomicAdd(&gn[old], -1);
+      for (int d = 0; d < KM_DIM; ++d) f[o][d] = A.feat[(size_t)d * A.n_total + i];
+      // the first center is taken whatever its distance; later parts start from
+      // nothing
+      best[o] = part == 0 ? 0 : -1;
+      dist[o] = part == 0 ? km_dist2(f[o], cen) : __builtin_inff();
     }
+    const int c1 = (k * (part + 1)) / S;
+#pragma unroll 4
+    for (int c = part == 0 ? 1 : (k * part) / S; c < c1; ++c) {
+      const float *cc = cen + (size_t)c * KM_DIM;
+#pragma unroll
+      for (int o = 0; o < O; ++o) {
+        const float e = km_dist2(f[o], cc);
+        if (e < dist[o]) {
+          dist[o] = e;
+          best[o] = c;
+        }
+      }
+    }
+    if constexpr (S > 1) {
+#pragma unroll
+      for (int o = 0; o < O; ++o) {
+        pd[wv][o][l] = dist[o];
+        pb[wv][o][l] = best[o];
+      }
+      __syncthreads();
+      if (part != 0) return;
+#pragma unroll
+      for (int o = 0; o < O; ++o)
+        for (int q = 1; q < S; ++q)
+          if (pd[wv + q][o][l] < dist[o]) {
+            dist[o] = pd[wv + q][o][l];
+            best[o] = pb[wv + q][o][l];
+          }
+    }
+#pragma unroll
+    for (int o = 0; o < O; ++o) {
+      int *m = A.memb + base + i0 + 64 * o;
+      const int old = has[o] ? *m : 0, now = best[o];
+      const bool move = has[o] && old != now;
+      changed += __popcll(__ballot(move));
+      if (!move) continue;
+      *m = now;
+      if constexpr (GATHER) {
+#pragma unroll
+        for (int d = 0; d < KM_DIM; ++d) {
+          const unsigned long long v = (unsigned long long)km_fixed(f[o][d]);
+          atomicAdd((unsigned long long *)&lsum[now * KM_DIM + d], v);
+          if (old >= 0) atomicAdd((unsigned long long *)&lsum[old * KM_DIM + d], 0ull - v);
+        }
+        atomicAdd(&lcnt[now], 1);
+        if (old >= 0) atomicAdd(&lcnt[old], -1);
+      } else {
+#pragma unroll
+        for (int d = 0; d < KM_DIM; ++d) {
+          const unsigned long long v = (unsigned long long)km_fixed(f[o][d]);
+          atomicAdd((unsigned long long *)&gs[now * KM_DIM + d], v);
+          if (old >= 0) atomicAdd((unsigned long long *)&gs[old * KM_DIM + d], 0ull - v);
+        }
+        atomicAdd(&gn[now], 1);
+        if (old >= 0) atomicAdd(&gn[old], -1);
+      }
+    }
+    t0 += 256 * O;
+    if (!GATHER || t0 >= t1) break;
   }
   if (l == 0 && changed) atomicAdd(A.delta + g, changed);
-  if constexpr (FIRST) {
+  if constexpr (GATHER) {
     __syncthreads();
-    for (int c = threadIdx.x; c < k; c += 256) {
-      if (!lcnt[c]) continue;
-      atomicAdd(gn + c, lcnt[c]);
-      for (int d = 0; d < KM_DIM; ++d)
-        if (lsum[c * KM_DIM + d])
-          atomicAdd((unsigned long long *)&gs[c * KM_DIM + d],
-                    (unsigned long long)lsum[c * KM_DIM + d]);
-    }
+    for (int c = threadIdx.x; c < k; c += 256)
+      if (lcnt[c]) atomicAdd(gn + c, lcnt[c]);
+    for (int j = threadIdx.x; j < k * KM_DIM; j += 256)
+      if (lsum[j]) atomicAdd((unsigned long long *)&gs[j], (unsigned long long)lsum[j]);
   }
 }
 
@@ -341,7 +353,7 @@ gd_status km_run(gd_ctx *ctx, int n_groups, const int64_t *off, const float *soa
   std::vector<float> cent((size_t)n_groups * k * KM_DIM, 0.0f);
   std::vector<int> done(n_groups, -1), init(k);
   std::vector<int> perm;
-  int64_t waves = 0;
+  int64_t waves = 0, n_live = 0;
   for (int g = 0; g < n_groups; ++g) {
     const int n = (int)(off[g + 1] - off[g]);
     if (passes) passes[g] = 0;
@@ -353,6 +365,7 @@ gd_status km_run(gd_ctx *ctx, int n_groups, const int64_t *off, const float *soa
       continue;
     }
     done[g] = INT32_MAX;
+    n_live += 1;
     waves += (n + 63) / 64;
     km_init_indices(n, k, g, level, seed, perm, init.data());
     for (int c = 0; c < k; ++c)
@@ -364,7 +377,15 @@ gd_status km_run(gd_ctx *ctx, int n_groups, const int64_t *off, const float *soa
   // waves per CU (and not for a handful of centers)
   const int o_lane = waves >= (int64_t)32 * ctx->n_cu ? 2 : 1;
   const int c_split = waves < (int64_t)2 * ctx->n_cu && k >= 16 ? 4 : 1;
-  const int tile = 64 * o_lane * (4 / c_split);
+  // a workgroup of few centers takes four tiles of groups of thousands of objects,
+  // where that leaves one for every other CU: four times as many flushes would
+  // meet on the same sums (10 groups of 20,000 objects, 3 centers, 43 us a pass,
+  // 33 so; 300 groups of 2,000, whose sums few meet on, would go from 20 to 23)
+  const int rounds = k <= KM_ROUNDS_K && waves >= (int64_t)8 * o_lane * ctx->n_cu &&
+                             waves >= (int64_t)64 * n_live
+                         ? 4
+                         : 1;
+  const int tile = 64 * o_lane * (4 / c_split) * rounds;
   for (int g = 0; g < n_groups; ++g) {
     if (done[g] < 0) continue;
     const int n = (int)(off[g + 1] - off[g]);
@@ -422,8 +443,9 @@ gd_status km_run(gd_ctx *ctx, int n_groups, const int64_t *off, const float *soa
   A.k = k;
   A.threshold = threshold;
   A.max_pass = max_pass;
-  // LDS sums of the first pass with unsplit centers
-  const size_t lds_first = (size_t)k * KM_DIM * 8 + (size_t)k * 4 + 16;
+  A.rounds = rounds;
+  // LDS sums of the gathering passes (unsplit centers)
+  const size_t lds_gather = (size_t)k * KM_DIM * 8 + (size_t)k * 4 + 16;
   void (*assign)(KmArgs, const float *, int) = nullptr, (*first)(KmArgs, const float *, int) = nullptr;
   if (c_split == 4) {
     assign = first = gd_km_assign_kernel<1, 4, false>;
@@ -434,17 +456,20 @@ gd_status km_run(gd_ctx *ctx, int n_groups, const int64_t *off, const float *soa
     assign = gd_km_assign_kernel<1, 1, false>;
     first = gd_km_assign_kernel<1, 1, true>;
   }
-  if (first != assign)
+  if (c_split == 1) {
     HIPCHK(hipFuncSetAttribute((const void *)first, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)lds_first));
+                               (int)lds_gather));
+    if (k <= KM_GATHER_K) assign = first;
+  }
   const dim3 upd((unsigned)n_groups, (unsigned)((k * KM_DIM + 255) / 256));
   HIPCHK(hipEventRecord(ctx->ev0, st));
   for (int p = 0; p < max_pass;) {
     const int batch = std::min(8, max_pass - p);
     for (int b = 0; b < batch; ++b, ++p) {
       if (b == batch - 1) HIPCHK(hipMemsetAsync(A.active, 0, 4, st));
-      hipLaunchKernelGGL(p == 0 ? first : assign, dim3(n_tiles), dim3(256),
-                         p == 0 && first != assign ? lds_first : 0, st, A, (const float *)A.cent, p);
+      const bool gather = c_split == 1 && (p == 0 || k <= KM_GATHER_K);
+      hipLaunchKernelGGL(p == 0 ? first : assign, dim3(n_tiles), dim3(256), gather ? lds_gather : 0,
+                         st, A, (const float *)A.cent, p);
       HIPCHK(hipGetLastError());
       hipLaunchKernelGGL(gd_km_update_kernel, upd, dim3(256), 0, st, A, p);
       HIPCHK(hipGetLastError());
