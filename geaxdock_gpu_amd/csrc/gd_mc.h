@@ -699,11 +699,13 @@ __device__ __forceinline__ void flat_pairs(const int *off, const Lds &S, int h,
 
 // Sum over MCS templates [m_begin, m_end) of tcc_m * sqrt(mean squared
 // distance of the template's atoms), src/kernel_cuda_l2_calcenergy.cu:274-313. Templates go
-// four at a time: their loads are issued together, one round ahead of their
+// Q at a time: their loads are issued together, one round ahead of their
 // use (a round waited out three dependent reads from L2 before: 196 templates
 // of a coarse receptor took 37,000 cycles of a step's 124,000 per wave), and
 // their lane sums share each butterfly step. Per template the additions are
-// the same as one template at a time.
+// the same as one template at a time. Lanes of three and four atoms take two
+// templates a round: four ahead hold 48 registers and more, which the step loop
+// then spilled (42 around the plain chunk loop of three atoms, 5 with two).
 template <int APL, int J>
 __device__ __forceinline__ float mcs_sum(const DevComplex &C, int lpr, const float (&x)[APL],
                                          const float (&y)[APL], const float (&z)[APL],
@@ -714,11 +716,12 @@ __device__ __forceinline__ float mcs_sum(const DevComplex &C, int lpr, const flo
   const gfloat4_p mcs = (gfloat4_p)C.mcs;
   const gfloat_p cnt = glob(C.mcs_cnt), tcc = glob(C.mcs_tcc);
   const int lna = C.lna;
-  f32x4_t M[4][APL];
-  float n[4], t[4];
+  constexpr int Q = APL >= 3 ? 2 : 4;
+  f32x4_t M[Q][APL];
+  float n[Q], t[Q];
   auto read = [&](int m0) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < Q; ++q) {
       const int m = min(m0 + q, m_end - 1);
 #pragma unroll
       for (int k = 0; k < APL; ++k) M[q][k] = mcs[(size_t)m * lna + li[k]];
@@ -727,10 +730,10 @@ __device__ __forceinline__ float mcs_sum(const DevComplex &C, int lpr, const flo
     }
   };
   read(m_begin);
-  for (int m0 = m_begin; m0 < m_end; m0 += 4) {
-    float s[4][J], nc[4], tc[4];
+  for (int m0 = m_begin; m0 < m_end; m0 += Q) {
+    float s[Q][J], nc[Q], tc[Q];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < Q; ++q) {
 #pragma unroll
       for (int j = 0; j < J; ++j) s[q][j] = 0.0f;
       nc[q] = n[q];
@@ -741,11 +744,14 @@ __device__ __forceinline__ float mcs_sum(const DevComplex &C, int lpr, const flo
         if (M[q][k][3] != 0.0f) s[q][k % J] += pair_d2(x[k], y[k], z[k], M[q][k][0], M[q][k][1], M[q][k][2]);
       }
     }
-    if (m0 + 4 < m_end) read(m0 + 4);
+    if (m0 + Q < m_end) read(m0 + Q);
 #pragma unroll
-    for (int j = 0; j < J; ++j) seg_sums(lpr, s[0][j], s[1][j], s[2][j], s[3][j]);
+    for (int j = 0; j < J; ++j) {
+      if constexpr (Q == 4) seg_sums(lpr, s[0][j], s[1][j], s[2][j], s[3][j]);
+      else seg_sums(lpr, s[0][j], s[1][j]);
+    }
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
+    for (int q = 0; q < Q; ++q)
       if (m0 + q < m_end && nc[q] > 0.0f) elhm += tc[q] * sqrtf(block_total(s[q]) / nc[q]);
   }
   return elhm;
