@@ -41,7 +41,7 @@ struct LaunchClass {
   KParams lay{};     // LDS offsets and exchange-buffer fields
   size_t lds_flat = 0;  // the same with the receptor as units of the flat
   KParams lay_flat{};   // pair loop (0: none)
-  bool near = false;  // plain chunk loop without distance tests (DA_NEAR)
+  bool near = false;  // chunk loop without distance tests (DA_NEAR)
 };
 
 struct HostComplex {
@@ -298,14 +298,16 @@ float far_share(const gd_complex_desc &d, float far2) {
 // where these cost more than they skip. At a wave per SIMD (blocks of at most
 // 256 lanes) nothing hides the tests' branches: 64 ladders of 4 replicas of 30
 // atoms, split 1, 2,000 points, 14.2 ms with tests and 12.1 without, 3,500 points
-// 22.8 and 20.4; one pose on 1,200 points 116 us and 106. At two waves per SIMD
+// 22.8 and 20.4; one pose on 1,200 points 116 us and 106; in tiles of 6,000 points
+// (share 0.84) 14 atoms 22.9 and 26.2. At two waves per SIMD
 // the tests pay from a share of far points on that falls with the atoms per
 // lane (batches and ladders, tests first): 1 atom, 2,000 points (share 0.6) 5.8 ms
 // and 5.5, 3,500 (0.77) 8.4 and 8.7; 2 atoms, 1,000 points (0.13) 65.8 and 63.1,
-// 2,000 (0.44) 10.6 and 10.4, 2,500 (0.52) 139.9 and 142.9; 3 atoms, 1,000 (0.14)
-// 43.2 and 43.1, 2,000 (0.46) 78.0 and 81.4.
+// 2,000 (0.44) 10.6 and 10.4, 2,500 (0.52) 139.9 and 142.9; 3 atoms, 800 points
+// (0.07) 6.98 and 6.81, 1,000 (0.14) 76.6 and 77.3, 2,000 (0.46) 78.0 and 81.4.
 constexpr int NEAR_BLOCK = 256;
-constexpr float NEAR_SHARE[4] = {0.65f, 0.45f, 0.3f, 0.3f};
+constexpr float NEAR_SHARE_1WAVE = 0.8f;
+constexpr float NEAR_SHARE[4] = {0.65f, 0.45f, 0.1f, 0.1f};
 
 // Lanes per replica and atoms per lane: the fewest lane slots lpr*apl that
 // hold lna atoms with apl <= 4, preferring 2..3 atoms per lane on ties (more
@@ -1214,7 +1216,7 @@ void pack_finish(const gd_ctx *ctx, PackSet &ps, int lpr = 0, int apl_of_lpr = 0
       all += cost[oe];
     }
     lc.end = (int)e;
-    lc.near = lc.block <= NEAR_BLOCK || far < NEAR_SHARE[lc.apl - 1] * all;
+    lc.near = far < (lc.block <= NEAR_BLOCK ? NEAR_SHARE_1WAVE : NEAR_SHARE[lc.apl - 1]) * all;
     lc.half_max = half_max;
     layout(lc.lay, &lc.lds, (pnp_max + 3) & ~3, pnk_max, nch_max, slots_max, lc.block, split,
            lc.tile);
@@ -1562,7 +1564,7 @@ hipError_t plan_classes(gd_ctx *ctx, const std::vector<LaunchClass> &classes, co
       P.n_queue = n_pk;
     }
     const int rec = lc.tile > 0 ? REC_TILED : flat ? REC_FLAT : REC_CHUNKS;
-    cl.f = mc_kernel_fn(lc.apl, da == 0 && rec == REC_CHUNKS && lc.near ? DA_NEAR : da, rec);
+    cl.f = mc_kernel_fn(lc.apl, lc.near && da <= 4 ? da | DA_NEAR : da, rec);
     out.push_back(cl);
   }
   // the dynamic LDS limit of every instance used is the device's: classes

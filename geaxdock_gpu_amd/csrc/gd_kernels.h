@@ -110,7 +110,8 @@ struct Pack {
 // MODE_TREE: the next n_steps MC steps by a tree of energies (gd_mc.h)
 enum { MODE_MC = 0, MODE_INIT = 1, MODE_EVAL = 2, MODE_SUREVAL = 3, MODE_TREE = 4 };
 // kernel instances besides the modes of delayed acceptance (see mc_kernel_handle)
-constexpr int DA_TREE = 5, DA_POSES = 6, DA_POSES2 = 7, DA_NEAR = 8;
+constexpr int DA_TREE = 5, DA_POSES = 6, DA_POSES2 = 7;
+constexpr int DA_NEAR = 16;  // added to a mode: pair loop without distance tests
 constexpr int TREE_DEPTH = 6;  // a wave's lanes hold the 2^depth - 1 energies
 
 struct KParams {
@@ -167,8 +168,9 @@ struct KParams {
 // mode `da` (0 plain, 1 delayed acceptance with the network per atom, 2 with
 // its tabulated outputs) and receptor layout; defined in gd_mc_inst.hip, one
 // object per APL. DA_POSES (2 or 3 atoms per lane) and DA_POSES2 (3) have
-// instances for REC_TILED and REC_FLAT, DA_NEAR for REC_CHUNKS, REC_FLAT none for
-// modes 1 and 3.
+// instances for REC_TILED and REC_FLAT, REC_FLAT none for modes 1 and 3. DA_NEAR
+// counts for modes 0, 2 and 4 of REC_CHUNKS and 0 of REC_TILED; others run as
+// they do without it (same bits).
 enum { REC_CHUNKS = 0, REC_TILED = 1, REC_FLAT = 2 };
 template <int APL>
 const void *mc_kernel_handle(int da, int rec);

@@ -1480,18 +1480,19 @@ __device__ __forceinline__ void tree_decide(const KParams &P, const DevComplex &
 }
 
 // DA: 0 plain Metropolis (DA_TREE: by a tree of energies, in instances of its
-// own, so that the step loop's registers stay as they are; DA_NEAR: without
-// distance tests; DA_POSES and
+// own, so that the step loop's registers stay as they are; DA_POSES and
 // DA_POSES2: poses with fewer lanes than the complex's shape has, slot k in
 // block k or k % 2 of block_total); delayed acceptance with the surrogate from
 // the network evaluated per atom (1) or from its tabulated outputs (2); 3 and 4
-// are 1 and 2 with the split groups' shared surrogate sums compiled in.
-template <int APL, int DA, bool TILE, bool FLAT>
+// are 1 and 2 with the split groups' shared surrogate sums compiled in. MODE is
+// DA, with DA_NEAR added where the pair loop goes without distance tests.
+template <int APL, int MODE, bool TILE, bool FLAT>
 __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const DevComplex &C, const Lds &S,
                          int lpr, int step0, int idx, int node, int &par) {
+  constexpr int DA = MODE & ~DA_NEAR;
+  constexpr bool SKIP = (MODE & DA_NEAR) == 0;
   constexpr bool TREE = DA == DA_TREE, POSES = DA == DA_POSES || DA == DA_POSES2;
-  constexpr bool SKIP = DA != DA_NEAR;
-  constexpr int DAM = TREE || POSES || !SKIP ? 0 : DA > 2 ? DA - 2 : DA;
+  constexpr int DAM = TREE || POSES ? 0 : DA > 2 ? DA - 2 : DA;
   constexpr int J = !POSES ? 1 : DA == DA_POSES2 ? 2 : APL;
   // the wide shape has one atom per lane (DA_POSES) or two
   constexpr int NP = group_points(DA == DA_POSES ? 1 : DA == DA_POSES2 ? 2 : APL);
@@ -1767,7 +1768,7 @@ __device__ __forceinline__ void run_pack(const KParams &P, const Pack &pk, const
       const bool eval = wave_active && __ballot(moved) != 0;
       if (eval) place(yv);
       gd_energy E;
-      pose_energy<APL, TILE, FLAT>(C, S, lpr, sp, eval, x, y, z, ox, oy, oz, lt, q, li, val, yv, E);
+      pose_energy<APL, TILE, FLAT, J, NP, SKIP>(C, S, lpr, sp, eval, x, y, z, ox, oy, oz, lt, q, li, val, yv, E);
       if (eval) {
         const float d1 = E.e[GD_MAXWEI - 1] - eo.e[GD_MAXWEI - 1];
         const float d2 = s_y - s_old;

@@ -10,11 +10,20 @@ namespace gd {
 // evaluation, 1 delayed acceptance with the network per atom, 2 with its
 // tabulated outputs, 3 and 4 the same with the receptor split's groups
 // sharing the surrogate's KDE and MCS sums, DA_TREE plain MC by a tree of
-// energies, DA_POSES poses with fewer lanes than the complex's shape, DA_NEAR 0
-// without the distance tests; rec: the receptor resident in LDS by chunks,
-// streamed through LDS tiles, or resident with unit lists.
+// energies, DA_POSES poses with fewer lanes than the complex's shape; DA_NEAR
+// added: without the distance tests; rec: the receptor resident in LDS by
+// chunks, streamed through LDS tiles, or resident with unit lists.
 template <>
 const void *mc_kernel_handle<GD_MC_APL>(int da, int rec) {
+  if (da & DA_NEAR) {
+    switch (rec == REC_CHUNKS ? da : rec == REC_TILED && da == DA_NEAR ? -1 : -2) {
+      case DA_NEAR: return (const void *)gd_mc_kernel<GD_MC_APL, DA_NEAR, false, false>;
+      case DA_NEAR + 2: return (const void *)gd_mc_kernel<GD_MC_APL, DA_NEAR + 2, false, false>;
+      case DA_NEAR + 4: return (const void *)gd_mc_kernel<GD_MC_APL, DA_NEAR + 4, false, false>;
+      case -1: return (const void *)gd_mc_kernel<GD_MC_APL, DA_NEAR, true, false>;
+      default: da &= ~DA_NEAR;
+    }
+  }
   if (rec == REC_TILED) {
     switch (da) {
       case 1: return (const void *)gd_mc_kernel<GD_MC_APL, 1, true, false>;
@@ -52,7 +61,6 @@ const void *mc_kernel_handle<GD_MC_APL>(int da, int rec) {
     case 3: return (const void *)gd_mc_kernel<GD_MC_APL, 3, false, false>;
     case 4: return (const void *)gd_mc_kernel<GD_MC_APL, 4, false, false>;
     case DA_TREE: return (const void *)gd_mc_kernel<GD_MC_APL, DA_TREE, false, false>;
-    case DA_NEAR: return (const void *)gd_mc_kernel<GD_MC_APL, DA_NEAR, false, false>;
     default: return (const void *)gd_mc_kernel<GD_MC_APL, 0, false, false>;
   }
 }

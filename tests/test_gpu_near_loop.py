@@ -8,7 +8,8 @@ a workgroup, agree bit for bit at the same split.
 import numpy as np
 import pytest
 
-from geaxdock_gpu_amd import abi, synth
+from geaxdock_gpu_amd import surrogate as sg
+from geaxdock_gpu_amd import synth
 
 pytestmark = pytest.mark.gpu
 
@@ -23,18 +24,26 @@ def gd():
 SHAPES = [(32, 1, 30, 4), (16, 2, 29, 8), (32, 2, 61, 4), (16, 3, 44, 8), (16, 4, 62, 8)]
 
 
-@pytest.mark.parametrize("pnp", [1, 700, 3501])
+@pytest.mark.parametrize("pnp,tile,pos,da", [(1, 0, 3, False), (700, 0, 3, False),
+                                             (3501, 0, 3, False), (3501, 256, 3, False),
+                                             (3501, 0, 3, True), (3501, 0, 40, True)])
 @pytest.mark.parametrize("lpr,apl,lna,n_tmp", SHAPES)
-def test_one_and_two_ladders_a_workgroup(gd, lpr, apl, lna, n_tmp, pnp):
-    cx = synth.make_complex(pnp, lna=lna, pnp=pnp, pnk=40, pos=3, mcs_atoms=5, n_lig=4, n_prt=2,
+def test_one_and_two_ladders_a_workgroup(gd, lpr, apl, lna, n_tmp, pnp, tile, pos, da):
+    cx = synth.make_complex(pnp, lna=lna, pnp=pnp, pnk=40, pos=pos, mcs_atoms=5, n_lig=4, n_prt=2,
                             n_tmp=n_tmp, void_radius=4.0)
     out = []
     for ladders in (1, 2):
-        with gd.Engine(seed=4, receptor_split=2, ladders_per_pack=ladders,
+        with gd.Engine(seed=4, receptor_split=2, ladders_per_pack=ladders, receptor_tile=tile,
                        lanes_per_replica=lpr, atoms_per_lane=apl) as e:
             e.add_complex(cx)
             recs = []
-            e.run(40, 20, sink=lambda c, r: recs.append(r))
+            if da:  # 40 templates: the split's groups share the surrogate's sums
+                e.sur_build_grids(1.0, 8.0)
+                e.sur_set_params(sg.pack_params(sg.init_params(2)))
+                e.sur_tabulate()
+                e.run_da(40, 20, 4, 2.0, sink=lambda c, r: recs.append(r))
+            else:
+                e.run(40, 20, sink=lambda c, r: recs.append(r))
             st = e.state(0)
             out.append([np.concatenate(recs).tobytes()] + [st[k].tobytes() for k in sorted(st)])
     assert out[0] == out[1]
