@@ -294,7 +294,7 @@ float far_share(const gd_complex_desc &d, float far2) {
   return (float)n / (float)d.pnp;
 }
 
-// Launches of the chunk loop go without its distance tests (DA_NEAR, same bits)
+// Launches by chunks or tiles go without the loop's distance tests (DA_NEAR, same bits)
 // where these cost more than they skip. At a wave per SIMD (blocks of at most
 // 256 lanes) nothing hides the tests' branches: 64 ladders of 4 replicas of 30
 // atoms, split 1, 2,000 points, 14.2 ms with tests and 12.1 without, 3,500 points
